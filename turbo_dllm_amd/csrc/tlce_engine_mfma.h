@@ -1,10 +1,10 @@
 // 256x256 bf16/f16 MFMA tile engines for gfx950 (CDNA4), wave64.
 //
-// Both compute C[i][j] = sum_k A[i][k] * B[j][k] for one 256x256 tile, A and B both
-// K-contiguous (row-major [rows, K]).  512 threads = 8 waves in a 2 (A rows) x
-// 4 (B rows) grid; each wave owns a 128x64 sub-tile as 4x2
-// v_mfma_f32_32x32x16 blocks (128 fp32 accumulator registers per lane), two
-// waves per SIMD.
+// Both compute C[i][j] = sum_k A[i][k] * B[j][k] for one 256x256 tile.  The
+// register-staged engine (any K that is a multiple of 8, operands K-contiguous,
+// row-major [rows, K]): 512 threads = 8 waves in a 2 (A rows) x 4 (B rows) grid; each
+// wave owns a 128x64 sub-tile as 4x2 v_mfma_f32_32x32x16 blocks (128 fp32
+// accumulator registers per lane), two waves per SIMD.
 //
 // LDS: two stages of (A 256x64 + B 256x64) 2-byte elements = 2 x 64 KiB of the
 // CU's 160 KiB.  A tile row is 128 bytes = eight 16-byte chunks; chunk c of
@@ -41,20 +41,18 @@ template <> struct MfmaOp<_Float16> {
   }
 };
 
-// Thread <-> tile-element mapping shared by the MFMA engines: 2 waves along
-// the A rows, kWavesN_ along the B rows, each wave 4 x kTN_ blocks of 32x32
-// (8 waves of 128x64, or 4 waves of 128x128).
-template <typename T_, int kWavesN_ = 4, int kTN_ = 2>
+// Its thread <-> tile-element mapping.
+template <typename T_>
 struct MfmaTileLayout {
   using T = T_;
   using Op = MfmaOp<T>;
   using V8 = typename Op::V8;
 
   static constexpr int kTile = 256;     // BM == BN
-  static constexpr int kWavesN = kWavesN_;   // waves along B rows
+  static constexpr int kWavesN = 4;     // waves along B rows
   static constexpr int kThreads = 2 * kWavesN * 64;
   static constexpr int kTM = 4;         // 32-row blocks per wave along A rows
-  static constexpr int kTN = kTN_;      // 32-col blocks per wave along B rows
+  static constexpr int kTN = 2;         // 32-col blocks per wave along B rows
   static constexpr int kCols = kTN;          // tile columns owned per thread
   static constexpr int kRows = kTM * 16;     // tile rows held per owned column
   static constexpr int kShare = 4;           // threads that hold the same column
@@ -79,11 +77,6 @@ struct MfmaTileLayout {
 
   __device__ __forceinline__ int col(int j) const {
     return wn * (kTN * 32) + j * 32 + (lane & 31);
-  }
-  // The tile columns that have owned index j in some thread: number t of them.
-  static constexpr int kTokensPerIndex = kWavesN * 32;
-  static __device__ __forceinline__ int token_of_index(int j, int t) {
-    return (t >> 5) * (kTN * 32) + j * 32 + (t & 31);
   }
   __device__ __forceinline__ int row(int i) const {
     return wm * 128 + (i >> 4) * 32 + ((i >> 2) & 3) * 8 + (lane >> 5) * 4 + (i & 3);
@@ -110,12 +103,6 @@ struct MfmaTileLayout {
     return v;
   }
   __device__ __forceinline__ bool col_leader() const { return (lane & 31) == 0; }
-  // Sum over the lanes of this wave that hold the same tile column (lanes l and
-  // l ^ 32 hold different rows of it); other waves keep their own sums.
-  __device__ __forceinline__ float reduce_over_rows_in_wave(float v) const {
-    return v + __shfl_xor(v, 32, 64);
-  }
-  __device__ __forceinline__ bool row_leader() const { return lane < 32; }
 };
 
 // Register-staged engine: global -> VGPR -> LDS, two 64-wide K stages.  Takes
@@ -241,11 +228,86 @@ struct MfmaEngine : MfmaTileLayout<T_> {
   }
 };
 
+// Thread <-> tile-element mapping of the direct-to-LDS engine: 4 waves (2 along the A
+// rows x 2 along the B rows), each 128x128 as 8x8 v_mfma_f32_16x16x32 blocks.
+//
+// Why 16x16x32 and not 32x32x16, whose operand registers are read half as often: with
+// real operand values the matrix pipes run at the part's power limit, and per FLOP the
+// 16x16x32 instruction moves its accumulator half as often (K = 32 per accumulation).
+// Measured on registers alone with normally distributed bf16 operands: 2050 against
+// 1780 TFLOP/s (2440 / 2480 with all-zero operands).  That holds only while the A
+// operand stays the same over a run of MFMAs (a change of A stalls the next issue by
+// about 5 cycles: 1820 TFLOP/s on zeros when A changes every time), hence 8 columns of
+// B per A fragment.
+//
+// Accumulator layout of one 16x16 block (lane l, register q of 4):
+//   row = 4*(l/16) + q,   col = l%16.
+// A/B fragment of one block for a 32-wide K slice: lane l supplies row l%16,
+// K = 8*(l/16) .. +8  (one 16-byte chunk).
+typedef float acc4_t __attribute__((ext_vector_type(4)));
+
+template <typename T_>
+struct DirectTileLayout {
+  using T = T_;
+  static constexpr int kTile = 256;
+  static constexpr int kThreads = 256;
+  static constexpr int kTM = 8;                  // 16-row blocks per wave along A rows
+  static constexpr int kTN = 8;                  // 16-row blocks per wave along B rows
+  static constexpr int kCols = kTN;              // tile columns owned per thread
+  static constexpr int kRows = kTM * 4;          // tile rows held per owned column
+  static constexpr int kShare = 8;               // threads that hold the same column
+  static constexpr int kStageCols = 2;           // owned columns per quarter of the tile
+  static constexpr bool kPrecise = false;
+
+  struct Acc { acc4_t c[kTM][kTN]; };
+
+  int lane, wave, wm, wn;
+
+  __device__ __forceinline__ DirectTileLayout() {
+    lane = threadIdx.x & 63;
+    wave = threadIdx.x >> 6;
+    wm = wave >> 1;
+    wn = wave & 1;
+  }
+  __device__ __forceinline__ void forget_lane_invariants() { asm volatile("" : "+v"(lane)); }
+  __device__ __forceinline__ int col(int j) const { return wn * 128 + j * 16 + (lane & 15); }
+  // The tile columns that have owned index j in some thread: number t of them.
+  static constexpr int kTokensPerIndex = 32;
+  static __device__ __forceinline__ int token_of_index(int j, int t) {
+    return (t >> 4) * 128 + j * 16 + (t & 15);
+  }
+  // Position of this lane's column among those with the same owned index.
+  __device__ __forceinline__ int position_in_index() const { return wn * 16 + (lane & 15); }
+  __device__ __forceinline__ int row(int i) const {
+    return wm * 128 + (i >> 2) * 16 + (lane >> 4) * 4 + (i & 3);
+  }
+  __device__ __forceinline__ int share_slot() const { return wm * 4 + (lane >> 4); }
+  static __device__ __forceinline__ float get(const Acc& a, int j, int i) {
+    return a.c[i >> 2][j][i & 3];
+  }
+  static __device__ __forceinline__ void set(Acc& a, int j, int i, float v) {
+    a.c[i >> 2][j][i & 3] = v;
+  }
+  static __device__ __forceinline__ void zero(Acc& a) {
+#pragma unroll
+    for (int tm = 0; tm < kTM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < kTN; ++tn) a.c[tm][tn] = acc4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  // Sum over the lanes that hold the same tile row (a group of 16 lanes).
+  __device__ __forceinline__ float reduce_over_cols(float v) const {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+  }
+  __device__ __forceinline__ bool col_leader() const { return (lane & 15) == 0; }
+};
+
 // Four-wave direct-to-LDS engine (K multiple of 64): 256 threads, each wave a
-// 128x128 sub-tile (4x4 MFMA blocks, 256 accumulator registers, one wave per
-// SIMD).  Operands go global -> LDS with global_load_lds_dwordx4 (no VGPR
-// staging, no ds_write) into two 64-wide K stages of 64 KiB; every wave load
-// instruction moves 1 KiB made of full 128-byte (or 512-byte) row segments.
+// 128x128 sub-tile (256 accumulator registers, one wave per SIMD).  Operands go
+// global -> LDS with global_load_lds_dwordx4 (no VGPR staging, no ds_write) into two
+// 64-wide K stages of 64 KiB; every wave load instruction moves 1 KiB made of full
+// 128-byte (or 512-byte) row segments.
 //
 // Either operand can be stored in one of two ways:
 //   K-contiguous  X[row][k]  (the projection's hidden and weight rows, the
@@ -257,11 +319,12 @@ struct MfmaEngine : MfmaTileLayout<T_> {
 //
 // LDS layouts of one operand stage (32 KiB):
 //   K-contiguous: 256 rows x 128 B; 16-byte chunk c of row r in slot
-//                 c ^ ((r >> 1) & 7).
+//                 c ^ ((r >> 1) & 7): any 16 consecutive rows of one chunk cover
+//                 all 64 banks.
 //   K-major:      64 K rows x 512 B; 16-byte chunk c of K row k in slot
-//                 c ^ (4 * (k & 3)): the four K rows x 64 bytes that half a
-//                 wave reads at once then fall into four different quarters
-//                 of the banks, and 64-byte runs stay contiguous.
+//                 c ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1)): the eight K rows (0..3 and
+//                 8..11) x 32 bytes that half a wave reads at once fall into eight
+//                 different eighths of the banks.
 // ds_read_b64_tr_b16 works on groups of 16 lanes: lane i of a group addresses
 // 4 consecutive elements, and lane l receives element l%4 of the chunks of
 // lanes l/4, 4 + l/4, 8 + l/4, 12 + l/4.  With lane i addressing K row i/4,
@@ -273,15 +336,34 @@ struct MfmaEngine : MfmaTileLayout<T_> {
 // once per tile, so a load costs three scalar instructions and no VALU work.
 //
 // Software pipeline of one wave (the only wave on its SIMD; it issues in
-// order and an MFMA occupies its pipe for 32 cycles): one K step = 64 MFMAs
-// = 16 groups of 4 (slice sl = g/4, A block q = g%4, B block t).  After every
-// MFMA at most one fragment read and one load instruction follow.
-//   reads : the fragments of the next slice, spread over the groups of the
-//           current one; slice 0 of the next tile is read in the two groups
-//           after the barrier, which sits in the middle of slice 3;
-//   loads : of the next tile's 16, six go out right after the barrier of the
-//           previous step, ten in the first groups of the step (two per group
-//           in groups 0..4, or one per group in groups 0..9).
+// order and an MFMA occupies its pipe for 16 cycles): one K step = 2 slices of 32 =
+// 2 x 8 groups of 8 MFMAs (A block q, B blocks 0..7).  After every MFMA at most one
+// fragment read or load instruction follows.
+//   reads : B fragments are held twice (all eight are needed by every group), those of
+//           the next slice are read in the first groups of the current one; an A
+//           fragment is needed by one group only, so its registers are refilled for
+//           the next slice right after that group.  The barrier that makes the next
+//           tile visible sits before group 2 of slice 1, when the last fragment of the
+//           current stage (A block 7, read in group 0) has arrived.
+//   loads : of the next tile's 16, kLoadsAfterBarrier go out in the groups right after
+//           the barrier of the previous step, the others in the first groups of the
+//           step, two per group: bunched four to a group the kernels lose 2 to 4 %, all
+//           16 right after the barrier 4 %, 6 there and 10 in the step 8 %.
+//   touches: the workgroups of an XCD share their operand strips through its L2, but all
+//           of them wait for whichever fetch misses it, and one tile of lead (about
+//           1 us) does not cover a fetch from beyond L2.  Once per step each wave reads
+//           one dword from 64 of the K tile's 128-byte lines, kTouchAhead tiles ahead,
+//           into a scrap of LDS nobody reads: neighbouring workgroups (even and odd tile
+//           index along the other operand) take the two halves of a strip, so between
+//           them the whole tile is in L2 before its loads are issued.
+//
+// Measured on one block of 8192 rows, H = 4096, V = 151936 (ms per contraction,
+// 32x32x16 engine -> 16x16x32 with the accumulators in AGPRs -> with touches):
+// exponentiated logits 8.1 -> 7.65 -> 7.3, grad_hidden 7.75 -> 7.25 -> 6.95, grad_weight
+// 7.85 -> 7.3 -> 7.25, forward statistics 7.8 -> 7.5 -> 7.2 (1.38 to 1.47 PFLOP/s;
+// grad_hidden's pipes are busy 0.835 of the cycles at 1.65 GHz, i.e. at the power
+// limit).  With no loads in the K loop grad_hidden takes 5.4 ms, with every load an L2
+// hit 6.2: what is left is the energy of moving operands.
 template <typename T>
 struct Operand {
   const T* ptr;   // matrix base
@@ -290,12 +372,35 @@ struct Operand {
   int rows;       // valid rows / columns of the matrix; accesses beyond are clamped
 };
 
+template <typename T> struct DirectMfma;
+// The MFMAs are written as asm so that the accumulators stay in the AGPR file: left to
+// the builtin, the allocator moves some of the 64 blocks through VGPRs inside the loop
+// (44 to 116 copies, each behind a full MFMA latency, per K step).  The waits for the
+// LDS reads that fill a and b are the compiler's, which tracks asm operands; what it
+// does not know is the result latency, so mainloop_ex ends on mfma_drain().
+template <> struct DirectMfma<__bf16> {
+  static __device__ __forceinline__ void mma(bf16x8_t a, bf16x8_t b, acc4_t& c) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  }
+  static __device__ __forceinline__ void mma_set(bf16x8_t a, bf16x8_t b, acc4_t& c) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+  }
+};
+template <> struct DirectMfma<_Float16> {
+  static __device__ __forceinline__ void mma(f16x8_t a, f16x8_t b, acc4_t& c) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  }
+  static __device__ __forceinline__ void mma_set(f16x8_t a, f16x8_t b, acc4_t& c) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
+  }
+};
+
 template <typename T_>
-struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
-  using Base = MfmaTileLayout<T_, 2, 4>;
+struct MfmaDirect4Engine : DirectTileLayout<T_> {
+  using Base = DirectTileLayout<T_>;
   using T = T_;
-  using Op = typename Base::Op;
-  using V8 = typename Base::V8;
+  using Op = DirectMfma<T_>;
+  using V8 = typename MfmaOp<T_>::V8;
   using Acc = typename Base::Acc;
   using Base::kTile;
   using Base::kTM;
@@ -307,8 +412,11 @@ struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
   static constexpr int kBK = 64;
   static constexpr int kOperandBytes = kTile * kBK * 2;      // 32768
   static constexpr int kStageBytes = 2 * kOperandBytes;      // 65536
-  static constexpr int kSmemBytes = 2 * kStageBytes;         // 131072
+  static constexpr int kTouchBytes = 4 * 256;                // where the L2 touches land
+  static constexpr int kSmemBytes = 2 * kStageBytes + kTouchBytes;
   static constexpr int kLoads = 8;                           // per wave, operand and K tile
+  static constexpr int kTouchAhead = 2;                      // K tiles
+    static constexpr int kLoadsAfterBarrier = 12;              // of the 16 of both operands
   static constexpr bool kHasKMajor = true;
 
   typedef short v4s_t __attribute__((ext_vector_type(4)));
@@ -322,6 +430,31 @@ struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
                  : "memory", "m0");
   }
 
+  static __device__ __forceinline__ void touch(unsigned lds_addr, unsigned byte_offset,
+                                               const char* base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(lds_addr), "v"(byte_offset), "s"(base)
+                 : "memory", "m0");
+  }
+
+  static __device__ __forceinline__ int64_t readfirstlane64(int64_t x) {
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)x);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(x >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+  }
+
+  // Per-lane byte offset of cache line `line` (0..255, 128 bytes each) of an operand's K tile.
+  template <bool kKMajor>
+  static __device__ __forceinline__ unsigned line_offset(const Operand<T>& x, int line) {
+    if (!kKMajor) {
+      return (unsigned)((int64_t)(min(x.row0 + line, x.rows - 1) - x.row0) * x.ld * 2);
+    } else {
+      const int last_chunk = x.rows / 8 - 1 - x.row0 / 8;
+      return (unsigned)((int64_t)(line >> 2) * x.ld * 2 + min((line & 3) * 8, last_chunk) * 16);
+    }
+  }
+
   // Loader state of one operand: where this wave's eight 1 KiB pieces of a K
   // tile come from and where they land.
   struct Loader {
@@ -332,10 +465,9 @@ struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
   };
 
   template <bool kKMajor>
-  __device__ __forceinline__ Loader make_loader(const Operand<T>& x, int k_begin, unsigned lds_op,
-                                                bool second_operand) const {
+  __device__ __forceinline__ Loader make_loader(const Operand<T>& x, int k_begin,
+                                                unsigned lds_op) const {
     Loader ld;
-    (void)second_operand;
     if (!kKMajor) {
       // this wave fills tile rows [64w, 64w+64), eight rows per instruction
 #pragma unroll
@@ -354,7 +486,7 @@ struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
 #pragma unroll
       for (int j = 0; j < kLoads; ++j) {
         const int kr = wave * 16 + j * 2 + (lane >> 5);
-        const int swz = 4 * (kr & 3);
+        const int swz = (4 * (kr & 3)) ^ (2 * ((kr >> 3) & 1));
         const int chunk = min((lane & 31) ^ swz, last_chunk);
         ld.off[j] = (unsigned)((int64_t)kr * x.ld * 2 + chunk * 16);
       }
@@ -365,44 +497,33 @@ struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
     return ld;
   }
 
-  // Fragment addressing of one operand for this lane.
-  struct Reader {
-    int base[4];   // LDS byte offset of block 0..3 within the operand stage
-  };
-
+  // Fragment addressing of one operand for this lane: LDS byte offset within the
+  // operand stage of block 0, K slice 0.
   template <bool kKMajor>
-  __device__ __forceinline__ Reader make_reader(int wave_block) const {
-    Reader rd;
+  __device__ __forceinline__ int reader_base(int wave_block) const {
     if (!kKMajor) {
-      const int swz = (lane >> 1) & 7;
-      (void)swz;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) rd.base[b] = (wave_block * 128 + b * 32 + (lane & 31)) * 128;
+      return (wave_block * 128 + (lane & 15)) * 128 +
+             (((lane >> 4) ^ ((lane >> 1) & 7)) * 16);
     } else {
-      const int g = lane >> 4;          // 16-lane group
+      const int g = lane >> 4;           // 16-lane group
       const int i = lane & 15;
-      const int hi = g >> 1;
-      const int swz = 4 * (i >> 2);      // = 4 * (K row & 3)
-      const int kr = 8 * hi + (i >> 2);  // K row within a 16-wide slice, first half
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int col = wave_block * 128 + b * 32 + 16 * (g & 1) + 4 * (i & 3);
-        const int slot = (col >> 3) ^ swz;
-        rd.base[b] = kr * 512 + slot * 16 + (col & 7) * 2;
-      }
+      const int kr = 8 * g + (i >> 2);   // K row within the 32-wide slice, first half
+      const int swz = (4 * (i >> 2)) ^ (2 * (g & 1));
+      const int chunk = wave_block * 16 + ((i & 3) >> 1);
+      return kr * 512 + (chunk ^ swz) * 16 + (i & 1) * 8;
     }
-    return rd;
   }
 
   template <bool kKMajor>
-  __device__ __forceinline__ V8 read_frag(const char* op_stage, const Reader& rd, int ks,
-                                          int b) const {
+  __device__ __forceinline__ V8 read_frag(const char* op_stage, int base, int ks, int b) const {
     if (!kKMajor) {
-      const int slot = ((2 * ks + (lane >> 5)) ^ ((lane >> 1) & 7)) * 16;
-      return __builtin_bit_cast(V8, *reinterpret_cast<const uint4*>(op_stage + rd.base[b] + slot));
+      // slice 1 is chunks 4..7: the slot's bit 2 flips; block b starts 16 rows further
+      return __builtin_bit_cast(
+          V8, *reinterpret_cast<const uint4*>(op_stage + ((base ^ (ks * 64)) + b * 16 * 128)));
     } else {
       typedef __attribute__((address_space(3))) v4s_t* lds_v4s_ptr;
-      const char* p0 = op_stage + rd.base[b] + ks * 16 * 512;
+      // block b is chunks 2b, 2b + 1 of the wave's 16: address bits 5..7
+      const char* p0 = op_stage + (base ^ (b * 32)) + ks * 32 * 512;
       const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
           (lds_v4s_ptr)(uintptr_t)(unsigned)(uintptr_t)p0);
       const v4s_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -414,7 +535,15 @@ struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
     }
   }
 
-  struct Frags { V8 a[kTM]; V8 b[kTN]; };
+  // Waits until the last MFMAs' results can be read (19 cycles for 16x16 blocks); takes
+  // the accumulators written last so that no read of them is moved above it.
+  static __device__ __forceinline__ void mfma_drain(Acc& acc) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 7"
+                 : "+a"(acc.c[7][0]), "+a"(acc.c[7][1]), "+a"(acc.c[7][2]), "+a"(acc.c[7][3]),
+                   "+a"(acc.c[7][4]), "+a"(acc.c[7][5]), "+a"(acc.c[7][6]), "+a"(acc.c[7][7]));
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // acc += A-tile * B-tile^T over K in [k_begin, k_end), a multiple of 64 wide.
   // K-contiguous operand: tile rows row0 .. row0+256 of x (rows clamped to
@@ -422,118 +551,136 @@ struct MfmaDirect4Engine : MfmaTileLayout<T_, 2, 4> {
   // column chunks clamped to the last valid one; x.rows is a multiple of 8);
   // all K rows in [k_begin, k_end) must exist.
   // kOverwrite: acc = A-tile * B-tile^T instead (the incoming acc is ignored: the
-  // first 16 MFMAs take a zero constant as their addend, which saves zeroing
+  // first 64 MFMAs take a zero constant as their addend, which saves zeroing
   // 256 accumulator registers per tile).
   template <bool kAKMajor, bool kBKMajor, bool kOverwrite = false>
   __device__ __forceinline__ void mainloop_ex(const Operand<T>& A, const Operand<T>& B,
                                               int k_begin, int k_end, Acc& acc,
                                               char* smem) const {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
-    Loader la = make_loader<kAKMajor>(A, k_begin, lds0, false);
-    Loader lb = make_loader<kBKMajor>(B, k_begin, lds0 + kOperandBytes, true);
-    const Reader ra = make_reader<kAKMajor>(wm);
-    const Reader rb = make_reader<kBKMajor>(wn);
+    Loader la = make_loader<kAKMajor>(A, k_begin, lds0);
+    Loader lb = make_loader<kBKMajor>(B, k_begin, lds0 + kOperandBytes);
+    const int ra = reader_base<kAKMajor>(wm);
+    const int rb = reader_base<kBKMajor>(wn);
 
-    // load number q (0..15) of the next K tile into `stage`, `ahead` K tiles
-    // past the loaders' current position: even q -> A, odd q -> B
-    auto issue_one = [&](int stage, int ahead, int q) {
+    // load number q (0..15) of the K tile the loaders stand at, into `stage`: even q -> A,
+    // odd q -> B
+    auto issue_one = [&](int stage, int q) {
       const unsigned s_off = (unsigned)(stage * kStageBytes) + (unsigned)((q >> 1) * 1024);
-      if (q & 1) load_to_lds(lb.fill + s_off, lb.off[q >> 1], lb.next + ahead * lb.step);
-      else load_to_lds(la.fill + s_off, la.off[q >> 1], la.next + ahead * la.step);
+      if (q & 1) load_to_lds(lb.fill + s_off, lb.off[q >> 1], lb.next);
+      else load_to_lds(la.fill + s_off, la.off[q >> 1], la.next);
     };
-    // fragment r (0..7) of a slice in the order the next slice consumes them:
-    // b0..b3 first (every MFMA group needs all four), then a0..a3
-    auto read_one = [&](Frags& f, int stage, int ks, int r) {
-      const char* st = smem + stage * kStageBytes;
-      if (r < 4) f.b[r] = read_frag<kBKMajor>(st + kOperandBytes, rb, ks, r);
-      else f.a[r - 4] = read_frag<kAKMajor>(st, ra, ks, r - 4);
+    V8 fa[kTM], fb[2][kTN];
+    auto read_a = [&](int stage, int ks, int i) {
+      fa[i] = read_frag<kAKMajor>(smem + stage * kStageBytes, ra, ks, i);
+    };
+    auto read_b = [&](int stage, int ks, int i) {
+      fb[ks][i] = read_frag<kBKMajor>(smem + stage * kStageBytes + kOperandBytes, rb, ks, i);
     };
 
     const int nk = (k_end - k_begin) / kBK;
-    constexpr bool kLoadsInPairs = !(kAKMajor && !kBKMajor);
-    auto step = [&](int k, Frags& fa, Frags& fb, auto has_next_tag, auto first_tag) {
-      constexpr bool kHasNext = decltype(has_next_tag)::value;
+    // This wave's share of the touches: 64 lines of A (waves 0, 1) or B (waves 2, 3), in
+    // the half of the tile's lines that the workgroup's neighbours leave to it.
+    const bool touch_b = wave >= 2;
+    const int line = (wave & 1) * 64 + lane +
+                     (((touch_b ? A.row0 : B.row0) / kTile) & 1) * 128;
+    const unsigned touch_off = touch_b ? line_offset<kBKMajor>(B, line) : line_offset<kAKMajor>(A, line);
+    const int64_t touch_step = readfirstlane64(touch_b ? lb.step : la.step);
+    const char* touch_base = reinterpret_cast<const char*>(
+        readfirstlane64(reinterpret_cast<int64_t>(touch_b ? lb.next : la.next)));
+    const unsigned touch_lds =
+        __builtin_amdgcn_readfirstlane(lds0 + 2 * kStageBytes + (unsigned)wave * 256);
+    auto touch_tile = [&](int k) {
+      touch(touch_lds, touch_off, touch_base + (int64_t)min(k, nk - 1) * touch_step);
+    };
+    // tiles_left: how many tiles follow (0, 1, or 2 for "two or more")
+    auto step = [&](int k, auto tiles_left_tag, auto first_tag) {
+      constexpr bool kHasNext = decltype(tiles_left_tag)::value >= 1;
+      constexpr bool kHasTwo = decltype(tiles_left_tag)::value >= 2;
       constexpr bool kFirst = decltype(first_tag)::value;   // first step of an overwriting loop
       const int cur = k & 1;
       const int nxt = cur ^ 1;
-      const bool more = (k + 2 < nk);
+      // fragments the allocator has moved between two steps with VALU copies: two wait
+      // states before an MFMA may read them, which the compiler does not add for asm
+      asm volatile("s_nop 1");
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int g = 0; g < 16; ++g) {
-        const int sl = g >> 2;
-        const int q = g & 3;
-        Frags& fcur = (sl & 1) ? fb : fa;
-        Frags& fnext = (sl & 1) ? fa : fb;
-        const bool after_barrier = kHasNext && sl == 3 && q >= 2;
-        if (kHasNext && sl == 3 && q == 2) {
+        const int s = g >> 3;
+        const int q = g & 7;
+        if (kHasNext && s == 1 && q == 2) {
           // tile k+1 is complete and visible from here on; stage `cur` is free
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          // (the one younger access is the touch of this step)
+          asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
           __syncthreads();
           la.next += la.step;
           lb.next += lb.step;
         }
 #pragma unroll
         for (int t = 0; t < kTN; ++t) {
-          if (kFirst && sl == 0) {
-            const f32x16_t zero = {};
-            acc.c[q][t] = Op::mma(fcur.a[q], fcur.b[t], zero);
-          } else {
-            acc.c[q][t] = Op::mma(fcur.a[q], fcur.b[t], acc.c[q][t]);
-          }
-          if (sl < 3) {
-            if (t == 0) read_one(fnext, cur, sl + 1, 2 * q);
-            if (t == 2) read_one(fnext, cur, sl + 1, 2 * q + 1);
+          if (kFirst && s == 0) Op::mma_set(fa[q], fb[s][t], acc.c[q][t]);
+          else Op::mma(fa[q], fb[s][t], acc.c[q][t]);
+          if (kHasNext && s == 0 && q == 4 && t == 3) touch_tile(k + kTouchAhead);
+          // last A block of this slice
+          if (q == 0 && t == 1) read_a(cur, s, kTM - 1);
+          if (s == 0) {
+            // slice 1 of this tile
+            if (q < 2 && (t == 3 || t == 5)) read_b(cur, 1, 2 * q + (t == 5));
+            if (q >= 2 && q < 6 && t == 5) read_b(cur, 1, q + 2);
+            if (q >= 1 && t == 2) read_a(cur, 1, q - 1);
             if (kHasNext) {
-              // loads 6..15 of the next tile: two per group in groups 0..4 (measured
-              // about 1 % faster), except for the K-major x K-contiguous pairing,
-              // which does better with one per group in groups 0..9
-              if (kLoadsInPairs) {
-                if ((t == 1 || t == 3) && g < 5) issue_one(nxt, 0, 6 + 2 * g + (t == 3));
-              } else {
-                if (t == 1 && g < 10) issue_one(nxt, 0, 6 + g);
-              }
+              constexpr int kRest = 16 - kLoadsAfterBarrier;
+              // two per group
+              if ((t == 0 || t == 4) && 2 * q + (t == 4) < kRest)
+                issue_one(nxt, kLoadsAfterBarrier + 2 * q + (t == 4));
             }
-          } else if (after_barrier) {
-            if (q == 2) {
-              if (t == 0) { read_one(fnext, nxt, 0, 0); read_one(fnext, nxt, 0, 1); }
-              else read_one(fnext, nxt, 0, t + 1);
-            } else {
-              if (t < 3) read_one(fnext, nxt, 0, 5 + t);
-            }
-            if (t >= 1 && more) issue_one(cur, 0, (q - 2) * 3 + (t - 1));
+          } else if (kHasNext && q >= 2) {
+            // slice 0 of the next tile
+            if (q < 4 && (t == 1 || t == 3 || t == 5)) read_b(nxt, 0, (q - 2) * 3 + (t >> 1));
+            if (q == 4 && (t == 1 || t == 3)) read_b(nxt, 0, 6 + (t >> 1));
+            if (q < 4 && t == 7) read_a(nxt, 0, q - 2);
+            if (q == 4 && t == 5) read_a(nxt, 0, 2);
+            if (q == 4 && t == 7) read_a(nxt, 0, 3);
+            if (q >= 5 && t == 3) read_a(nxt, 0, q - 1);
+            if (kHasTwo && (t == 2 || t == 6) && 2 * (q - 2) + (t == 6) < kLoadsAfterBarrier)
+              issue_one(cur, 2 * (q - 2) + (t == 6));
           }
           __builtin_amdgcn_sched_barrier(0);
         }
       }
     };
 
-    // tile 0 entirely, then the first six loads of tile 1 (la.next / lb.next
-    // always point at the tile whose loads are being issued)
+    // tile 0 entirely, then the first loads of tile 1 (la.next / lb.next always point at
+    // the tile whose loads are being issued)
 #pragma unroll
-    for (int q = 0; q < 16; ++q) issue_one(0, 0, q);
+    for (int q = 0; q < 16; ++q) issue_one(0, q);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     la.next += la.step;
     lb.next += lb.step;
     if (nk > 1) {
 #pragma unroll
-      for (int q = 0; q < 6; ++q) issue_one(1, 0, q);
+      for (int q = 0; q < kLoadsAfterBarrier; ++q) issue_one(1, q);
     }
-    Frags f0, f1;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) read_one(f0, 0, 0, r);
-    // a step consumes slices from f0,f1,f0,f1 and leaves the next tile's slice 0 in f0
+    for (int r = 0; r < kTN; ++r) read_b(0, 0, r);
+#pragma unroll
+    for (int r = 0; r + 1 < kTM; ++r) read_a(0, 0, r);
+    using Left0 = std::integral_constant<int, 0>;
+    using Left1 = std::integral_constant<int, 1>;
+    using Left2 = std::integral_constant<int, 2>;
+    int k = 0;
     if constexpr (kOverwrite) {
-      if (nk > 1) {
-        step(0, f0, f1, std::true_type{}, std::true_type{});
-        for (int k = 1; k + 1 < nk; ++k) step(k, f0, f1, std::true_type{}, std::false_type{});
-        step(nk - 1, f0, f1, std::false_type{}, std::false_type{});
-      } else {
-        step(0, f0, f1, std::false_type{}, std::true_type{});
-      }
-    } else {
-      for (int k = 0; k + 1 < nk; ++k) step(k, f0, f1, std::true_type{}, std::false_type{});
-      step(nk - 1, f0, f1, std::false_type{}, std::false_type{});
+      if (nk > 2) step(0, Left2{}, std::true_type{});
+      else if (nk == 2) step(0, Left1{}, std::true_type{});
+      else step(0, Left0{}, std::true_type{});
+      k = 1;
     }
+    for (; k + 2 < nk; ++k) step(k, Left2{}, std::false_type{});
+    if (k + 2 == nk) step(k++, Left1{}, std::false_type{});
+    if (k < nk) step(k, Left0{}, std::false_type{});
+    mfma_drain(acc);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last touches have landed
     __syncthreads();
   }
 

@@ -77,7 +77,7 @@ template <class E, bool kSoftcap, bool kPlain = false>
 __global__ __launch_bounds__(E::kThreads) void lce_exp_logits_panel_kernel(ExpPanelArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
-  static_assert(E::kHasKMajor && sizeof(T) == 2 && E::kCols == 4,
+  static_assert(E::kHasKMajor && sizeof(T) == 2,
                 "written for the four-wave direct-to-LDS engine");
   if (p.run_flag != nullptr && *p.run_flag == 0) return;
   if (p.m_dev != nullptr) {
@@ -160,12 +160,13 @@ __global__ __launch_bounds__(E::kThreads) void lce_exp_logits_panel_kernel(ExpPa
       }
       col_sum[j] = s;
       col_max[j] = mx;
+      if (j % E::kStageCols != E::kStageCols - 1) continue;
       __syncthreads();
-      constexpr int kPieces = E::kTokensPerIndex * 32;   // 16-byte pieces of this quarter
+      constexpr int kPieces = E::kTokensPerIndex * 32;   // 16-byte pieces per owned index
 #pragma unroll
-      for (int it = 0; it < kPieces / E::kThreads; ++it) {
+      for (int it = 0; it < E::kStageCols * kPieces / E::kThreads; ++it) {
         const int c = it * E::kThreads + threadIdx.x;
-        const int t = E::token_of_index(j, c >> 5);
+        const int t = E::token_of_index(j + 1 - E::kStageCols + c / kPieces, (c % kPieces) >> 5);
         const int ch = c & 31;
         const uint4 val = *reinterpret_cast<const uint4*>(smem + t * 512 + ((ch ^ (t & 31)) * 16));
         stream_store16(panel + ((int64_t)tt * E::kTile + t) * p.ld + pcol + ch * 8, val);

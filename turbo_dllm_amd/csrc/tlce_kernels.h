@@ -529,12 +529,13 @@ __global__ __launch_bounds__(E::kThreads) void lce_grad_logits_panel_kernel(Grad
                                         (vq & 1) * 8);
           store4<T>(dst, g4[0], g4[1], g4[2], g4[3]);
         }
+        if (j % E::kStageCols != E::kStageCols - 1) continue;
         __syncthreads();
-        constexpr int kPieces = E::kTokensPerIndex * 32;   // 16-byte pieces of this quarter
+        constexpr int kPieces = E::kTokensPerIndex * 32;   // 16-byte pieces per owned index
 #pragma unroll
-        for (int it = 0; it < kPieces / E::kThreads; ++it) {
+        for (int it = 0; it < E::kStageCols * kPieces / E::kThreads; ++it) {
           const int c = it * E::kThreads + threadIdx.x;
-          const int t = E::token_of_index(j, c >> 5);
+          const int t = E::token_of_index(j + 1 - E::kStageCols + c / kPieces, (c % kPieces) >> 5);
           const int ch = c & 31;
           const uint4 val =
               *reinterpret_cast<const uint4*>(smem + t * 512 + ((ch ^ (t & 31)) * 16));
@@ -815,17 +816,20 @@ __global__ __launch_bounds__(E::kThreads) void lce_kl_panel_kernel(KlPanelArgs p
         process(j, i4, t, g);
         if (grad || kEmit) store4<T>(cell, g[0], g[1], g[2], g[3]);
       }
-      if (grad || kEmit) {
-        // the tokens with owned index j are complete: their rows go out while
-        // the next quarter of the tile is being processed
+      if ((grad || kEmit) && j % E::kStageCols == E::kStageCols - 1) {
+        // the tokens of this quarter of the tile are complete: their rows go out while
+        // the next quarter is being processed
         __syncthreads();
         constexpr int kPieces = E::kTokensPerIndex * 32;
-        constexpr int kMine = kPieces / E::kThreads;
+        constexpr int kMine = E::kStageCols * kPieces / E::kThreads;
+        auto token_of = [&](int c) {
+          return E::token_of_index(j + 1 - E::kStageCols + c / kPieces, (c % kPieces) >> 5);
+        };
         uint4 val[kMine];   // LDS reads first, then the stores: one wait per quarter
 #pragma unroll
         for (int it = 0; it < kMine; ++it) {
           const int c = it * E::kThreads + threadIdx.x;
-          const int tok = E::token_of_index(j, c >> 5);
+          const int tok = token_of(c);
           const int ch = c & 31;
           val[it] = *reinterpret_cast<const uint4*>(smem + tok * 512 + ((ch ^ (tok & 31)) * 16));
         }
@@ -833,7 +837,7 @@ __global__ __launch_bounds__(E::kThreads) void lce_kl_panel_kernel(KlPanelArgs p
 #pragma unroll
         for (int it = 0; it < kMine; ++it) {
           const int c = it * E::kThreads + threadIdx.x;
-          const int tok = E::token_of_index(j, c >> 5);
+          const int tok = token_of(c);
           const int ch = c & 31;
           stream_store16(panel + ((int64_t)tt * E::kTile + tok) * p.ld + prow + ch * 8, val[it]);
         }
@@ -943,21 +947,20 @@ __global__ __launch_bounds__(E::kThreads) void lce_logits_panel_kernel(LogitsPan
     }
     return make_float4(z[0], z[1], z[2], z[3]);
   };
-  if constexpr (E::kHasKMajor && E::kCols == 4) {
+  if constexpr (E::kHasKMajor) {
     // The float32 tile is twice the engine's LDS: it is staged and written in two
-    // halves (the tokens of two owned column indices = 128 rows of 1 KiB, 16-byte
+    // halves (the tokens of half the owned column indices = 128 rows of 1 KiB, 16-byte
     // chunk c of staged row s in slot c ^ (s & 63)), so that G leaves in whole
     // 1 KiB rows instead of 16-byte pieces a row apart.
-    constexpr int kPerIndex = E::kTokensPerIndex;     // 64 tokens per owned index
+    constexpr int kPerIndex = E::kTokensPerIndex;
+    constexpr int kHalf = E::kCols / 2;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       if (half) __syncthreads();                      // the first half has been read out
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj) {
-        const int j = 2 * half + jj;
-        // position of this lane's token among those with index j, as token_of_index counts
-        const int t = (eng.col(j) / (E::kTile / 2)) * 32 + (eng.col(j) & 31);
-        const int s_row = jj * kPerIndex + t;
+      for (int jj = 0; jj < kHalf; ++jj) {
+        const int j = kHalf * half + jj;
+        const int s_row = jj * kPerIndex + eng.position_in_index();
 #pragma unroll
         for (int i4 = 0; i4 < E::kRows; i4 += 4) {
           const int c = eng.row(i4) >> 2;
@@ -967,11 +970,11 @@ __global__ __launch_bounds__(E::kThreads) void lce_logits_panel_kernel(LogitsPan
       }
       __syncthreads();
 #pragma unroll 4
-      for (int it = 0; it < (2 * kPerIndex * 64) / E::kThreads; ++it) {
+      for (int it = 0; it < (kHalf * kPerIndex * 64) / E::kThreads; ++it) {
         const int idx = it * E::kThreads + threadIdx.x;
         const int s_row = idx >> 6;
         const int ch = idx & 63;
-        const int tok = E::token_of_index(2 * half + s_row / kPerIndex, s_row % kPerIndex);
+        const int tok = E::token_of_index(kHalf * half + s_row / kPerIndex, s_row % kPerIndex);
         const uint4 val =
             *reinterpret_cast<const uint4*>(smem + s_row * 1024 + ((ch ^ (s_row & 63)) * 16));
         stream_store16(p.panel + ((int64_t)tt * E::kTile + tok) * p.ld + prow + ch * 4, val);
@@ -1155,7 +1158,7 @@ constexpr int kSplitMajorBelowTiles = 64;
 // instead of 64 pieces 16 or 8 bytes long in 64 different rows.
 //
 // float32 output (the grad_hidden slabs): the tile is 256 KiB, twice the LDS, and
-// goes in two halves, the rows of two owned column indices each (128 rows of
+// goes in two halves, the rows of half the owned column indices each (128 rows of
 // 1 KiB, 16-byte chunk c of staged row s in slot c ^ (s & 63)).  kAdd: the slab's
 // old values of a half are requested before its rows are staged, so their
 // latency passes under the staging.
@@ -1166,7 +1169,8 @@ __device__ __forceinline__ void store_tile_f32_by_rows(const E& eng, const typen
                                                        int row0, int col0, int c_rows,
                                                        int c_cols) {
   constexpr int kPerIndex = E::kTokensPerIndex;                 // rows per owned index
-  constexpr int kMine = (2 * kPerIndex * 64) / E::kThreads;     // 16-byte pieces per thread
+  constexpr int kHalf = E::kCols / 2;
+  constexpr int kMine = (kHalf * kPerIndex * 64) / E::kThreads; // 16-byte pieces per thread
   constexpr int kBatch = 8;
   constexpr int kBatches = kMine / kBatch;
   constexpr int kAhead = 2;                                     // batches of old values in flight
@@ -1178,7 +1182,7 @@ __device__ __forceinline__ void store_tile_f32_by_rows(const E& eng, const typen
       const int idx = it * E::kThreads + threadIdx.x;
       *s_row = idx >> 6;
       *ch = idx & 63;
-      *out_row = row0 + E::token_of_index(2 * half + *s_row / kPerIndex, *s_row % kPerIndex);
+      *out_row = row0 + E::token_of_index(kHalf * half + *s_row / kPerIndex, *s_row % kPerIndex);
       *out_col = col0 + *ch * 4;
       return *out_row < c_rows && *out_col < c_cols;
     };
@@ -1199,10 +1203,9 @@ __device__ __forceinline__ void store_tile_f32_by_rows(const E& eng, const typen
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int j = 2 * half + jj;
-      const int t = (eng.col(j) / (E::kTile / 2)) * 32 + (eng.col(j) & 31);
-      const int s_row = jj * kPerIndex + t;
+    for (int jj = 0; jj < kHalf; ++jj) {
+      const int j = kHalf * half + jj;
+      const int s_row = jj * kPerIndex + eng.position_in_index();
 #pragma unroll
       for (int i4 = 0; i4 < E::kRows; i4 += 4) {
         const int chunk = eng.row(i4) >> 2;
@@ -1346,7 +1349,7 @@ __global__ __launch_bounds__(E::kThreads) void lce_gemm_nt_kernel(GemmArgs p) {
                      acc, smem);
   }
 
-  if constexpr (E::kHasKMajor && sizeof(T) == 2 && E::kCols == 4) {
+  if constexpr (E::kHasKMajor && sizeof(T) == 2) {
     // The direct engine is only planned for hidden sizes that are multiples of 64
     // and its outputs (workspace slabs, rows of grad_weight) are 16-byte aligned:
     // whole output rows leave through LDS (the main loop has ended on a barrier).
