@@ -45,15 +45,39 @@ static inline int64_t align256(int64_t x) { return round_up(x, 256); }
 
 static inline int dtype_bytes(int dtype) { return dtype == TLCE_DTYPE_F32 ? 4 : 2; }
 
-// Forward launch shape: token tiles x vocabulary splits workgroups, at most (and
-// close to) four whole waves of 256 workgroups on a 256-CU MI355X.  Shared by
-// the host plan and by the kernels that derive the plan from a row count that
-// only the device knows.
+// Forward launch shape: token tiles x vocabulary splits workgroups, at most four whole
+// rounds of 256 workgroups on a 256-CU MI355X.  Shared by the host plan and by the
+// kernels that derive the plan from a row count that only the device knows.
+//
+// A split loops over ceil(n_vtiles / splits) tiles, so the launch lasts about
+// rounds x (that + 1/8 for a workgroup's start and merge) tile times; of one to four
+// rounds the cheapest is taken, ties going to fewer (longer loops keep the workgroups
+// of an XCD in step).  Fewer than four splits leave an XCD's 32 workgroups more
+// distinct operand strips than the usual 12, which costs time: 2 splits measured 9 %.
+// Measured (ms, H = 4096, V = 151936; always four rounds -> this rule): 1610 rows
+// 1.72 -> 1.60, 6357 rows 6.43 -> 5.62; 12000 rows over H = 2048, V = 65536 2.42 -> 2.37
+// (three rounds); 32768 rows over V = 16384 keep 2.98 (one round of two splits 3.26).
 constexpr int kTargetWorkgroups = 1024;
 __host__ __device__ static inline int forward_vocab_splits(int n_ttiles, int n_vtiles) {
-  const int want = n_ttiles > 0 ? kTargetWorkgroups / n_ttiles : kTargetWorkgroups;
-  const int s = want < 1 ? 1 : want;
-  return s < n_vtiles ? s : n_vtiles;
+  int pick = 1;
+  int64_t best = -1;
+  for (int rounds = 1; rounds <= kTargetWorkgroups / 256; ++rounds) {
+    int splits = n_ttiles > 0 ? rounds * 256 / n_ttiles : rounds * 256;
+    splits = splits < 1 ? 1 : (splits < n_vtiles ? splits : n_vtiles);
+    const int64_t launched = ((int64_t)n_ttiles * splits + 255) / 256;
+    const int64_t tiles = (n_vtiles + splits - 1) / splits;
+    const int strips = splits >= 8   ? 100
+                       : splits >= 4 ? 102
+                       : splits == 3 ? 104
+                       : splits == 2 ? 110
+                                     : 133;
+    const int64_t cost = launched * (8 * tiles + 1) * strips;
+    if (best < 0 || cost < best) {
+      best = cost;
+      pick = splits;
+    }
+  }
+  return pick;
 }
 
 // K splits of the grad_hidden contraction: `tiles` output tiles per panel, each a
@@ -121,24 +145,14 @@ __device__ __forceinline__ int xcd_logical_block_of(int bid, int tiles) {
   return logical < tiles ? logical : -1;
 }
 
-// Grouped tile order: consecutive logical ids walk `group` tiles along i, then
-// step j, so the ~32 workgroups resident on one XCD cover a group x (32/group)
-// block of tiles and share both operands through that XCD's L2.
+// Grouped tile order: consecutive logical ids walk a group of at most `group` tiles
+// along i, then step j, so the ~32 workgroups resident on one XCD cover a group x
+// (32/group) block of tiles and share both operands through that XCD's L2.  The groups
+// are balanced: ceil(ni / group) groups whose sizes differ by at most one (13 tiles in
+// groups of at most 4: 4, 3, 3, 3 instead of 4, 4, 4, 1; a group of one tile has its 32
+// workgroups fetch 33 strips instead of 12: 9 token tiles in groups of 4, 4, 1 took the
+// forward 1.51 ms against 1.28 balanced, 5 hidden tiles grad_weight 0.65 against 0.59).
 __device__ __forceinline__ void grouped_tile(int logical, int ni, int nj, int group,
-                                             int* ti, int* tj) {
-  const int width = group * nj;
-  const int gid = logical / width;
-  const int first = gid * group;
-  const int gsize = min(ni - first, group);
-  const int within = logical - gid * width;
-  *ti = first + within % gsize;
-  *tj = within / gsize;
-}
-
-// The same order with the groups along i balanced: ceil(ni / group) groups whose
-// sizes differ by at most one (13 tiles in groups of at most 4: 4, 3, 3, 3 instead
-// of 4, 4, 4, 1), for launches whose ni is small and not a multiple of the group.
-__device__ __forceinline__ void balanced_grouped_tile(int logical, int ni, int nj, int group,
                                                       int* ti, int* tj) {
   const int n_groups = (ni + group - 1) / group;
   const int base = ni / n_groups, extra = ni % n_groups;   // the first `extra` groups hold base + 1

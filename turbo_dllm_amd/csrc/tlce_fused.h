@@ -87,7 +87,7 @@ __global__ __launch_bounds__(E::kThreads) void lce_exp_logits_panel_kernel(ExpPa
   const int logical = xcd_logical_block_of(blockIdx.x, p.n_ttiles * p.n_vtiles);
   if (logical < 0) return;
   int tt, vt;
-  balanced_grouped_tile(logical, p.n_ttiles, p.n_vtiles, 4, &tt, &vt);
+  grouped_tile(logical, p.n_ttiles, p.n_vtiles, 4, &tt, &vt);
 
   E eng;
   typename E::Acc acc;

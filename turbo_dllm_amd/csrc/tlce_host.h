@@ -113,8 +113,7 @@ inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_gr
   p.n_ttiles = (int)(p.mp / p.tile);
   p.n_vtiles = (int)(p.vp / p.tile);
   p.n_htiles = (int)ceil_div(h, p.tile);
-  // forward: token tiles x vocabulary splits workgroups, at most (and close to)
-  // four whole waves of 256 workgroups
+  // forward: token tiles x vocabulary splits workgroups, whole rounds of 256
   p.nsplit = forward_vocab_splits(p.n_ttiles, p.n_vtiles);
   if (panel_bytes <= 0) panel_bytes = kDefaultPanelBytes;
   const int64_t col_bytes = p.mp * dtype_bytes(dtype) * ((weight_grad && !p.kmajor) ? 2 : 1);
