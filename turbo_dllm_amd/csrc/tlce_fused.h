@@ -84,10 +84,9 @@ __global__ __launch_bounds__(E::kThreads) void lce_exp_logits_panel_kernel(ExpPa
     p.m = effective_block_rows(p.m, p.m_dev, p.row0);
     p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
   }
-  const int logical = xcd_logical_block_of(blockIdx.x, p.n_ttiles * p.n_vtiles);
-  if (logical < 0) return;
   int tt, vt;
-  grouped_tile(logical, p.n_ttiles, p.n_vtiles, 4, &tt, &vt);
+  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_vtiles, (int64_t)E::kTile * p.h * sizeof(T), &tt, &vt))
+    return;
 
   E eng;
   typename E::Acc acc;

@@ -401,10 +401,9 @@ __global__ __launch_bounds__(E::kThreads) void lce_grad_logits_panel_kernel(Grad
     p.m = effective_rows(p.m, p.m_dev);
     p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
   }
-  const int logical = xcd_logical_block_of(blockIdx.x, p.n_ttiles * p.n_ptiles);
-  if (logical < 0) return;
   int tt, pv;
-  grouped_tile(logical, p.n_ttiles, p.n_ptiles, 4, &tt, &pv);
+  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_ptiles, (int64_t)E::kTile * p.h * sizeof(T), &tt, &pv))
+    return;
 
   E eng;
   const T* hidden = static_cast<const T*>(p.hidden);
@@ -676,10 +675,9 @@ __global__ __launch_bounds__(E::kThreads) void lce_kl_panel_kernel(KlPanelArgs p
   static_assert(kEmit || !kNoTeacher, "kNoTeacher belongs to the emitting pass");
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
-  const int logical = xcd_logical_block(blockIdx.x, gridDim.x);
-  if (logical >= p.n_ttiles * p.n_ptiles) return;
   int tt, pv;
-  grouped_tile(logical, p.n_ttiles, p.n_ptiles, 4, &tt, &pv);
+  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_ptiles, (int64_t)E::kTile * p.h * sizeof(T), &tt, &pv))
+    return;
 
   E eng;
   typename E::Acc acc;
@@ -926,10 +924,9 @@ template <class E, bool kSoftcap>
 __global__ __launch_bounds__(E::kThreads) void lce_logits_panel_kernel(LogitsPanelArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
-  const int logical = xcd_logical_block(blockIdx.x, gridDim.x);
-  if (logical >= p.n_ttiles * p.n_ptiles) return;
   int tt, pv;
-  grouped_tile(logical, p.n_ttiles, p.n_ptiles, 4, &tt, &pv);
+  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_ptiles, (int64_t)E::kTile * p.h * sizeof(T), &tt, &pv))
+    return;
   E eng;
   typename E::Acc acc;
   const int vbase = p.v0 + pv * E::kTile;
@@ -1302,18 +1299,18 @@ __global__ __launch_bounds__(E::kThreads) void lce_gemm_nt_kernel(GemmArgs p) {
       if (p.k == 0 && p.mode == kAddF32) return;
     }
   }
-  int logical, split;
+  int split, ti, tj;
   const int tiles = p.ni * p.nj;
   if (gridDim.y == 1 || tiles >= kSplitMajorBelowTiles) {
-    // every split deals its tiles to the 8 XCDs in contiguous runs of tiles / 8
     split = blockIdx.y;
     if (split >= n_splits) return;
-    logical = xcd_logical_block_of(blockIdx.x, tiles);
-    if (logical < 0) return;
+    if (!xcd_tile(blockIdx.x, p.ni, p.nj, (int64_t)E::kTile * min(p.k, p.k_per_split) * sizeof(T),
+                  &ti, &tj))
+      return;
   } else {
     // Few output tiles under many K splits (a small head, the last rows of a call
-    // whose row count is on the device): a run of tiles / 8 would be 2 or 3 tiles, and
-    // all 8 XCDs would fetch every K range of both operands.  The (split, tile) pairs
+    // whose row count is on the device): an XCD's share of a split would be 2 or 3 tiles,
+    // and all 8 XCDs would fetch every K range of both operands.  The (split, tile) pairs
     // in split-major order are dealt to the XCDs in 8 contiguous, equally long runs
     // instead, so the tiles that stream one K range sit on one XCD (or two) and share
     // it through that L2.
@@ -1324,10 +1321,8 @@ __global__ __launch_bounds__(E::kThreads) void lce_gemm_nt_kernel(GemmArgs p) {
     const int last = (int)((int64_t)(xcd + 1) * total / kXcds);
     if (slot >= last - first) return;
     split = (first + slot) / tiles;
-    logical = (first + slot) - split * tiles;
+    grouped_tile((first + slot) - split * tiles, p.ni, p.nj, 4, &ti, &tj);
   }
-  int ti, tj;
-  grouped_tile(logical, p.ni, p.nj, 4, &ti, &tj);
   // each K split owns its own output slab: no atomics, reproducible sums; a
   // split whose K range is empty still writes its (zero) tile
   const int k_begin = split * p.k_per_split;
