@@ -612,8 +612,9 @@ int tlce_grad_weight_from_panel(const void* hidden, const int64_t* row_idx,
 /* ---- introspection used by the benchmark and the tests -------------------
  * Tile plan the host scheduler would use for a problem; any pointer may be
  * NULL.  `engine` is 2 for the bf16/f16 MFMA kernels with direct-to-LDS loads
- * (h a multiple of 32), 1 for the register-staged MFMA kernels (h a multiple of
- * 8), 0 for the generic float32-FMA kernels (float32 inputs, other h). */
+ * (h a multiple of 64), 1 for the register-staged MFMA kernels (h a multiple of
+ * 8), 3 for the float32 MFMA kernels (float32 inputs, h a multiple of 4, v at
+ * least 64), 0 for the generic float32-FMA kernels (the rest). */
 int tlce_query_plan(int64_t m, int64_t h, int64_t v, int dtype,
                     int compute_weight_grad, int64_t panel_bytes,
                     int* engine, int64_t* tile, int64_t* forward_vocab_splits,

@@ -49,3 +49,35 @@ def check(dev, m, h, v, dtype, mode, seed=5, **kw):
 ])
 def test_direct_engine_edges(gpu_device, m, h, v, dtype, mode):
     check(gpu_device, m, h, v, dtype, mode)
+
+
+@pytest.mark.parametrize("m,h,v,kw", [
+    (1, 4, 64, {}),                                 # one piece of one K stage
+    (3, 4, 63, {}),                                 # the last vocabulary of the generic engine
+    (31, 36, 127, dict(logit_softcap=30.0)),        # a K stage and a remainder
+    (128, 32, 128, {}),                             # whole tiles, one K stage
+    (129, 100, 257, dict(exclude_index=7)),         # a row and a vocabulary row past tiles
+    (260, 260, 3001, {}),                           # K splits of grad_hidden, odd vocabulary
+    (700, 64, 4099, dict(logit_softcap=20.0)),
+])
+def test_float32_engine_edges(gpu_device, m, h, v, kw):
+    check(gpu_device, m, h, v, torch.float32, "recompute", **kw)
+
+
+def test_float32_engine_with_bias_matches_the_oracle(gpu_device):
+    gen = torch.Generator().manual_seed(3)
+    m, h, v = 130, 68, 300
+    hidden = torch.randn(m, h, generator=gen)
+    weight = torch.randn(v, h, generator=gen) * 0.05
+    bias = torch.randn(v, generator=gen) * 0.1
+    labels = torch.randint(0, v, (m,), generator=gen)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (hidden, weight, bias)]
+    loss = tiled_linear_cross_entropy(leaves[0], leaves[1], labels.to(gpu_device),
+                                      bias=leaves[2], dtype=torch.float32)
+    loss.backward()
+    ref = [t.clone().requires_grad_(True) for t in (hidden, weight, bias)]
+    expected = torch.nn.functional.cross_entropy(ref[0] @ ref[1].t() + ref[2], labels)
+    expected.backward()
+    assert abs(float(loss.detach()) - float(expected.detach())) <= 2e-5 * float(expected.detach())
+    for got, want in zip(leaves, ref):
+        assert oracle.relative_max_error(got.grad, want.grad) <= 3e-5

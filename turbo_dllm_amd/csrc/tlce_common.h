@@ -45,6 +45,13 @@ static inline int64_t align256(int64_t x) { return round_up(x, 256); }
 
 static inline int dtype_bytes(int dtype) { return dtype == TLCE_DTYPE_F32 ? 4 : 2; }
 
+// Workgroups of a tile engine that the 256 CUs hold at once: the float32 MFMA engine
+// (128x128 tiles) fits two on a CU, the 256x256 ones take a CU each, and the generic
+// 64x64 one is planned like those.
+__host__ __device__ static inline int resident_workgroups(int tile) {
+  return tile == 128 ? 512 : 256;
+}
+
 // Forward launch shape: token tiles x vocabulary splits workgroups, at most four whole
 // rounds of 256 workgroups on a 256-CU MI355X.  Shared by the host plan and by the
 // kernels that derive the plan from a row count that only the device knows.
@@ -58,13 +65,14 @@ static inline int dtype_bytes(int dtype) { return dtype == TLCE_DTYPE_F32 ? 4 : 
 // 1.72 -> 1.60, 6357 rows 6.43 -> 5.62; 12000 rows over H = 2048, V = 65536 2.42 -> 2.37
 // (three rounds); 32768 rows over V = 16384 keep 2.98 (one round of two splits 3.26).
 constexpr int kTargetWorkgroups = 1024;
-__host__ __device__ static inline int forward_vocab_splits(int n_ttiles, int n_vtiles) {
+__host__ __device__ static inline int forward_vocab_splits(int n_ttiles, int n_vtiles,
+                                                           int resident) {
   int pick = 1;
   int64_t best = -1;
-  for (int rounds = 1; rounds <= kTargetWorkgroups / 256; ++rounds) {
-    int splits = n_ttiles > 0 ? rounds * 256 / n_ttiles : rounds * 256;
+  for (int rounds = 1; rounds <= kTargetWorkgroups / resident; ++rounds) {
+    int splits = n_ttiles > 0 ? rounds * resident / n_ttiles : rounds * resident;
     splits = splits < 1 ? 1 : (splits < n_vtiles ? splits : n_vtiles);
-    const int64_t launched = ((int64_t)n_ttiles * splits + 255) / 256;
+    const int64_t launched = ((int64_t)n_ttiles * splits + resident - 1) / resident;
     const int64_t tiles = (n_vtiles + splits - 1) / splits;
     const int strips = splits >= 8   ? 100
                        : splits >= 4 ? 102
@@ -89,12 +97,13 @@ __host__ __device__ static inline int forward_vocab_splits(int n_ttiles, int n_v
 // Ties go to fewer splits.  Integer arithmetic only: the host plan and the
 // kernels that re-plan for a row count known on the device must agree.
 __host__ __device__ static inline int grad_hidden_k_splits(int64_t tiles, int max_split,
-                                                           int64_t k_steps, int64_t slab_elems) {
+                                                           int64_t k_steps, int64_t slab_elems,
+                                                           int resident = 256) {
   const int64_t per_slab = (slab_elems >> 20) > 1 ? (slab_elems >> 20) : 1;
   int pick = 1;
   int64_t best = -1;
   for (int ks = 1; ks <= max_split; ++ks) {
-    const int64_t rounds = (tiles * ks + 255) / 256;
+    const int64_t rounds = (tiles * ks + resident - 1) / resident;
     const int64_t cost = rounds * ((k_steps + ks - 1) / ks + 8) + ks * per_slab;
     if (best < 0 || cost < best) {
       best = cost;

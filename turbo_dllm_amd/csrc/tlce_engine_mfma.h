@@ -56,6 +56,7 @@ struct MfmaTileLayout {
   static constexpr int kCols = kTN;          // tile columns owned per thread
   static constexpr int kRows = kTM * 16;     // tile rows held per owned column
   static constexpr int kShare = 4;           // threads that hold the same column
+  static constexpr int kWavesPerSimd = 1;
   static constexpr bool kPrecise = false;    // hardware exp / rcp approximations in the epilogues
   static_assert(kWavesN * kTN * 32 == kTile, "waves must tile the 256 B rows");
 
@@ -257,6 +258,7 @@ struct DirectTileLayout {
   static constexpr int kRows = kTM * 4;          // tile rows held per owned column
   static constexpr int kShare = 8;               // threads that hold the same column
   static constexpr int kStageCols = 2;           // owned columns per quarter of the tile
+  static constexpr int kWavesPerSimd = 1;
   static constexpr bool kPrecise = false;
 
   struct Acc { acc4_t c[kTM][kTN]; };

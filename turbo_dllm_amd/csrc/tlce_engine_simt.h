@@ -1,5 +1,6 @@
-// 64x64x16 float32-FMA tile engine: the generic path for float32 inputs and for
-// shapes the MFMA engine cannot take (hidden size not a multiple of 8).
+// 64x64x16 float32-FMA tile engine: the generic path for shapes the MFMA engines cannot
+// take (hidden size not a multiple of 8, of 4 for float32) and for float32 vocabularies
+// of fewer than 64 entries.
 //
 // Same contract as MfmaEngine: C[i][j] = sum_k A[i][k] * B[j][k] over one tile,
 // A and B K-contiguous.  256 threads; thread t owns tile column t%64 and the 16
@@ -18,6 +19,7 @@ struct SimtEngine {
   static constexpr int kTile = 64;
   static constexpr int kBK = 16;
   static constexpr int kThreads = 256;
+  static constexpr int kWavesPerSimd = 1;
   static constexpr int kPad = kBK + 1;
   static constexpr int kSmemBytes = 2 * kTile * kPad * 4;  // A and B slabs, float32
   static constexpr int kCols = 1;

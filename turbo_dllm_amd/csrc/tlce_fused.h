@@ -74,7 +74,7 @@ struct ExpPanelArgs {
 // kPlain: the panel receives exp(z - c) itself, without the soft cap's derivative
 // (a forward value, the unnormalised softmax, not a logit gradient).
 template <class E, bool kSoftcap, bool kPlain = false>
-__global__ __launch_bounds__(E::kThreads) void lce_exp_logits_panel_kernel(ExpPanelArgs p) {
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_panel_kernel(ExpPanelArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
   static_assert(E::kHasKMajor && sizeof(T) == 2,

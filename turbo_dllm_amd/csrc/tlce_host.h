@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "tlce_common.h"
+#include "tlce_engine_f32.h"
 #include "tlce_engine_mfma.h"
 #include "tlce_engine_simt.h"
 #include "tlce_kernels.h"
@@ -77,7 +78,7 @@ struct ScopedTimer {
 constexpr int64_t kDefaultPanelBytes = 1ll << 30;
 
 struct Plan {
-  int engine;   // 2 = direct-to-LDS MFMA, 1 = register-staged MFMA, 0 = generic
+  int engine;   // 3 = float32 MFMA, 2 = direct-to-LDS MFMA, 1 = register-staged MFMA, 0 = generic
   bool kmajor;  // gradient contractions read K-major operands in place
   int tile;
   int bk;
@@ -91,22 +92,27 @@ struct Plan {
 };
 
 inline int engine_class(int64_t h, int dtype) {
-  if (dtype == TLCE_DTYPE_F32 || (h % 8) != 0) return 0;
+  if (dtype == TLCE_DTYPE_F32) return (h % 4) == 0 ? 3 : 0;
+  if ((h % 8) != 0) return 0;
   return (h % 64) == 0 ? 2 : 1;
 }
 
 inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_grad,
-               int64_t panel_bytes, int max_engine = 2) {
+               int64_t panel_bytes, int max_engine = 3) {
   Plan p;
-  // 2: four-wave direct-to-LDS MFMA (h % 64 == 0), 1: register-staged MFMA
-  // (h % 8 == 0), 0: generic float32-FMA tiles
+  // 16-bit inputs: 2: four-wave direct-to-LDS MFMA (h % 64 == 0), 1: register-staged MFMA
+  // (h % 8 == 0); float32: 3: float32 MFMA (h % 4 == 0); 0: generic float32-FMA tiles
   p.engine = std::min(engine_class(h, dtype), max_engine);
+  // a float32 vocabulary that one generic tile holds would leave most of a 128x128 tile
+  // and of its matrix instructions empty (both take about 10 us there)
+  if (p.engine == 3 && v < 64) p.engine = 0;
   // The direct engine reads weight, hidden and the logit-gradient panel in
   // their stored form for the gradient contractions (no transposed copies) as
-  // long as every 64-row K slab of weight exists.
-  p.kmajor = (p.engine == 2) && (v % 64) == 0;
-  p.tile = p.engine ? 256 : 64;
-  p.bk = p.engine ? 64 : 16;
+  // long as every 64-row K slab of weight exists; the float32 engine always does (it
+  // takes what is past the K range as zeros).
+  p.kmajor = p.engine == 3 || ((p.engine == 2) && (v % 64) == 0);
+  p.tile = p.engine == 3 ? 128 : p.engine ? 256 : 64;
+  p.bk = p.engine == 3 ? 32 : p.engine ? 64 : 16;
   const int64_t mm = std::max<int64_t>(m, 1);
   p.mp = round_up(mm, p.tile);
   p.vp = round_up(v, p.tile);
@@ -114,7 +120,7 @@ inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_gr
   p.n_vtiles = (int)(p.vp / p.tile);
   p.n_htiles = (int)ceil_div(h, p.tile);
   // forward: token tiles x vocabulary splits workgroups, whole rounds of 256
-  p.nsplit = forward_vocab_splits(p.n_ttiles, p.n_vtiles);
+  p.nsplit = forward_vocab_splits(p.n_ttiles, p.n_vtiles, resident_workgroups(p.tile));
   if (panel_bytes <= 0) panel_bytes = kDefaultPanelBytes;
   const int64_t col_bytes = p.mp * dtype_bytes(dtype) * ((weight_grad && !p.kmajor) ? 2 : 1);
   int64_t tiles_per_panel = std::max<int64_t>(1, panel_bytes / col_bytes / p.tile);
@@ -140,7 +146,7 @@ inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_gr
   if (p.engine) {
     p.dh_max_ksplit = (int)std::max<int64_t>(1, std::min<int64_t>(16, p.vc / p.bk / 8));
     p.dh_ksplit = grad_hidden_k_splits((int64_t)p.n_ttiles * p.n_htiles, p.dh_max_ksplit,
-                                       p.vc / p.bk, p.mp * h);
+                                       p.vc / p.bk, p.mp * h, resident_workgroups(p.tile));
   }
   return p;
 }
@@ -201,7 +207,7 @@ inline BackwardLayout backward_layout(const Plan& p, int64_t m, int64_t h, int d
   l.ht = off;
   if (weight_grad) {
     if (!p.kmajor) off += align256(h * p.mp * es);
-    else if (m % 64 != 0) off += align256(round_up(m, 64) * h * es);
+    else if (p.engine == 2 && m % 64 != 0) off += align256(round_up(m, 64) * h * es);
   }
   l.g = off;     off += align256(p.mp * p.vc * es);
   l.gt = off;    off += (weight_grad && !p.kmajor) ? align256(p.vc * p.mp * es) : 0;
@@ -329,7 +335,7 @@ int launch_gemm(GemmArgs a, int ksplit, int cls, hipStream_t stream) {
   static LdsOptIn lds;
   if (int rc = enable_large_lds(lce_gemm_nt_kernel<E, kAKMajor, kBKMajor>, E::kSmemBytes, lds))
     return rc;
-  const int ksteps = a.k / E::kBK;
+  const int ksteps = (int)ceil_div(a.k, E::kBK);
   a.k_per_split = (int)ceil_div(ksteps, ksplit) * E::kBK;
   // ksplit is the number of splits launched; with a device-side row count the
   // kernel may use fewer of them (a.slab_budget then bounds splits x slab)
@@ -447,7 +453,9 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
   const T* hidden_t = static_cast<const T*>(hidden);
   const T* weight_t = static_cast<const T*>(weight);
   const T* hidden_k = hidden_t;          // K-major operand of grad_weight
-  const int64_t m64 = round_up(m, 64);
+  // the direct engine takes whole 64-row K slabs, the float32 engine any K
+  constexpr int kSlab = sizeof(T) == 2 ? 64 : 1;
+  const int64_t m64 = round_up(m, kSlab);
   if (!p.kmajor) {
     // K-contiguous copies for engines that cannot read K-major operands
     if (int rc = launch_transpose<T>(weight_t, h, v, h, wt, p.vp, p.vp, stream)) return rc;
@@ -496,7 +504,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
         // The head is stored [h, v].  grad_hidden: A = its columns [v0, v0+K), which
         // are K-contiguous rows of the stored matrix; B = G.
         dh.a = weight_t + v0; dh.lda = v; dh.a_rows = (int)h;
-        dh.k = (int)round_up(rows_valid, 64);
+        dh.k = (int)round_up(rows_valid, kSlab);
         if (int rc = launch_gemm<E, false, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
           return rc;
         if (weight_grad) {
@@ -516,7 +524,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
       if (p.kmajor) {
         // grad_hidden: A = weight rows [v0, v0+K) as stored (K-major), B = G
         dh.a = weight_t + v0 * h; dh.lda = h; dh.a_rows = (int)h;
-        dh.k = (int)round_up(rows_valid, 64);
+        dh.k = (int)round_up(rows_valid, kSlab);
         if (int rc = launch_gemm<E, true, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
           return rc;
         if (weight_grad) {

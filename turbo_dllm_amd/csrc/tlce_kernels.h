@@ -44,13 +44,13 @@ struct ForwardArgs {
 // (fused_linear_ce.cpp:104 `weight_dim_first`) and read in place as a K-major
 // operand, K = the hidden axis; v is then a multiple of 8.
 template <class E, bool kSoftcap, bool kBias, bool kWDimFirst = false>
-__global__ __launch_bounds__(E::kThreads) void lce_forward_stats_kernel(ForwardArgs p) {
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_forward_stats_kernel(ForwardArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
   if (p.m_dev != nullptr) {
     p.m = effective_rows(p.m, p.m_dev);
     p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
-    p.nsplit = forward_vocab_splits(p.n_ttiles, p.n_vtiles);
+    p.nsplit = forward_vocab_splits(p.n_ttiles, p.n_vtiles, resident_workgroups(E::kTile));
     p.part_ld = p.n_ttiles * E::kTile;
   }
   const int logical = xcd_logical_block_of(blockIdx.x, p.n_ttiles * p.nsplit);
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(256) void lce_combine_loss_kernel(CombineArgs p) {
   if (p.m_dev != nullptr) {
     p.m = effective_rows(p.m, p.m_dev);
     const int n_ttiles = (p.m + p.tile - 1) / p.tile;
-    p.nsplit = forward_vocab_splits(n_ttiles, p.n_vtiles);
+    p.nsplit = forward_vocab_splits(n_ttiles, p.n_vtiles, resident_workgroups(p.tile));
     p.part_ld = n_ttiles * p.tile;
   }
   int wave_valid = 0;
@@ -394,7 +394,7 @@ __device__ __forceinline__ void stream_store16(void* dst, uint4 v) {
 }
 
 template <class E, bool kSoftcap, bool kBias, bool kWDimFirst = false>
-__global__ __launch_bounds__(E::kThreads) void lce_grad_logits_panel_kernel(GradLogitsArgs p) {
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits_panel_kernel(GradLogitsArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
   if (p.m_dev != nullptr) {
@@ -670,7 +670,7 @@ struct KlPanelArgs {
 };
 
 template <class E, bool kSoftcap, bool kGrad, bool kEmit = false, bool kNoTeacher = false>
-__global__ __launch_bounds__(E::kThreads) void lce_kl_panel_kernel(KlPanelArgs p) {
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_kernel(KlPanelArgs p) {
   static_assert(!(kGrad && kEmit), "kEmit belongs to the loss mode");
   static_assert(kEmit || !kNoTeacher, "kNoTeacher belongs to the emitting pass");
   extern __shared__ __align__(16) char smem[];
@@ -921,7 +921,7 @@ struct LogitsPanelArgs {
 };
 
 template <class E, bool kSoftcap>
-__global__ __launch_bounds__(E::kThreads) void lce_logits_panel_kernel(LogitsPanelArgs p) {
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_logits_panel_kernel(LogitsPanelArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
   int tt, pv;
@@ -944,7 +944,7 @@ __global__ __launch_bounds__(E::kThreads) void lce_logits_panel_kernel(LogitsPan
     }
     return make_float4(z[0], z[1], z[2], z[3]);
   };
-  if constexpr (E::kHasKMajor) {
+  if constexpr (E::kHasKMajor && sizeof(T) == 2) {
     // The float32 tile is twice the engine's LDS: it is staged and written in two
     // halves (the tokens of half the owned column indices = 128 rows of 1 KiB, 16-byte
     // chunk c of staged row s in slot c ^ (s & 63)), so that G leaves in whole
@@ -1138,7 +1138,8 @@ __device__ __forceinline__ int dynamic_k_splits(int n_ttiles, int n_htiles, int 
                                                 int launched, int64_t slab_budget, int k_steps,
                                                 int64_t* stride) {
   const int64_t slab = (int64_t)n_ttiles * tile * h;
-  int ks = grad_hidden_k_splits((int64_t)n_ttiles * n_htiles, launched, k_steps, slab);
+  int ks = grad_hidden_k_splits((int64_t)n_ttiles * n_htiles, launched, k_steps, slab,
+                                resident_workgroups(tile));
   while (ks > 1 && ks * slab > slab_budget) --ks;
   *stride = slab;
   return ks;
@@ -1281,7 +1282,7 @@ __device__ __forceinline__ void store_tile_t_by_rows(const E& eng, const typenam
 }
 
 template <class E, bool kAKMajor, bool kBKMajor>
-__global__ __launch_bounds__(E::kThreads) void lce_gemm_nt_kernel(GemmArgs p) {
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_kernel(GemmArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
   int n_splits = gridDim.y;
@@ -1291,7 +1292,7 @@ __global__ __launch_bounds__(E::kThreads) void lce_gemm_nt_kernel(GemmArgs p) {
       p.nj = (p.c_rows + E::kTile - 1) / E::kTile;
       n_splits = dynamic_k_splits(p.nj, p.ni, E::kTile, (int)p.ldc, (int)gridDim.y,
                                   p.slab_budget, p.k_steps_plan, &p.c_split_stride);
-      p.k_per_split = (p.k / E::kBK + n_splits - 1) / n_splits * E::kBK;
+      p.k_per_split = ((p.k + E::kBK - 1) / E::kBK + n_splits - 1) / n_splits * E::kBK;
     } else if (p.m_role == kKFollows) {
       const int rows = effective_block_rows(p.k, p.m_dev, p.m_dev_offset);
       p.k = (rows + p.m_round - 1) / p.m_round * p.m_round;

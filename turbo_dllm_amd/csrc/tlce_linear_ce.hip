@@ -161,6 +161,7 @@ TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaDirect4Engine<__bf16>)
 TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaDirect4Engine<_Float16>)
 TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaEngine<__bf16>)
 TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaEngine<_Float16>)
+TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaF32Engine)
 TLCE_ENGINE_ENTRY_POINTS(extern template, SimtEngine<float>)
 TLCE_ENGINE_ENTRY_POINTS(extern template, SimtEngine<__bf16>)
 TLCE_ENGINE_ENTRY_POINTS(extern template, SimtEngine<_Float16>)
@@ -171,6 +172,7 @@ using namespace tlce;
 
 #define TLCE_DISPATCH(plan, dtype, CALL)                                                   \
   do {                                                                                     \
+    if ((plan).engine == 3) { using E = MfmaF32Engine; return CALL; }                      \
     if ((plan).engine == 2) {                                                              \
       if ((dtype) == TLCE_DTYPE_BF16) { using E = MfmaDirect4Engine<__bf16>; return CALL; } \
       { using E = MfmaDirect4Engine<_Float16>; return CALL; }                              \
