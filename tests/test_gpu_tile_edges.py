@@ -51,6 +51,23 @@ def test_direct_engine_edges(gpu_device, m, h, v, dtype, mode):
     check(gpu_device, m, h, v, dtype, mode)
 
 
+@pytest.mark.parametrize("mode", options.GRADIENT_MODES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,h,v,kw", [
+    (1, 64, 2, {}),                                 # the tail is the whole K range
+    (65, 64, 63, {}),                               # and holds all but one of its rows
+    (130, 128, 65, dict(exclude_index=64)),         # one slab and a tail of one row
+    (257, 192, 191, {}),                            # two slabs and a tail
+    (300, 256, 4099, dict(logit_softcap=20.0)),     # the tail in the last of the K splits
+    (1030, 320, 32003, {}),                         # two panels of the recomputing backward
+])
+def test_direct_engine_ragged_vocabularies(gpu_device, m, h, v, kw, dtype, mode):
+    """Vocabularies (K of the grad_hidden contraction) and row counts (K of grad_weight)
+    that end inside a 64-row K slab."""
+    with options.panel_budget((32 << 20) if v > 30000 and mode == "recompute" else 0):
+        check(gpu_device, m, h, v, dtype, mode, **kw)
+
+
 @pytest.mark.parametrize("m,h,v,kw", [
     (1, 4, 64, {}),                                 # one piece of one K stage
     (3, 4, 63, {}),                                 # the last vocabulary of the generic engine

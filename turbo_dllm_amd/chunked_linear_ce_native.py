@@ -465,7 +465,7 @@ def forward(
 def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
                               bias: torch.Tensor | None, weight_dim_first: bool) -> bool:
     """Whether ``forward_with_gradients`` takes these operands: bf16 inputs on the
-    GPU, head stored [V, H], no bias, H and V multiples of 64.  (f16's exponent
+    GPU, head stored [V, H], no bias, H a multiple of 64.  (f16's exponent
     range cannot hold exp(logit - reference) and its row sums.)"""
     if bias is not None or weight_dim_first or not hidden.is_cuda:
         return False
@@ -473,7 +473,7 @@ def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
         return False
     if hidden.dim() != 2 or weight.dim() != 2 or weight.shape[1] != hidden.shape[1]:
         return False
-    return bool(_lib.library().tlce_fused_gradients_supported(
+    return bool(_lib.library().tlce_gradients_in_forward_supported(
         hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
 
 
@@ -513,8 +513,8 @@ def forward_with_gradients(
     device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
     if not fused_gradients_supported(hidden, weight, None, False):
         raise RuntimeError(
-            "forward_with_gradients needs bf16 operands, a [V, H] head and H, V multiples "
-            "of 64; use forward / backward for other inputs"
+            "forward_with_gradients needs bf16 operands, a [V, H] head and hidden sizes that "
+            "are multiples of 64; use forward / backward for other inputs"
         )
     hidden = _dense(hidden)
     weight = _dense(weight)
@@ -568,7 +568,7 @@ def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
     """Whether ``forward_with_gradients`` takes ``m`` rows as one block under the
     panel budget in force, so that its grad_weight contraction can be postponed to
     the backward (``grad_weight_from_panel``)."""
-    if dtype != torch.bfloat16 or not _lib.library().tlce_fused_gradients_supported(
+    if dtype != torch.bfloat16 or not _lib.library().tlce_gradients_in_forward_supported(
             h, v, _lib.DTYPE_BF16):
         return False
     return _lib.query_fused_plan(m, h, v, _lib.DTYPE_BF16, get_panel_bytes())["n_blocks"] == 1
@@ -1243,7 +1243,7 @@ def dflash_kl_forward(
 def kl_gradient_in_forward_supported(draft_hidden, draft_weight, teacher_hidden,
                                      logit_softcap: float) -> bool:
     """Whether ``dflash_kl_forward_with_gradient`` takes these operands (bf16, a soft cap
-    between 10 and 40 or none, hidden sizes and V multiples of 64; rows go in blocks of the
+    between 10 and 40 or none, hidden sizes multiples of 64; rows go in blocks of the
     panel budget)."""
     if draft_hidden.dtype != torch.bfloat16 or draft_hidden.shape[0] == 0:
         return False
@@ -1400,7 +1400,7 @@ def dflash_ce_topk_forward(
 
 def ce_topk_gradient_in_forward_supported(hidden: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether ``dflash_ce_topk_forward_with_gradient`` takes these operands: bf16,
-    H and V multiples of 64 (rows are taken in blocks of the panel of exponentiated
+    H a multiple of 64 (rows are taken in blocks of the panel of exponentiated
     logits, 2.5 GiB over the whole vocabulary: 8192 rows at V = 151936)."""
     if hidden.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or hidden.shape[0] == 0:
         return False

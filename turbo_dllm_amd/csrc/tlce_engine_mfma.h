@@ -333,6 +333,12 @@ struct DirectTileLayout {
 // columns 4*(i%4).. of a 4 x 16 block, lane l ends up with 4 consecutive K
 // values of column l: half an MFMA fragment.
 //
+// A K range that ends inside a 64-row slab of a K-major operand (a vocabulary or row
+// count that is no multiple of 64) takes its last tile from a zero-padded copy of those
+// rows: the scalar base of the last tile is another pointer, nothing else changes.
+// Before, such vocabularies went through transposed copies of the head and of the
+// logit-gradient panel and four contractions.
+//
 // Loads use the scalar-base form: tile base and K position live in SGPRs, the
 // per-lane byte offsets (row clamp and slot swizzle folded in) are computed
 // once per tile, so a load costs three scalar instructions and no VALU work.
@@ -372,6 +378,10 @@ struct Operand {
   int64_t ld;     // elements between consecutive stored rows
   int row0;       // first tile row (K-contiguous) or first tile column (K-major)
   int rows;       // valid rows / columns of the matrix; accesses beyond are clamped
+  // K-major: K rows from k_full on (a multiple of 64; the matrix has fewer than 64 more)
+  // are read from `tail`, a [64, ld] copy of them with zero rows after the last.
+  const T* tail = nullptr;
+  int k_full = 0x7fffffff;
 };
 
 template <typename T> struct DirectMfma;
@@ -418,7 +428,7 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
   static constexpr int kSmemBytes = 2 * kStageBytes + kTouchBytes;
   static constexpr int kLoads = 8;                           // per wave, operand and K tile
   static constexpr int kTouchAhead = 2;                      // K tiles
-    static constexpr int kLoadsAfterBarrier = 12;              // of the 16 of both operands
+  static constexpr int kLoadsAfterBarrier = 12;              // of the 16 of both operands
   static constexpr bool kHasKMajor = true;
 
   typedef short v4s_t __attribute__((ext_vector_type(4)));
@@ -464,10 +474,12 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     unsigned fill;          // LDS address of this wave's first piece in stage 0
     const char* next;       // base address of the next K tile to request
     int64_t step;           // bytes between consecutive K tiles
+    const char* last;       // K-major: base address of the last K tile (the operand's tail
+                            // when the K range ends inside a 64-row slab)
   };
 
   template <bool kKMajor>
-  __device__ __forceinline__ Loader make_loader(const Operand<T>& x, int k_begin,
+  __device__ __forceinline__ Loader make_loader(const Operand<T>& x, int k_begin, int nk,
                                                 unsigned lds_op) const {
     Loader ld;
     if (!kKMajor) {
@@ -482,6 +494,7 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
       ld.fill = __builtin_amdgcn_readfirstlane(lds_op + (unsigned)(wave * 64 * 128));
       ld.next = reinterpret_cast<const char*>(x.ptr + (int64_t)x.row0 * x.ld + k_begin);
       ld.step = kBK * 2;
+      ld.last = nullptr;
     } else {
       // this wave fills K rows [16w, 16w+16) of the slab, two rows per instruction
       const int last_chunk = x.rows / 8 - 1 - x.row0 / 8;   // relative to the tile
@@ -493,7 +506,11 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
         ld.off[j] = (unsigned)((int64_t)kr * x.ld * 2 + chunk * 16);
       }
       ld.fill = __builtin_amdgcn_readfirstlane(lds_op + (unsigned)(wave * 16 * 512));
-      ld.next = reinterpret_cast<const char*>(x.ptr + (int64_t)k_begin * x.ld + x.row0);
+      const int k_last = k_begin + (nk - 1) * kBK;
+      ld.last = reinterpret_cast<const char*>(
+          (k_last >= x.k_full ? x.tail : x.ptr + (int64_t)k_last * x.ld) + x.row0);
+      ld.next = nk == 1 ? ld.last
+                        : reinterpret_cast<const char*>(x.ptr + (int64_t)k_begin * x.ld + x.row0);
       ld.step = (int64_t)kBK * x.ld * 2;
     }
     return ld;
@@ -550,8 +567,8 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
   // acc += A-tile * B-tile^T over K in [k_begin, k_end), a multiple of 64 wide.
   // K-contiguous operand: tile rows row0 .. row0+256 of x (rows clamped to
   // x.rows - 1).  K-major operand: tile columns row0 .. row0+256 of x (16-byte
-  // column chunks clamped to the last valid one; x.rows is a multiple of 8);
-  // all K rows in [k_begin, k_end) must exist.
+  // column chunks clamped to the last valid one; x.rows is a multiple of 8); the K
+  // rows in [k_begin, k_end) must exist up to k_full, and in the tail from there on.
   // kOverwrite: acc = A-tile * B-tile^T instead (the incoming acc is ignored: the
   // first 64 MFMAs take a zero constant as their addend, which saves zeroing
   // 256 accumulator registers per tile).
@@ -560,8 +577,14 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
                                               int k_begin, int k_end, Acc& acc,
                                               char* smem) const {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
-    Loader la = make_loader<kAKMajor>(A, k_begin, lds0);
-    Loader lb = make_loader<kBKMajor>(B, k_begin, lds0 + kOperandBytes);
+    const int nk = (k_end - k_begin) / kBK;
+    Loader la = make_loader<kAKMajor>(A, k_begin, nk, lds0);
+    Loader lb = make_loader<kBKMajor>(B, k_begin, nk, lds0 + kOperandBytes);
+    // the loaders move on to K tile `k`
+    auto advance = [&](int k) {
+      la.next = kAKMajor && k == nk - 1 ? la.last : la.next + la.step;
+      lb.next = kBKMajor && k == nk - 1 ? lb.last : lb.next + lb.step;
+    };
     const int ra = reader_base<kAKMajor>(wm);
     const int rb = reader_base<kBKMajor>(wn);
 
@@ -580,7 +603,6 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
       fb[ks][i] = read_frag<kBKMajor>(smem + stage * kStageBytes + kOperandBytes, rb, ks, i);
     };
 
-    const int nk = (k_end - k_begin) / kBK;
     // This wave's share of the touches: 64 lines of A (waves 0, 1) or B (waves 2, 3), in
     // the half of the tile's lines that the workgroup's neighbours leave to it.
     const bool touch_b = wave >= 2;
@@ -592,8 +614,11 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
         readfirstlane64(reinterpret_cast<int64_t>(touch_b ? lb.next : la.next)));
     const unsigned touch_lds =
         __builtin_amdgcn_readfirstlane(lds0 + 2 * kStageBytes + (unsigned)wave * 256);
+    // (a tail is small and in L2 already; the tile before it is touched again)
+    const bool ragged = touch_b ? kBKMajor && k_end > B.k_full : kAKMajor && k_end > A.k_full;
+    const int touch_last = __builtin_amdgcn_readfirstlane(nk - 1 - (ragged ? 1 : 0));
     auto touch_tile = [&](int k) {
-      touch(touch_lds, touch_off, touch_base + (int64_t)min(k, nk - 1) * touch_step);
+      touch(touch_lds, touch_off, touch_base + (int64_t)min(k, touch_last) * touch_step);
     };
     // tiles_left: how many tiles follow (0, 1, or 2 for "two or more")
     auto step = [&](int k, auto tiles_left_tag, auto first_tag) {
@@ -615,8 +640,7 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
           // (the one younger access is the touch of this step)
           asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
           __syncthreads();
-          la.next += la.step;
-          lb.next += lb.step;
+          if (kHasTwo) advance(k + 2);
         }
 #pragma unroll
         for (int t = 0; t < kTN; ++t) {
@@ -658,9 +682,8 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     for (int q = 0; q < 16; ++q) issue_one(0, q);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    la.next += la.step;
-    lb.next += lb.step;
     if (nk > 1) {
+      advance(1);
 #pragma unroll
       for (int q = 0; q < kLoadsAfterBarrier; ++q) issue_one(1, q);
     }

@@ -327,6 +327,7 @@ int launch_scale_cast(const ScaleCastArgs& a, hipStream_t stream);
 
 // ------------------------------------------------------------------- plan ----
 struct FusedPlan {
+  int64_t v;
   int64_t vp;           // panel columns: the vocabulary rounded up to whole tiles
   int n_vtiles, n_htiles;
   int64_t block_rows;   // rows per block, a multiple of the tile
@@ -334,12 +335,17 @@ struct FusedPlan {
   int dh_ksplit;        // K splits of the grad_hidden contraction of a full block
 };
 
-inline bool fused_gradients_supported(int64_t h, int64_t v, int dtype) {
-  return dtype == TLCE_DTYPE_BF16 && engine_class(h, dtype) == 2 && (v % 64) == 0;
+// Any vocabulary: the contraction over it takes the rows of an incomplete last 64-row
+// slab from a padded copy (k_tail_bytes).  Against the recomputing sequence, which alone
+// took vocabularies that are no multiple of 64 before: 2741 rows, H = 2048, V = 32003
+// 1.56 -> 1.08 ms a step (three contractions, no transposed copies).
+inline bool gradients_in_forward_supported(int64_t h, int dtype) {
+  return dtype == TLCE_DTYPE_BF16 && engine_class(h, dtype) == 2;
 }
 
 inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int64_t panel_bytes) {
   FusedPlan p;
+  p.v = v;
   const int64_t tile = 256;
   p.vp = round_up(v, tile);
   p.n_vtiles = (int)(p.vp / tile);
@@ -364,7 +370,7 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
 
 struct FusedLayout {
   int64_t panel, part_sum, part_max, target, ref, ref_next, row_scale, scaled_hidden, slabs,
-      redo, total;
+      redo, k_tail, total;
 };
 
 inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dtype,
@@ -384,8 +390,25 @@ inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dt
   if (weight_grad) off += align256(p.block_rows * h * es);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
   l.redo = off;       off += align256((int64_t)p.n_blocks * 4);
+  l.k_tail = off;     off += k_tail_bytes(p.v, h);
   l.total = off;
   return l;
+}
+
+// The head as the K-major operand of a contraction over the vocabulary.  `k_tail`: where
+// prepare_k_tail has put the rows of an incomplete last slab.
+inline int prepare_k_tail(const void* weight, int64_t v, int64_t h, char* k_tail,
+                          hipStream_t stream) {
+  return v % 64 != 0 ? launch_k_tail(weight, v, h, k_tail, stream) : 0;
+}
+inline void set_head_operand(GemmArgs& g, const void* weight, int64_t v, int64_t h,
+                             const char* k_tail) {
+  g.a = weight; g.lda = h; g.a_rows = (int)h;
+  g.k = (int)round_up(v, 64);
+  if (g.k != v) {
+    g.a_tail = k_tail;
+    g.a_k_full = g.k - 64;
+  }
 }
 
 // Options of the fused sequence beyond the operator's own arguments.
@@ -427,6 +450,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
   la.ignore = ignore; la.exclude = exclude; la.softcap = softcap; la.logit_scale = opt.logit_scale;
   la.target = target; la.ref = ref; la.valid_count = valid_count; la.m_dev = m_dev;
   if (int rc = launch_label_logit(la, stream)) return rc;
+  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
 
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
@@ -478,9 +502,8 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
 
     // grad_hidden of the block: A = weight as stored (K-major, K = vocabulary), B = panel
     GemmArgs dh;
-    dh.a = weight; dh.lda = h; dh.a_rows = (int)h;
+    set_head_operand(dh, weight, v, h, ws + l.k_tail);
     dh.b = panel; dh.ldb = p.vp; dh.b_rows = (int)rows_p;
-    dh.k = (int)round_up(v, 64);
     dh.k_per_split = 0;
     dh.ni = p.n_htiles; dh.nj = n_ttiles;
     dh.c = slabs; dh.ldc = h; dh.c_rows = (int)rows_p; dh.c_cols = (int)h;
@@ -584,6 +607,7 @@ int soft_embedding_fused_impl(const FusedPlan& p, const void* hidden, const void
   float* row_scale = reinterpret_cast<float*>(ws + l.row_scale);
   float* slabs = reinterpret_cast<float*>(ws + l.slabs);
   const T* hidden_t = static_cast<const T*>(hidden);
+  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
     const int64_t rows = std::min<int64_t>(p.block_rows, m - r0);
@@ -610,9 +634,9 @@ int soft_embedding_fused_impl(const FusedPlan& p, const void* hidden, const void
     // the contraction of grad_hidden in the forward that leaves the gradients: K = the
     // vocabulary, K splits into slabs for few rows
     GemmArgs g;
-    g.a = weight; g.lda = h; g.a_rows = (int)h;
+    set_head_operand(g, weight, v, h, ws + l.k_tail);
     g.b = panel; g.ldb = p.vp; g.b_rows = (int)rows_p;
-    g.k = (int)round_up(v, 64); g.k_per_split = 0;
+    g.k_per_split = 0;
     g.ni = p.n_htiles; g.nj = n_ttiles;
     g.c = slabs; g.ldc = h; g.c_rows = (int)rows_p; g.c_cols = (int)h;
     g.c_split_stride = p.block_rows * h;
@@ -678,7 +702,7 @@ int launch_topk_row_scale(const TopkRowScaleArgs& a, hipStream_t stream);
 int launch_topk_apply(const TopkApplyArgs& a, hipStream_t stream);
 
 struct TopkFusedLayout {
-  int64_t forward, panel, ref_used, row_scale, slabs, total;
+  int64_t forward, panel, ref_used, row_scale, slabs, k_tail, total;
 };
 
 // Rows are taken in blocks of the panel budget of the forward that leaves the gradients
@@ -686,7 +710,8 @@ struct TopkFusedLayout {
 // so a block is a call of its own on a part of every per-row buffer.
 inline bool topk_gradient_in_forward_supported(int64_t m, int64_t h, int64_t v, int dtype) {
   (void)m;
-  return fused_gradients_supported(h, v, dtype);
+  (void)v;
+  return gradients_in_forward_supported(h, dtype);
 }
 
 // Rows per block of the objectives that take whole blocks of rows one after the other.
@@ -702,6 +727,7 @@ inline TopkFusedLayout topk_fused_layout(const TopkPlan& t, const FusedPlan& p, 
   l.ref_used = off;   off += align256((int64_t)t.n_fpanels * p.block_rows * 4);
   l.row_scale = off;  off += align256(p.block_rows * 4);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
+  l.k_tail = off;     off += k_tail_bytes(p.v, h);
   l.total = off;
   return l;
 }
@@ -741,10 +767,11 @@ int topk_forward_with_gradient_impl(const TopkPlan& t, const FusedPlan& p, const
   sa.row_scale = row_scale;
   if (int rc = launch_topk_row_scale(sa, stream)) return rc;
 
+  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
   GemmArgs g;
-  g.a = weight; g.lda = h; g.a_rows = (int)h;
+  set_head_operand(g, weight, v, h, ws + l.k_tail);
   g.b = panel; g.ldb = p.vp; g.b_rows = m_pad;
-  g.k = (int)round_up(v, 64); g.k_per_split = 0;
+  g.k_per_split = 0;
   g.ni = p.n_htiles; g.nj = m_pad / E::kTile;
   g.c = slabs; g.ldc = h; g.c_rows = m_pad; g.c_cols = (int)h;
   g.c_split_stride = p.block_rows * h;
@@ -808,7 +835,7 @@ int launch_kl_grad_from_exp(const KlGradFromExpArgs& a, int n_vtiles, hipStream_
 constexpr float kKlMinCap = 10.0f;
 
 struct KlFusedLayout {
-  int64_t kl, teacher_parts, teacher, exp_panel, slabs, total;
+  int64_t kl, teacher_parts, teacher, exp_panel, slabs, k_tail, total;
 };
 
 template <class E, bool kSoftcap, bool kNoTeacher>
@@ -846,7 +873,8 @@ inline bool kl_gradient_in_forward_supported(int64_t m, int64_t hd, int64_t ht, 
   // left (measured: 2 % of the gradient's largest entry at cap 3): caps below 10 keep the
   // sequence that evaluates cap' on the float32 logit
   const bool cap_ok = softcap <= 0.0f || (softcap >= kKlMinCap && softcap <= kSoftEmbeddingMaxCap);
-  return cap_ok && fused_gradients_supported(hd, v, dtype) && engine_class(ht, dtype) == 2;
+  (void)v;
+  return cap_ok && gradients_in_forward_supported(hd, dtype) && engine_class(ht, dtype) == 2;
 }
 
 inline KlFusedLayout kl_fused_layout(const KlLayout& kl, const Plan& pd, const FusedPlan& p,
@@ -858,6 +886,7 @@ inline KlFusedLayout kl_fused_layout(const KlLayout& kl, const Plan& pd, const F
   l.teacher = off;    off += align256(pd.mp * pd.vp * 2);
   l.exp_panel = off;  off += align256(pd.mp * pd.vp * 2);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * pd.mp * hd * 4);
+  l.k_tail = off;     off += k_tail_bytes(p.v, hd);
   l.total = off;
   return l;
 }
@@ -944,10 +973,11 @@ int kl_forward_with_gradient_impl(const Plan& pd, const Plan& pt, const KlLayout
   ga.t_part_max = t_part_max; ga.t_lse = teacher_lse;
   if (int rc = launch_kl_grad_from_exp(ga, pd.n_vtiles, stream)) return rc;
 
+  if (int rc = prepare_k_tail(draft_weight, v, hd, ws + l.k_tail, stream)) return rc;
   GemmArgs g;
-  g.a = draft_weight; g.lda = hd; g.a_rows = (int)hd;
+  set_head_operand(g, draft_weight, v, hd, ws + l.k_tail);
   g.b = exp_panel; g.ldb = pd.vp; g.b_rows = (int)pd.mp;
-  g.k = (int)round_up(v, 64); g.k_per_split = 0;
+  g.k_per_split = 0;
   g.ni = fp.n_htiles; g.nj = (int)(pd.mp / E::kTile);
   g.c = slabs; g.ldc = hd; g.c_rows = (int)pd.mp; g.c_cols = (int)hd;
   g.c_split_stride = pd.mp * hd;
@@ -978,6 +1008,7 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
   float* row_scale = reinterpret_cast<float*>(ws + l.row_scale);
   float* slabs = reinterpret_cast<float*>(ws + l.slabs);
   const T* hidden_t = static_cast<const T*>(hidden);
+  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
     const int64_t rows = std::min<int64_t>(p.block_rows, m - r0);
@@ -1009,9 +1040,9 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
     if (int rc = launch_kl_grad_from_exp(ga, p.n_vtiles, stream)) return rc;
 
     GemmArgs g;
-    g.a = weight; g.lda = h; g.a_rows = (int)h;
+    set_head_operand(g, weight, v, h, ws + l.k_tail);
     g.b = panel; g.ldb = p.vp; g.b_rows = (int)rows_p;
-    g.k = (int)round_up(v, 64); g.k_per_split = 0;
+    g.k_per_split = 0;
     g.ni = p.n_htiles; g.nj = n_ttiles;
     g.c = slabs; g.ldc = h; g.c_rows = (int)rows_p; g.c_cols = (int)h;
     g.c_split_stride = p.block_rows * h;

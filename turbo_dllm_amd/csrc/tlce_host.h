@@ -78,6 +78,7 @@ struct ScopedTimer {
 constexpr int64_t kDefaultPanelBytes = 1ll << 30;
 
 struct Plan {
+  int64_t v;    // vocabulary rows
   int engine;   // 3 = float32 MFMA, 2 = direct-to-LDS MFMA, 1 = register-staged MFMA, 0 = generic
   bool kmajor;  // gradient contractions read K-major operands in place
   int tile;
@@ -100,17 +101,18 @@ inline int engine_class(int64_t h, int dtype) {
 inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_grad,
                int64_t panel_bytes, int max_engine = 3) {
   Plan p;
+  p.v = v;
   // 16-bit inputs: 2: four-wave direct-to-LDS MFMA (h % 64 == 0), 1: register-staged MFMA
   // (h % 8 == 0); float32: 3: float32 MFMA (h % 4 == 0); 0: generic float32-FMA tiles
   p.engine = std::min(engine_class(h, dtype), max_engine);
   // a float32 vocabulary that one generic tile holds would leave most of a 128x128 tile
   // and of its matrix instructions empty (both take about 10 us there)
   if (p.engine == 3 && v < 64) p.engine = 0;
-  // The direct engine reads weight, hidden and the logit-gradient panel in
-  // their stored form for the gradient contractions (no transposed copies) as
-  // long as every 64-row K slab of weight exists; the float32 engine always does (it
-  // takes what is past the K range as zeros).
-  p.kmajor = p.engine == 3 || ((p.engine == 2) && (v % 64) == 0);
+  // The direct and the float32 engine read weight, hidden and the logit-gradient panel
+  // in their stored form for the gradient contractions (no transposed copies).  The
+  // direct one takes whole 64-row K slabs: of a last, incomplete slab of weight or
+  // hidden a zero-padded copy is made (launch_k_tail).
+  p.kmajor = p.engine >= 2;
   p.tile = p.engine == 3 ? 128 : p.engine ? 256 : 64;
   p.bk = p.engine == 3 ? 32 : p.engine ? 64 : 16;
   const int64_t mm = std::max<int64_t>(m, 1);
@@ -194,21 +196,24 @@ inline ForwardLayout forward_layout(const Plan& p, bool dynamic_rows = false,
 struct BackwardLayout {
   int64_t scale, acc32, wt, ht, g, gt, total;
 };
-// wt / gt exist only on the transposed-copy path; ht is hidden^T there and, on
-// the K-major path, a copy of hidden padded to a multiple of 64 rows (only when
-// m is not one already).
+// Bytes of the zero-padded copy of a 16-bit [rows, h] matrix's last K slab that a
+// direct-engine contraction over its rows needs (none: all slabs are whole).
+inline int64_t k_tail_bytes(int64_t rows, int64_t h) {
+  return rows % 64 != 0 ? align256(64 * h * 2) : 0;
+}
+
+// wt / ht / gt are transposed copies on the path of the engines without K-major
+// operands; on the direct engine's path wt and ht are the K tails of weight and hidden.
 inline BackwardLayout backward_layout(const Plan& p, int64_t m, int64_t h, int dtype, bool weight_grad) {
   BackwardLayout l;
   const int64_t es = dtype_bytes(dtype);
   int64_t off = 0;
   l.scale = off; off += align256(p.mp * 4);
   l.acc32 = off; off += align256(p.mp * h * 4 * p.dh_ksplit);   // one slab per K split
-  l.wt = off;    off += p.kmajor ? 0 : align256(h * p.vp * es);
+  const bool direct = p.engine == 2;
+  l.wt = off;    off += direct ? k_tail_bytes(p.v, h) : p.kmajor ? 0 : align256(h * p.vp * es);
   l.ht = off;
-  if (weight_grad) {
-    if (!p.kmajor) off += align256(h * p.mp * es);
-    else if (p.engine == 2 && m % 64 != 0) off += align256(round_up(m, 64) * h * es);
-  }
+  if (weight_grad) off += direct ? k_tail_bytes(m, h) : p.kmajor ? 0 : align256(h * p.mp * es);
   l.g = off;     off += align256(p.mp * p.vc * es);
   l.gt = off;    off += (weight_grad && !p.kmajor) ? align256(p.vc * p.mp * es) : 0;
   l.total = off;
@@ -362,6 +367,7 @@ int launch_transpose(const T* in, int64_t ld_in, int64_t rows, int64_t cols, T* 
 // Launchers of the engine-independent kernels (tlce_row_kernels.h), defined
 // beside the C ABI.
 int fill_zero(void* dst, int64_t bytes, hipStream_t stream);
+int launch_k_tail(const void* matrix, int64_t rows, int64_t h, void* tail, hipStream_t stream);
 int launch_token_scale(const ScaleArgs& sa, hipStream_t stream);
 int launch_kl_finish(float* losses, const float* loss_part, const float* tsum_part, int n_tiles,
                      int64_t part_ld, const float* lse, int64_t m, hipStream_t stream);
@@ -452,7 +458,6 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
 
   const T* hidden_t = static_cast<const T*>(hidden);
   const T* weight_t = static_cast<const T*>(weight);
-  const T* hidden_k = hidden_t;          // K-major operand of grad_weight
   // the direct engine takes whole 64-row K slabs, the float32 engine any K
   constexpr int kSlab = sizeof(T) == 2 ? 64 : 1;
   const int64_t m64 = round_up(m, kSlab);
@@ -463,12 +468,14 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
       if (int rc = launch_transpose<T>(hidden_t, h, m, h, ht, p.mp, p.mp, stream, m_dev))
         return rc;
     }
-  } else if (weight_grad && m64 != m && m_dev == nullptr) {
-    // whole 64-row K slabs must exist: pad hidden with zero rows
-    TLCE_HIP(hipMemcpyAsync(ht, hidden_t, (size_t)(m * h * sizeof(T)), hipMemcpyDeviceToDevice,
-                            stream));
-    if (int rc = fill_zero(ht + m * h, (m64 - m) * h * (int64_t)sizeof(T), stream)) return rc;
-    hidden_k = ht;
+  } else {
+    if (v % kSlab != 0) {
+      if (int rc = launch_k_tail(weight_t, v, h, wt, stream)) return rc;
+    }
+    // (with a device-side row count the caller's buffer holds the padding rows)
+    if (weight_grad && m_dev == nullptr && m % kSlab != 0) {
+      if (int rc = launch_k_tail(hidden_t, m, h, ht, stream)) return rc;
+    }
   }
 
   for (int panel = 0; panel < p.n_panels; ++panel) {
@@ -512,8 +519,12 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
           // becomes the output's rows: A = G (its panel columns), B = hidden, both K-major
           GemmArgs dwt = dw;
           dwt.a = g; dwt.lda = p.vc; dwt.a_rows = (int)width;
-          dwt.b = hidden_k; dwt.ldb = h; dwt.b_rows = (int)h;
+          dwt.b = hidden_t; dwt.ldb = h; dwt.b_rows = (int)h;
           dwt.k = (int)m64;
+          if (m64 != m && m_dev == nullptr) {
+            dwt.b_tail = ht;
+            dwt.b_k_full = (int)(m64 - kSlab);
+          }
           dwt.ni = (int)(width / p.tile); dwt.nj = p.n_htiles;
           dwt.c = static_cast<T*>(grad_weight) + v0; dwt.ldc = v;
           dwt.c_rows = (int)h; dwt.c_cols = (int)rows_valid;
@@ -525,13 +536,21 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
         // grad_hidden: A = weight rows [v0, v0+K) as stored (K-major), B = G
         dh.a = weight_t + v0 * h; dh.lda = h; dh.a_rows = (int)h;
         dh.k = (int)round_up(rows_valid, kSlab);
+        if (dh.k != rows_valid) {
+          dh.a_tail = wt;
+          dh.a_k_full = dh.k - kSlab;
+        }
         if (int rc = launch_gemm<E, true, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
           return rc;
         if (weight_grad) {
           // grad_weight: A = hidden as stored, B = G as stored, both K-major (K = token)
-          dw.a = hidden_k; dw.lda = h; dw.a_rows = (int)h;
+          dw.a = hidden_t; dw.lda = h; dw.a_rows = (int)h;
           dw.b = g; dw.ldb = p.vc; dw.b_rows = (int)width;
           dw.k = (int)m64;
+          if (m64 != m && m_dev == nullptr) {
+            dw.a_tail = ht;
+            dw.a_k_full = (int)(m64 - kSlab);
+          }
           if (int rc = launch_gemm<E, true, true>(dw, 1, kClassGradWeight, stream)) return rc;
         }
         continue;

@@ -492,7 +492,6 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
   };
 
   T* g_out = static_cast<T*>(p.g);
-  T* gt_out = static_cast<T*>(p.gt);
   const int prow = pv * E::kTile;  // first panel column of this tile
   if constexpr (E::kHasKMajor && sizeof(T) == 2) {
     // The MFMA engine's LDS is free after the main loop: the tile is staged there
@@ -553,17 +552,6 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
     } else {
       emit(std::false_type{}, std::false_type{});
     }
-    if (gt_out != nullptr) {
-      // transposed copy for the contractions that cannot read G K-major (vocabulary
-      // not a multiple of 64): the whole tile is still staged; thread = token
-      const int tok = threadIdx.x % E::kTile;
-      for (int vrow = threadIdx.x / E::kTile; vrow < E::kTile; vrow += E::kThreads / E::kTile) {
-        const T val = *reinterpret_cast<const T*>(smem + tok * 512 +
-                                                  (((vrow >> 3) ^ (tok & 31)) * 16) +
-                                                  (vrow & 7) * 2);
-        gt_out[(int64_t)(prow + vrow) * p.ldgt + (int64_t)tt * E::kTile + tok] = val;
-      }
-    }
   } else {
     auto transform = [&](auto edge_tag, auto onehot_tag) {
       constexpr bool kEdge = decltype(edge_tag)::value;
@@ -598,6 +586,8 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
                   E::get(acc, j, i + 1), E::get(acc, j, i + 2), E::get(acc, j, i + 3));
       }
     }
+    // transposed copy for the contractions of the engines that cannot read G K-major
+    T* gt_out = static_cast<T*>(p.gt);
     if (gt_out != nullptr) {
 #pragma unroll
       for (int j = 0; j < E::kCols; ++j) {
@@ -1129,6 +1119,11 @@ struct GemmArgs {
   int64_t m_dev_offset = 0;  // the operand's first token row is row m_dev_offset of the counted rows
   int64_t slab_budget = 0;   // kRowsFollow: float32 elements all K-split slabs may take
   int k_steps_plan = 0;      // kRowsFollow: K steps of a full panel, what the split rule plans on
+  // K-major operands whose K rows end inside a 64-row slab (Operand::tail)
+  const void* a_tail = nullptr;
+  int a_k_full = 0x7fffffff;
+  const void* b_tail = nullptr;
+  int b_k_full = 0x7fffffff;
 };
 
 // K splits and slab stride the grad_hidden contraction uses for a device-side
@@ -1336,8 +1331,10 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
   if (k_begin >= k_end) {
     E::zero(acc);   // nothing to accumulate
   } else if constexpr (E::kHasKMajor) {
-    const Operand<T> a = {static_cast<const T*>(p.a), p.lda, ti * E::kTile, p.a_rows};
-    const Operand<T> b = {static_cast<const T*>(p.b), p.ldb, tj * E::kTile, p.b_rows};
+    const Operand<T> a = {static_cast<const T*>(p.a), p.lda, ti * E::kTile, p.a_rows,
+                          static_cast<const T*>(p.a_tail), p.a_k_full};
+    const Operand<T> b = {static_cast<const T*>(p.b), p.ldb, tj * E::kTile, p.b_rows,
+                          static_cast<const T*>(p.b_tail), p.b_k_full};
     eng.template mainloop_ex<kAKMajor, kBKMajor, true>(a, b, k_begin, k_end, acc, smem);
   } else {
     eng.mainloop_set(static_cast<const T*>(p.a), p.lda, ti * E::kTile, p.a_rows,

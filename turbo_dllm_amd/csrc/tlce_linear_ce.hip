@@ -37,6 +37,19 @@ int fill_zero(void* dst, int64_t bytes, hipStream_t stream) {
   return 0;
 }
 
+// `tail` [64, h] receives the last rows % 64 rows of a 16-bit [rows, h] matrix (h a
+// multiple of 8) and zero rows: what a contraction over the rows reads as its last slab.
+int launch_k_tail(const void* matrix, int64_t rows, int64_t h, void* tail, hipStream_t stream) {
+  const int64_t kept = rows % 64;
+  const int n16 = (int)(64 * h / 8);
+  ScopedTimer timer(kClassOther, stream);
+  lce_k_tail_kernel<<<(int)ceil_div(n16, 256), 256, 0, stream>>>(
+      reinterpret_cast<const uint4*>(static_cast<const char*>(matrix) + (rows - kept) * h * 2),
+      (int)(kept * h / 8), static_cast<uint4*>(tail), n16);
+  TLCE_LAUNCH_CHECK();
+  return 0;
+}
+
 int launch_token_scale(const ScaleArgs& sa, hipStream_t stream) {
   ScopedTimer timer(kClassOther, stream);
   lce_token_scale_kernel<<<(int)ceil_div(sa.mp, 256), 256, 0, stream>>>(sa);
@@ -537,7 +550,7 @@ extern "C" int64_t tlce_soft_embedding_workspace_bytes(int64_t m, int64_t h, int
   const Plan bp = make_plan(m, h, v, dtype, false, panel_bytes);
   int64_t need = soft_embedding_layout(fp, bp, m, h, dtype).total;
   // the soft cap is not known here: enough for either sequence
-  if (fused_gradients_supported(h, v, dtype)) {
+  if (gradients_in_forward_supported(h, dtype)) {
     const FusedPlan p = make_fused_plan(m, h, v, dtype, panel_bytes);
     need = std::max(need, fused_layout(p, m, h, dtype, false).total);
   }
@@ -553,7 +566,7 @@ extern "C" int tlce_soft_embedding(const void* hidden, const void* weight, int64
   if (m == 0) return 0;
   TLCE_REQUIRE(out != nullptr && workspace != nullptr, "soft_embedding: null pointer");
   TLCE_REQUIRE(((uintptr_t)out & 15) == 0, "soft_embedding: out must be 16-byte aligned");
-  if (fused_gradients_supported(h, v, dtype) && embedding_scale > 0.0f) {
+  if (gradients_in_forward_supported(h, dtype) && embedding_scale > 0.0f) {
     // two contractions instead of three: under a soft cap of at most 40 no row maximum is
     // needed at all; otherwise one pass emits entries relative to exact tile maxima
     const bool capped = logit_softcap > 0.0f && logit_softcap <= kSoftEmbeddingMaxCap;
@@ -682,7 +695,7 @@ extern "C" int tlce_kl_forward_with_gradient(
   if (m == 0) return 0;
   TLCE_REQUIRE(kl_gradient_in_forward_supported(m, h_draft, h_teacher, v, dtype, logit_softcap),
                "kl_forward_with_gradient: needs bf16 inputs, a soft cap of at most 40 or none, both "
-               "hidden sizes and v multiples of 64 (h_draft=%lld, h_teacher=%lld, v=%lld)",
+               "hidden sizes multiples of 64 (h_draft=%lld, h_teacher=%lld, v=%lld)",
                (long long)h_draft, (long long)h_teacher, (long long)v);
   TLCE_REQUIRE(losses && draft_lse && teacher_lse && unit_grad_hidden_f32 && workspace,
                "kl_forward_with_gradient: null pointer");
@@ -816,7 +829,7 @@ extern "C" int tlce_ce_topk_forward_with_gradient(
   if (int rc = topk_validate(hidden, weight, labels, m, h, v, dtype, top_k)) return rc;
   if (m == 0) return 0;
   TLCE_REQUIRE(topk_gradient_in_forward_supported(m, h, v, dtype),
-               "ce_topk_forward_with_gradient: needs bf16 inputs with h and v multiples of 64 "
+               "ce_topk_forward_with_gradient: needs bf16 inputs and hidden sizes that are multiples of 64 "
                "(h=%lld, v=%lld)", (long long)h, (long long)v);
   TLCE_REQUIRE(losses && probabilities && top_values && top_ids && lse && unit_grad_hidden_f32 &&
                    workspace,
@@ -916,15 +929,19 @@ extern "C" int tlce_segment_weighted_sum(const float* values, const float* weigh
 
 // ------------------------------------ forward that leaves the gradients ----
 extern "C" int tlce_fused_gradients_supported(int64_t h, int64_t v, int dtype) {
-  return (h > 0 && v > 0 && fused_gradients_supported(h, v, dtype)) ? 1 : 0;
+  return (h > 0 && v > 0 && (v % 64) == 0 && gradients_in_forward_supported(h, dtype)) ? 1 : 0;
+}
+
+extern "C" int tlce_gradients_in_forward_supported(int64_t h, int64_t v, int dtype) {
+  return (h > 0 && v > 0 && gradients_in_forward_supported(h, dtype)) ? 1 : 0;
 }
 
 extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
                                      int64_t panel_bytes, int64_t* block_rows, int* n_blocks,
                                      int* grad_hidden_k_splits) {
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0, "query_fused_plan: bad shape");
-  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
-               "query_fused_plan: needs bf16 inputs with h and v multiples of 64");
+  TLCE_REQUIRE(gradients_in_forward_supported(h, dtype),
+               "query_fused_plan: needs bf16 inputs and hidden sizes that are multiples of 64");
   const FusedPlan p = make_fused_plan(m, h, v, dtype, panel_bytes);
   if (block_rows) *block_rows = p.block_rows;
   if (n_blocks) *n_blocks = p.n_blocks;
@@ -935,7 +952,7 @@ extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
 extern "C" int64_t tlce_forward_with_gradients_workspace_bytes(int64_t m, int64_t h, int64_t v,
                                                                int dtype, int compute_weight_grad,
                                                                int64_t panel_bytes) {
-  if (m < 0 || h <= 0 || v <= 0 || !fused_gradients_supported(h, v, dtype)) return -1;
+  if (m < 0 || h <= 0 || v <= 0 || !gradients_in_forward_supported(h, dtype)) return -1;
   return fused_layout(make_fused_plan(m, h, v, dtype, panel_bytes), m, h, dtype,
                       compute_weight_grad != 0).total;
 }
@@ -949,8 +966,8 @@ extern "C" int tlce_forward_with_gradients(
     int64_t panel_bytes, void* workspace, int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
-  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
-               "forward_with_gradients: needs bf16 inputs with h and v multiples of 64 "
+  TLCE_REQUIRE(gradients_in_forward_supported(h, dtype),
+               "forward_with_gradients: needs bf16 inputs and hidden sizes that are multiples of 64 "
                "(h=%lld v=%lld dtype=%d)", (long long)h, (long long)v, dtype);
   TLCE_REQUIRE(valid_count != nullptr, "forward_with_gradients: valid_count is null");
   TLCE_REQUIRE(logit_multiplier > 0.0f,
@@ -1054,8 +1071,8 @@ extern "C" int tlce_grad_weight_from_panel(const void* hidden, const int64_t* ro
                                            int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0, "grad_weight_from_panel: bad shape");
-  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
-               "grad_weight_from_panel: needs bf16 inputs with h and v multiples of 64");
+  TLCE_REQUIRE(gradients_in_forward_supported(h, dtype),
+               "grad_weight_from_panel: needs bf16 inputs and hidden sizes that are multiples of 64");
   TLCE_REQUIRE(reduction_code == TLCE_REDUCTION_SUM || reduction_code == TLCE_REDUCTION_MEAN ||
                    reduction_code == TLCE_REDUCTION_NONE,
                "grad_weight_from_panel: unknown reduction code %d", reduction_code);

@@ -345,6 +345,15 @@ __global__ __launch_bounds__(256) void lce_topk_scan_kernel(TopkScanArgs p) {
   }
 }
 
+// The first `valid16` 16-byte pieces of src, then zeros (the zero-padded copy of a
+// matrix's last rows).
+__global__ __launch_bounds__(256) void lce_k_tail_kernel(const uint4* __restrict__ src,
+                                                         int valid16, uint4* __restrict__ dst,
+                                                         int n16) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n16) dst[i] = i < valid16 ? src[i] : make_uint4(0u, 0u, 0u, 0u);
+}
+
 __global__ __launch_bounds__(256) void lce_fill_zero_kernel(uint4* __restrict__ dst16,
                                                             int64_t n16, unsigned char* tail,
                                                             int ntail) {
