@@ -586,6 +586,14 @@ def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
 _STEP_PANEL_SHARE = 24
 _DEFAULT_PANEL_BYTES = 5 << 29    # what the library takes for a budget of 0
 
+# Steps with a trainable head of fewer multiply-adds per contraction whose vocabulary is no
+# multiple of 64 keep the recomputing backward: they are bound by launches and host calls,
+# of which it has fewer, and its grad_weight does not depend on the panel budget.  Measured
+# (gradients in the forward / recomputed, us a step): 600 rows, H = 256, V = 3000 293 / 264;
+# 64 rows, H = 1024, V = 32003 (2.1e9 multiply-adds) 282 / 260; 600 rows, H = 256, V = 50257
+# (7.7e9) 287 / 335; 600 rows, H = 1024, V = 32003 298 / 343.
+_RAGGED_STEP_MIN_MACS = 1 << 32
+
 
 def _step_panel_budgets(m: int, v: int, device: torch.device) -> tuple[int, ...]:
     """Panel budgets a step with a trainable head tries in turn: the context's if it
@@ -613,6 +621,8 @@ def training_forward(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.T
     if not compute_weight_grad:
         out = forward_with_gradients(hidden, weight, labels, compute_weight_grad=False, **kw)
         return out, False, get_panel_bytes()
+    if v % 64 != 0 and m * h * v < _RAGGED_STEP_MIN_MACS:
+        return None
     budgets = _step_panel_budgets(m, v, hidden.device)
     for budget in budgets:
         with panel_budget(budget):

@@ -71,17 +71,20 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             and get_gradient_mode() == "forward"
             and native.fused_gradients_supported(rows, weight, bias, False)
         )
+        step = None
         if ctx.fused:
-            rows = rows[:m]
-            out, ctx.postponed, ctx.panel_bytes = native.training_forward(
-                rows, weight, targets[:m], compute_weight_grad=bool(ctx.needs_input_grad[1]),
+            step = native.training_forward(
+                rows[:m], weight, targets[:m], compute_weight_grad=bool(ctx.needs_input_grad[1]),
                 per_token=False, ignore_index=-100, exclude_index=exclude_index,
                 logit_softcap=logit_softcap,
                 token_weights=None if token_weights is None else token_weights[:m],
                 logit_multiplier=multiplier,
                 row_idx=row_idx, n_out=n, row_count=row_count if mode == "device" else None,
             )
-            losses, _, valid_count, grad_rows32, grad_weight32 = out
+            ctx.fused = step is not None
+        if ctx.fused:
+            rows = rows[:m]
+            (losses, _, valid_count, grad_rows32, grad_weight32), ctx.postponed, ctx.panel_bytes = step
             ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx,
                                   row_count if mode == "device" else None,
                                   rows if ctx.postponed else None)
