@@ -90,7 +90,7 @@ int launch_label_logit(const LabelLogitArgs& a, hipStream_t stream) {
 int launch_fused_rows(const FusedRowsArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassCombine, stream);
   lce_fused_rows_kernel<__bf16>
-      <<<(int)ceil_div(a.m_pad, kFusedRowsPerBlock), 256, 0, stream>>>(a);
+      <<<(int)ceil_div(a.m_pad, kFusedRowsPerBlock), 64 * kFusedRowsWaves, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
