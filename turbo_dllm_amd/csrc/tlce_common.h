@@ -91,20 +91,26 @@ __host__ __device__ static inline int forward_vocab_splits(int n_ttiles, int n_v
 // K splits of the grad_hidden contraction: `tiles` output tiles per panel, each a
 // loop of `k_steps` K steps when unsplit; every split accumulates into a float32
 // slab of its own (`slab_elems` elements), summed by the final cast.  Picks the
-// count in [1, max_split] with the least estimated time, in units of one K step:
-//   rounds of 256 workgroups x (K steps per split + 8 for a tile's start and output)
-//   + splits x the time the final cast needs to read one more slab.
-// Ties go to fewer splits.  Integer arithmetic only: the host plan and the
-// kernels that re-plan for a row count known on the device must agree.
+// count in [1, max_split] with the least estimated time, in eighths of a K step:
+//   rounds of `resident` workgroups x (K steps per split + 8 for a tile's start and output)
+//   + splits x the time the slab's write and its read by the final cast take.
+// Up to 64 splits: 64 rows over H = 1024 are four tiles, whose K loop of 500 steps (V =
+// 32000) ran on 64 CUs with at most 16 splits, 49 us; now 25.
+// Ties go to fewer splits.  Integer arithmetic only (divisions in 32 bits: a K step is 64
+// or 32 wide): the host plan and the kernels that re-plan for a row count known on the
+// device must agree.
+constexpr int kMaxKSplits = 64;
 __host__ __device__ static inline int grad_hidden_k_splits(int64_t tiles, int max_split,
                                                            int64_t k_steps, int64_t slab_elems,
                                                            int resident = 256) {
-  const int64_t per_slab = (slab_elems >> 20) > 1 ? (slab_elems >> 20) : 1;
+  const int64_t per_slab = (slab_elems >> 17) > 1 ? (slab_elems >> 17) : 1;
+  const int shift = resident == 512 ? 9 : 8;
   int pick = 1;
   int64_t best = -1;
   for (int ks = 1; ks <= max_split; ++ks) {
-    const int64_t rounds = (tiles * ks + resident - 1) / resident;
-    const int64_t cost = rounds * ((k_steps + ks - 1) / ks + 8) + ks * per_slab;
+    const int64_t rounds = (tiles * ks + resident - 1) >> shift;
+    const int64_t steps = ((uint32_t)k_steps + (uint32_t)ks - 1) / (uint32_t)ks;
+    const int64_t cost = rounds * 8 * (steps + 8) + ks * per_slab;
     if (best < 0 || cost < best) {
       best = cost;
       pick = ks;

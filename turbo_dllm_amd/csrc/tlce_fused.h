@@ -362,9 +362,9 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
   p.block_rows = per * tile;
   p.n_blocks = (int)ceil_div(total, per);
   const int64_t k_steps = p.vp / 64;
-  const int max_split = (int)std::max<int64_t>(1, std::min<int64_t>(16, k_steps / 8));
+  const int max_split = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxKSplits, k_steps / 8));
   p.dh_ksplit = grad_hidden_k_splits((p.block_rows / tile) * p.n_htiles, max_split, k_steps,
-                                     p.block_rows * h);
+                                     std::min(p.block_rows, std::max<int64_t>(m, 1)) * h);
   return p;
 }
 
@@ -506,14 +506,14 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     dh.b = panel; dh.ldb = p.vp; dh.b_rows = (int)rows_p;
     dh.k_per_split = 0;
     dh.ni = p.n_htiles; dh.nj = n_ttiles;
-    dh.c = slabs; dh.ldc = h; dh.c_rows = (int)rows_p; dh.c_cols = (int)h;
+    dh.c = slabs; dh.ldc = h; dh.c_rows = (int)rows; dh.c_cols = (int)h;
     dh.c_split_stride = p.block_rows * h;
     dh.mode = kStoreF32;
     int ksplit = (rows_p == p.block_rows)
                      ? p.dh_ksplit
                      : std::min(p.dh_ksplit,
                                 grad_hidden_k_splits((int64_t)n_ttiles * p.n_htiles, p.dh_ksplit,
-                                                     p.vp / 64, rows_p * h));
+                                                     p.vp / 64, rows * h));
     ReduceSlabsArgs rs;
     if (m_dev != nullptr) {
       // The block may hold far fewer rows than it was sized for (down to none): up to 16
@@ -638,14 +638,14 @@ int soft_embedding_fused_impl(const FusedPlan& p, const void* hidden, const void
     g.b = panel; g.ldb = p.vp; g.b_rows = (int)rows_p;
     g.k_per_split = 0;
     g.ni = p.n_htiles; g.nj = n_ttiles;
-    g.c = slabs; g.ldc = h; g.c_rows = (int)rows_p; g.c_cols = (int)h;
+    g.c = slabs; g.ldc = h; g.c_rows = (int)rows; g.c_cols = (int)h;
     g.c_split_stride = p.block_rows * h;
     g.mode = kStoreF32;
     const int ksplit = (rows_p == p.block_rows)
                            ? p.dh_ksplit
                            : std::min(p.dh_ksplit,
                                       grad_hidden_k_splits((int64_t)n_ttiles * p.n_htiles,
-                                                           p.dh_ksplit, p.vp / 64, rows_p * h));
+                                                           p.dh_ksplit, p.vp / 64, rows * h));
     if (int rc = launch_gemm<E, true, false>(g, ksplit, kClassGradHidden, stream)) return rc;
     ReduceSlabsArgs rs;
     rs.slabs = slabs; rs.n_splits = ksplit; rs.split_stride = p.block_rows * h;
@@ -773,7 +773,7 @@ int topk_forward_with_gradient_impl(const TopkPlan& t, const FusedPlan& p, const
   g.b = panel; g.ldb = p.vp; g.b_rows = m_pad;
   g.k_per_split = 0;
   g.ni = p.n_htiles; g.nj = m_pad / E::kTile;
-  g.c = slabs; g.ldc = h; g.c_rows = m_pad; g.c_cols = (int)h;
+  g.c = slabs; g.ldc = h; g.c_rows = (int)m; g.c_cols = (int)h;
   g.c_split_stride = p.block_rows * h;
   g.mode = kStoreF32;
   if (int rc = launch_gemm<E, true, false>(g, p.dh_ksplit, kClassGradHidden, stream)) return rc;
@@ -979,7 +979,7 @@ int kl_forward_with_gradient_impl(const Plan& pd, const Plan& pt, const KlLayout
   g.b = exp_panel; g.ldb = pd.vp; g.b_rows = (int)pd.mp;
   g.k_per_split = 0;
   g.ni = fp.n_htiles; g.nj = (int)(pd.mp / E::kTile);
-  g.c = slabs; g.ldc = hd; g.c_rows = (int)pd.mp; g.c_cols = (int)hd;
+  g.c = slabs; g.ldc = hd; g.c_rows = (int)m; g.c_cols = (int)hd;
   g.c_split_stride = pd.mp * hd;
   g.mode = kStoreF32;
   if (int rc = launch_gemm<E, true, false>(g, fp.dh_ksplit, kClassGradHidden, stream)) return rc;
@@ -1044,14 +1044,14 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
     g.b = panel; g.ldb = p.vp; g.b_rows = (int)rows_p;
     g.k_per_split = 0;
     g.ni = p.n_htiles; g.nj = n_ttiles;
-    g.c = slabs; g.ldc = h; g.c_rows = (int)rows_p; g.c_cols = (int)h;
+    g.c = slabs; g.ldc = h; g.c_rows = (int)rows; g.c_cols = (int)h;
     g.c_split_stride = p.block_rows * h;
     g.mode = kStoreF32;
     const int ksplit = (rows_p == p.block_rows)
                            ? p.dh_ksplit
                            : std::min(p.dh_ksplit,
                                       grad_hidden_k_splits((int64_t)n_ttiles * p.n_htiles,
-                                                           p.dh_ksplit, p.vp / 64, rows_p * h));
+                                                           p.dh_ksplit, p.vp / 64, rows * h));
     if (int rc = launch_gemm<E, true, false>(g, ksplit, kClassGradHidden, stream)) return rc;
     ReduceSlabsArgs rs;
     rs.slabs = slabs; rs.n_splits = ksplit; rs.split_stride = p.block_rows * h;

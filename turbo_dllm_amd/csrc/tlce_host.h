@@ -146,7 +146,7 @@ inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_gr
   p.dh_ksplit = 1;
   p.dh_max_ksplit = 1;
   if (p.engine) {
-    p.dh_max_ksplit = (int)std::max<int64_t>(1, std::min<int64_t>(16, p.vc / p.bk / 8));
+    p.dh_max_ksplit = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxKSplits, p.vc / p.bk / 8));
     p.dh_ksplit = grad_hidden_k_splits((int64_t)p.n_ttiles * p.n_htiles, p.dh_max_ksplit,
                                        p.vc / p.bk, p.mp * h, resident_workgroups(p.tile));
   }
@@ -488,7 +488,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     dh.b = g; dh.ldb = p.vc; dh.b_rows = (int)p.mp;
     dh.k_per_split = 0;
     dh.ni = p.n_htiles; dh.nj = p.n_ttiles;
-    dh.c = acc32; dh.ldc = h; dh.c_rows = (int)p.mp; dh.c_cols = (int)h;
+    dh.c = acc32; dh.ldc = h; dh.c_rows = (int)m; dh.c_cols = (int)h;
     dh.c_split_stride = p.mp * h;
     dh.mode = (panel == 0) ? kStoreF32 : kAddF32;
     dh.m_dev = m_dev; dh.m_role = kRowsFollow;

@@ -1459,6 +1459,7 @@ __global__ __launch_bounds__(256) void lce_finalize_grad_hidden_kernel(
     // four hidden entries per thread: 16-byte loads of every slab, one vector store
     for (int k = threadIdx.x * 4; k < h; k += 256 * 4) {
       f32x4_t sum = *reinterpret_cast<const f32x4_t*>(src + k);
+#pragma unroll 8
       for (int s = 1; s < n_splits; ++s)
         sum += *reinterpret_cast<const f32x4_t*>(src + (int64_t)s * split_stride + k);
       store4<T>(dst + k, sum[0], sum[1], sum[2], sum[3]);
