@@ -980,24 +980,37 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_logits_pane
 
 // One workgroup per row: folds `width` float32 logits of the row (vocabulary ids
 // v0 .. v0 + width) into run_max / run_sum (natural-log units) and into the
-// row's sorted list of the k largest pairs, 16384 logits at a time (64 per
+// row's sorted list of the k largest pairs, 16384 logits at a time (32 per
 // thread, in registers).  Logits above the list's current k-th value (for a
 // row's first logits: at least the k-th largest per-thread maximum) are
 // gathered in LDS and merged with the list by rank; when there are too many
 // of them, k rounds of "the best pair after the previous pick" run over the
 // whole chunk instead.  Ties go to the smaller id.  k <= 256.
+//
+// With `exp_out` it also writes exp(logit - reference) * cap' of the chunk, rounded to
+// bf16, into a panel over the whole vocabulary, the operand of the gradient contraction
+// formed in the forward.  The reference is the row's largest logit so far, this chunk's
+// included, so every entry is at most 1; it is kept per (chunk, row) in `ref_used`.
+constexpr int kTopkChunk = 16384;
+constexpr int kTopkScanThreads = 512;
 struct TopkScanArgs {
-  const float* panel;
+  const float* panel;   // [m, ld]; columns from the vocabulary's end to `stored` hold -inf
   int64_t ld;
   int m;
   int64_t v0;
   int width;
+  int stored;           // columns of this panel that were written, a multiple of 64
   int k;
   int first;            // 1: the lists and statistics are empty
   float* run_max;
   float* run_sum;
   float* top_values;    // [m, k]
   int64_t* top_ids;     // [m, k]
+  void* exp_out = nullptr;     // bf16 [m_pad, ld_out]; this panel goes to columns v0 ...
+  int64_t ld_out = 0;
+  int m_pad = 0;               // rows of exp_out to define (zeros from m on)
+  float softcap = 0.0f;
+  float* ref_used = nullptr;   // [chunks of this panel, m_pad]
 };
 
 // One wave per row: lse, the label's logit as a direct dot product, loss and

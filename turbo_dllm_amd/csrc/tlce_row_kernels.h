@@ -123,7 +123,7 @@ __device__ __forceinline__ bool topk_before(float va, int64_t ia, float vb, int6
   return va > vb || (va == vb && ia < ib);
 }
 
-// The best (value, id) pair over the workgroup's 256 threads, returned to all
+// The best (value, id) pair over the workgroup's threads, returned to all
 // of them; ends on a barrier-free read of red_*, so callers synchronise before
 // the next call.
 __device__ __forceinline__ void topk_workgroup_best(float& best_val, int64_t& best_id,
@@ -146,7 +146,7 @@ __device__ __forceinline__ void topk_workgroup_best(float& best_val, int64_t& be
   best_val = red_val[0];
   best_id = red_id[0];
 #pragma unroll
-  for (int w = 1; w < 4; ++w) {
+  for (int w = 1; w < kTopkScanThreads / 64; ++w) {
     if (topk_before(red_val[w], red_id[w], best_val, best_id)) {
       best_val = red_val[w];
       best_id = red_id[w];
@@ -154,23 +154,43 @@ __device__ __forceinline__ void topk_workgroup_best(float& best_val, int64_t& be
   }
 }
 
-__global__ __launch_bounds__(256) void lce_topk_scan_kernel(TopkScanArgs p) {
-  constexpr int kPerThread = 64;
-  constexpr int kChunk = kPerThread * 256;
-  constexpr int kSlots = 3;                       // gathered pairs per thread
-  constexpr int kCapacity = kSlots * 256;
+// What bounds it is reading the logits once (and, with kEmit, writing half as many bytes):
+// every thread loads 8 pieces of four consecutive logits per chunk, and the exponentials of
+// the running sum are the entries that are written.  Measured on 8192 rows, V = 151936,
+// k = 16 in five panels: 2.44 ms (7.5 GB, 3.1 TB/s) against 2.32 for the scan (256 threads of
+// 64 logits in scalar loads) and 1.41 for a pass of its own that read the logits again and
+// wrote the entries.  512 threads of 32 logits: with 64 a thread the entries spill or leave
+// one wave per SIMD (4.8 ms).
+template <bool kEmit>
+__global__ __launch_bounds__(kTopkScanThreads, 6) void lce_topk_scan_kernel(TopkScanArgs p) {
+  constexpr int kThreads = kTopkScanThreads;
+  constexpr int kWaves = kThreads / 64;
+  constexpr int kChunk = kTopkChunk;
+  constexpr int kPerThread = kChunk / kThreads;
+  constexpr int kSlots = 2;                       // gathered pairs per thread
+  constexpr int kCapacity = kSlots * kThreads;
   __shared__ float list_val[256];
   __shared__ int64_t list_id[256];
   __shared__ float cand_val[kCapacity];
   __shared__ int64_t cand_id[kCapacity];
-  __shared__ float red_val[4];
-  __shared__ int64_t red_id[4];
-  __shared__ float red_f[4];
-  __shared__ int wave_total[4];
-  __shared__ float tmax[256];
+  __shared__ float red_val[kWaves];
+  __shared__ int64_t red_id[kWaves];
+  __shared__ float wave_high[kWaves];
+  __shared__ float wave_exp[kWaves];
+  __shared__ float wave_kth[kWaves];
+  __shared__ int wave_total[kWaves];
+  __shared__ __align__(16) float tmax[kThreads];
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
   const int row = blockIdx.x;
+  __bf16* exp_row = nullptr;
+  if constexpr (kEmit) {
+    exp_row = static_cast<__bf16*>(p.exp_out) + (int64_t)row * p.ld_out + p.v0;
+    if (row >= p.m) {
+      for (int c = 4 * t; c < p.stored; c += 4 * kThreads) store4<__bf16>(exp_row + c, 0.0f, 0.0f, 0.0f, 0.0f);
+      return;
+    }
+  }
   const float* src = p.panel + (int64_t)row * p.ld;
   float run_max = p.first ? -INFINITY : p.run_max[row];
   float run_sum = p.first ? 0.0f : p.run_sum[row];
@@ -181,66 +201,114 @@ __global__ __launch_bounds__(256) void lce_topk_scan_kernel(TopkScanArgs p) {
   }
   __syncthreads();
 
-  for (int c0 = 0; c0 < p.width; c0 += kChunk) {
+  for (int c0 = 0; c0 < p.stored; c0 += kChunk) {
+    // element i of this thread is column c0 + column(i); the empty asm keeps the compiler
+    // from holding what depends on the columns in registers over the whole loop
+    int t4 = 4 * t;
+    asm volatile("" : "+v"(t4));
+    auto column = [&](int i) { return t4 + 4 * kThreads * (i >> 2) + (i & 3); };
     float vals[kPerThread];
+#pragma unroll
+    for (int i = 0; i < kPerThread; i += 4) {
+      f32x4_t z = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (c0 + column(i) < p.stored) z = *reinterpret_cast<const f32x4_t*>(src + c0 + column(i));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vals[i + e] = z[e];
+    }
     float local_max = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < kPerThread; ++i) {
-      const int idx = c0 + t + 256 * i;
-      vals[i] = idx < p.width ? src[idx] : -INFINITY;
-      local_max = fmaxf(local_max, vals[i]);
-    }
+    for (int i = 0; i < kPerThread; ++i) local_max = fmaxf(local_max, vals[i]);
     // running softmax statistics
     const float m = wave_max(local_max);
-    if (lane == 0) red_f[wave] = m;
+    if (lane == 0) wave_high[wave] = m;
     __syncthreads();
-    const float new_max =
-        fmaxf(run_max, fmaxf(fmaxf(red_f[0], red_f[1]), fmaxf(red_f[2], red_f[3])));
-    __syncthreads();
-    float local_sum = 0.0f;
-    if (new_max > -INFINITY) {
+    float new_max = run_max;
 #pragma unroll
-      for (int i = 0; i < kPerThread; ++i) local_sum += __expf(vals[i] - new_max);
+    for (int w = 0; w < kWaves; ++w) new_max = fmaxf(new_max, wave_high[w]);
+    float local_sum = 0.0f;
+    const bool any = new_max > -INFINITY;
+    const float inv_cap = kEmit && p.softcap > 0.0f ? 1.0f / p.softcap : 0.0f;
+#pragma unroll
+    for (int i = 0; i < kPerThread; i += 4) {
+      float e[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float z = vals[i + u];
+        const float x = any ? __expf(z - new_max) : 0.0f;   // (-inf gives 0)
+        local_sum += x;
+        if constexpr (kEmit) {
+          e[u] = x;
+          if (p.softcap > 0.0f) {
+            const float q = z * inv_cap;
+            e[u] = z > -INFINITY ? x * (1.0f - q * q) : 0.0f;
+          }
+        }
+      }
+      if constexpr (kEmit) {
+        if (c0 + column(i) < p.stored) store4<__bf16>(exp_row + c0 + column(i), e[0], e[1], e[2], e[3]);
+      }
     }
+    if (kEmit && t == 0) p.ref_used[(int64_t)(c0 / kChunk) * p.m_pad + row] = new_max;
     local_sum = wave_sum(local_sum);
-    if (lane == 0) red_f[wave] = local_sum;
-    __syncthreads();
-    run_sum = (run_max > -INFINITY ? run_sum * __expf(run_max - new_max) : 0.0f) +
-              (red_f[0] + red_f[1] + red_f[2] + red_f[3]);
-    run_max = new_max;
+    if (lane == 0) wave_exp[wave] = local_sum;
 
     // the list entry this thread carries into the selection
     const float own_val = t < p.k ? list_val[t] : -INFINITY;
     const int64_t own_id = t < p.k ? list_id[t] : INT64_MAX;
     float kth = list_val[p.k - 1];
     bool inclusive = false;
-    if (kth == -INFINITY && p.k <= 256) {
-      // nothing to compare with yet (a row's first logits): the k-th largest
-      // of the 256 per-thread maxima is a value at least k logits reach
-      __syncthreads();
-      tmax[t] = local_max;
-      __syncthreads();
-      int before = 0;
-      for (int j = 0; j < 256; ++j) {
-        const float other = tmax[j];
-        before += (other > local_max || (other == local_max && j < t)) ? 1 : 0;
+    if (kth == -INFINITY) {
+      // nothing to compare with yet (a row's first logits): a value that at least k logits
+      // reach, the k-th largest of the per-thread maxima of some wave (k <= 32; a quarter of
+      // the work of the next, and a few times k logits beat it) or of all threads
+      if (p.k <= 32) {
+        int before = 0;
+#pragma unroll 8
+        for (int l = 0; l < 64; ++l) {
+          const float other = __uint_as_float(
+              __builtin_amdgcn_readlane(__float_as_uint(local_max), l));
+          before += (other > local_max || (other == local_max && l < lane)) ? 1 : 0;
+        }
+        if (before == p.k - 1) wave_kth[wave] = local_max;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) kth = fmaxf(kth, wave_kth[w]);
+      } else {
+        tmax[t] = local_max;
+        __syncthreads();
+        int before = 0;
+#pragma unroll 4
+        for (int j = 0; j < kThreads; j += 4) {
+          const f32x4_t other = *reinterpret_cast<const f32x4_t*>(tmax + j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            before += (other[e] > local_max || (other[e] == local_max && j + e < t)) ? 1 : 0;
+        }
+        if (before == p.k - 1) wave_kth[0] = local_max;
+        __syncthreads();
+        kth = wave_kth[0];
       }
-      if (before == p.k - 1) red_f[0] = local_max;
-      __syncthreads();
-      kth = red_f[0];
       inclusive = true;
-      __syncthreads();
     }
     auto beats = [&](float v) { return inclusive ? v >= kth : v > kth; };
-    auto chunk_id = [&](int i) -> int64_t {
-      return (c0 + t + 256 * i < p.width) ? p.v0 + c0 + t + 256 * i : INT64_MAX;
-    };
-    // gather the logits that beat the current k-th value: count per thread,
-    // exclusive prefix over the workgroup (no atomics), then write
-    int mine = 0;
+    // gather the logits that beat the current k-th value: count per thread, exclusive
+    // prefix over the workgroup (no atomics), then write.  The few threads that have one
+    // read their logits again: kept in registers until here they would cost half of the
+    // waves in flight.
+    auto for_each_candidate = [&](auto&& take) {
+      if (!beats(local_max)) return;
+#pragma unroll 1
+      for (int i = 0; i < kPerThread; i += 4) {
+        const int c = c0 + column(i);
+        if (c >= p.width) break;
+        const f32x4_t z = *reinterpret_cast<const f32x4_t*>(src + c);
 #pragma unroll
-    for (int i = 0; i < kPerThread; ++i)
-      mine += (beats(vals[i]) && c0 + t + 256 * i < p.width) ? 1 : 0;
+        for (int e = 0; e < 4; ++e)
+          if (beats(z[e]) && c + e < p.width) take(z[e], p.v0 + c + e);
+      }
+    };
+    int mine = 0;
+    for_each_candidate([&](float, int64_t) { ++mine; });
     int scan = mine;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -251,16 +319,23 @@ __global__ __launch_bounds__(256) void lce_topk_scan_kernel(TopkScanArgs p) {
     __syncthreads();
     int offset = scan - mine;
     for (int w = 0; w < wave; ++w) offset += wave_total[w];
-    const int n_cand = wave_total[0] + wave_total[1] + wave_total[2] + wave_total[3];
-    if (n_cand <= kCapacity && mine > 0) {
+    int n_cand = 0;
+    float chunk_sum = 0.0f;
 #pragma unroll
-      for (int i = 0; i < kPerThread; ++i) {
-        if (beats(vals[i]) && c0 + t + 256 * i < p.width) {
-          cand_val[offset] = vals[i];
-          cand_id[offset] = chunk_id(i);
-          ++offset;
-        }
-      }
+    for (int w = 0; w < kWaves; ++w) {
+      n_cand += wave_total[w];
+      chunk_sum += wave_exp[w];
+    }
+    run_sum = (run_max > -INFINITY ? run_sum * __expf(run_max - new_max) : 0.0f) + chunk_sum;
+    run_max = new_max;
+    if (n_cand == 0) continue;   // (the list and what the waves left are not written again
+                                 //  before the next chunk's first barrier)
+    if (n_cand <= kCapacity && mine > 0) {
+      for_each_candidate([&](float z, int64_t id) {
+        cand_val[offset] = z;
+        cand_id[offset] = id;
+        ++offset;
+      });
     }
     __syncthreads();
     if (n_cand > kCapacity) {
@@ -276,7 +351,7 @@ __global__ __launch_bounds__(256) void lce_topk_scan_kernel(TopkScanArgs p) {
           best_id = own_id;
         }
         for (int i = 0; i < kPerThread; ++i) {
-          const int idx = c0 + t + 256 * i;
+          const int idx = c0 + t + kThreads * i;
           if (idx >= p.width) break;
           const float v = src[idx];
           const int64_t d = p.v0 + idx;
@@ -307,7 +382,7 @@ __global__ __launch_bounds__(256) void lce_topk_scan_kernel(TopkScanArgs p) {
       int64_t gi[kSlots];
 #pragma unroll
       for (int q = 0; q < kSlots; ++q) {
-        const int pos = t + 256 * q;
+        const int pos = t + kThreads * q;
         rank[q] = p.k;
         if (pos < n_cand) {
           gv[q] = cand_val[pos];
