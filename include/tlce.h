@@ -325,7 +325,7 @@ int tlce_backward_local(const void* hidden, const void* weight, const float* bia
  * forward-only, without a logits buffer: the forward tile loop yields lse, the
  * probability panels (rounded to `dtype`, as the reference rounds them before
  * its second matmul) are contracted with the weight rows in float32: three
- * contractions.  Under a soft cap of at most 40 (bf16, h a multiple of 64)
+ * contractions.  Under a soft cap of at most 40 (bf16, h and v multiples of 64)
  * two suffice: capped logits lie in [-cap, cap], so exp(logit - cap) needs no
  * row maximum; it is written for a block of rows over the whole vocabulary
  * into a panel of panel_bytes (0: 2.5 GiB), contracted with the weight rows, and
@@ -544,9 +544,7 @@ int tlce_segment_weighted_sum(const float* values, const float* weights,
  * upstream gradient inside its contraction, is only available through
  * tlce_grad_weight_from_panel, i.e. when all rows form one block
  * (grad_weight_f32 must be NULL here).  No bias, head stored [v, h], bf16 inputs
- * with h a multiple of 64 (tlce_gradients_in_forward_supported;
- * tlce_fused_gradients_supported answers for vocabularies of whole 64-row slabs
- * only, of which no padded copy of the last rows is made); everything else
+ * with h and v multiples of 64 (tlce_fused_gradients_supported); everything else
  * goes through tlce_forward / tlce_backward (f16 included: its exponent range
  * cannot hold exp(logit - reference) and the row sums of it).
  *
@@ -563,7 +561,6 @@ int tlce_segment_weighted_sum(const float* values, const float* weights,
  * tlce_masked_loss_*, workgroups past the count exit at once and nothing needs
  * the host, so compaction, this call and tlce_apply_grad_output record into one
  * HIP graph that serves any mask. */
-int tlce_gradients_in_forward_supported(int64_t h, int64_t v, int dtype);
 int tlce_fused_gradients_supported(int64_t h, int64_t v, int dtype);
 
 int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,

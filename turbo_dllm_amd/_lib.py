@@ -103,7 +103,6 @@ SIGNATURES = {
             c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
         ],
     ),
-    "tlce_gradients_in_forward_supported": (c_int, [c_int64, c_int64, c_int]),
     "tlce_fused_gradients_supported": (c_int, [c_int64, c_int64, c_int]),
     "tlce_query_fused_plan": (
         c_int, [c_int64, c_int64, c_int64, c_int, c_int64, c_void_p, c_void_p, c_void_p]

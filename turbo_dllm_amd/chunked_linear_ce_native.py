@@ -465,7 +465,7 @@ def forward(
 def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
                               bias: torch.Tensor | None, weight_dim_first: bool) -> bool:
     """Whether ``forward_with_gradients`` takes these operands: bf16 inputs on the
-    GPU, head stored [V, H], no bias, H a multiple of 64.  (f16's exponent
+    GPU, head stored [V, H], no bias, H and V multiples of 64.  (f16's exponent
     range cannot hold exp(logit - reference) and its row sums.)"""
     if bias is not None or weight_dim_first or not hidden.is_cuda:
         return False
@@ -473,7 +473,7 @@ def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
         return False
     if hidden.dim() != 2 or weight.dim() != 2 or weight.shape[1] != hidden.shape[1]:
         return False
-    return bool(_lib.library().tlce_gradients_in_forward_supported(
+    return bool(_lib.library().tlce_fused_gradients_supported(
         hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
 
 
@@ -513,8 +513,8 @@ def forward_with_gradients(
     device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
     if not fused_gradients_supported(hidden, weight, None, False):
         raise RuntimeError(
-            "forward_with_gradients needs bf16 operands, a [V, H] head and hidden sizes that "
-            "are multiples of 64; use forward / backward for other inputs"
+            "forward_with_gradients needs bf16 operands, a [V, H] head and H, V multiples "
+            "of 64; use forward / backward for other inputs"
         )
     hidden = _dense(hidden)
     weight = _dense(weight)
@@ -568,7 +568,7 @@ def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
     """Whether ``forward_with_gradients`` takes ``m`` rows as one block under the
     panel budget in force, so that its grad_weight contraction can be postponed to
     the backward (``grad_weight_from_panel``)."""
-    if dtype != torch.bfloat16 or not _lib.library().tlce_gradients_in_forward_supported(
+    if dtype != torch.bfloat16 or not _lib.library().tlce_fused_gradients_supported(
             h, v, _lib.DTYPE_BF16):
         return False
     return _lib.query_fused_plan(m, h, v, _lib.DTYPE_BF16, get_panel_bytes())["n_blocks"] == 1
@@ -585,14 +585,6 @@ def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
 # 57.9 (recomputing backward) -> 43.2 ms.
 _STEP_PANEL_SHARE = 24
 _DEFAULT_PANEL_BYTES = 5 << 29    # what the library takes for a budget of 0
-
-# Steps with a trainable head of fewer multiply-adds per contraction whose vocabulary is no
-# multiple of 64 keep the recomputing backward: they are bound by launches and host calls,
-# of which it has fewer, and its grad_weight does not depend on the panel budget.  Measured
-# (gradients in the forward / recomputed, us a step): 600 rows, H = 256, V = 3000 293 / 264;
-# 64 rows, H = 1024, V = 32003 (2.1e9 multiply-adds) 282 / 260; 600 rows, H = 256, V = 50257
-# (7.7e9) 287 / 335; 600 rows, H = 1024, V = 32003 298 / 343.
-_RAGGED_STEP_MIN_MACS = 1 << 32
 
 
 def _step_panel_budgets(m: int, v: int, device: torch.device) -> tuple[int, ...]:
@@ -621,8 +613,6 @@ def training_forward(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.T
     if not compute_weight_grad:
         out = forward_with_gradients(hidden, weight, labels, compute_weight_grad=False, **kw)
         return out, False, get_panel_bytes()
-    if v % 64 != 0 and m * h * v < _RAGGED_STEP_MIN_MACS:
-        return None
     budgets = _step_panel_budgets(m, v, hidden.device)
     for budget in budgets:
         with panel_budget(budget):

@@ -335,11 +335,24 @@ struct FusedPlan {
   int dh_ksplit;        // K splits of the grad_hidden contraction of a full block
 };
 
-// Any vocabulary: the contraction over it takes the rows of an incomplete last 64-row
-// slab from a padded copy (k_tail_bytes).  Against the recomputing sequence, which alone
-// took vocabularies that are no multiple of 64 before: 2741 rows, H = 2048, V = 32003
-// 1.56 -> 1.08 ms a step (three contractions, no transposed copies).
-inline bool gradients_in_forward_supported(int64_t h, int dtype) {
+// Cross entropies and soft embeddings whose panel entries are formed in the forward:
+// vocabularies of whole 64-row slabs.  Others keep the sequences that recompute the
+// logits, which are more exact: their logit gradients are rounded with the upstream factor
+// in them, and grad_weight contracts the hidden rows as they are, not a rounded product of
+// them with a row factor.  2-norm errors against float64, recomputed / in the forward,
+// 1500 rows, H = 1024, V = 32003: grad_weight 2.42e-3 / 2.83e-3, grad_hidden under a frozen
+// head 2.21e-3 / 2.36e-3 (reduction "sum" 2.07e-3 / 2.36e-3), soft embeddings 2.25e-3 /
+// 2.25e-3 (H = 3840, V = 40001, a soft cap of 30: 2.25e-3 / 2.31e-3).  A step of 2741 rows over
+// H = 2048 takes 1.32 ms recomputed (1.55 from transposed copies) and took 1.04 in the forward.
+inline bool fused_gradients_supported(int64_t h, int64_t v, int dtype) {
+  return dtype == TLCE_DTYPE_BF16 && engine_class(h, dtype) == 2 && (v % 64) == 0;
+}
+
+// KL and CE with top-k take any vocabulary: the contraction over it reads the rows of an
+// incomplete last 64-row slab from a padded copy (k_tail_bytes).  They are the more exact
+// of their two sequences (recomputed -> in the forward, same sizes: KL losses 5.4e-4 ->
+// 4.5e-5, its grad_hidden 4.61e-3 -> 2.40e-3, top-k's 1.667e-3 -> 1.658e-3).
+inline bool objective_gradient_in_forward_supported(int64_t h, int dtype) {
   return dtype == TLCE_DTYPE_BF16 && engine_class(h, dtype) == 2;
 }
 
@@ -370,7 +383,7 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
 
 struct FusedLayout {
   int64_t panel, part_sum, part_max, target, ref, ref_next, row_scale, scaled_hidden, slabs,
-      redo, k_tail, total;
+      redo, total;
 };
 
 inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dtype,
@@ -390,19 +403,18 @@ inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dt
   if (weight_grad) off += align256(p.block_rows * h * es);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
   l.redo = off;       off += align256((int64_t)p.n_blocks * 4);
-  l.k_tail = off;     off += k_tail_bytes(p.v, h);
   l.total = off;
   return l;
 }
 
 // The head as the K-major operand of a contraction over the vocabulary.  `k_tail`: where
-// prepare_k_tail has put the rows of an incomplete last slab.
+// prepare_k_tail has put the rows of an incomplete last slab (null: v is a multiple of 64).
 inline int prepare_k_tail(const void* weight, int64_t v, int64_t h, char* k_tail,
                           hipStream_t stream) {
   return v % 64 != 0 ? launch_k_tail(weight, v, h, k_tail, stream) : 0;
 }
 inline void set_head_operand(GemmArgs& g, const void* weight, int64_t v, int64_t h,
-                             const char* k_tail) {
+                             const char* k_tail = nullptr) {
   g.a = weight; g.lda = h; g.a_rows = (int)h;
   g.k = (int)round_up(v, 64);
   if (g.k != v) {
@@ -450,7 +462,6 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
   la.ignore = ignore; la.exclude = exclude; la.softcap = softcap; la.logit_scale = opt.logit_scale;
   la.target = target; la.ref = ref; la.valid_count = valid_count; la.m_dev = m_dev;
   if (int rc = launch_label_logit(la, stream)) return rc;
-  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
 
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
@@ -502,7 +513,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
 
     // grad_hidden of the block: A = weight as stored (K-major, K = vocabulary), B = panel
     GemmArgs dh;
-    set_head_operand(dh, weight, v, h, ws + l.k_tail);
+    set_head_operand(dh, weight, v, h);
     dh.b = panel; dh.ldb = p.vp; dh.b_rows = (int)rows_p;
     dh.k_per_split = 0;
     dh.ni = p.n_htiles; dh.nj = n_ttiles;
@@ -607,7 +618,6 @@ int soft_embedding_fused_impl(const FusedPlan& p, const void* hidden, const void
   float* row_scale = reinterpret_cast<float*>(ws + l.row_scale);
   float* slabs = reinterpret_cast<float*>(ws + l.slabs);
   const T* hidden_t = static_cast<const T*>(hidden);
-  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
     const int64_t rows = std::min<int64_t>(p.block_rows, m - r0);
@@ -634,7 +644,7 @@ int soft_embedding_fused_impl(const FusedPlan& p, const void* hidden, const void
     // the contraction of grad_hidden in the forward that leaves the gradients: K = the
     // vocabulary, K splits into slabs for few rows
     GemmArgs g;
-    set_head_operand(g, weight, v, h, ws + l.k_tail);
+    set_head_operand(g, weight, v, h);
     g.b = panel; g.ldb = p.vp; g.b_rows = (int)rows_p;
     g.k_per_split = 0;
     g.ni = p.n_htiles; g.nj = n_ttiles;
@@ -711,7 +721,7 @@ struct TopkFusedLayout {
 inline bool topk_gradient_in_forward_supported(int64_t m, int64_t h, int64_t v, int dtype) {
   (void)m;
   (void)v;
-  return gradients_in_forward_supported(h, dtype);
+  return objective_gradient_in_forward_supported(h, dtype);
 }
 
 // Rows per block of the objectives that take whole blocks of rows one after the other.
@@ -877,7 +887,7 @@ inline bool kl_gradient_in_forward_supported(int64_t m, int64_t hd, int64_t ht, 
   // sequence that evaluates cap' on the float32 logit
   const bool cap_ok = softcap <= 0.0f || (softcap >= kKlMinCap && softcap <= kSoftEmbeddingMaxCap);
   (void)v;
-  return cap_ok && gradients_in_forward_supported(hd, dtype) && engine_class(ht, dtype) == 2;
+  return cap_ok && objective_gradient_in_forward_supported(hd, dtype) && engine_class(ht, dtype) == 2;
 }
 
 inline KlFusedLayout kl_fused_layout(const KlLayout& kl, const Plan& pd, const FusedPlan& p,
@@ -1011,7 +1021,6 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
   float* row_scale = reinterpret_cast<float*>(ws + l.row_scale);
   float* slabs = reinterpret_cast<float*>(ws + l.slabs);
   const T* hidden_t = static_cast<const T*>(hidden);
-  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
     const int64_t rows = std::min<int64_t>(p.block_rows, m - r0);
@@ -1043,7 +1052,7 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
     if (int rc = launch_kl_grad_from_exp(ga, p.n_vtiles, stream)) return rc;
 
     GemmArgs g;
-    set_head_operand(g, weight, v, h, ws + l.k_tail);
+    set_head_operand(g, weight, v, h);
     g.b = panel; g.ldb = p.vp; g.b_rows = (int)rows_p;
     g.k_per_split = 0;
     g.ni = p.n_htiles; g.nj = n_ttiles;

@@ -543,7 +543,7 @@ extern "C" int64_t tlce_soft_embedding_workspace_bytes(int64_t m, int64_t h, int
   const Plan bp = make_plan(m, h, v, dtype, false, panel_bytes);
   int64_t need = soft_embedding_layout(fp, bp, m, h, dtype).total;
   // the soft cap is not known here: enough for either sequence
-  if (gradients_in_forward_supported(h, dtype)) {
+  if (fused_gradients_supported(h, v, dtype)) {
     const FusedPlan p = make_fused_plan(m, h, v, dtype, panel_bytes);
     need = std::max(need, fused_layout(p, m, h, dtype, false).total);
   }
@@ -559,7 +559,7 @@ extern "C" int tlce_soft_embedding(const void* hidden, const void* weight, int64
   if (m == 0) return 0;
   TLCE_REQUIRE(out != nullptr && workspace != nullptr, "soft_embedding: null pointer");
   TLCE_REQUIRE(((uintptr_t)out & 15) == 0, "soft_embedding: out must be 16-byte aligned");
-  if (gradients_in_forward_supported(h, dtype) && embedding_scale > 0.0f) {
+  if (fused_gradients_supported(h, v, dtype) && embedding_scale > 0.0f) {
     // two contractions instead of three: under a soft cap of at most 40 no row maximum is
     // needed at all; otherwise one pass emits entries relative to exact tile maxima
     const bool capped = logit_softcap > 0.0f && logit_softcap <= kSoftEmbeddingMaxCap;
@@ -922,19 +922,15 @@ extern "C" int tlce_segment_weighted_sum(const float* values, const float* weigh
 
 // ------------------------------------ forward that leaves the gradients ----
 extern "C" int tlce_fused_gradients_supported(int64_t h, int64_t v, int dtype) {
-  return (h > 0 && v > 0 && (v % 64) == 0 && gradients_in_forward_supported(h, dtype)) ? 1 : 0;
-}
-
-extern "C" int tlce_gradients_in_forward_supported(int64_t h, int64_t v, int dtype) {
-  return (h > 0 && v > 0 && gradients_in_forward_supported(h, dtype)) ? 1 : 0;
+  return (h > 0 && v > 0 && fused_gradients_supported(h, v, dtype)) ? 1 : 0;
 }
 
 extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
                                      int64_t panel_bytes, int64_t* block_rows, int* n_blocks,
                                      int* grad_hidden_k_splits) {
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0, "query_fused_plan: bad shape");
-  TLCE_REQUIRE(gradients_in_forward_supported(h, dtype),
-               "query_fused_plan: needs bf16 inputs and hidden sizes that are multiples of 64");
+  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
+               "query_fused_plan: needs bf16 inputs with h and v multiples of 64");
   const FusedPlan p = make_fused_plan(m, h, v, dtype, panel_bytes);
   if (block_rows) *block_rows = p.block_rows;
   if (n_blocks) *n_blocks = p.n_blocks;
@@ -945,7 +941,7 @@ extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
 extern "C" int64_t tlce_forward_with_gradients_workspace_bytes(int64_t m, int64_t h, int64_t v,
                                                                int dtype, int compute_weight_grad,
                                                                int64_t panel_bytes) {
-  if (m < 0 || h <= 0 || v <= 0 || !gradients_in_forward_supported(h, dtype)) return -1;
+  if (m < 0 || h <= 0 || v <= 0 || !fused_gradients_supported(h, v, dtype)) return -1;
   return fused_layout(make_fused_plan(m, h, v, dtype, panel_bytes), m, h, dtype,
                       compute_weight_grad != 0).total;
 }
@@ -959,8 +955,8 @@ extern "C" int tlce_forward_with_gradients(
     int64_t panel_bytes, void* workspace, int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
-  TLCE_REQUIRE(gradients_in_forward_supported(h, dtype),
-               "forward_with_gradients: needs bf16 inputs and hidden sizes that are multiples of 64 "
+  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
+               "forward_with_gradients: needs bf16 inputs with h and v multiples of 64 "
                "(h=%lld v=%lld dtype=%d)", (long long)h, (long long)v, dtype);
   TLCE_REQUIRE(valid_count != nullptr, "forward_with_gradients: valid_count is null");
   TLCE_REQUIRE(logit_multiplier > 0.0f,
@@ -1064,8 +1060,8 @@ extern "C" int tlce_grad_weight_from_panel(const void* hidden, const int64_t* ro
                                            int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0, "grad_weight_from_panel: bad shape");
-  TLCE_REQUIRE(gradients_in_forward_supported(h, dtype),
-               "grad_weight_from_panel: needs bf16 inputs and hidden sizes that are multiples of 64");
+  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
+               "grad_weight_from_panel: needs bf16 inputs with h and v multiples of 64");
   TLCE_REQUIRE(reduction_code == TLCE_REDUCTION_SUM || reduction_code == TLCE_REDUCTION_MEAN ||
                    reduction_code == TLCE_REDUCTION_NONE,
                "grad_weight_from_panel: unknown reduction code %d", reduction_code);

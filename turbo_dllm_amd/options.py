@@ -42,7 +42,7 @@ _panel_bytes = contextvars.ContextVar("tlce_panel_bytes", default=0)
 #   "forward"   (default) during the forward, while the logits of a block of rows
 #               exist: 3 contractions per step instead of 4.  Taken where the
 #               library supports it (bf16 inputs, no bias, head stored [V, H], H
-#               a multiple of 64) and a gradient is required; other calls
+#               and V multiples of 64) and a gradient is required; other calls
 #               fall back to "recompute".  The forward then holds the float32
 #               grad_hidden [M, H] and either the float32 grad_weight [V, H] or,
 #               when all rows fit one block, its workspace, until the backward
