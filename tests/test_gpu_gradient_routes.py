@@ -88,3 +88,45 @@ def test_ragged_soft_embedding_rounds_normalised_probabilities(gpu_device, softc
     if softcap is not None:
         z = softcap * torch.tanh(z / softcap)
     assert relative_norm(got, z.softmax(1) @ weight.double()) <= TWO_ROUNDINGS
+
+
+# 10240 rows over V = 151936: two blocks of the default panel of 2.5 GiB
+BLOCKED = (10240, 64, 151936)
+
+
+def test_rows_beyond_the_default_panel_hold_no_panel_until_the_backward(gpu_device):
+    """Between forward and backward, where a model's activations are live, only the float32
+    gradients may be held; the panel of the step (3.1 GB in one block) is released."""
+    m, h, v = BLOCKED
+    hidden, weight, labels, _ = operands(gpu_device, m, h, v)
+    x, w = hidden.requires_grad_(True), weight.requires_grad_(True)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    with _lib.kernel_profile() as prof:
+        loss = tiled_linear_cross_entropy(x, w, labels, reduction="mean", dtype=torch.bfloat16)
+    held = torch.cuda.memory_allocated() - before
+    gradients = 4 * h * (m + v)
+    print("[case] held", held, "float32 gradients", gradients, flush=True)
+    assert prof.launches["grad_weight_gemm"] == 2
+    assert held <= gradients + (1 << 20)
+    loss.backward()
+    torch.cuda.synchronize()
+    ones = torch.full((m,), 1.0 / m, dtype=torch.float64, device=gpu_device)
+    # (gradients formed in the forward: three roundings of grad_weight, 2.87e-3, and 8 % for the
+    # spread of one sample)
+    assert relative_norm(w.grad, exact_grad_weight(hidden.detach(), weight.detach(), labels, ones)) <= 3.1e-3
+
+
+def test_per_token_losses_beyond_one_block_recompute(gpu_device):
+    m, h, v = BLOCKED
+    hidden, weight, labels, up = operands(gpu_device, m, h, v)
+    with _lib.kernel_profile() as prof:
+        got = step(hidden, weight, labels, up, "none")
+    assert prof.launches["exp_logits_panel"] == 0
+    with options.gradient_mode("recompute"):
+        want = step(hidden, weight, labels, up, "none")
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    error = relative_norm(got[2], exact_grad_weight(hidden, weight, labels, up.double()))
+    print("[case] grad_weight error", error, flush=True)
+    assert error <= TWO_ROUNDINGS

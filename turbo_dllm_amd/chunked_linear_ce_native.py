@@ -574,62 +574,6 @@ def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
     return _lib.query_fused_plan(m, h, v, _lib.DTYPE_BF16, get_panel_bytes())["n_blocks"] == 1
 
 
-# The panel of exponentiated logits of a training step may take this share of the GPU's
-# memory when the context sets no budget of its own: 12 GiB of 288, 42 K rows at
-# V = 151936.  All rows are then one block: grad_weight waits for the upstream gradient
-# and is stored once in the input dtype, instead of a float32 [V, H] accumulator that
-# every further block reads and writes and a last pass rounds; and per-token losses,
-# whose upstream gradients grad_weight needs inside its contraction, keep the three
-# contractions.  Measured (H = 4096, V = 151936, blocks of the library's 2.5 GiB ->
-# one block): 32768 rows, mean loss 88.5 -> 86.0 ms; 16384 rows, per-token losses
-# 57.9 (recomputing backward) -> 43.2 ms.
-_STEP_PANEL_SHARE = 24
-_DEFAULT_PANEL_BYTES = 5 << 29    # what the library takes for a budget of 0
-
-
-def _step_panel_budgets(m: int, v: int, device: torch.device) -> tuple[int, ...]:
-    """Panel budgets a step with a trainable head tries in turn: the context's if it
-    has one, else what makes all rows one block (where that is within the share above)
-    and then the library's default, for a GPU whose memory is taken otherwise."""
-    budget = get_panel_bytes()
-    if budget:
-        return (budget,)
-    whole = -(-m // 256) * 256 * (-(-v // 256) * 256) * 2
-    if whole <= _DEFAULT_PANEL_BYTES or whole > torch.cuda.get_device_properties(device).total_memory // _STEP_PANEL_SHARE:
-        return (0,)
-    return (whole, 0)
-
-
-def training_forward(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor, *,
-                     compute_weight_grad: bool, per_token: bool, **kw):
-    """``forward_with_gradients`` as the autograd functions run it: under the panel
-    budget of ``_step_panel_budgets``, with grad_weight postponed when all rows form one
-    block.  ``per_token``: the upstream gradient will have one value per token, so a
-    trainable head needs the postponed contraction.  Returns the outputs of
-    ``forward_with_gradients``, whether grad_weight is postponed, and the panel budget
-    (for ``grad_weight_from_panel``); or None when the recomputing backward must serve."""
-    m, h = hidden.shape
-    v = weight.shape[0]
-    if not compute_weight_grad:
-        out = forward_with_gradients(hidden, weight, labels, compute_weight_grad=False, **kw)
-        return out, False, get_panel_bytes()
-    budgets = _step_panel_budgets(m, v, hidden.device)
-    for budget in budgets:
-        with panel_budget(budget):
-            postpone = weight_grad_can_wait(m, h, v, hidden.dtype)
-            if per_token and not postpone:
-                continue
-            try:
-                out = forward_with_gradients(hidden, weight, labels, compute_weight_grad=True,
-                                             postpone_weight_grad=postpone, **kw)
-            except torch.cuda.OutOfMemoryError:
-                if budget == budgets[-1]:
-                    raise
-                continue
-            return out, postpone, budget
-    return None
-
-
 def _upstream_gradient(grad_output: torch.Tensor, reduction_code: int, n_out: int) -> torch.Tensor:
     """The upstream gradient as the library reads it: float32, one element for a
     scalar reduction, one per output row for reduction "none"."""

@@ -71,23 +71,22 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             and get_gradient_mode() == "forward"
             and native.fused_gradients_supported(rows, weight, bias, False)
         )
-        step = None
         if ctx.fused:
-            step = native.training_forward(
-                rows[:m], weight, targets[:m], compute_weight_grad=bool(ctx.needs_input_grad[1]),
-                per_token=False, ignore_index=-100, exclude_index=exclude_index,
-                logit_softcap=logit_softcap,
+            rows = rows[:m]
+            ctx.postponed = bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
+                m, rows.shape[1], weight.shape[0], rows.dtype)
+            losses, _, valid_count, grad_rows32, grad_weight32 = native.forward_with_gradients(
+                rows, weight, targets[:m], ignore_index=-100, exclude_index=exclude_index,
+                logit_softcap=logit_softcap, compute_weight_grad=bool(ctx.needs_input_grad[1]),
                 token_weights=None if token_weights is None else token_weights[:m],
                 logit_multiplier=multiplier,
                 row_idx=row_idx, n_out=n, row_count=row_count if mode == "device" else None,
+                postpone_weight_grad=ctx.postponed,
             )
-            ctx.fused = step is not None
-        if ctx.fused:
-            rows = rows[:m]
-            (losses, _, valid_count, grad_rows32, grad_weight32), ctx.postponed, ctx.panel_bytes = step
             ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx,
                                   row_count if mode == "device" else None,
                                   rows if ctx.postponed else None)
+            ctx.panel_bytes = native.get_panel_bytes()
             ctx.hidden_shape = hidden.shape
             ctx.n_rows, ctx.m = n, m
             ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]

@@ -281,23 +281,27 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
         wants_grad and options.get_gradient_mode() == "forward"
         and native.fused_gradients_supported(rows, weight_vf, bias, in_place or weight_dim_first)
     )
-    step = None
+    can_wait = ctx.fused and bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
+        m, rows.shape[1], weight_vf.shape[0], rows.dtype)
+    if reduction == "none" and bool(ctx.needs_input_grad[1]) and not can_wait:
+        ctx.fused = False
     if ctx.fused:
         # (rows compacted with the count read back carry up to 63 zero rows of padding)
-        step = native.training_forward(
-            rows[:m], weight_vf, targets[:m], compute_weight_grad=bool(ctx.needs_input_grad[1]),
-            per_token=reduction == "none", ignore_index=ignore_index,
-            exclude_index=exclude_index, logit_softcap=float(logit_softcap), row_idx=row_idx,
-            n_out=n, row_count=row_count if mode == "device" else None,
-        )
-        ctx.fused = step is not None
-    if ctx.fused:
+        rows, targets = rows[:m], targets[:m]
         # all rows in one block: the grad_weight contraction waits for the upstream
         # gradient and is stored in the input dtype at once (no float32 [V, H] buffer)
-        (losses, lse, valid_count, grad_rows32, grad_weight32), ctx.postponed, ctx.panel_bytes = step
+        ctx.postponed = can_wait
+        losses, lse, valid_count, grad_rows32, grad_weight32 = native.forward_with_gradients(
+            rows, weight_vf, targets, ignore_index=ignore_index, exclude_index=exclude_index,
+            logit_softcap=float(logit_softcap),
+            compute_weight_grad=bool(ctx.needs_input_grad[1]), row_idx=row_idx, n_out=n,
+            row_count=row_count if mode == "device" else None,
+            postpone_weight_grad=ctx.postponed,
+        )
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx,
                               row_count if mode == "device" else None,
-                              rows[:m] if ctx.postponed else None)
+                              rows if ctx.postponed else None)
+        ctx.panel_bytes = native.get_panel_bytes()
         ctx.hidden_shape = hidden.shape
         ctx.n_rows, ctx.m = n, m
         ctx.reduction = reduction
