@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import linear_ce_oracle as oracle
+from turbo_dllm_amd import chunked_linear_ce_native as native
 from turbo_dllm_amd import options
 from turbo_dllm_amd.dflash_linear_topk import frozen_linear_ce_topk
 
@@ -60,3 +61,29 @@ def test_scan_edges(gpu_device, m, v, k, panel_tiles, softcap):
     error = oracle.relative_max_error(x.grad, grad)
     print("[case] gradient error", error, flush=True)
     assert error <= 1e-2
+
+
+def test_entries_of_one_logits_panel_are_rounded_once(gpu_device):
+    """Three chunks of the scan in one float32 logits panel, the row maximum in the last of
+    them: the entries of the gradient panel are exp(logit - maximum of the panel) rounded to
+    bf16 once, so d lse / d hidden is as far from float64 as that one rounding makes it (5 %
+    for hardware exponentials that round the other way; entries rounded in the chunk they
+    are scanned in, and again for the final maximum, are about 1.4 times as far)."""
+    m, h, v = 64, 64, 49152
+    gen = torch.Generator().manual_seed(7)
+    hidden = (torch.randint(-8, 9, (m, h), generator=gen) / 8).bfloat16().to(gpu_device)
+    weight = (torch.randint(-2, 3, (v, h), generator=gen) / 8).bfloat16().to(gpu_device)
+    weight[:, 0] += (torch.arange(v, device=gpu_device) // 16384) * 0.5   # later words are likelier
+    hidden[:, 0] = 1.0
+    labels = torch.randint(0, v, (m,), generator=gen).to(gpu_device)
+    unit = native.dflash_ce_topk_forward_with_gradient(
+        hidden, weight, labels, top_k=4, output_multiplier=1.0, logit_softcap=0.0)[5]
+    z = hidden.double() @ weight.double().t()
+    maxima = [z[:, c:c + 16384].amax(1) for c in range(0, v, 16384)]
+    assert float((maxima[0] < maxima[2]).double().mean()) > 0.5
+    e = (z - z.amax(1, keepdim=True)).exp()
+    exact = (e @ weight.double()) / e.sum(1, keepdim=True)
+    once = (e.bfloat16().double() @ weight.double()) / e.sum(1, keepdim=True)
+    error, bound = float((unit.double() - exact).norm()), float((once - exact).norm())
+    print("[case] error", error / float(exact.norm()), "one rounding", bound / float(exact.norm()), flush=True)
+    assert error <= 1.05 * bound

@@ -669,21 +669,21 @@ int soft_embedding_fused_impl(const FusedPlan& p, const void* hidden, const void
 // ---- frozen-head cross entropy with top-k: the gradient formed in the forward ----
 // The backward of tlce_ce_topk_* recomputes the logits to form the softmax panel
 // (3 contractions per step).  Here the forward, which stages float32 logits panels
-// anyway, also writes e = exp(z - reference) * cap' of every scan chunk in bf16 into a
+// anyway, also writes e = exp(z - reference) * cap' of every panel in bf16 into a
 // panel over the whole vocabulary and contracts it with the weight rows once:
 //   unit[r, :] = (multiplier / sum_r) * (e . weight)[r, :] = d lse_r / d hidden[r, :]
-// (2 contractions).  The reference of a chunk is the row's largest logit so far, so e <= 1;
-// chunks written before a row's maximum grew are multiplied by exp(old - final) afterwards (lce_rescale_exp_rows_kernel).  The
+// (2 contractions).  The reference of a panel is the row's largest logit so far (known
+// after the panel's scan), so e <= 1; panels written before a row's maximum grew are
+// multiplied by exp(old - final) afterwards (lce_rescale_exp_rows_kernel).  The
 // backward is then one pass over rows: ce_scale[r] * unit[r, :] plus the single-row
 // terms of the label and the top-k ids, rounded once.
 struct RescaleExpArgs {
   void* panel;             // bf16 [m_pad, ld]
   int64_t ld;
   int m, m_pad;
-  const float* ref_used;   // [panels * panel_chunks, m_pad]
+  const float* ref_used;   // [n_panels, m_pad]
   const float* run_max;    // [m] the final row maxima
   int64_t panel_width;     // columns per logits panel
-  int panel_chunks;        // scan chunks per logits panel
   int64_t total_width;     // columns of the whole panel
 };
 
@@ -707,7 +707,7 @@ struct TopkApplyArgs {
   void* grad_hidden;               // bf16 [m, h]
 };
 
-int launch_rescale_exp_rows(const RescaleExpArgs& a, int n_chunks, hipStream_t stream);
+int launch_rescale_exp_rows(const RescaleExpArgs& a, int n_panels, hipStream_t stream);
 int launch_topk_row_scale(const TopkRowScaleArgs& a, hipStream_t stream);
 int launch_topk_apply(const TopkApplyArgs& a, hipStream_t stream);
 
@@ -734,7 +734,7 @@ inline TopkFusedLayout topk_fused_layout(const TopkPlan& t, const FusedPlan& p, 
   int64_t off = 0;
   l.forward = off;    off += align256(t.forward_total);
   l.panel = off;      off += align256(p.block_rows * p.vp * 2);
-  l.ref_used = off;   off += align256((int64_t)t.n_fpanels * topk_chunks_per_panel(t) * p.block_rows * 4);
+  l.ref_used = off;   off += align256((int64_t)t.n_fpanels * p.block_rows * 4);
   l.row_scale = off;  off += align256(p.block_rows * 4);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
   l.k_tail = off;     off += k_tail_bytes(p.v, h);
@@ -765,15 +765,12 @@ int topk_forward_with_gradient_impl(const TopkPlan& t, const FusedPlan& p, const
     return rc;
   const float* run_max = reinterpret_cast<const float*>(fws + t.run_max);
   const float* run_sum = reinterpret_cast<const float*>(fws + t.run_sum);
-  const int chunks = topk_chunks_per_panel(t);
-  const int last_chunks = (int)ceil_div(t.plan.vp - (int64_t)(t.n_fpanels - 1) * t.vcf, kTopkChunk);
-  const int n_chunks = (t.n_fpanels - 1) * chunks + last_chunks;
-  if (n_chunks > 1) {
+  if (t.n_fpanels > 1) {
     RescaleExpArgs ra;
     ra.panel = panel; ra.ld = p.vp; ra.m = (int)m; ra.m_pad = m_pad;
     ra.ref_used = ref_used; ra.run_max = run_max;
-    ra.panel_width = t.vcf; ra.panel_chunks = chunks; ra.total_width = p.vp;
-    if (int rc = launch_rescale_exp_rows(ra, n_chunks - 1, stream)) return rc;
+    ra.panel_width = t.vcf; ra.total_width = p.vp;
+    if (int rc = launch_rescale_exp_rows(ra, t.n_fpanels - 1, stream)) return rc;
   }
   TopkRowScaleArgs sa;
   sa.run_sum = run_sum; sa.multiplier = multiplier; sa.m = (int)m; sa.m_pad = m_pad;

@@ -260,19 +260,49 @@ __global__ __launch_bounds__(256) void lce_kl_grad_from_exp_kernel(KlGradFromExp
   *reinterpret_cast<v8_t*>(e) = out;
 }
 
-// blockIdx.y = scan chunk (all but the last, which was written with the final maxima): rows
-// whose maximum grew after the chunk was written are brought to the final reference.
+// One row and 2048 columns per workgroup, 8 columns per thread.
+__global__ __launch_bounds__(256) void lce_exp_from_logits_kernel(ExpFromLogitsArgs p) {
+  const int r = blockIdx.x;
+  const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
+  if (c >= p.width) return;
+  __bf16* dst = static_cast<__bf16*>(p.out) + (int64_t)r * p.ld_out + p.col0 + c;
+  if (r >= p.m) {
+    store4<__bf16>(dst, 0.0f, 0.0f, 0.0f, 0.0f);
+    store4<__bf16>(dst + 4, 0.0f, 0.0f, 0.0f, 0.0f);
+    return;
+  }
+  const float ref = p.run_max[r];
+  if (c == 0) p.ref_used[r] = ref;
+  const float* src = p.logits + (int64_t)r * p.ld + c;
+  const f32x4_t z0 = *reinterpret_cast<const f32x4_t*>(src);
+  const f32x4_t z1 = *reinterpret_cast<const f32x4_t*>(src + 4);
+  float e[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float z = i < 4 ? z0[i] : z1[i - 4];
+    float x = __expf(z - ref);            // -inf (past the vocabulary) gives 0
+    if (p.softcap > 0.0f) {
+      const float t = z / p.softcap;
+      x = (z > -INFINITY) ? x * (1.0f - t * t) : 0.0f;
+    }
+    e[i] = x;
+  }
+  store4<__bf16>(dst, e[0], e[1], e[2], e[3]);
+  store4<__bf16>(dst + 4, e[4], e[5], e[6], e[7]);
+}
+
+// blockIdx.y = logits panel (all but the last, which was written with the final
+// maxima): rows whose maximum grew after the panel was written are brought to the
+// final reference.
 __global__ __launch_bounds__(256) void lce_rescale_exp_rows_kernel(RescaleExpArgs p) {
   const int r = blockIdx.x;
   const int j = blockIdx.y;
-  const int64_t first = (int64_t)(j / p.panel_chunks) * p.panel_width;   // its logits panel
-  const int64_t c0 = first + (int64_t)(j % p.panel_chunks) * kTopkChunk;
-  const int64_t c1 = min(min(c0 + kTopkChunk, first + p.panel_width), p.total_width);
-  if (c0 >= c1) return;
   const float used = p.ref_used[(int64_t)j * p.m_pad + r];
   const float fin = p.run_max[r];
   if (used == fin) return;
   const float f = __expf(used - fin);
+  const int64_t c0 = (int64_t)j * p.panel_width;
+  const int64_t c1 = min(c0 + p.panel_width, p.total_width);
   __bf16* row = static_cast<__bf16*>(p.panel) + (int64_t)r * p.ld;
   typedef __bf16 v8_t __attribute__((ext_vector_type(8)));
   for (int64_t c = c0 + threadIdx.x * 8; c < c1; c += 256 * 8) {

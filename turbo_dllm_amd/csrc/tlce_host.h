@@ -846,13 +846,27 @@ int launch_logits_panel_variant(const LogitsPanelArgs& a, hipStream_t stream) {
   return 0;
 }
 
-inline int topk_chunks_per_panel(const TopkPlan& t) { return (int)ceil_div(t.vcf, kTopkChunk); }
+// After the scan of a float32 logits panel: exp(logit - the row's largest logit so
+// far) * cap' of that panel, rounded to bf16, into a panel over the whole vocabulary
+// (the operand of the gradient contraction formed in the forward).
+struct ExpFromLogitsArgs {
+  const float* logits;   // [m, ld] float32 (columns past the vocabulary hold -inf)
+  int64_t ld;
+  int m, m_pad;          // rows with logits; rows of `out` to define (zeros from m on)
+  int width;             // columns of this logits panel, a multiple of 8
+  float softcap;
+  const float* run_max;  // [m] the reference: the row's largest logit so far
+  float* ref_used;       // [m] out: the reference this panel was written with
+  void* out;             // bf16 [m_pad, ld_out]; this panel goes to columns col0 ...
+  int64_t ld_out, col0;
+};
+int launch_exp_from_logits(const ExpFromLogitsArgs& a, hipStream_t stream);
 
 struct TopkExpHook {
   void* panel;           // bf16 [m_pad, ld]
   int64_t ld;
   int m_pad;
-  float* ref_used;       // [n_fpanels * chunks per panel, m_pad]
+  float* ref_used;       // [n_fpanels, m_pad]
 };
 
 template <class E>
@@ -885,12 +899,15 @@ int topk_forward_impl(const TopkPlan& t, const void* hidden, const void* weight,
     sa.panel = panel; sa.ld = t.vcf; sa.m = (int)m; sa.v0 = v0; sa.width = (int)valid;
     sa.stored = (int)width; sa.k = top_k; sa.first = pi == 0;
     sa.run_max = run_max; sa.run_sum = run_sum; sa.top_values = top_values; sa.top_ids = top_ids;
-    if (hook != nullptr) {
-      sa.exp_out = hook->panel; sa.ld_out = hook->ld; sa.m_pad = hook->m_pad;
-      sa.softcap = softcap;
-      sa.ref_used = hook->ref_used + (int64_t)pi * topk_chunks_per_panel(t) * hook->m_pad;
-    }
     if (int rc = launch_topk_scan(sa, stream)) return rc;
+    if (hook != nullptr) {
+      ExpFromLogitsArgs xa;
+      xa.logits = panel; xa.ld = t.vcf; xa.m = (int)m; xa.m_pad = hook->m_pad;
+      xa.width = (int)width; xa.softcap = softcap;
+      xa.run_max = run_max; xa.ref_used = hook->ref_used + (int64_t)pi * hook->m_pad;
+      xa.out = hook->panel; xa.ld_out = hook->ld; xa.col0 = v0;
+      if (int rc = launch_exp_from_logits(xa, stream)) return rc;
+    }
   }
   TopkFinishArgs fa;
   fa.hidden = hidden; fa.weight = weight; fa.labels = labels; fa.m = (int)m; fa.h = (int)h;

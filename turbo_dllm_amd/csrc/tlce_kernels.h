@@ -986,11 +986,6 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_logits_pane
 // gathered in LDS and merged with the list by rank; when there are too many
 // of them, k rounds of "the best pair after the previous pick" run over the
 // whole chunk instead.  Ties go to the smaller id.  k <= 256.
-//
-// With `exp_out` it also writes exp(logit - reference) * cap' of the chunk, rounded to
-// bf16, into a panel over the whole vocabulary, the operand of the gradient contraction
-// formed in the forward.  The reference is the row's largest logit so far, this chunk's
-// included, so every entry is at most 1; it is kept per (chunk, row) in `ref_used`.
 constexpr int kTopkChunk = 16384;
 constexpr int kTopkScanThreads = 512;
 struct TopkScanArgs {
@@ -1006,11 +1001,6 @@ struct TopkScanArgs {
   float* run_sum;
   float* top_values;    // [m, k]
   int64_t* top_ids;     // [m, k]
-  void* exp_out = nullptr;     // bf16 [m_pad, ld_out]; this panel goes to columns v0 ...
-  int64_t ld_out = 0;
-  int m_pad = 0;               // rows of exp_out to define (zeros from m on)
-  float softcap = 0.0f;
-  float* ref_used = nullptr;   // [chunks of this panel, m_pad]
 };
 
 // One wave per row: lse, the label's logit as a direct dot product, loss and

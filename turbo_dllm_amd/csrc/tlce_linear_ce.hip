@@ -67,8 +67,7 @@ int launch_kl_finish(float* losses, const float* loss_part, const float* tsum_pa
 
 int launch_topk_scan(const TopkScanArgs& sa, hipStream_t stream) {
   ScopedTimer timer(kClassOther, stream);
-  if (sa.exp_out != nullptr) lce_topk_scan_kernel<true><<<sa.m_pad, kTopkScanThreads, 0, stream>>>(sa);
-  else lce_topk_scan_kernel<false><<<sa.m, kTopkScanThreads, 0, stream>>>(sa);
+  lce_topk_scan_kernel<<<sa.m, kTopkScanThreads, 0, stream>>>(sa);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
@@ -111,10 +110,18 @@ int launch_kl_grad_from_exp(const KlGradFromExpArgs& a, int n_vtiles, hipStream_
   return 0;
 }
 
-int launch_rescale_exp_rows(const RescaleExpArgs& a, int n_chunks, hipStream_t stream) {
-  if (n_chunks <= 0 || a.m <= 0) return 0;
+int launch_exp_from_logits(const ExpFromLogitsArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassOther, stream);
-  lce_rescale_exp_rows_kernel<<<dim3((unsigned)a.m, (unsigned)n_chunks), 256, 0, stream>>>(a);
+  lce_exp_from_logits_kernel<<<dim3((unsigned)a.m_pad, (unsigned)ceil_div(a.width, 2048)), 256, 0,
+                               stream>>>(a);
+  TLCE_LAUNCH_CHECK();
+  return 0;
+}
+
+int launch_rescale_exp_rows(const RescaleExpArgs& a, int n_panels, hipStream_t stream) {
+  if (n_panels <= 0 || a.m <= 0) return 0;
+  ScopedTimer timer(kClassOther, stream);
+  lce_rescale_exp_rows_kernel<<<dim3((unsigned)a.m, (unsigned)n_panels), 256, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }

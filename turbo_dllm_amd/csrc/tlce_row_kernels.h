@@ -154,14 +154,14 @@ __device__ __forceinline__ void topk_workgroup_best(float& best_val, int64_t& be
   }
 }
 
-// What bounds it is reading the logits once (and, with kEmit, writing half as many bytes):
-// every thread loads 8 pieces of four consecutive logits per chunk, and the exponentials of
-// the running sum are the entries that are written.  Measured on 8192 rows, V = 151936,
-// k = 16 in five panels: 2.44 ms (7.5 GB, 3.1 TB/s) against 2.32 for the scan (256 threads of
-// 64 logits in scalar loads) and 1.41 for a pass of its own that read the logits again and
-// wrote the entries.  512 threads of 32 logits: with 64 a thread the entries spill or leave
-// one wave per SIMD (4.8 ms).
-template <bool kEmit>
+// What bounds it is reading the logits once: every thread loads 8 pieces of four consecutive
+// logits per chunk, and the few threads that hold a candidate read their logits again.
+// Measured on 8192 rows, V = 151936, k = 16 in five panels: 2.32 ms with 256 threads of 64
+// logits in scalar loads, 2.03 now (2.5 TB/s).  512 threads of 32 logits: with 64 a thread one wave
+// per SIMD is left.  The entries of the gradient panel are not written here but by a pass of
+// their own after a whole panel's scan (1.41 ms): written chunk by chunk, more of them are
+// rounded a second time when a row's maximum grows (d lse / d hidden in float32 against
+// float64, 1500 rows, H = 512: 1.24e-4 per panel, 1.54e-4 per chunk).
 __global__ __launch_bounds__(kTopkScanThreads, 6) void lce_topk_scan_kernel(TopkScanArgs p) {
   constexpr int kThreads = kTopkScanThreads;
   constexpr int kWaves = kThreads / 64;
@@ -183,14 +183,6 @@ __global__ __launch_bounds__(kTopkScanThreads, 6) void lce_topk_scan_kernel(Topk
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
   const int row = blockIdx.x;
-  __bf16* exp_row = nullptr;
-  if constexpr (kEmit) {
-    exp_row = static_cast<__bf16*>(p.exp_out) + (int64_t)row * p.ld_out + p.v0;
-    if (row >= p.m) {
-      for (int c = 4 * t; c < p.stored; c += 4 * kThreads) store4<__bf16>(exp_row + c, 0.0f, 0.0f, 0.0f, 0.0f);
-      return;
-    }
-  }
   const float* src = p.panel + (int64_t)row * p.ld;
   float run_max = p.first ? -INFINITY : p.run_max[row];
   float run_sum = p.first ? 0.0f : p.run_sum[row];
@@ -226,29 +218,10 @@ __global__ __launch_bounds__(kTopkScanThreads, 6) void lce_topk_scan_kernel(Topk
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) new_max = fmaxf(new_max, wave_high[w]);
     float local_sum = 0.0f;
-    const bool any = new_max > -INFINITY;
-    const float inv_cap = kEmit && p.softcap > 0.0f ? 1.0f / p.softcap : 0.0f;
+    if (new_max > -INFINITY) {
 #pragma unroll
-    for (int i = 0; i < kPerThread; i += 4) {
-      float e[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float z = vals[i + u];
-        const float x = any ? __expf(z - new_max) : 0.0f;   // (-inf gives 0)
-        local_sum += x;
-        if constexpr (kEmit) {
-          e[u] = x;
-          if (p.softcap > 0.0f) {
-            const float q = z * inv_cap;
-            e[u] = z > -INFINITY ? x * (1.0f - q * q) : 0.0f;
-          }
-        }
-      }
-      if constexpr (kEmit) {
-        if (c0 + column(i) < p.stored) store4<__bf16>(exp_row + c0 + column(i), e[0], e[1], e[2], e[3]);
-      }
+      for (int i = 0; i < kPerThread; ++i) local_sum += __expf(vals[i] - new_max);   // (-inf gives 0)
     }
-    if (kEmit && t == 0) p.ref_used[(int64_t)(c0 / kChunk) * p.m_pad + row] = new_max;
     local_sum = wave_sum(local_sum);
     if (lane == 0) wave_exp[wave] = local_sum;
 
