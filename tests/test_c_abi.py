@@ -89,6 +89,16 @@ def test_workspace_sizes_and_plan():
     assert tight["n_panels"] > plan["n_panels"]
 
 
+@pytest.mark.parametrize("m,v", [(1, 100), (64, 87424), (300, 16384), (1000, 16384), (70000, 700)])
+def test_generic_engine_forward_has_four_workgroups_per_cu(m, v):
+    """64x64 tiles of which a CU needs four to hide their loads: token tiles x vocabulary
+    splits come to 1024 where the vocabulary has that many tiles."""
+    plan = _lib.query_plan(m, 1001, v, _lib.DTYPE_BF16, False)
+    assert plan["engine"] == "generic" and plan["tile"] == 64
+    ttiles, vtiles = -(-m // 64), -(-v // 64)
+    assert plan["forward_vocab_splits"] == min(max(1024 // ttiles, 1), vtiles)
+
+
 def test_bad_arguments_report_errors_without_a_gpu():
     lib = _lib.library()
     rc = lib.tlce_query_plan(1, 0, 5, _lib.DTYPE_BF16, 1, 0, None, None, None, None, None, None)

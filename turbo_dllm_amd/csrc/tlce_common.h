@@ -45,11 +45,12 @@ static inline int64_t align256(int64_t x) { return round_up(x, 256); }
 
 static inline int dtype_bytes(int dtype) { return dtype == TLCE_DTYPE_F32 ? 4 : 2; }
 
-// Workgroups of a tile engine that the 256 CUs hold at once: the float32 MFMA engine
-// (128x128 tiles) fits two on a CU, the 256x256 ones take a CU each, and the generic
-// 64x64 one is planned like those.
+// Workgroups of a tile engine that the 256 CUs hold at once: the 256x256 engines take a CU
+// each, the float32 MFMA engine (128x128 tiles) fits two on one.  The generic engine (64x64,
+// 9 KiB of LDS) needs four on a CU to hide its loads: planned for one, its forward took 2.73
+// instead of 1.18 ms (1000 bf16 rows, H = 1001, V = 16384).
 __host__ __device__ static inline int resident_workgroups(int tile) {
-  return tile == 128 ? 512 : 256;
+  return tile == 64 ? 1024 : tile == 128 ? 512 : 256;
 }
 
 // Forward launch shape: token tiles x vocabulary splits workgroups, at most four whole
@@ -104,7 +105,7 @@ __host__ __device__ static inline int grad_hidden_k_splits(int64_t tiles, int ma
                                                            int64_t k_steps, int64_t slab_elems,
                                                            int resident = 256) {
   const int64_t per_slab = (slab_elems >> 17) > 1 ? (slab_elems >> 17) : 1;
-  const int shift = resident == 512 ? 9 : 8;
+  const int shift = 31 - __builtin_clz(resident);
   int pick = 1;
   int64_t best = -1;
   for (int ks = 1; ks <= max_split; ++ks) {
