@@ -43,6 +43,7 @@ struct MfmaF32Engine {
   static constexpr int kSmemBytes = 2 * kStageBytes;           // 65536
   static constexpr bool kHasKMajor = true;
   static constexpr bool kPrecise = true;
+  static constexpr bool kReadsWhereUsed = false;
 
   struct Acc { acc4_t c[kTM][kTN]; };
 

@@ -58,6 +58,7 @@ struct MfmaTileLayout {
   static constexpr int kShare = 4;           // threads that hold the same column
   static constexpr int kWavesPerSimd = 1;
   static constexpr bool kPrecise = false;    // hardware exp / rcp approximations in the epilogues
+  static constexpr bool kReadsWhereUsed = false;
   static_assert(kWavesN * kTN * 32 == kTile, "waves must tile the 256 B rows");
 
   struct Acc { f32x16_t c[kTM][kTN]; };
@@ -260,6 +261,7 @@ struct DirectTileLayout {
   static constexpr int kStageCols = 2;           // owned columns per quarter of the tile
   static constexpr int kWavesPerSimd = 1;
   static constexpr bool kPrecise = false;
+  static constexpr bool kReadsWhereUsed = true;   // has read()
 
   struct Acc { acc4_t c[kTM][kTN]; };
 
@@ -286,6 +288,13 @@ struct DirectTileLayout {
   __device__ __forceinline__ int share_slot() const { return wm * 4 + (lane >> 4); }
   static __device__ __forceinline__ float get(const Acc& a, int j, int i) {
     return a.c[i >> 2][j][i & 3];
+  }
+  // The same, copied to a VGPR at this place: left to itself the compiler copies all 256
+  // accumulators at once where the first is used.
+  static __device__ __forceinline__ float read(const Acc& a, int j, int i) {
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a.c[i >> 2][j][i & 3]));
+    return v;
   }
   static __device__ __forceinline__ void set(Acc& a, int j, int i, float v) {
     a.c[i >> 2][j][i & 3] = v;

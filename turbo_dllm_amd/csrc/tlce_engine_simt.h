@@ -27,6 +27,7 @@ struct SimtEngine {
   static constexpr int kShare = 4;
   static constexpr bool kHasKMajor = false;
   static constexpr bool kPrecise = sizeof(T_) == 4;   // float32 inputs: library exp / tanh
+  static constexpr bool kReadsWhereUsed = false;
 
   struct Acc { float c[kRows]; };
 

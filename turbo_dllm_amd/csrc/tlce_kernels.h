@@ -92,49 +92,93 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_forward_sta
                        acc, smem);
     }
     const int vbase = vt * E::kTile;
-    if (kBias) {
-#pragma unroll
-      for (int i = 0; i < E::kRows; ++i) {
-        const float b = p.bias[min(vbase + eng.row(i), p.v - 1)];
-#pragma unroll
-        for (int j = 0; j < E::kCols; ++j)
-          E::set(acc, j, i, fmaf(E::get(acc, j, i), p.logit_scale, b));
-      }
-    }
     // Only the last vocabulary tile (rows past v) and the tile that holds the
     // excluded column need per-element masking: a workgroup-uniform branch.
     const bool edge = (vbase + E::kTile > p.v) ||
                       (p.exclude >= vbase && p.exclude < vbase + E::kTile);
-    if (kSoftcap || edge) {
-      asm volatile("" ::: "memory");   // keep this a real branch, not per-element selects
-      const int excluded = (int)p.exclude;
+    const int excluded = (int)p.exclude;
+    // online (max, sum-exp) in the base-2 domain: exp(z - m) = exp2(z*log2e - m2), one
+    // owned column after the other; `logit` makes a logit of accumulator element i
+    auto fold = [&](auto&& logit) {
+      auto element = [&](int j, int i) {
+        if constexpr (E::kReadsWhereUsed) return E::read(acc, j, i);
+        else return E::get(acc, j, i);
+      };
 #pragma unroll
-      for (int i = 0; i < E::kRows; ++i) {
-        const int v = vbase + eng.row(i);
-        const bool ok = (v < p.v) && (v != excluded);
+      for (int j = 0; j < E::kCols; ++j) {
+        float z[E::kRows];
+        float tile_max = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < E::kCols; ++j) {
-          float z = E::get(acc, j, i);
-          if (kSoftcap) z = p.softcap * tanh_of<E::kPrecise>(z * inv_cap);
-          E::set(acc, j, i, ok ? z : -INFINITY);
+        for (int i = 0; i < E::kRows; ++i) {
+          z[i] = logit(i, element(j, i));
+          tile_max = fmaxf(tile_max, z[i]);
         }
-      }
-    }
-    // online (max, sum-exp) in the base-2 domain: exp(z - m) = exp2(z*log2e - m2)
-#pragma unroll
-    for (int j = 0; j < E::kCols; ++j) {
-      float tile_max = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < E::kRows; ++i) tile_max = fmaxf(tile_max, E::get(acc, j, i));
-      const float new_max = fmaxf(run_max[j], tile_max * log2e_scaled);
-      if (new_max > -INFINITY) {
-        float s = run_sum[j] * exp2_of<E::kPrecise>(run_max[j] - new_max);
+        const float new_max = fmaxf(run_max[j], tile_max * log2e_scaled);
+        const bool any = new_max > -INFINITY;
+        const float base = any ? new_max : 0.0f;
+        float s = run_sum[j] * exp2_of<E::kPrecise>(run_max[j] - base);
 #pragma unroll
         for (int i = 0; i < E::kRows; ++i)
-          s += exp2_of<E::kPrecise>(fmaf(E::get(acc, j, i), log2e_scaled, -new_max));
-        run_sum[j] = s;
+          s += exp2_of<E::kPrecise>(fmaf(z[i], log2e_scaled, -base));
+        run_sum[j] = any ? s : run_sum[j];
         run_max[j] = new_max;
+        if (E::kReadsWhereUsed) __builtin_amdgcn_sched_barrier(0);
       }
+    };
+    if constexpr (E::kReadsWhereUsed) {
+      // Bias, soft cap and mask as the elements are read: masked in place, the compiler
+      // copied all 256 accumulators at once and kept the running pairs in scratch memory,
+      // a round trip per column and tile.  A tile takes 3.2 us beside its K loop, was 8.1
+      // (9000 rows, V = 131072: H = 512 1.40 -> 1.06 ms, H = 1600 3.09 -> 2.82).
+      float bias[kBias ? E::kRows : 1];
+      if (kBias) {
+#pragma unroll
+        for (int i = 0; i < E::kRows; ++i) bias[i] = p.bias[min(vbase + eng.row(i), p.v - 1)];
+        // waited for here: loads that may still be pending at the next tile would have
+        // the compiler wait for all of its K loop's loads in every step
+#pragma unroll
+        for (int i = 0; i < E::kRows; ++i) asm volatile("" : "+v"(bias[i]));
+      }
+      auto logit = [&](int i, float z) {
+        if (kBias) z = fmaf(z, p.logit_scale, bias[i]);
+        if (kSoftcap) z = p.softcap * tanh_of<E::kPrecise>(z * inv_cap);
+        return z;
+      };
+      if (edge) {
+        fold([&](int i, float z) {
+          const int v = vbase + eng.row(i);
+          const bool ok = (v < p.v) & (v != excluded);
+          z = logit(i, z);
+          return ok ? z : -INFINITY;
+        });
+      } else {
+        fold(logit);
+      }
+    } else {
+      if (kBias) {
+#pragma unroll
+        for (int i = 0; i < E::kRows; ++i) {
+          const float b = p.bias[min(vbase + eng.row(i), p.v - 1)];
+#pragma unroll
+          for (int j = 0; j < E::kCols; ++j)
+            E::set(acc, j, i, fmaf(E::get(acc, j, i), p.logit_scale, b));
+        }
+      }
+      if (kSoftcap || edge) {
+        asm volatile("" ::: "memory");   // keep this a real branch, not per-element selects
+#pragma unroll
+        for (int i = 0; i < E::kRows; ++i) {
+          const int v = vbase + eng.row(i);
+          const bool ok = (v < p.v) && (v != excluded);
+#pragma unroll
+          for (int j = 0; j < E::kCols; ++j) {
+            float z = E::get(acc, j, i);
+            if (kSoftcap) z = p.softcap * tanh_of<E::kPrecise>(z * inv_cap);
+            E::set(acc, j, i, ok ? z : -INFINITY);
+          }
+        }
+      }
+      fold([](int, float z) { return z; });
     }
   }
 
