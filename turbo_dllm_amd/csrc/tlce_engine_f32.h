@@ -111,11 +111,11 @@ struct MfmaF32Engine {
     }
   }
 
-  template <bool kAKMajor, bool kBKMajor, bool kOverwrite = false>
+  template <bool kAKMajor, bool kBKMajor>
   __device__ __forceinline__ void mainloop_ex(const Operand<float>& A, const Operand<float>& B,
                                               int k_begin, int k_end, Acc& acc,
                                               char* smem) const {
-    if (kOverwrite) zero(acc);
+    zero(acc);
     acc4_t ra[4], rb[4];
     const int slot = (lane >> 4) ^ ((lane >> 1) & 7);
     const char* a_base = smem + (wm * 64 + (lane & 15)) * 128;
@@ -168,7 +168,7 @@ struct MfmaF32Engine {
                                                Acc& acc, char* smem) const {
     const Operand<float> a = {A, lda, a_row0, a_rows};
     const Operand<float> b = {B, ldb, b_row0, b_rows};
-    mainloop_ex<false, false, true>(a, b, k_begin, k_end, acc, smem);
+    mainloop_ex<false, false>(a, b, k_begin, k_end, acc, smem);
   }
 };
 

@@ -573,15 +573,14 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // acc += A-tile * B-tile^T over K in [k_begin, k_end), a multiple of 64 wide.
+  // acc = A-tile * B-tile^T over K in [k_begin, k_end), a multiple of 64 wide and not empty
+  // (the first 64 MFMAs take a zero constant as their addend, which saves zeroing 256
+  // accumulator registers per tile).
   // K-contiguous operand: tile rows row0 .. row0+256 of x (rows clamped to
   // x.rows - 1).  K-major operand: tile columns row0 .. row0+256 of x (16-byte
   // column chunks clamped to the last valid one; x.rows is a multiple of 8); the K
   // rows in [k_begin, k_end) must exist up to k_full, and in the tail from there on.
-  // kOverwrite: acc = A-tile * B-tile^T instead (the incoming acc is ignored: the
-  // first 64 MFMAs take a zero constant as their addend, which saves zeroing
-  // 256 accumulator registers per tile).
-  template <bool kAKMajor, bool kBKMajor, bool kOverwrite = false>
+  template <bool kAKMajor, bool kBKMajor>
   __device__ __forceinline__ void mainloop_ex(const Operand<T>& A, const Operand<T>& B,
                                               int k_begin, int k_end, Acc& acc,
                                               char* smem) const {
@@ -633,7 +632,7 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     auto step = [&](int k, auto tiles_left_tag, auto first_tag) {
       constexpr bool kHasNext = decltype(tiles_left_tag)::value >= 1;
       constexpr bool kHasTwo = decltype(tiles_left_tag)::value >= 2;
-      constexpr bool kFirst = decltype(first_tag)::value;   // first step of an overwriting loop
+      constexpr bool kFirst = decltype(first_tag)::value;   // the first step sets the accumulators
       const int cur = k & 1;
       const int nxt = cur ^ 1;
       // fragments the allocator has moved between two steps with VALU copies: two wait
@@ -703,13 +702,10 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     using Left0 = std::integral_constant<int, 0>;
     using Left1 = std::integral_constant<int, 1>;
     using Left2 = std::integral_constant<int, 2>;
-    int k = 0;
-    if constexpr (kOverwrite) {
-      if (nk > 2) step(0, Left2{}, std::true_type{});
-      else if (nk == 2) step(0, Left1{}, std::true_type{});
-      else step(0, Left0{}, std::true_type{});
-      k = 1;
-    }
+    if (nk > 2) step(0, Left2{}, std::true_type{});
+    else if (nk == 2) step(0, Left1{}, std::true_type{});
+    else step(0, Left0{}, std::true_type{});
+    int k = 1;
     for (; k + 2 < nk; ++k) step(k, Left2{}, std::false_type{});
     if (k + 2 == nk) step(k++, Left1{}, std::false_type{});
     if (k < nk) step(k, Left0{}, std::false_type{});
@@ -718,23 +714,14 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     __syncthreads();
   }
 
-  __device__ __forceinline__ void mainloop(const T* __restrict__ A, int64_t lda, int a_row0,
-                                           int a_rows, const T* __restrict__ B, int64_t ldb,
-                                           int b_row0, int b_rows, int k_begin, int k_end,
-                                           Acc& acc, char* smem) const {
-    const Operand<T> a = {A, lda, a_row0, a_rows};
-    const Operand<T> b = {B, ldb, b_row0, b_rows};
-    mainloop_ex<false, false>(a, b, k_begin, k_end, acc, smem);
-  }
-
-  // acc = A * B^T over a non-empty K range (same operands as mainloop).
+  // The same with both operands K-contiguous.
   __device__ __forceinline__ void mainloop_set(const T* __restrict__ A, int64_t lda, int a_row0,
                                                int a_rows, const T* __restrict__ B, int64_t ldb,
                                                int b_row0, int b_rows, int k_begin, int k_end,
                                                Acc& acc, char* smem) const {
     const Operand<T> a = {A, lda, a_row0, a_rows};
     const Operand<T> b = {B, ldb, b_row0, b_rows};
-    mainloop_ex<false, false, true>(a, b, k_begin, k_end, acc, smem);
+    mainloop_ex<false, false>(a, b, k_begin, k_end, acc, smem);
   }
 };
 

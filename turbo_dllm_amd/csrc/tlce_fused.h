@@ -527,9 +527,9 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
                                                      p.vp / 64, rows * h));
     ReduceSlabsArgs rs;
     if (m_dev != nullptr) {
-      // The block may hold far fewer rows than it was sized for (down to none): up to 16
-      // splits are launched and the kernel takes as many as the real rows call for,
-      // within the slab memory the plan allocated; the others exit at once.
+      // The block may hold far fewer rows than it was sized for (down to none): at least
+      // 16 splits (or the plan's, if more) are launched and the kernel takes as many as the
+      // real rows call for, within the slab memory the plan allocated; the others exit at once.
       dh.m_dev = m_dev; dh.m_role = kRowsFollow; dh.m_dev_offset = r0;
       dh.slab_budget = (int64_t)p.dh_ksplit * p.block_rows * h;
       dh.k_steps_plan = (int)(p.vp / 64);

@@ -284,10 +284,14 @@ int launch_forward(const Plan& p, const ForwardArgs& a, hipStream_t stream) {
   return launch_forward_variant<E, false, false>(p, a, stream);
 }
 
-// The same over a head stored [h, v] (engines with K-major operand loaders).
+// The engine that takes a head stored [h, v] in place (dim_first_in_place).
+template <class E>
+constexpr bool kTakesDimFirst = E::kHasKMajor && sizeof(typename E::T) == 2;
+
+// The same over a head stored [h, v].
 template <class E>
 int launch_forward_dim_first(const Plan& p, const ForwardArgs& a, hipStream_t stream) {
-  if constexpr (E::kHasKMajor) {
+  if constexpr (kTakesDimFirst<E>) {
     const bool softcap = a.softcap > 0.0f, bias = a.bias != nullptr;
     if (softcap && bias) return launch_forward_variant<E, true, true, true>(p, a, stream);
     if (softcap) return launch_forward_variant<E, true, false, true>(p, a, stream);
@@ -312,10 +316,10 @@ int launch_grad_logits_variant(const GradLogitsArgs& a, hipStream_t stream) {
   return 0;
 }
 
-// The logit-gradient panel over a head stored [h, v] (engines with K-major loaders).
+// The logit-gradient panel over a head stored [h, v].
 template <class E>
 int launch_grad_logits_dim_first(const GradLogitsArgs& a, hipStream_t stream) {
-  if constexpr (E::kHasKMajor) {
+  if constexpr (kTakesDimFirst<E>) {
     const bool softcap = a.softcap > 0.0f, bias = a.bias != nullptr;
     if (softcap && bias) return launch_grad_logits_variant<E, true, true, true>(a, stream);
     if (softcap) return launch_grad_logits_variant<E, true, false, true>(a, stream);
@@ -492,8 +496,8 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     dh.c_split_stride = p.mp * h;
     dh.mode = (panel == 0) ? kStoreF32 : kAddF32;
     dh.m_dev = m_dev; dh.m_role = kRowsFollow;
-    // device-side row count: up to four K splits are launched and the kernel picks
-    // how many to use for the real count, within the slabs the plan allocated
+    // device-side row count: at least four K splits (or the plan's, if more) are launched
+    // and the kernel picks how many to use for the real count, within the slabs the plan allocated
     const int dh_launch_ksplit =
         m_dev == nullptr ? p.dh_ksplit : std::max(p.dh_ksplit, std::min(4, p.dh_max_ksplit));
     dh.slab_budget = (int64_t)p.dh_ksplit * p.mp * h;
@@ -507,30 +511,32 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     dw.c_split_stride = 0;
     dw.mode = kStoreT;
     if constexpr (E::kHasKMajor) {
-      if (p.kmajor && dim_first) {
-        // The head is stored [h, v].  grad_hidden: A = its columns [v0, v0+K), which
-        // are K-contiguous rows of the stored matrix; B = G.
-        dh.a = weight_t + v0; dh.lda = v; dh.a_rows = (int)h;
-        dh.k = (int)round_up(rows_valid, kSlab);
-        if (int rc = launch_gemm<E, false, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
-          return rc;
-        if (weight_grad) {
-          // grad_weight [h, v]: the roles of the operands swap so that the hidden axis
-          // becomes the output's rows: A = G (its panel columns), B = hidden, both K-major
-          GemmArgs dwt = dw;
-          dwt.a = g; dwt.lda = p.vc; dwt.a_rows = (int)width;
-          dwt.b = hidden_t; dwt.ldb = h; dwt.b_rows = (int)h;
-          dwt.k = (int)m64;
-          if (m64 != m && m_dev == nullptr) {
-            dwt.b_tail = ht;
-            dwt.b_k_full = (int)(m64 - kSlab);
+      if constexpr (kTakesDimFirst<E>) {
+        if (dim_first) {
+          // The head is stored [h, v].  grad_hidden: A = its columns [v0, v0+K), which
+          // are K-contiguous rows of the stored matrix; B = G.
+          dh.a = weight_t + v0; dh.lda = v; dh.a_rows = (int)h;
+          dh.k = (int)round_up(rows_valid, kSlab);
+          if (int rc = launch_gemm<E, false, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
+            return rc;
+          if (weight_grad) {
+            // grad_weight [h, v]: the roles of the operands swap so that the hidden axis
+            // becomes the output's rows: A = G (its panel columns), B = hidden, both K-major
+            GemmArgs dwt = dw;
+            dwt.a = g; dwt.lda = p.vc; dwt.a_rows = (int)width;
+            dwt.b = hidden_t; dwt.ldb = h; dwt.b_rows = (int)h;
+            dwt.k = (int)m64;
+            if (m64 != m && m_dev == nullptr) {
+              dwt.b_tail = ht;
+              dwt.b_k_full = (int)(m64 - kSlab);
+            }
+            dwt.ni = (int)(width / p.tile); dwt.nj = p.n_htiles;
+            dwt.c = static_cast<T*>(grad_weight) + v0; dwt.ldc = v;
+            dwt.c_rows = (int)h; dwt.c_cols = (int)rows_valid;
+            if (int rc = launch_gemm<E, true, true>(dwt, 1, kClassGradWeight, stream)) return rc;
           }
-          dwt.ni = (int)(width / p.tile); dwt.nj = p.n_htiles;
-          dwt.c = static_cast<T*>(grad_weight) + v0; dwt.ldc = v;
-          dwt.c_rows = (int)h; dwt.c_cols = (int)rows_valid;
-          if (int rc = launch_gemm<E, true, true>(dwt, 1, kClassGradWeight, stream)) return rc;
+          continue;
         }
-        continue;
       }
       if (p.kmajor) {
         // grad_hidden: A = weight rows [v0, v0+K) as stored (K-major), B = G

@@ -86,7 +86,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_forward_sta
     if constexpr (kWDimFirst) {
       const Operand<T> a = {weight, p.v, vt * E::kTile, p.v};
       const Operand<T> b = {hidden, p.h, tt * E::kTile, p.m};
-      eng.template mainloop_ex<true, false, true>(a, b, 0, p.h, acc, smem);
+      eng.template mainloop_ex<true, false>(a, b, 0, p.h, acc, smem);
     } else {
       eng.mainloop_set(weight, p.h, vt * E::kTile, p.v, hidden, p.h, tt * E::kTile, p.m, 0, p.h,
                        acc, smem);
@@ -478,7 +478,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
   if constexpr (kWDimFirst) {   // the head as stored, [h, v]: a K-major operand
     const Operand<T> a = {weight, p.v, vbase, p.v};
     const Operand<T> b = {hidden, p.h, tt * E::kTile, p.m};
-    eng.template mainloop_ex<true, false, true>(a, b, 0, p.h, acc, smem);
+    eng.template mainloop_ex<true, false>(a, b, 0, p.h, acc, smem);
   } else {
     eng.mainloop_set(weight, p.h, vbase, p.v, hidden, p.h, tt * E::kTile, p.m, 0, p.h, acc, smem);
   }
@@ -1149,8 +1149,9 @@ struct GemmArgs {
   const void* b;
   int64_t ldb;
   int b_rows;
-  int k;            // padded K, multiple of the engine's BK
-  int k_per_split;  // multiple of BK
+  int k;            // K; a multiple of 64 for the direct engine, of 256 for the staged and of 64
+                    // for the generic one (padded copies), any for the float32 engine
+  int k_per_split;  // multiple of the engine's BK
   int ni, nj;       // tiles along A rows / B rows
   void* c;          // [c_rows, ldc]: row = B row, column = A row
   int64_t ldc;
@@ -1382,7 +1383,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
                           static_cast<const T*>(p.a_tail), p.a_k_full};
     const Operand<T> b = {static_cast<const T*>(p.b), p.ldb, tj * E::kTile, p.b_rows,
                           static_cast<const T*>(p.b_tail), p.b_k_full};
-    eng.template mainloop_ex<kAKMajor, kBKMajor, true>(a, b, k_begin, k_end, acc, smem);
+    eng.template mainloop_ex<kAKMajor, kBKMajor>(a, b, k_begin, k_end, acc, smem);
   } else {
     eng.mainloop_set(static_cast<const T*>(p.a), p.lda, ti * E::kTile, p.a_rows,
                      static_cast<const T*>(p.b), p.ldb, tj * E::kTile, p.b_rows, k_begin, k_end,
