@@ -103,3 +103,47 @@ def test_main_loops_wait_for_no_more_than_the_tile_they_need(kernels):
             waits = [b for b in body if b.startswith("s_waitcnt") and "vmcnt" in b]
             assert waits == ["s_waitcnt vmcnt(1)"], (name, waits)
     assert loops >= len(kernels) // 2
+
+
+def _registers(operand):
+    """v5, v[4:7], a[0:3] -> {("v", 5)} ..."""
+    match = re.fullmatch(r"([va])(?:(\d+)|\[(\d+):(\d+)\])", operand.strip())
+    if not match:
+        return frozenset()
+    first = int(match[2] or match[3])
+    return frozenset((match[1], r) for r in range(first, int(match[4] or first) + 1))
+
+
+def _operands(line):
+    return [_registers(part) for part in line.partition(" ")[2].split(",")]
+
+
+def _issued(line):
+    """Wait states an instruction stands for (a 16x16x32 MFMA holds its pipe for four)."""
+    return int(line.split()[1]) + 1 if line.startswith("s_nop") else 4 if line.startswith("v_mfma") else 1
+
+
+def test_wait_states_around_the_asm_matrix_instructions(kernels):
+    """The compiler adds no wait states for instructions in asm statements: an MFMA must not
+    follow a vector instruction that writes one of its operands by less than two of them,
+    and its result must not be read by another kind of instruction for 19."""
+    checked = 0
+    for name, (_, code) in kernels.items():
+        parsed = [_operands(line) for line in code]
+        for at, line in enumerate(code):
+            matrix = line.startswith("v_mfma")
+            stores = not line.startswith("v_")
+            sources = frozenset().union(*parsed[at][0 if stores else 1:])
+            if not matrix:
+                sources = frozenset(r for r in sources if r[0] == "a")
+            if not sources:
+                continue
+            checked += 1
+            waited, back = 0, at - 1
+            while back >= 0 and waited < (2 if matrix else 19):
+                before = code[back]
+                if before.startswith("v_mfma" if not matrix else "v_") and before.startswith("v_mfma") != matrix:
+                    assert not parsed[back][0] & sources, (name, before, line)
+                waited += _issued(before)
+                back -= 1
+    assert checked > 100 * len(kernels)
