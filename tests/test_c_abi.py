@@ -74,7 +74,7 @@ def test_workspace_sizes_and_plan():
     assert frozen <= bwd
     # float32 grad_hidden accumulators + one bf16 panel + per-row scales, nothing else
     assert bwd == 32768 * 4096 * 4 + plan["panel_columns"] * 32768 * 2 + 32768 * 4
-    # a vocabulary that is not a multiple of 64 falls back to transposed operand copies
+    # a vocabulary that is not a multiple of 64 needs a padded copy of the head's last rows
     assert lib.tlce_backward_workspace_bytes(32768, 4096, 151937, _lib.DTYPE_BF16, 1, 0, 0) > bwd
     # few loss rows: the grad-hidden contraction splits K to fill the GPU
     small = _lib.query_plan(1750, 4096, 151936, _lib.DTYPE_BF16, True)

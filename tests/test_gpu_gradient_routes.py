@@ -10,7 +10,10 @@ backward are held to the middle of the two, 2.6e-3."""
 import pytest
 import torch
 
+import linear_ce_oracle as oracle
 from turbo_dllm_amd import _lib, options
+from turbo_dllm_amd.dflash_kl import frozen_linear_kl
+from turbo_dllm_amd.dflash_linear_topk import frozen_linear_ce_topk
 from turbo_dllm_amd.streaming_soft_embedding import streaming_soft_embedding
 from turbo_dllm_amd.tiled_linear_cross_entropy import tiled_linear_cross_entropy
 
@@ -130,3 +133,94 @@ def test_per_token_losses_beyond_one_block_recompute(gpu_device):
     error = relative_norm(got[2], exact_grad_weight(hidden, weight, labels, up.double()))
     print("[case] grad_weight error", error, flush=True)
     assert error <= TWO_ROUNDINGS
+
+
+# KL and CE with top-k form their gradients in the forward over any vocabulary: the last K
+# slab of the contraction over it comes from a zero-padded copy of the head's last rows
+RAGGED = [(1, 64, 2), (65, 64, 63), (130, 128, 65), (257, 192, 191), (300, 256, 4099)]
+
+
+@pytest.mark.parametrize("softcap", [None, 20.0])
+@pytest.mark.parametrize("m,h,v", RAGGED)
+def test_ragged_kl_gradient_in_the_forward(gpu_device, m, h, v, softcap):
+    """Loss and gradient at the operator's bars for bf16 (rtol 2e-2 / atol 1e-3, relative
+    max-norm 2e-2 of the float64 oracle)."""
+    print("[case]", m, h, v, softcap, flush=True)
+    gen = torch.Generator().manual_seed(m + v)
+    cpu = [(torch.randn(n, h, generator=gen) * std).bfloat16()
+           for n, std in ((m, 1.0), (v, 0.2), (m, 1.0), (v, 0.2))]
+    ops = [t.to(gpu_device) for t in cpu]
+    up = torch.rand(m, generator=gen) + 0.1
+    x = ops[0].clone().requires_grad_(True)
+    with _lib.kernel_profile() as prof:
+        losses = frozen_linear_kl(x, *ops[1:], logit_softcap=softcap)
+    assert prof.launches["grad_hidden_gemm"] == 1
+    losses.backward(up.to(gpu_device))
+    torch.cuda.synchronize()
+    want = oracle.dense_frozen_kl(*cpu, logit_softcap=softcap)
+    torch.testing.assert_close(losses.detach().cpu().double(), want, rtol=2e-2, atol=1e-3)
+    grad = oracle.dense_frozen_kl_grad(*cpu, up, logit_softcap=softcap)
+    assert oracle.relative_max_error(x.grad, grad) <= 2e-2
+
+
+@pytest.mark.parametrize("softcap", [None, 20.0])
+@pytest.mark.parametrize("m,h,v", RAGGED)
+def test_ragged_top_k_gradient_in_the_forward(gpu_device, m, h, v, softcap):
+    print("[case]", m, h, v, softcap, flush=True)
+    k = min(v, 7)
+    gen = torch.Generator().manual_seed(m + v)
+    hidden = torch.randn(m, h, generator=gen).bfloat16()
+    weight = (torch.randn(v, h, generator=gen) * 0.2).bfloat16()
+    labels = torch.randint(0, v, (m,), generator=gen)
+    up = torch.rand(3, m, generator=gen)
+    x = hidden.to(gpu_device).requires_grad_(True)
+    with _lib.kernel_profile() as prof:
+        loss, prob, values, ids = frozen_linear_ce_topk(
+            x, weight.to(gpu_device), labels.to(gpu_device), top_k=k, logit_softcap=softcap)
+    assert prof.launches["grad_hidden_gemm"] == 1
+    g = up.to(gpu_device)
+    (loss * g[0] + prob * g[1] + values.mean(1) * g[2]).sum().backward()
+    torch.cuda.synchronize()
+    z = hidden.double() @ weight.double().t()
+    z = z if softcap is None else softcap * torch.tanh(z / softcap)
+    want = torch.logsumexp(z, 1) - z.gather(1, labels[:, None])[:, 0]
+    torch.testing.assert_close(loss.detach().cpu().double(), want, rtol=1e-4, atol=1e-4)
+    grad = oracle.dense_ce_topk_grad(hidden, weight, labels, ids.cpu(), up[0], up[1],
+                                     up[2][:, None].expand(m, k) / k, logit_softcap=softcap)
+    assert oracle.relative_max_error(x.grad, grad) <= 2e-2
+
+
+def test_ragged_objectives_in_several_blocks_of_rows(gpu_device):
+    """V = 150001, 9000 rows: two blocks of the 2.5 GiB panel for each objective.  Gradients
+    against float64 in the 2-norm: entries rounded twice at most (when written, and where a
+    maximum moved) and the result once, 2.87e-3, and 8 % for the spread of one sample."""
+    m, h, v = 9000, 64, 150001
+    hidden, weight, labels, up = operands(gpu_device, m, h, v)
+    teacher, teacher_weight, _, _ = operands(gpu_device, m, h, v, seed=4)
+    x = hidden.clone().requires_grad_(True)
+    with _lib.kernel_profile() as prof:
+        losses = frozen_linear_kl(x, weight, teacher, teacher_weight)
+    assert prof.launches["grad_hidden_gemm"] == 2
+    losses.backward(up)
+    y = hidden.clone().requires_grad_(True)
+    with _lib.kernel_profile() as prof:
+        ce, _, _, _ = frozen_linear_ce_topk(y, weight, labels, top_k=4)
+    assert prof.launches["grad_hidden_gemm"] == 2
+    ce.backward(up)
+    w, tw = weight.double(), teacher_weight.double()
+    wants = [[], [], [], []]
+    for lo in range(0, m, 500):
+        part = slice(lo, lo + 500)
+        draft, factor = (hidden[part].double() @ w.t()).log_softmax(1), up[part, None].double()
+        target = (teacher[part].double() @ tw.t()).log_softmax(1)
+        wants[0].append((target.exp() * (target - draft)).sum(1))
+        wants[1].append(((draft.exp() - target.exp()) * factor) @ w)
+        wants[2].append(-draft.gather(1, labels[part, None])[:, 0])
+        wants[3].append(factor * (draft.exp() @ w - w[labels[part]]))
+    kl, kl_grad, nll, nll_grad = (torch.cat(t) for t in wants)
+    for got, want in ((losses, kl), (ce, nll)):
+        torch.testing.assert_close(got.detach().double(), want, rtol=1e-3, atol=1e-3)
+    for got, want in ((x.grad, kl_grad), (y.grad, nll_grad)):
+        error = relative_norm(got, want)
+        print("[case] gradient error", error, flush=True)
+        assert error <= 3.1e-3

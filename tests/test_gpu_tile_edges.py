@@ -63,7 +63,8 @@ def test_direct_engine_edges(gpu_device, m, h, v, dtype, mode):
 ])
 def test_direct_engine_ragged_vocabularies(gpu_device, m, h, v, kw, dtype, mode):
     """Vocabularies (K of the grad_hidden contraction) and row counts (K of grad_weight)
-    that end inside a 64-row K slab."""
+    that end inside a 64-row K slab, in the recomputing backward, which such heads take in
+    either mode."""
     with options.panel_budget((32 << 20) if v > 30000 and mode == "recompute" else 0):
         check(gpu_device, m, h, v, dtype, mode, **kw)
 
