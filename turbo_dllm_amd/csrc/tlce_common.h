@@ -169,7 +169,7 @@ __device__ __forceinline__ int xcd_logical_block_of(int bid, int tiles) {
 // workgroups fetch 33 strips instead of 12: 9 token tiles in groups of 4, 4, 1 took the
 // forward 1.51 ms against 1.28 balanced, 5 hidden tiles grad_weight 0.65 against 0.59).
 __device__ __forceinline__ void grouped_tile(int logical, int ni, int nj, int group,
-                                                      int* ti, int* tj) {
+                                             int* ti, int* tj) {
   const int n_groups = (ni + group - 1) / group;
   const int base = ni / n_groups, extra = ni % n_groups;   // the first `extra` groups hold base + 1
   const int big = (base + 1) * nj;
@@ -205,12 +205,26 @@ __device__ __forceinline__ void grouped_tile(int logical, int ni, int nj, int gr
 //               further groups, from the last-level cache, where all the i strips stay.
 //               Four tiles along j when only those fit beside the i strips.
 // By groups where the eighths are aligned, unless the strips are so short that the cache
-// holds them anyway.  Measured, ms by groups / by blocks (H, V = 4096, 151936 unless
-// stated): exponentiated logits of 32 token tiles 7.12 / 7.21, of 128 28.4 / 29.3, of 25
-// tiles 6.00 / 5.73, of 33 tiles over H = 3840, V = 262144 13.65 / 12.15, of 16 tiles
-// over H = 1024, V = 131072 1.06 / 1.01; grad_hidden of 15 hidden tiles 13.6 / 12.7;
-// grad_weight of 16 hidden tiles and 8192 rows 7.04 / 7.24, 1610 rows 1.71 / 1.62, of 15
-// hidden tiles 12.5 / 11.9.
+// holds them anyway.  The two limits, on the strips that eight tiles per XCD and all of i
+// make, are where the measured pairs cross (ms, bf16, V = 151936, H = 4096 unless stated;
+// E: exponentiated logits, W: grad_weight of 16 or, unaligned, of 15 hidden tiles, H = 3840).
+// By groups / by blocks of eight, aligned:
+//   40 MiB  E 4096 rows, H = 1024    1.36 / 1.30      90 MiB  E 4096, H = 2304   2.23 / 2.29
+//   50 MiB  W 1280 rows              1.49 / 1.40     100 MiB  W 2560             2.53 / 2.55
+//   60 MiB  E 4096, H = 1536         1.68 / 1.66     120 MiB  E 8192, H = 2560   4.81 / 4.89
+//   70 MiB  W 1792                   1.88 / 1.88     144 MiB  E 8192, H = 3072   5.57 / 5.65
+//   80 MiB  E 4096, H = 2048         2.04 / 2.04     192 MiB  E 8192             7.26 / 7.39
+//   96 MiB  E 8192, H = 2048         3.98 / 3.99     320 MiB  W 8192             7.35 / 7.65
+// By groups / blocks of eight / blocks of four, unaligned:
+//  165 MiB  E 6144 rows, H = 3840    5.31 / 5.29 / 5.28
+//  198 MiB  W 5120                   4.50 / 4.42 / 4.40
+//  206 MiB  E 8448, H = 4352         8.58 / 8.18 / 8.25
+//  242 MiB  E 8448, H = 5120        10.08 / 9.73 / 9.66
+//  316 MiB  W 8192                   7.27 / 7.21 / 6.98
+//  326 MiB  W 8448                   7.48 / 7.40 / 7.16
+// (past 224 MiB for blocks of four too, eight are taken: 12288 rows W 10.71 / 10.87 / 10.65,
+// grad_hidden over the whole vocabulary 10.61 / 10.87 / 10.99, in 15 hidden tiles of 8448
+// rows 7.65 / 7.12 / 7.22)
 __device__ __forceinline__ bool xcd_tile(int bid, int ni, int nj, int64_t strip, int* ti,
                                          int* tj) {
   const int64_t total = (int64_t)ni * nj;
