@@ -142,8 +142,9 @@ int tlce_forward(const void* hidden, const void* weight, const float* bias,
 /* tlce_forward for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has
  * no counterpart in the reference.  Same arguments and results as tlce_forward
- * minus the workspace: the per-split softmax partials, the forward's only
- * scratch memory, live in a device array of TLCE_FORWARD_NOALLOC_SCRATCH_BYTES
+ * minus the workspace: the per-split softmax partials, its only scratch
+ * memory (float32 stays on the float32 kernels here, where tlce_forward may
+ * lay its operands out in bf16 planes: other roundings), live in a device array of TLCE_FORWARD_NOALLOC_SCRATCH_BYTES
  * that is part of the library image (every GPU the library runs on holds its
  * copy until the process ends).  The call allocates and frees nothing.
  *   - m beyond TLCE_FORWARD_NOALLOC_MAX_ROWS (more partials than the array
@@ -614,7 +615,9 @@ int tlce_grad_weight_from_panel(const void* hidden, const int64_t* row_idx,
  * NULL.  `engine` is 2 for the bf16/f16 MFMA kernels with direct-to-LDS loads
  * (h a multiple of 64), 1 for the register-staged MFMA kernels (h a multiple of
  * 8), 3 for the float32 MFMA kernels (float32 inputs, h a multiple of 4, v at
- * least 64), 0 for the generic float32-FMA kernels (the rest). */
+ * least 64), 0 for the generic float32-FMA kernels (the rest).  Float32 cross
+ * entropies of some size (more than 384 rows, h >= 512) run instead on the bf16
+ * matrix units, on operands in three planes; their plan is not shown here. */
 int tlce_query_plan(int64_t m, int64_t h, int64_t v, int dtype,
                     int compute_weight_grad, int64_t panel_bytes,
                     int* engine, int64_t* tile, int64_t* forward_vocab_splits,

@@ -27,7 +27,9 @@ LIBRARY_PATH = PACKAGE_DIR / LIBRARY_NAME
 # per engine, and once per kernel family for the two direct-to-LDS MFMA engines,
 # whose kernels take the longest to compile.
 _SPLIT_ENGINES = {"direct_bf16": "MfmaDirect4Engine<__bf16>",
-                  "direct_f16": "MfmaDirect4Engine<_Float16>"}
+                  "direct_f16": "MfmaDirect4Engine<_Float16>",
+                  # float32 operands as three bf16 planes: cross entropies only
+                  "split_f32": "SplitF32Engine"}
 _WHOLE_ENGINES = {"staged_bf16": "MfmaEngine<__bf16>", "staged_f16": "MfmaEngine<_Float16>",
                   "mfma_f32": "MfmaF32Engine", "generic_f32": "SimtEngine<float>",
                   "generic_bf16": "SimtEngine<__bf16>", "generic_f16": "SimtEngine<_Float16>"}
@@ -36,16 +38,19 @@ _PARTS = {2: "grad_logits", 7: "grad_logits_cap", 8: "grad_logits_bias", 9: "gra
           10: "forward_dim_first", 11: "grad_logits_dim_first", 12: "exp_panel"}
 # the forward that leaves the gradients (part 12 and its launch sequence) exists for bf16 only
 _FUSED_ENGINES = ("direct_bf16",)
+_SPLIT_F32_PARTS = (1, 2, 3, 7, 8, 9)   # its launch sequences are tlce_split_f32.hip
 UNITS = (
     [(f"engine_{tag}_{name}", "tlce_engine_unit.hip",
       (f"-DTLCE_UNIT_ENGINE={engine}", f"-DTLCE_UNIT_PART={part}")
       + (("-DTLCE_UNIT_FUSED=1",) if tag in _FUSED_ENGINES else ()))
      for tag, engine in _SPLIT_ENGINES.items() for part, name in _PARTS.items()
-     if part != 12 or tag in _FUSED_ENGINES]
+     if (part in _SPLIT_F32_PARTS if tag == "split_f32"
+         else part != 12 or tag in _FUSED_ENGINES)]
     + [(f"engine_{tag}", "tlce_engine_unit.hip",
         (f"-DTLCE_UNIT_ENGINE={engine}", "-DTLCE_UNIT_PART=0"))
        for tag, engine in _WHOLE_ENGINES.items()]
-    + [("linear_ce", "tlce_linear_ce.hip", ()), ("compact", "tlce_compact.hip", ())]
+    + [("linear_ce", "tlce_linear_ce.hip", ()), ("split_f32", "tlce_split_f32.hip", ()),
+       ("compact", "tlce_compact.hip", ())]
 )
 OFFLOAD_ARCH = "gfx950"
 

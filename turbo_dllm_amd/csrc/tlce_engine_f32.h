@@ -1,5 +1,6 @@
 // 128x128 float32 MFMA tile engine: float32 inputs whose hidden size is a multiple of 4
-// (16-byte rows); others take the generic engine.
+// (16-byte rows); others take the generic engine.  Cross entropies of some size run on
+// the bf16 matrix units instead (tlce_split_f32.h).
 //
 // Same contract as the other engines: C[i][j] = sum_k A[i][k] * B[j][k] over one tile,
 // every product and sum in float32 (v_mfma_f32_16x16x4_f32), operands K-contiguous
@@ -32,6 +33,7 @@ struct MfmaF32Engine {
   using T = float;
   static constexpr int kTile = 128;
   static constexpr int kThreads = 256;
+  static constexpr int kPlanes = 1;
   static constexpr int kWavesPerSimd = 2;
   static constexpr int kBK = 32;
   static constexpr int kTM = 4, kTN = 4;             // 16-row blocks per wave

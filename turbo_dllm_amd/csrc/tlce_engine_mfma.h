@@ -56,6 +56,7 @@ struct MfmaTileLayout {
   static constexpr int kCols = kTN;          // tile columns owned per thread
   static constexpr int kRows = kTM * 16;     // tile rows held per owned column
   static constexpr int kShare = 4;           // threads that hold the same column
+  static constexpr int kPlanes = 1;
   static constexpr int kWavesPerSimd = 1;
   static constexpr bool kPrecise = false;    // hardware exp / rcp approximations in the epilogues
   static constexpr bool kReadsWhereUsed = false;
@@ -416,10 +417,18 @@ template <> struct DirectMfma<_Float16> {
   }
 };
 
-template <typename T_>
-struct MfmaDirect4Engine : DirectTileLayout<T_> {
+template <typename T_, int kPlanes_>
+struct DirectToLdsEngine : DirectTileLayout<T_> {
   using Base = DirectTileLayout<T_>;
   using T = T_;
+  // The K loop's passes over the planes of the operands (kPlanes == 1: one over the
+  // matrices themselves).  Plane of A and of B in pass s: nibble s of these.
+  static constexpr int kPlanes = kPlanes_;
+  static constexpr int kPasses = kPlanes == 1 ? 1 : 6;
+  static constexpr unsigned kPassPlaneA = kPlanes == 1 ? 0u : 0x001102u;
+  static constexpr unsigned kPassPlaneB = kPlanes == 1 ? 0u : 0x010120u;
+  static_assert(kPlanes == 1 || kPlanes == 3, "matrices as they are, or float32 in three planes");
+  static constexpr bool kPrecise = kPlanes > 1;              // float32 in, float32 epilogues
   using Op = DirectMfma<T_>;
   using V8 = typename MfmaOp<T_>::V8;
   using Acc = typename Base::Acc;
@@ -469,10 +478,11 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
   template <bool kKMajor>
   static __device__ __forceinline__ unsigned line_offset(const Operand<T>& x, int line) {
     if (!kKMajor) {
-      return (unsigned)((int64_t)(min(x.row0 + line, x.rows - 1) - x.row0) * x.ld * 2);
+      return (unsigned)((int64_t)(min(x.row0 + line, x.rows - 1) - x.row0) * x.ld * kPlanes * 2);
     } else {
       const int last_chunk = x.rows / 8 - 1 - x.row0 / 8;
-      return (unsigned)((int64_t)(line >> 2) * x.ld * 2 + min((line & 3) * 8, last_chunk) * 16);
+      return (unsigned)((int64_t)(line >> 2) * x.ld * kPlanes * 2 +
+                        min((line & 3) * 8, last_chunk) * 16);
     }
   }
 
@@ -485,6 +495,8 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     int64_t step;           // bytes between consecutive K tiles
     const char* last;       // K-major: base address of the last K tile (the operand's tail
                             // when the K range ends inside a 64-row slab)
+    const char* begin;      // base address of the first K tile in plane 0
+    int64_t plane;          // bytes from one plane to the next
   };
 
   template <bool kKMajor>
@@ -498,10 +510,10 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
         const int r = wave * 64 + j * 8 + (lane >> 3);
         const int chunk = (lane & 7) ^ ((r >> 1) & 7);
         const int rr = min(x.row0 + r, x.rows - 1) - x.row0;
-        ld.off[j] = (unsigned)((int64_t)rr * x.ld * 2 + chunk * 16);
+        ld.off[j] = (unsigned)((int64_t)rr * x.ld * kPlanes * 2 + chunk * 16);
       }
       ld.fill = __builtin_amdgcn_readfirstlane(lds_op + (unsigned)(wave * 64 * 128));
-      ld.next = reinterpret_cast<const char*>(x.ptr + (int64_t)x.row0 * x.ld + k_begin);
+      ld.next = reinterpret_cast<const char*>(x.ptr + (int64_t)x.row0 * x.ld * kPlanes + k_begin);
       ld.step = kBK * 2;
       ld.last = nullptr;
     } else {
@@ -512,16 +524,20 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
         const int kr = wave * 16 + j * 2 + (lane >> 5);
         const int swz = (4 * (kr & 3)) ^ (2 * ((kr >> 3) & 1));
         const int chunk = min((lane & 31) ^ swz, last_chunk);
-        ld.off[j] = (unsigned)((int64_t)kr * x.ld * 2 + chunk * 16);
+        ld.off[j] = (unsigned)((int64_t)kr * x.ld * kPlanes * 2 + chunk * 16);
       }
       ld.fill = __builtin_amdgcn_readfirstlane(lds_op + (unsigned)(wave * 16 * 512));
       const int k_last = k_begin + (nk - 1) * kBK;
       ld.last = reinterpret_cast<const char*>(
           (k_last >= x.k_full ? x.tail : x.ptr + (int64_t)k_last * x.ld) + x.row0);
-      ld.next = nk == 1 ? ld.last
-                        : reinterpret_cast<const char*>(x.ptr + (int64_t)k_begin * x.ld + x.row0);
-      ld.step = (int64_t)kBK * x.ld * 2;
+      ld.next = kPlanes == 1 && nk == 1
+                    ? ld.last
+                    : reinterpret_cast<const char*>(x.ptr + (int64_t)k_begin * x.ld * kPlanes +
+                                                    x.row0);
+      ld.step = (int64_t)kBK * x.ld * kPlanes * 2;
     }
+    ld.begin = ld.next;
+    ld.plane = x.ld * 2;
     return ld;
   }
 
@@ -585,13 +601,44 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
                                               int k_begin, int k_end, Acc& acc,
                                               char* smem) const {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
-    const int nk = (k_end - k_begin) / kBK;
+    const int pass_tiles = (k_end - k_begin) / kBK;   // K tiles of one pass
+    const int nk = pass_tiles * kPasses;
     Loader la = make_loader<kAKMajor>(A, k_begin, nk, lds0);
     Loader lb = make_loader<kBKMajor>(B, k_begin, nk, lds0 + kOperandBytes);
-    // the loaders move on to K tile `k`
+    // The place of a K tile among the passes, advanced one tile at a time.
+    struct Place { int pass, tile; };
+    auto next_place = [&](Place& at) {
+      if (++at.tile == pass_tiles) {
+        at.tile = 0;
+        ++at.pass;
+      }
+    };
+    // where a pass starts in an operand (no multiplication: the compiler forms 64-bit
+    // products in vector registers, and the loads take their base from scalar ones)
+    auto pass_start = [](const char* begin, int64_t plane, unsigned pass_planes, int pass) {
+      const unsigned which = (pass_planes >> (4 * pass)) & 15u;
+      return which == 0 ? begin : which == 1 ? begin + plane : begin + plane + plane;
+    };
+    Place load_at = {0, 0};
+    if constexpr (kPlanes > 1) {
+      la.next = pass_start(la.begin, la.plane, kPassPlaneA, 0);
+      lb.next = pass_start(lb.begin, lb.plane, kPassPlaneB, 0);
+    }
+    // the loaders move on to K tile `k`, the next one
     auto advance = [&](int k) {
-      la.next = kAKMajor && k == nk - 1 ? la.last : la.next + la.step;
-      lb.next = kBKMajor && k == nk - 1 ? lb.last : lb.next + lb.step;
+      if constexpr (kPlanes == 1) {
+        la.next = kAKMajor && k == nk - 1 ? la.last : la.next + la.step;
+        lb.next = kBKMajor && k == nk - 1 ? lb.last : lb.next + lb.step;
+      } else {
+        next_place(load_at);
+        if (load_at.tile != 0) {
+          la.next += la.step;
+          lb.next += lb.step;
+        } else {
+          la.next = pass_start(la.begin, la.plane, kPassPlaneA, load_at.pass);
+          lb.next = pass_start(lb.begin, lb.plane, kPassPlaneB, load_at.pass);
+        }
+      }
     };
     const int ra = reader_base<kAKMajor>(wm);
     const int rb = reader_base<kBKMajor>(wn);
@@ -619,14 +666,35 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     const unsigned touch_off = touch_b ? line_offset<kBKMajor>(B, line) : line_offset<kAKMajor>(A, line);
     const int64_t touch_step = readfirstlane64(touch_b ? lb.step : la.step);
     const char* touch_base = reinterpret_cast<const char*>(
-        readfirstlane64(reinterpret_cast<int64_t>(touch_b ? lb.next : la.next)));
+        readfirstlane64(reinterpret_cast<int64_t>(touch_b ? lb.begin : la.begin)));
     const unsigned touch_lds =
         __builtin_amdgcn_readfirstlane(lds0 + 2 * kStageBytes + (unsigned)wave * 256);
     // (a tail is small and in L2 already; the tile before it is touched again)
     const bool ragged = touch_b ? kBKMajor && k_end > B.k_full : kAKMajor && k_end > A.k_full;
     const int touch_last = __builtin_amdgcn_readfirstlane(nk - 1 - (ragged ? 1 : 0));
+    const unsigned touch_planes =
+        __builtin_amdgcn_readfirstlane(touch_b ? kPassPlaneB : kPassPlaneA);
+    const int64_t touch_plane = readfirstlane64(touch_b ? lb.plane : la.plane);
+    Place touch_at = {0, 0};
+    const char* touch_next = pass_start(touch_base, touch_plane, touch_planes, 0);
+    auto next_touch = [&] {
+      next_place(touch_at);
+      touch_next = touch_at.tile != 0
+                       ? touch_next + touch_step
+                       : pass_start(touch_base, touch_plane, touch_planes, touch_at.pass);
+    };
+    if constexpr (kPlanes > 1) {
+#pragma unroll
+      for (int t = 0; t < kTouchAhead; ++t) next_touch();
+    }
     auto touch_tile = [&](int k) {
-      touch(touch_lds, touch_off, touch_base + (int64_t)min(k, touch_last) * touch_step);
+      if constexpr (kPlanes == 1) {
+        touch(touch_lds, touch_off, touch_base + (int64_t)min(k, touch_last) * touch_step);
+      } else {
+        // called for K tiles kTouchAhead, + 1, ...: past the last one the first again
+        touch(touch_lds, touch_off, k < nk ? touch_next : touch_base);
+        next_touch();
+      }
     };
     // tiles_left: how many tiles follow (0, 1, or 2 for "two or more")
     auto step = [&](int k, auto tiles_left_tag, auto first_tag) {
@@ -724,5 +792,15 @@ struct MfmaDirect4Engine : DirectTileLayout<T_> {
     mainloop_ex<false, false>(a, b, k_begin, k_end, acc, smem);
   }
 };
+
+// 16-bit matrices as they are stored.
+template <typename T_>
+struct MfmaDirect4Engine : DirectToLdsEngine<T_, 1> {};
+
+// Float32 matrices in three bf16 planes (tlce_split_f32.h): an operand's row holds its
+// planes one after the other, so `ld` is the distance of two planes and a third of the
+// distance of two rows.  The K loop runs once per pair of planes,
+//   lo.hi  hi.lo  mid.mid  mid.hi  hi.mid  hi.hi
+struct SplitF32Engine : DirectToLdsEngine<__bf16, 3> {};
 
 }  // namespace tlce

@@ -16,6 +16,7 @@ template <typename T_>
 struct SimtEngine {
   using T = T_;
 
+  static constexpr int kPlanes = 1;
   static constexpr int kTile = 64;
   static constexpr int kBK = 16;
   static constexpr int kThreads = 256;

@@ -15,6 +15,7 @@
 //                        6: the launch sequences over them.
 #include "tlce_host.h"
 #include "tlce_fused.h"
+#include "tlce_split_f32.h"
 
 #ifndef TLCE_UNIT_ENGINE
 #error "define TLCE_UNIT_ENGINE and TLCE_UNIT_PART (see turbo_dllm_amd/build.py)"

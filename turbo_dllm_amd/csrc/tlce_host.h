@@ -387,6 +387,30 @@ struct ShardStats {
   float* target_logits = nullptr;
 };
 
+// Merge of the forward's partials into lse, loss and (when asked for) the weighted loss sum;
+// ca holds the operands, the partials and the plain outputs.  `weighted`: [m] scratch.
+template <typename T>
+int launch_combine(CombineArgs ca, int n_vtiles, int tile, int64_t m, const ShardStats& shard,
+                   char* weighted, const RowOptions& opt, hipStream_t stream) {
+  ca.label_offset = shard.vocab_start;
+  ca.local_max = shard.local_max; ca.local_sum = shard.local_sum;
+  ca.target_logits = shard.target_logits;
+  ca.logit_scale = opt.logit_scale; ca.token_weights = opt.token_weights;
+  ca.n_vtiles = n_vtiles; ca.tile = tile; ca.m_dev = opt.row_count;
+  ca.weight_dim_first = opt.weight_dim_first;
+  if (opt.weighted_sum != nullptr) {
+    ca.weighted = reinterpret_cast<float*>(weighted);
+    ca.weighted_rows = (int)m;
+  }
+  {
+    ScopedTimer timer(kClassCombine, stream);
+    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock), 256, 0, stream>>>(ca);
+  }
+  TLCE_LAUNCH_CHECK();
+  if (opt.weighted_sum != nullptr) return launch_sum(ca.weighted, m, opt.weighted_sum, stream);
+  return 0;
+}
+
 template <class E>
 int forward_impl(const Plan& p, const void* hidden, const void* weight, const float* bias,
                  const int64_t* labels, const int64_t* row_idx, int64_t m, int64_t h, int64_t v,
@@ -419,24 +443,7 @@ int forward_impl(const Plan& p, const void* hidden, const void* weight, const fl
   ca.part_max = fa.part_max; ca.part_sum = fa.part_sum;
   ca.part_ld = fa.part_ld; ca.nsplit = p.nsplit;
   ca.losses = losses; ca.lse = lse; ca.valid_count = valid_count;
-  ca.label_offset = shard.vocab_start;
-  ca.local_max = shard.local_max; ca.local_sum = shard.local_sum;
-  ca.target_logits = shard.target_logits;
-  ca.logit_scale = opt.logit_scale; ca.token_weights = opt.token_weights;
-  ca.n_vtiles = p.n_vtiles; ca.tile = p.tile; ca.m_dev = opt.row_count;
-  ca.weight_dim_first = opt.weight_dim_first;
-  float* weighted = reinterpret_cast<float*>(ws + l.weighted);
-  if (opt.weighted_sum != nullptr) {
-    ca.weighted = weighted;
-    ca.weighted_rows = (int)m;
-  }
-  {
-    ScopedTimer timer(kClassCombine, stream);
-    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock), 256, 0, stream>>>(ca);
-  }
-  TLCE_LAUNCH_CHECK();
-  if (opt.weighted_sum != nullptr) return launch_sum(weighted, m, opt.weighted_sum, stream);
-  return 0;
+  return launch_combine<T>(ca, p.n_vtiles, p.tile, m, shard, ws + l.weighted, opt, stream);
 }
 
 // ---------------------------------------------------------------- backward --

@@ -437,6 +437,17 @@ __device__ __forceinline__ void stream_store16(void* dst, uint4 v) {
   __builtin_nontemporal_store(x, reinterpret_cast<u4_t*>(dst));
 }
 
+// A float32 value as the sum of three bf16 numbers, each the next rounded to nearest:
+// exact (8 + 8 + 8 significant bits) down to the smallest normal numbers.  A value that
+// would round to infinity keeps its leading bits instead, infinities and NaN have no rest.
+__device__ __forceinline__ void split_planes(float x, float (&part)[3]) {
+  part[0] = to_float<__bf16>(from_float<__bf16>(x));
+  if (fabsf(part[0]) > 3.4e38f) part[0] = __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+  float rest = fabsf(part[0]) <= 3.4e38f ? x - part[0] : 0.0f;
+  part[1] = to_float<__bf16>(from_float<__bf16>(rest));
+  part[2] = rest - part[1];
+}
+
 template <class E, bool kSoftcap, bool kBias, bool kWDimFirst = false>
 __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits_panel_kernel(GradLogitsArgs p) {
   extern __shared__ __align__(16) char smem[];
@@ -446,7 +457,8 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
     p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
   }
   int tt, pv;
-  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_ptiles, (int64_t)E::kTile * p.h * sizeof(T), &tt, &pv))
+  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_ptiles,
+                (int64_t)E::kTile * p.h * E::kPlanes * sizeof(T), &tt, &pv))
     return;
 
   E eng;
@@ -537,7 +549,69 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
 
   T* g_out = static_cast<T*>(p.g);
   const int prow = pv * E::kTile;  // first panel column of this tile
-  if constexpr (E::kHasKMajor && sizeof(T) == 2) {
+  if constexpr (E::kPlanes == 3) {
+    // The same as below for float32 gradients in three bf16 planes ([token][plane][vocab]):
+    // a quarter of the tile, 64 tokens of all planes (96 KiB of LDS), at a time.
+    auto emit = [&](auto edge_tag, auto onehot_tag) {
+      constexpr bool kEdge = decltype(edge_tag)::value;
+      asm volatile("" ::: "memory");
+      float row_sum[kBias ? E::kRows : 1];
+      if (kBias) {
+#pragma unroll
+        for (int i = 0; i < E::kRows; ++i) row_sum[i] = 0.0f;
+      }
+      constexpr int kTokens = E::kStageCols * E::kTokensPerIndex;   // 64
+      constexpr int kPlaneBytes = kTokens * 512;
+#pragma unroll
+      for (int j = 0; j < E::kCols; ++j) {
+        const int slot = (j % E::kStageCols) * E::kTokensPerIndex + eng.position_in_index();
+#pragma unroll
+        for (int i = 0; i < E::kRows; i += 4) {
+          float part[4][3];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int row = eng.row(i + q);
+            const bool vok = !kEdge || ((vbase + row < p.v) && (vbase + row != excluded));
+            const float g = grad_of(E::get(acc, j, i + q), j, row, vok, edge_tag, onehot_tag);
+            if (kBias) row_sum[i + q] += g;
+            split_planes(g, part[q]);
+          }
+          const int vq = eng.row(i) >> 2;
+          char* dst = smem + slot * 512 + (((vq >> 1) ^ (slot & 31)) * 16) + (vq & 1) * 8;
+#pragma unroll
+          for (int pl = 0; pl < 3; ++pl)
+            store4<T>(reinterpret_cast<T*>(dst + pl * kPlaneBytes), part[0][pl], part[1][pl],
+                      part[2][pl], part[3][pl]);
+        }
+        if (j % E::kStageCols != E::kStageCols - 1) continue;
+        __syncthreads();
+        constexpr int kPieces = kTokens * 32;   // 16-byte pieces per plane
+#pragma unroll 4
+        for (int it = 0; it < 3 * kPieces / E::kThreads; ++it) {
+          const int c = it * E::kThreads + threadIdx.x;
+          const int pl = c / kPieces, sl = (c % kPieces) >> 5, ch = c & 31;
+          const int t = E::token_of_index(j + 1 - E::kStageCols + sl / E::kTokensPerIndex,
+                                          sl % E::kTokensPerIndex);
+          const uint4 val = *reinterpret_cast<const uint4*>(smem + pl * kPlaneBytes + sl * 512 +
+                                                            ((ch ^ (sl & 31)) * 16));
+          stream_store16(g_out + (((int64_t)tt * E::kTile + t) * 3 + pl) * p.ldg + prow + ch * 8,
+                         val);
+        }
+        if (j + 1 < E::kCols) __syncthreads();   // the stage has been read out
+      }
+      if (kBias) {
+#pragma unroll
+        for (int i = 0; i < E::kRows; ++i) add_grad_bias(eng.row(i), row_sum[i]);
+      }
+    };
+    if (edge) {
+      emit(std::true_type{}, std::true_type{});
+    } else if (onehot) {
+      emit(std::false_type{}, std::true_type{});
+    } else {
+      emit(std::false_type{}, std::false_type{});
+    }
+  } else if constexpr (E::kHasKMajor && sizeof(T) == 2) {
     // The MFMA engine's LDS is free after the main loop: the tile is staged there
     // as [token][vocab] (512-byte rows, 16-byte chunk c of token t in slot
     // c ^ (t & 31)) and G is written in whole 512-byte rows.  The work goes by
@@ -1348,8 +1422,8 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
   if (gridDim.y == 1 || tiles >= kSplitMajorBelowTiles) {
     split = blockIdx.y;
     if (split >= n_splits) return;
-    if (!xcd_tile(blockIdx.x, p.ni, p.nj, (int64_t)E::kTile * min(p.k, p.k_per_split) * sizeof(T),
-                  &ti, &tj))
+    if (!xcd_tile(blockIdx.x, p.ni, p.nj,
+                  (int64_t)E::kTile * min(p.k, p.k_per_split) * E::kPlanes * sizeof(T), &ti, &tj))
       return;
   } else {
     // Few output tiles under many K splits (a small head, the last rows of a call

@@ -6,6 +6,7 @@
 #include "tlce_host.h"
 #include "tlce_row_kernels.h"
 #include "tlce_fused_rows.h"
+#include "tlce_split_f32.h"
 
 namespace tlce {
 
@@ -231,19 +232,40 @@ extern "C" int tlce_query_plan(int64_t m, int64_t h, int64_t v, int dtype, int c
   return 0;
 }
 
+namespace {
+
+int64_t forward_workspace(int64_t m, int64_t h, int64_t v, int dtype, bool dynamic_rows,
+                          bool weighted, bool no_split = false) {
+  if (!no_split && split_forward_taken(m, h, v, dtype, dynamic_rows))
+    return split_forward_layout(make_split_plan(m, h, v, 0), dynamic_rows, weighted).total;
+  return forward_layout(make_plan(m, h, v, dtype, false, 0), dynamic_rows, weighted).total;
+}
+
+int64_t backward_workspace(int64_t m, int64_t h, int64_t v, int dtype, bool weight_grad,
+                           int64_t panel_bytes) {
+  if (split_f32_supported(m, h, v, dtype))
+    return split_backward_layout(make_split_plan(m, h, v, panel_bytes), h).total;
+  const Plan p = make_plan(m, h, v, dtype, weight_grad, panel_bytes);
+  return backward_layout(p, m, h, dtype, weight_grad).total;
+}
+
+}  // namespace
+
 extern "C" int64_t tlce_forward_workspace_bytes(int64_t m, int64_t h, int64_t v, int dtype) {
   if (m < 0 || h <= 0 || v <= 0) return -1;
-  return forward_layout(make_plan(m, h, v, dtype, false, 0)).total;
+  return forward_workspace(m, h, v, dtype, false, false);
 }
 
 namespace {
 
+// no_split: float32 stays on the float32 engine (callers without room for planes)
 int forward_entry(const void* hidden, const void* weight, const float* bias,
                   const int64_t* labels, const int64_t* row_idx, int64_t m, int64_t n_out,
                   int64_t h, int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index,
                   float logit_softcap, float* losses, float* lse, float* valid_count,
                   const ShardStats& shard, void* workspace, int64_t workspace_bytes,
-                  hipStream_t stream, const RowOptions& opt = RowOptions{}) {
+                  hipStream_t stream, const RowOptions& opt = RowOptions{},
+                  bool no_split = false) {
   const bool local = shard.local_max != nullptr;
   const bool fused = opt.weighted_sum != nullptr;   // the masked-token loss entry point
   if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
@@ -267,11 +289,16 @@ int forward_entry(const void* hidden, const void* weight, const float* bias,
   if (m == 0) return 0;
   TLCE_REQUIRE(labels && workspace && (local || ((losses || fused) && lse)),
                "forward: null pointer");
-  const Plan p = make_plan(m, h, v, dtype, false, 0);
-  const int64_t need = forward_layout(p, opt.row_count != nullptr, fused).total;
+  const bool dynamic = opt.row_count != nullptr;
+  const int64_t need = forward_workspace(m, h, v, dtype, dynamic, fused, no_split);
   TLCE_REQUIRE(workspace_bytes >= need, "forward: workspace too small (%lld < %lld)",
                (long long)workspace_bytes, (long long)need);
   TLCE_REQUIRE(((uintptr_t)workspace & 255) == 0, "forward: workspace must be 256-byte aligned");
+  if (!no_split && split_forward_taken(m, h, v, dtype, dynamic))
+    return split_forward(make_split_plan(m, h, v, 0), hidden, weight, bias, labels, row_idx, m, h,
+                         v, ignore_index, exclude_index, logit_softcap, losses, lse, valid_count,
+                         shard, static_cast<char*>(workspace), stream, opt);
+  const Plan p = make_plan(m, h, v, dtype, false, 0);
   TLCE_DISPATCH(p, dtype,
                 forward_impl<E>(p, hidden, weight, bias, labels, row_idx, m, h, v, ignore_index,
                                 exclude_index, logit_softcap, losses, lse, valid_count, shard,
@@ -348,7 +375,7 @@ extern "C" int tlce_forward_noalloc(const void* hidden, const void* weight, cons
                                     float* valid_count, void* stream) {
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0, "forward_noalloc: bad shape m=%lld h=%lld v=%lld",
                (long long)m, (long long)h, (long long)v);
-  const int64_t need = forward_layout(make_plan(m, h, v, dtype, false, 0)).total;
+  const int64_t need = forward_workspace(m, h, v, dtype, false, false, true);
   TLCE_REQUIRE(need <= (int64_t)TLCE_FORWARD_NOALLOC_SCRATCH_BYTES,
                "forward_noalloc: m=%lld needs %lld bytes of softmax partials, the static scratch "
                "array holds %lld (at most %lld rows); use tlce_forward with a workspace",
@@ -359,7 +386,7 @@ extern "C" int tlce_forward_noalloc(const void* hidden, const void* weight, cons
   return forward_entry(hidden, weight, bias, labels, row_idx, m, n_out, h, v, dtype, ignore_index,
                        exclude_index, logit_softcap, losses, lse, valid_count, ShardStats{}, ptr,
                        (int64_t)TLCE_FORWARD_NOALLOC_SCRATCH_BYTES,
-                       static_cast<hipStream_t>(stream));
+                       static_cast<hipStream_t>(stream), RowOptions{}, true);
 }
 
 extern "C" int tlce_forward_local(const void* hidden, const void* weight, const float* bias,
@@ -389,8 +416,7 @@ extern "C" int64_t tlce_backward_workspace_bytes(int64_t m, int64_t h, int64_t v
                                                  int64_t panel_bytes) {
   (void)has_bias;
   if (m < 0 || h <= 0 || v <= 0) return -1;
-  const Plan p = make_plan(m, h, v, dtype, compute_weight_grad != 0, panel_bytes);
-  return backward_layout(p, m, h, dtype, compute_weight_grad != 0).total;
+  return backward_workspace(m, h, v, dtype, compute_weight_grad != 0, panel_bytes);
 }
 
 namespace {
@@ -430,11 +456,17 @@ int backward_entry(const void* hidden, const void* weight, const float* bias,
                "backward: the mean reduction needs valid_count");
   TLCE_REQUIRE(((uintptr_t)grad_hidden & 15) == 0 && ((uintptr_t)grad_weight & 15) == 0,
                "backward: gradients must be 16-byte aligned");
-  const Plan p = make_plan(m, h, v, dtype, grad_weight != nullptr, panel_bytes);
-  const int64_t need = backward_layout(p, m, h, dtype, grad_weight != nullptr).total;
+  const int64_t need = backward_workspace(m, h, v, dtype, grad_weight != nullptr, panel_bytes);
   TLCE_REQUIRE(workspace_bytes >= need, "backward: workspace too small (%lld < %lld)",
                (long long)workspace_bytes, (long long)need);
   TLCE_REQUIRE(((uintptr_t)workspace & 255) == 0, "backward: workspace must be 256-byte aligned");
+  if (split_f32_supported(m, h, v, dtype))
+    return split_backward(make_split_plan(m, h, v, panel_bytes), hidden, weight, bias, labels,
+                          row_idx, lse, valid_count, grad_output, m, n_out, h, v, reduction_code,
+                          ignore_index, exclude_index, logit_softcap, vocab_start, grad_hidden,
+                          grad_weight, (bias != nullptr) ? grad_bias : nullptr,
+                          static_cast<char*>(workspace), stream, opt);
+  const Plan p = make_plan(m, h, v, dtype, grad_weight != nullptr, panel_bytes);
   TLCE_DISPATCH(p, dtype,
                 backward_impl<E>(p, hidden, weight, bias, labels, row_idx, lse, valid_count,
                                  grad_output, m, n_out, h, v, dtype, reduction_code, ignore_index,
@@ -495,7 +527,10 @@ extern "C" int tlce_backward_local(const void* hidden, const void* weight, const
 extern "C" int64_t tlce_masked_loss_forward_workspace_bytes(int64_t m, int64_t h, int64_t v,
                                                             int dtype, int dynamic_rows) {
   if (m < 0 || h <= 0 || v <= 0) return -1;
-  return forward_layout(make_plan(m, h, v, dtype, false, 0), dynamic_rows != 0, true).total;
+  // (a size asked for rows counted on the device serves calls that know theirs too)
+  const int64_t fixed = forward_workspace(m, h, v, dtype, false, true);
+  if (dynamic_rows == 0) return fixed;
+  return std::max(fixed, forward_workspace(m, h, v, dtype, true, true));
 }
 
 extern "C" int tlce_masked_loss_forward(const void* hidden, const void* weight, const float* bias,
