@@ -590,6 +590,36 @@ int tlce_apply_grad_output(const float* grad_hidden_f32, const float* grad_weigh
                            int64_t h, int64_t v, int dtype, int reduction_code,
                            void* grad_hidden, void* grad_weight, void* stream);
 
+/* The pair for float32 operands whose products run on the bf16 matrix units
+ * (tlce_f32_gradients_in_forward_supported: more than 128 rows, h a multiple of 4
+ * and at least 512, 96 or more tiles of 256 x 256, 1 GiB or less of planes, six
+ * bytes an element, for the head).  Same arguments and results without a dtype; the
+ * panel holds exp(logit - reference) in three bf16 planes and every gradient is
+ * float32.  grad_weight cannot be postponed. */
+int tlce_f32_gradients_in_forward_supported(int64_t m, int64_t h, int64_t v);
+
+int64_t tlce_forward_with_gradients_f32_workspace_bytes(int64_t m, int64_t h, int64_t v,
+                                                        int compute_weight_grad,
+                                                        int64_t panel_bytes);
+
+int tlce_forward_with_gradients_f32(const float* hidden, const float* weight,
+                                    const int64_t* labels, const int64_t* row_idx,
+                                    const float* token_weights, const int64_t* row_count,
+                                    int64_t m, int64_t n_out, int64_t h, int64_t v,
+                                    int64_t ignore_index, int64_t exclude_index,
+                                    float logit_softcap, float logit_multiplier,
+                                    float* losses, float* lse, float* valid_count,
+                                    float* grad_hidden, float* grad_weight,
+                                    int64_t panel_bytes, void* workspace,
+                                    int64_t workspace_bytes, void* stream);
+
+int tlce_apply_grad_output_f32(const float* grad_hidden_in, const float* grad_weight_in,
+                               const int64_t* row_idx, const int64_t* row_count,
+                               const float* grad_output, const float* valid_count,
+                               int64_t m, int64_t n_out, int64_t h, int64_t v,
+                               int reduction_code, float* grad_hidden, float* grad_weight,
+                               void* stream);
+
 /* One block of rows only (tlce_query_fused_plan: n_blocks == 1): the grad_weight
  * contraction of tlce_forward_with_gradients postponed until the upstream
  * gradient is known.  Call the forward with grad_weight_f32 = NULL (as for a

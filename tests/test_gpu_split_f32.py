@@ -153,3 +153,86 @@ def test_scratch_of_the_planes_is_bounded():
     assert lib.tlce_forward_workspace_bytes(2048, 4096, 262144, f32) < 1024 * mib + hidden + 4 * mib
     backward = lib.tlce_backward_workspace_bytes(2048, 4096, 262144, f32, 1, 0, 0)
     assert backward < 2 * 1024 * mib + hidden + 64 * 2048 * 4096 * 4
+
+
+def launches_of(call):
+    """Launches per kernel class of what `call` runs (forward only: this thread)."""
+    with _lib.kernel_profile() as prof:
+        result = call()
+        torch.cuda.synchronize()
+    return result, prof
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["sync", "device", "none"])
+@pytest.mark.parametrize("case", [
+    dict(m=129, h=512, v=24449, reduction="mean"),
+    dict(m=1500, h=580, v=8190, reduction="sum", softcap=15.0, exclude=8189, ignored=0.3),
+    dict(m=1030, h=580, v=8190, reduction="none", frozen=True),
+    # blocks of 256 rows, the last of one row
+    dict(m=1025, h=640, v=8191, reduction="mean", panel=14 << 20),
+    # losses beyond the first try's window in some rows
+    dict(m=520, h=512, v=16384, reduction="sum", far=True),
+], ids=lambda c: f"{c['m']}x{c['h']}x{c['v']}-{c['reduction']}")
+def test_gradients_left_by_the_forward(gpu_device, case, mode):
+    m, h, v = case["m"], case["h"], case["v"]
+    print("[case]", case, mode, flush=True)
+    hidden, weight, labels = operands(gpu_device, m, h, v, m, case.get("ignored", 0.0))
+    if case.get("far"):
+        hidden[::7] *= 20.0
+        labels[::7] = (labels[::7] + 1) % v
+    valid = labels != -100
+    cap, exclude = case.get("softcap", 0.0), case.get("exclude", -1)
+    upstream = torch.ones(m, device=gpu_device)
+    if case["reduction"] == "mean":
+        upstream /= valid.sum()
+    if case["reduction"] == "none":
+        upstream = (torch.rand(m, generator=torch.Generator().manual_seed(2)) + 0.5).to(gpu_device)
+    want = exact(hidden, weight, labels, upstream, None, cap, exclude)
+    x = hidden.clone().requires_grad_()
+    w = weight.clone().requires_grad_(not case.get("frozen", False))
+    with options.panel_budget(case.get("panel", 0)):
+        loss, prof = launches_of(lambda: tiled_linear_cross_entropy(
+            x, w, labels, reduction=case["reduction"], logit_softcap=cap or None,
+            exclude_index=exclude if exclude >= 0 else None, compaction=mode))
+        assert prof.launches["exp_logits_panel"] > 0
+        for again in (False, True):   # a second backward over one graph
+            x.grad = w.grad = None
+            (loss * upstream).sum().backward(retain_graph=True) \
+                if case["reduction"] == "none" else loss.backward(retain_graph=True)
+            # (an entry is formed from two sums over the vocabulary, a hidden one and a factor)
+            assert off(x.grad, want[1]) < 2 * bound(m, h, v)
+            assert case.get("frozen") or off(w.grad, want[2]) < 2 * bound(m, h, v)
+    total = want[0] if case["reduction"] == "none" else (want[0] * upstream).sum()
+    assert off(loss.detach(), total) < bound(m, h, v)
+
+
+@pytest.mark.gpu
+def test_masked_token_loss_in_planes(gpu_device):
+    """Token weights and the output multiplier, which enter the row factors."""
+    from turbo_dllm_amd.loss import masked_token_loss
+    m, h, v = 700, 512, 16001
+    hidden, weight, labels = operands(gpu_device, m, h, v, 4, 0.1)
+    weights = (torch.rand(m, generator=torch.Generator().manual_seed(6)) + 0.5).to(gpu_device)
+    head = torch.nn.Linear(h, v, bias=False, device=gpu_device)
+    head.weight = torch.nn.Parameter(weight)
+    x = hidden.clone().requires_grad_()
+    loss = masked_token_loss(x, labels, weights, head, valid_token_count=100.0,
+                             mask_token_id=v - 1, output_multiplier=0.5)
+    loss.backward()
+    want = exact(hidden * 0.5, weight, labels, weights / 100.0, exclude=v - 1)
+    assert off(loss.detach(), (want[0] * weights / 100.0).sum()) < bound(m, h, v)
+    assert off(x.grad, 0.5 * want[1]) < 2 * bound(m, h, v)
+    assert off(head.weight.grad, want[2]) < 2 * bound(m, h, v)
+
+
+def test_which_float32_calls_leave_their_gradients_in_the_forward():
+    taken = _lib.library().tlce_f32_gradients_in_forward_supported
+    assert taken(1024, 1024, 32000) and taken(385, 512, 16641)
+    assert taken(129, 1024, 32000) and not taken(128, 1024, 32000)      # rows
+    assert not taken(1024, 1024, 5888)            # tiles
+    assert not taken(2048, 4096, 151936)          # a head of more than 1 GiB of planes
+    assert not taken(1024, 1022, 32000)           # hidden size
+    size = _lib.library().tlce_forward_with_gradients_f32_workspace_bytes
+    assert size(128, 1024, 32000, 1, 0) == -1
+    assert 0 < size(65536, 1024, 32000, 1, 0) < (5 << 29) + (2 << 30)

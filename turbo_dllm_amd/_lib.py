@@ -122,6 +122,31 @@ SIGNATURES = {
             c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
         ],
     ),
+    "tlce_f32_gradients_in_forward_supported": (c_int, [c_int64, c_int64, c_int64]),
+    "tlce_forward_with_gradients_f32_workspace_bytes": (
+        c_int64, [c_int64, c_int64, c_int64, c_int, c_int64]
+    ),
+    "tlce_forward_with_gradients_f32": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,   # hidden weight labels row_idx weights
+            c_void_p,                                           # row_count
+            c_int64, c_int64, c_int64, c_int64,                 # m n_out h v
+            c_int64, c_int64, c_float, c_float,                 # ignore exclude softcap multiplier
+            c_void_p, c_void_p, c_void_p,                       # losses lse valid_count
+            c_void_p, c_void_p,                                 # grad_hidden grad_weight
+            c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
+        ],
+    ),
+    "tlce_apply_grad_output_f32": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_void_p, c_void_p,             # dh dw row_idx row_count
+            c_void_p, c_void_p,                                 # grad_output valid_count
+            c_int64, c_int64, c_int64, c_int64, c_int,          # m n_out h v reduction
+            c_void_p, c_void_p, c_void_p,                       # grad_hidden grad_weight stream
+        ],
+    ),
     "tlce_ce_topk_gradient_in_forward_supported": (c_int, [c_int64, c_int64, c_int64, c_int]),
     "tlce_ce_topk_forward_with_gradient_workspace_bytes": (
         c_int64, [c_int64, c_int64, c_int64, c_int, c_int64]),

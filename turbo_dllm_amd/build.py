@@ -38,11 +38,12 @@ _PARTS = {2: "grad_logits", 7: "grad_logits_cap", 8: "grad_logits_bias", 9: "gra
           10: "forward_dim_first", 11: "grad_logits_dim_first", 12: "exp_panel"}
 # the forward that leaves the gradients (part 12 and its launch sequence) exists for bf16 only
 _FUSED_ENGINES = ("direct_bf16",)
-_SPLIT_F32_PARTS = (1, 2, 3, 7, 8, 9)   # its launch sequences are tlce_split_f32.hip
+_SPLIT_F32_PARTS = (1, 2, 3, 7, 8, 9, 12)   # its launch sequences are tlce_split_f32.hip
 UNITS = (
     [(f"engine_{tag}_{name}", "tlce_engine_unit.hip",
       (f"-DTLCE_UNIT_ENGINE={engine}", f"-DTLCE_UNIT_PART={part}")
-      + (("-DTLCE_UNIT_FUSED=1",) if tag in _FUSED_ENGINES else ()))
+      + (("-DTLCE_UNIT_FUSED=1",) if tag in _FUSED_ENGINES else ())
+      + (("-DTLCE_UNIT_PLANES=1",) if tag == "split_f32" else ()))
      for tag, engine in _SPLIT_ENGINES.items() for part, name in _PARTS.items()
      if (part in _SPLIT_F32_PARTS if tag == "split_f32"
          else part != 12 or tag in _FUSED_ENGINES)]

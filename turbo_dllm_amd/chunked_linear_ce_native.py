@@ -477,6 +477,22 @@ def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
         hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
 
 
+def f32_gradients_in_forward_supported(m: int, hidden: torch.Tensor, weight: torch.Tensor,
+                                       bias: torch.Tensor | None,
+                                       weight_dim_first: bool) -> bool:
+    """Whether ``forward_with_gradients_f32`` takes ``m`` rows of these operands: float32
+    on the GPU, head stored [V, H], no bias, and sizes at which float32 products run on
+    the bf16 matrix units."""
+    if bias is not None or weight_dim_first or not hidden.is_cuda:
+        return False
+    if hidden.dtype != torch.float32 or weight.dtype != hidden.dtype:
+        return False
+    if hidden.dim() != 2 or weight.dim() != 2 or weight.shape[1] != hidden.shape[1]:
+        return False
+    return bool(_lib.library().tlce_f32_gradients_in_forward_supported(
+        m, hidden.shape[1], weight.shape[0]))
+
+
 def forward_with_gradients(
     hidden: torch.Tensor,
     weight: torch.Tensor,
@@ -510,12 +526,49 @@ def forward_with_gradients(
     known and stores it directly in the input dtype.  The last element returned
     is then the workspace to hand to that call instead of a float32 gradient.
     """
-    device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
     if not fused_gradients_supported(hidden, weight, None, False):
+        _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
         raise RuntimeError(
             "forward_with_gradients needs bf16 operands, a [V, H] head and H, V multiples "
             "of 64; use forward / backward for other inputs"
         )
+    return _forward_with_gradients(
+        hidden, weight, labels, ignore_index, exclude_index, logit_softcap, compute_weight_grad,
+        token_weights, logit_multiplier, row_idx, n_out, row_count, postpone_weight_grad)
+
+
+def forward_with_gradients_f32(
+    hidden: torch.Tensor,
+    weight: torch.Tensor,
+    labels: torch.Tensor,
+    *,
+    ignore_index: int,
+    exclude_index: int,
+    logit_softcap: float,
+    compute_weight_grad: bool,
+    token_weights: torch.Tensor | None = None,
+    logit_multiplier: float = 1.0,
+    row_idx: torch.Tensor | None = None,
+    n_out: int | None = None,
+    row_count: torch.Tensor | None = None,
+):
+    """``forward_with_gradients`` for float32 operands that
+    ``f32_gradients_in_forward_supported`` names; grad_weight is never postponed."""
+    if hidden.dim() != 2 or not f32_gradients_in_forward_supported(
+            hidden.shape[0], hidden, weight, None, False):
+        _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
+        raise RuntimeError("forward_with_gradients_f32 does not take these operands "
+                           "(f32_gradients_in_forward_supported)")
+    return _forward_with_gradients(
+        hidden, weight, labels, ignore_index, exclude_index, logit_softcap, compute_weight_grad,
+        token_weights, logit_multiplier, row_idx, n_out, row_count, False)
+
+
+def _forward_with_gradients(hidden, weight, labels, ignore_index, exclude_index, logit_softcap,
+                            compute_weight_grad, token_weights, logit_multiplier, row_idx, n_out,
+                            row_count, postpone_weight_grad):
+    device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
+    f32 = hidden.dtype == torch.float32
     hidden = _dense(hidden)
     weight = _dense(weight)
     labels = labels.reshape(-1).to(torch.long).contiguous()
@@ -544,22 +597,22 @@ def forward_with_gradients(
                                "one block of the forward (weight_grad_can_wait)")
         grad_weight32 = (torch.empty((v, h), dtype=torch.float32, device=device)
                          if compute_weight_grad and not postpone else None)
-        ws = _workspace(
-            lib.tlce_forward_with_gradients_workspace_bytes(
-                m, h, v, code, int(compute_weight_grad), panel),
-            device,
-        )
+        entry = lib.tlce_forward_with_gradients_f32 if f32 else lib.tlce_forward_with_gradients
+        size = (lib.tlce_forward_with_gradients_f32_workspace_bytes if f32
+                else lib.tlce_forward_with_gradients_workspace_bytes)
+        sizes = (m, h, v) if f32 else (m, h, v, code)
+        ws = _workspace(size(*sizes, int(compute_weight_grad), panel), device)
         _lib.check(
-            lib.tlce_forward_with_gradients(
+            entry(
                 _ptr(hidden), _ptr(weight), _ptr(labels), _ptr(row_idx), _ptr(token_weights),
-                _ptr(row_count), m, n_out, h, v, code,
+                _ptr(row_count), m, n_out, *sizes[1:],
                 int(ignore_index), int(exclude_index), float(logit_softcap),
                 float(logit_multiplier),
                 _ptr(losses), _ptr(lse), valid_count.data_ptr(),
                 _ptr(grad_hidden32), _ptr(grad_weight32),
                 panel, ws.data_ptr(), ws.numel(), _stream(device),
             ),
-            "tlce_forward_with_gradients",
+            "tlce_forward_with_gradients_f32" if f32 else "tlce_forward_with_gradients",
         )
     return losses, lse, valid_count, grad_hidden32, (ws if postpone else grad_weight32)
 
@@ -663,18 +716,51 @@ def apply_grad_output(
         raise RuntimeError("row_idx must be int64 with one entry per row of grad_hidden32")
     if dtype != torch.bfloat16:
         raise RuntimeError("apply_grad_output writes bf16 gradients only")
-    code = _lib.DTYPE_BF16
+    return _apply_grad_output(grad_hidden32, grad_weight32, grad_output, valid_count,
+                              reduction_code, dtype, row_idx, n_out, v, row_count)
+
+
+def apply_grad_output_f32(
+    grad_hidden32: torch.Tensor,
+    grad_weight32: torch.Tensor | None,
+    grad_output: torch.Tensor,
+    valid_count: torch.Tensor,
+    *,
+    reduction: str,
+    row_idx: torch.Tensor | None = None,
+    n_out: int | None = None,
+    vocab: int | None = None,
+    row_count: torch.Tensor | None = None,
+) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """``apply_grad_output`` for what ``forward_with_gradients_f32`` left: float32 gradients."""
+    _require_device(grad_hidden32, grad_weight32, grad_output, valid_count, row_idx)
+    reduction_code = _reduction_code(reduction)
+    v = grad_weight32.shape[0] if grad_weight32 is not None else int(vocab or 1)
+    n_out = grad_hidden32.shape[0] if n_out is None else int(n_out)
+    return _apply_grad_output(
+        grad_hidden32, grad_weight32, _upstream_gradient(grad_output, reduction_code, n_out),
+        valid_count, reduction_code, torch.float32, row_idx, n_out, v, row_count)
+
+
+def _apply_grad_output(grad_hidden32, grad_weight32, grad_output, valid_count, reduction_code,
+                       dtype, row_idx, n_out, v, row_count):
+    device = grad_hidden32.device
+    m, h = grad_hidden32.shape
+    lib = _lib.library()
+    f32 = dtype == torch.float32
+    entry = lib.tlce_apply_grad_output_f32 if f32 else lib.tlce_apply_grad_output
+    codes = (reduction_code,) if f32 else (_lib.DTYPE_BF16, reduction_code)
     with torch.cuda.device(device):
         grad_hidden = torch.empty((n_out, h), dtype=dtype, device=device)
         grad_weight = (torch.empty((v, h), dtype=dtype, device=device)
                        if grad_weight32 is not None else None)
         _lib.check(
-            _lib.library().tlce_apply_grad_output(
+            entry(
                 _ptr(grad_hidden32), _ptr(grad_weight32), _ptr(row_idx), _ptr(row_count),
-                _ptr(grad_output), _ptr(valid_count), m, n_out, h, v, code, reduction_code,
+                _ptr(grad_output), _ptr(valid_count), m, n_out, h, v, *codes,
                 _ptr(grad_hidden), _ptr(grad_weight), _stream(device),
             ),
-            "tlce_apply_grad_output",
+            "tlce_apply_grad_output_f32" if f32 else "tlce_apply_grad_output",
         )
     return grad_hidden, grad_weight
 

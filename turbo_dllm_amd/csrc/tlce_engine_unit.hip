@@ -11,7 +11,8 @@
 //                        panels over a head stored [h, v],
 //                        12: the exponentiated-logits panel of the forward that
 //                        leaves the gradients (with TLCE_UNIT_FUSED, which also adds
-//                        that sequence to part 6: the bf16 direct engine only),
+//                        that sequence to part 6: the bf16 direct engine only; with
+//                        TLCE_UNIT_PLANES its cross-entropy variants: float32 in planes),
 //                        6: the launch sequences over them.
 #include "tlce_host.h"
 #include "tlce_fused.h"
@@ -83,6 +84,11 @@ TLCE_LAUNCHERS_GRAD_LOGITS_DIM_FIRST(extern template, UnitEngine)
 TLCE_LAUNCHERS_EXP_PANEL(template, UnitEngine)
 #else
 TLCE_LAUNCHERS_EXP_PANEL(extern template, UnitEngine)
+#endif
+#endif
+#ifdef TLCE_UNIT_PLANES
+#if TLCE_UNIT_PART == 12
+TLCE_LAUNCHERS_EXP_GRADIENTS(template, UnitEngine)
 #endif
 #endif
 #if TLCE_UNIT_PART == 6

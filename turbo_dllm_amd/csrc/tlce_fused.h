@@ -32,6 +32,7 @@
 #pragma once
 
 #include "tlce_host.h"
+#include "tlce_split_f32.h"
 
 namespace tlce {
 
@@ -85,7 +86,8 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
     p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
   }
   int tt, vt;
-  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_vtiles, (int64_t)E::kTile * p.h * sizeof(T), &tt, &vt))
+  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_vtiles,
+                (int64_t)E::kTile * p.h * E::kPlanes * sizeof(T), &tt, &vt))
     return;
 
   E eng;
@@ -120,13 +122,18 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
 
   // The tile is staged in LDS (free after the main loop) as [token][vocab]:
   // 512-byte rows, 16-byte chunk c of token t in slot c ^ (t & 31), and leaves in
-  // whole rows, a quarter of the tokens (one owned column index) at a time.
+  // whole rows, a quarter of the tokens (one owned column index) at a time.  Entries in
+  // three planes ([token][plane][vocab]) take 96 KiB a quarter, each in the same place.
+  constexpr int kQuarter = E::kStageCols * E::kTokensPerIndex;   // tokens
+  constexpr int kPlaneBytes = kQuarter * 512;
   auto emit = [&](auto edge_tag) {
     constexpr bool kEdge = decltype(edge_tag)::value;
     asm volatile("" ::: "memory");   // one real branch per variant
 #pragma unroll
     for (int j = 0; j < E::kCols; ++j) {
-      const int tok = eng.col(j);
+      const int tok = E::kPlanes > 1
+                          ? (j % E::kStageCols) * E::kTokensPerIndex + eng.position_in_index()
+                          : eng.col(j);
       float s = 0.0f, mx = -INFINITY;
 #pragma unroll
       for (int i = 0; i < E::kRows; i += 4) {
@@ -153,14 +160,38 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
           e4[q] = (kSoftcap && !kPlain) ? e * dcap : e;
         }
         const int vq = eng.row(i) >> 2;
-        T* dst = reinterpret_cast<T*>(smem + tok * 512 + (((vq >> 1) ^ (tok & 31)) * 16) +
-                                      (vq & 1) * 8);
-        store4<T>(dst, e4[0], e4[1], e4[2], e4[3]);
+        char* dst = smem + tok * 512 + (((vq >> 1) ^ (tok & 31)) * 16) + (vq & 1) * 8;
+        if constexpr (E::kPlanes > 1) {
+          float part[4][3];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) split_planes(e4[q], part[q]);
+#pragma unroll
+          for (int pl = 0; pl < 3; ++pl)
+            store4<T>(reinterpret_cast<T*>(dst + pl * kPlaneBytes), part[0][pl], part[1][pl],
+                      part[2][pl], part[3][pl]);
+        } else {
+          store4<T>(reinterpret_cast<T*>(dst), e4[0], e4[1], e4[2], e4[3]);
+        }
       }
       col_sum[j] = s;
       col_max[j] = mx;
       if (j % E::kStageCols != E::kStageCols - 1) continue;
       __syncthreads();
+      if constexpr (E::kPlanes > 1) {
+#pragma unroll 4
+        for (int it = 0; it < 3 * kQuarter * 32 / E::kThreads; ++it) {
+          const int c = it * E::kThreads + threadIdx.x;
+          const int pl = c / (kQuarter * 32), sl = (c % (kQuarter * 32)) >> 5, ch = c & 31;
+          const int t = E::token_of_index(j + 1 - E::kStageCols + sl / E::kTokensPerIndex,
+                                          sl % E::kTokensPerIndex);
+          const uint4 val = *reinterpret_cast<const uint4*>(smem + pl * kPlaneBytes + sl * 512 +
+                                                            ((ch ^ (sl & 31)) * 16));
+          stream_store16(panel + (((int64_t)tt * E::kTile + t) * 3 + pl) * p.ld + pcol + ch * 8,
+                         val);
+        }
+        if (j + 1 < E::kCols) __syncthreads();   // the quarter has been read out
+        continue;
+      }
       constexpr int kPieces = E::kTokensPerIndex * 32;   // 16-byte pieces per owned index
 #pragma unroll
       for (int it = 0; it < E::kStageCols * kPieces / E::kThreads; ++it) {
@@ -246,14 +277,15 @@ struct FusedRowsArgs {
   int part_ld, n_vtiles;
   int m, m_pad;                // rows of the block; rows of `scaled_hidden` to define (zeros past m)
   int h, v;
+  int hp = 0;                  // float32 in planes: elements of a plane of scaled_hidden's rows
   int64_t ignore, exclude;
   float softcap, logit_scale, window;
-  void* panel;                 // [.., ld]
+  void* panel;                 // [.., ld], or [.., 3, ld] in planes
   int64_t ld;
   float* lse;                  // [m]
   float* losses;               // scattered, or null
   float* row_scale;            // [m_pad]
-  void* scaled_hidden;         // [m_pad, h] or null (no grad_weight)
+  void* scaled_hidden;         // [m_pad, h] or [m_pad, 3, hp], or null (no grad_weight)
   float* ref_next;             // [m] reference of the second try
   int* redo;                   // [1] set when some row needs the second try
   const int* run_flag;         // non-null: run only when *run_flag != 0
@@ -319,11 +351,12 @@ struct SoftRowsArgs {
 };
 
 int launch_soft_rows(const SoftRowsArgs& a, hipStream_t stream);
-int launch_label_logit(const LabelLogitArgs& a, hipStream_t stream);
+// T: the operands' type, __bf16 or float (whose panel and scaled rows are in planes)
+template <typename T> int launch_label_logit(const LabelLogitArgs& a, hipStream_t stream);
 int launch_scale_rows(const ScaleRowsArgs& a, hipStream_t stream);
-int launch_fused_rows(const FusedRowsArgs& a, hipStream_t stream);
+template <typename T> int launch_fused_rows(const FusedRowsArgs& a, hipStream_t stream);
 int launch_reduce_slabs(const ReduceSlabsArgs& a, hipStream_t stream);
-int launch_scale_cast(const ScaleCastArgs& a, hipStream_t stream);
+template <typename T> int launch_scale_cast(const ScaleCastArgs& a, hipStream_t stream);
 
 // ------------------------------------------------------------------- plan ----
 struct FusedPlan {
@@ -333,7 +366,11 @@ struct FusedPlan {
   int64_t block_rows;   // rows per block, a multiple of the tile
   int n_blocks;
   int dh_ksplit;        // K splits of the grad_hidden contraction of a full block
+  int64_t k_steps;      // of its K loop, unsplit
 };
+
+// Float32 entries are three bf16 planes.
+inline int panel_entry_bytes(int dtype) { return dtype == TLCE_DTYPE_F32 ? 6 : 2; }
 
 // Cross entropies and soft embeddings whose panel entries are formed in the forward:
 // vocabularies of whole 64-row slabs.  Others keep the sequences that recompute the
@@ -365,8 +402,7 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
   p.n_htiles = (int)ceil_div(h, tile);
   if (panel_bytes <= 0) panel_bytes = kDefaultFusedPanelBytes;
   const int64_t total = ceil_div(std::max<int64_t>(m, 1), tile);   // token tiles
-  const int64_t budget =
-      std::max<int64_t>(1, panel_bytes / (p.vp * dtype_bytes(dtype) * tile));
+  const int64_t budget = std::max<int64_t>(1, panel_bytes / (p.vp * panel_entry_bytes(dtype) * tile));
   p.n_blocks = (int)ceil_div(total, budget);
   int64_t per = ceil_div(total, p.n_blocks);   // balanced blocks
   // several blocks: 16 token tiles x 16 hidden tiles make whole rounds of 256
@@ -374,22 +410,25 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
   if (p.n_blocks > 1 && round_up(per, 16) <= budget) per = round_up(per, 16);
   p.block_rows = per * tile;
   p.n_blocks = (int)ceil_div(total, per);
-  const int64_t k_steps = p.vp / 64;
-  const int max_split = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxKSplits, k_steps / 8));
-  p.dh_ksplit = grad_hidden_k_splits((p.block_rows / tile) * p.n_htiles, max_split, k_steps,
+  // (in planes, six steps of the K loop per 64 vocabulary rows)
+  p.k_steps = p.vp / 64 * (dtype == TLCE_DTYPE_F32 ? SplitF32Engine::kPasses : 1);
+  const int max_split = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxKSplits, p.k_steps / 8));
+  p.dh_ksplit = grad_hidden_k_splits((p.block_rows / tile) * p.n_htiles, max_split, p.k_steps,
                                      std::min(p.block_rows, std::max<int64_t>(m, 1)) * h);
   return p;
 }
 
 struct FusedLayout {
   int64_t panel, part_sum, part_max, target, ref, ref_next, row_scale, scaled_hidden, slabs,
-      redo, total;
+      redo, hidden_planes, weight_planes, total;
 };
 
 inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dtype,
                                 bool weight_grad) {
   FusedLayout l;
-  const int64_t es = dtype_bytes(dtype);
+  const int64_t es = panel_entry_bytes(dtype);
+  const bool planes = dtype == TLCE_DTYPE_F32;
+  const int64_t hp = round_up(h, 64);   // (h itself without planes)
   const int64_t mp = round_up(std::max<int64_t>(m, 1), 256);
   int64_t off = 0;
   l.panel = off;      off += align256(p.block_rows * p.vp * es);
@@ -400,9 +439,13 @@ inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dt
   l.ref_next = off;   off += align256(p.block_rows * 4);
   l.row_scale = off;  off += align256(p.block_rows * 4);
   l.scaled_hidden = off;
-  if (weight_grad) off += align256(p.block_rows * h * es);
+  if (weight_grad) off += align256(p.block_rows * hp * es);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
   l.redo = off;       off += align256((int64_t)p.n_blocks * 4);
+  l.hidden_planes = off;
+  if (planes) off += align256(mp * hp * es);
+  l.weight_planes = off;
+  if (planes) off += align256(p.vp * hp * es);
   l.total = off;
   return l;
 }
@@ -423,6 +466,21 @@ inline void set_head_operand(GemmArgs& g, const void* weight, int64_t v, int64_t
   }
 }
 
+// Float32 cross entropies leave their gradients in the forward where they run in planes and
+// the whole head's fit their bound.  Nothing is lost by it: what the row factors add are
+// float32 roundings.  Per-token losses of a trainable head (whose grad_weight would have to
+// wait, and the panel with it) keep the recomputing backward.  One contraction less and the
+// head split once lower the sizes from which planes pay.  Forward and backward in us, float32
+// engine / recomputing in planes / this (2-norm errors 2e-7 to 7e-7, on the engine 5e-7 to 3e-6):
+//   1024 rows, H = 1024, V = 32000   2300 / 1439 / 1149     2048 rows  4446 / 2621 / 2017
+//    512 rows, H = 2048, V = 50001   3800 / 2602 / 2071      512, H = 512, V = 16384  390 / 387 / 335
+//    300 rows, H = 1024, V = 32000    992 /  -   / 668       300, H = 512, V = 16384  347 / - / 310
+//    129 rows, H = 1024, V = 50001   1027 /  -   / 763       129, H = 512, V = 33000  454 / - / 388
+inline bool f32_gradients_in_forward_supported(int64_t m, int64_t h, int64_t v) {
+  return split_f32_supported(m, h, v, TLCE_DTYPE_F32, 128, 96) &&
+         round_up(v, 256) * round_up(h, 64) * 6 <= kSplitWeightBytes;
+}
+
 // Options of the fused sequence beyond the operator's own arguments.
 struct FusedOptions {
   float logit_scale = 1.0f;
@@ -441,6 +499,8 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
   // take the real count from the device and the workgroups past it exit at once
   const int64_t* m_dev = opt.row_count;
   using T = typename E::T;
+  constexpr int kPlanes = E::kPlanes;
+  using In = std::conditional_t<kPlanes == 1, T, float>;
   const bool weight_grad = grad_weight32 != nullptr;
   const FusedLayout l = fused_layout(p, m, h, dtype, weight_grad);
   T* panel = reinterpret_cast<T*>(ws + l.panel);
@@ -453,7 +513,25 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
   T* scaled_hidden = weight_grad ? reinterpret_cast<T*>(ws + l.scaled_hidden) : nullptr;
   float* slabs = reinterpret_cast<float*>(ws + l.slabs);
   int* redo = reinterpret_cast<int*>(ws + l.redo);
-  const T* hidden_t = static_cast<const T*>(hidden);
+  const In* hidden_in = static_cast<const In*>(hidden);
+  // the operands of the contractions, hp elements a row (and plane): the matrices
+  // themselves, or their planes
+  const int64_t hp = kPlanes == 1 ? h : round_up(h, 64);
+  const T* hidden_t;
+  const void* weight_t;
+  if constexpr (kPlanes == 1) {
+    hidden_t = hidden_in;
+    weight_t = weight;
+  } else {
+    if (int rc = launch_split_planes(hidden_in, m, round_up(m, 256), h, hp, ws + l.hidden_planes,
+                                     stream))
+      return rc;
+    if (int rc = launch_split_planes(static_cast<const float*>(weight), v, p.vp, h, hp,
+                                     ws + l.weight_planes, stream))
+      return rc;
+    hidden_t = reinterpret_cast<const T*>(ws + l.hidden_planes);
+    weight_t = ws + l.weight_planes;
+  }
 
   if (int rc = fill_zero(redo, (int64_t)p.n_blocks * 4, stream)) return rc;
   LabelLogitArgs la;
@@ -461,7 +539,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
   la.m = (int)m; la.h = (int)h; la.v = (int)v;
   la.ignore = ignore; la.exclude = exclude; la.softcap = softcap; la.logit_scale = opt.logit_scale;
   la.target = target; la.ref = ref; la.valid_count = valid_count; la.m_dev = m_dev;
-  if (int rc = launch_label_logit(la, stream)) return rc;
+  if (int rc = launch_label_logit<In>(la, stream)) return rc;
 
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
@@ -472,8 +550,8 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     const int64_t rows64 = round_up(rows, 64);
 
     ExpPanelArgs ea;
-    ea.hidden = hidden_t + r0 * h; ea.weight = weight;
-    ea.m = (int)rows; ea.h = (int)h; ea.v = (int)v;
+    ea.hidden = hidden_t + r0 * hp * kPlanes; ea.weight = weight_t;
+    ea.m = (int)rows; ea.h = (int)hp; ea.v = (int)v;
     ea.exclude = exclude; ea.softcap = softcap; ea.logit_scale = opt.logit_scale;
     ea.n_ttiles = n_ttiles; ea.n_vtiles = p.n_vtiles;
     ea.panel = panel; ea.ld = p.vp;
@@ -481,13 +559,13 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     ea.m_dev = m_dev; ea.row0 = r0;
 
     FusedRowsArgs ra;
-    ra.hidden = hidden_t + r0 * h; ra.labels = labels + r0;
+    ra.hidden = hidden_in + r0 * h; ra.labels = labels + r0;
     ra.target = target + r0;
     ra.token_weights = opt.token_weights ? opt.token_weights + r0 : nullptr;
     ra.row_idx = row_idx ? row_idx + r0 : nullptr; ra.loss_row0 = r0;
     ra.part_sum = part_sum; ra.part_max = part_max;
     ra.part_ld = (int)p.block_rows; ra.n_vtiles = p.n_vtiles;
-    ra.m = (int)rows; ra.m_pad = (int)rows_p; ra.h = (int)h; ra.v = (int)v;
+    ra.m = (int)rows; ra.m_pad = (int)rows_p; ra.h = (int)h; ra.v = (int)v; ra.hp = (int)hp;
     ra.ignore = ignore; ra.exclude = exclude; ra.softcap = softcap;
     ra.logit_scale = opt.logit_scale;
     ra.window = kRefWindow;
@@ -508,12 +586,14 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
       ra.ref = ea.ref;
       ra.run_flag = ea.run_flag;
       // the second try must not mark the block again: it reads the flag the first set
-      if (int rc = launch_fused_rows(ra, stream)) return rc;
+      if (int rc = launch_fused_rows<In>(ra, stream)) return rc;
     }
 
-    // grad_hidden of the block: A = weight as stored (K-major, K = vocabulary), B = panel
+    // grad_hidden of the block: A = weight as stored or its planes (K-major, K = vocabulary),
+    // B = panel
     GemmArgs dh;
-    set_head_operand(dh, weight, v, h);
+    dh.a = weight_t; dh.lda = hp; dh.a_rows = (int)hp;
+    dh.k = (int)round_up(v, 64);   // (planes have zero rows up to there)
     dh.b = panel; dh.ldb = p.vp; dh.b_rows = (int)rows_p;
     dh.k_per_split = 0;
     dh.ni = p.n_htiles; dh.nj = n_ttiles;
@@ -524,7 +604,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
                      ? p.dh_ksplit
                      : std::min(p.dh_ksplit,
                                 grad_hidden_k_splits((int64_t)n_ttiles * p.n_htiles, p.dh_ksplit,
-                                                     p.vp / 64, rows * h));
+                                                     p.k_steps, rows * h));
     ReduceSlabsArgs rs;
     if (m_dev != nullptr) {
       // The block may hold far fewer rows than it was sized for (down to none): at least
@@ -532,7 +612,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
       // real rows call for, within the slab memory the plan allocated; the others exit at once.
       dh.m_dev = m_dev; dh.m_role = kRowsFollow; dh.m_dev_offset = r0;
       dh.slab_budget = (int64_t)p.dh_ksplit * p.block_rows * h;
-      dh.k_steps_plan = (int)(p.vp / 64);
+      dh.k_steps_plan = (int)p.k_steps;
       ksplit = (int)std::max<int64_t>(p.dh_ksplit, std::min<int64_t>(16, p.vp / 64 / 8));
       rs.n_htiles = p.n_htiles; rs.tile = E::kTile; rs.launched_splits = ksplit;
       rs.k_steps = dh.k_steps_plan; rs.slab_budget = dh.slab_budget;
@@ -547,7 +627,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     if (weight_grad) {
       // grad_weight += panel^T . (s * hidden): both operands K-major, K = the block's rows
       GemmArgs dw;
-      dw.a = scaled_hidden; dw.lda = h; dw.a_rows = (int)h;
+      dw.a = scaled_hidden; dw.lda = hp; dw.a_rows = (int)hp;
       dw.b = panel; dw.ldb = p.vp; dw.b_rows = (int)p.vp;
       dw.k = (int)rows64;
       dw.k_per_split = 0;
@@ -1071,16 +1151,20 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
   return 0;
 }
 
+#define TLCE_LAUNCHERS_EXP_GRADIENTS(X, E)                                              \
+  X int launch_exp_panel_variant<E, false, false>(const ExpPanelArgs&, hipStream_t);    \
+  X int launch_exp_panel_variant<E, true, false>(const ExpPanelArgs&, hipStream_t);
 #define TLCE_LAUNCHERS_EXP_PANEL(X, E)                                                  \
   X int launch_kl_panel_emit<E>(const KlPanelArgs&, hipStream_t);                       \
-  X int launch_exp_panel_variant<E, false, false>(const ExpPanelArgs&, hipStream_t);    \
-  X int launch_exp_panel_variant<E, true, false>(const ExpPanelArgs&, hipStream_t);     \
+  TLCE_LAUNCHERS_EXP_GRADIENTS(X, E)                                                    \
   X int launch_exp_panel_variant<E, true, true>(const ExpPanelArgs&, hipStream_t);
-#define TLCE_FUSED_ENTRY_POINTS(X, E)                                                            \
+#define TLCE_FUSED_GRADIENTS(X, E)                                                               \
   X int fused_gradients_impl<E>(const FusedPlan&, const void*, const void*, const int64_t*,      \
                                 const int64_t*, int64_t, int64_t, int64_t, int, int64_t,         \
                                 int64_t, float, float*, float*, float*, float*, float*, char*,   \
-                                hipStream_t, const FusedOptions&);                               \
+                                hipStream_t, const FusedOptions&);
+#define TLCE_FUSED_ENTRY_POINTS(X, E)                                                            \
+  TLCE_FUSED_GRADIENTS(X, E)                                                                     \
   X int soft_embedding_fused_impl<E>(const FusedPlan&, const void*, const void*, int64_t,        \
                                      int64_t, int64_t, int, float, float, void*, char*,          \
                                      hipStream_t);                                               \

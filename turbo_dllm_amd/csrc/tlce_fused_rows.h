@@ -120,7 +120,15 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
           dcap = 1.0f - t * t;
         }
         const float entry = (expf(target - c) - sum) * dcap;
-        static_cast<T*>(p.panel)[(int64_t)r * p.ld + label] = from_float<T>(entry);
+        if constexpr (sizeof(T) == 4) {
+          float part[3];
+          split_planes(entry, part);
+          __bf16* at = static_cast<__bf16*>(p.panel) + (int64_t)r * 3 * p.ld + label;
+#pragma unroll
+          for (int pl = 0; pl < 3; ++pl) at[pl * p.ld] = from_float<__bf16>(part[pl]);
+        } else {
+          static_cast<T*>(p.panel)[(int64_t)r * p.ld + label] = from_float<T>(entry);
+        }
       }
     }
     if (r < p.m_pad) p.row_scale[r] = factor;
@@ -129,6 +137,28 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
   T* scaled = static_cast<T*>(p.scaled_hidden);
   if (scaled == nullptr) return;
   __syncthreads();
+  if constexpr (sizeof(T) == 4) {
+    // float32: in planes of hp elements, zeros from h on (h a multiple of 4)
+    for (int i = 0; i < kFusedRowsPerBlock / kFusedRowsWaves; ++i) {
+      const int rr = wave * (kFusedRowsPerBlock / kFusedRowsWaves) + i;
+      const int r = row0 + rr;
+      if (r >= p.m_pad) return;
+      const float factor = sh_factor[rr];
+      const float* hrow = static_cast<const float*>(p.hidden) + (int64_t)min(r, p.m - 1) * p.h;
+      __bf16* out = static_cast<__bf16*>(p.scaled_hidden) + (int64_t)r * 3 * p.hp;
+      for (int k = lane * 4; k < p.hp; k += 64 * 4) {
+        f32x4_t x = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (k < p.h && r < p.m) x = *reinterpret_cast<const f32x4_t*>(hrow + k);
+        float part[4][3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) split_planes(x[e] * factor, part[e]);
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl)
+          store4<__bf16>(out + pl * p.hp + k, part[0][pl], part[1][pl], part[2][pl], part[3][pl]);
+      }
+    }
+    return;
+  }
   for (int i = 0; i < kFusedRowsPerBlock / kFusedRowsWaves; ++i) {
     const int rr = wave * (kFusedRowsPerBlock / kFusedRowsWaves) + i;
     const int r = row0 + rr;

@@ -81,16 +81,18 @@ int launch_sum(const float* x, int64_t n, float* out, hipStream_t stream) {
 }
 
 // ---- row kernels of the forward that leaves the gradients (tlce_fused_rows.h) ----
+template <typename T>
 int launch_label_logit(const LabelLogitArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassCombine, stream);
-  lce_label_logit_kernel<__bf16><<<(int)ceil_div(a.m, 16), 256, 0, stream>>>(a);
+  lce_label_logit_kernel<T><<<(int)ceil_div(a.m, 16), 256, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
 
+template <typename T>
 int launch_fused_rows(const FusedRowsArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassCombine, stream);
-  lce_fused_rows_kernel<__bf16>
+  lce_fused_rows_kernel<T>
       <<<(int)ceil_div(a.m_pad, kFusedRowsPerBlock), 64 * kFusedRowsWaves, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
@@ -162,15 +164,21 @@ int launch_reduce_slabs(const ReduceSlabsArgs& a, hipStream_t stream) {
   return 0;
 }
 
+template <typename T>
 int launch_scale_cast(const ScaleCastArgs& a, hipStream_t stream) {
   if (a.rows <= 0) return 0;
   ScopedTimer timer(kClassOther, stream);
-  lce_scale_cast_rows_kernel<__bf16><<<(unsigned)a.rows, 256, 0, stream>>>(a);
+  lce_scale_cast_rows_kernel<T><<<(unsigned)a.rows, 256, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
+template int launch_label_logit<__bf16>(const LabelLogitArgs&, hipStream_t);
+template int launch_label_logit<float>(const LabelLogitArgs&, hipStream_t);
+template int launch_fused_rows<__bf16>(const FusedRowsArgs&, hipStream_t);
+template int launch_fused_rows<float>(const FusedRowsArgs&, hipStream_t);
 
 TLCE_FUSED_ENTRY_POINTS(extern template, MfmaDirect4Engine<__bf16>)
+TLCE_FUSED_GRADIENTS(extern template, SplitF32Engine)
 TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaDirect4Engine<__bf16>)
 TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaDirect4Engine<_Float16>)
 TLCE_ENGINE_ENTRY_POINTS(extern template, MfmaEngine<__bf16>)
@@ -988,18 +996,15 @@ extern "C" int64_t tlce_forward_with_gradients_workspace_bytes(int64_t m, int64_
                       compute_weight_grad != 0).total;
 }
 
-extern "C" int tlce_forward_with_gradients(
+namespace {
+
+int forward_with_gradients_entry(
     const void* hidden, const void* weight, const int64_t* labels, const int64_t* row_idx,
     const float* token_weights, const int64_t* row_count, int64_t m, int64_t n_out, int64_t h,
     int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
     float logit_multiplier,
     float* losses, float* lse, float* valid_count, float* grad_hidden_f32, float* grad_weight_f32,
-    int64_t panel_bytes, void* workspace, int64_t workspace_bytes, void* stream_) {
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
-  if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
-  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
-               "forward_with_gradients: needs bf16 inputs with h and v multiples of 64 "
-               "(h=%lld v=%lld dtype=%d)", (long long)h, (long long)v, dtype);
+    int64_t panel_bytes, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
   TLCE_REQUIRE(valid_count != nullptr, "forward_with_gradients: valid_count is null");
   TLCE_REQUIRE(logit_multiplier > 0.0f,
                "forward_with_gradients: the logit multiplier must be positive");
@@ -1035,21 +1040,23 @@ extern "C" int tlce_forward_with_gradients(
   opt.logit_scale = logit_multiplier;
   opt.token_weights = token_weights;
   opt.row_count = row_count;
+  if (dtype == TLCE_DTYPE_F32)
+    return fused_gradients_impl<SplitF32Engine>(
+        p, hidden, weight, labels, row_idx, m, h, v, dtype, ignore_index, exclude_index,
+        logit_softcap, losses, lse, valid_count, grad_hidden_f32, grad_weight_f32,
+        static_cast<char*>(workspace), stream, opt);
   return fused_gradients_impl<MfmaDirect4Engine<__bf16>>(
       p, hidden, weight, labels, row_idx, m, h, v, dtype, ignore_index, exclude_index,
       logit_softcap, losses, lse, valid_count, grad_hidden_f32, grad_weight_f32,
       static_cast<char*>(workspace), stream, opt);
 }
 
-extern "C" int tlce_apply_grad_output(const float* grad_hidden_f32, const float* grad_weight_f32,
-                                      const int64_t* row_idx, const int64_t* row_count,
-                                      const float* grad_output,
-                                      const float* valid_count, int64_t m, int64_t n_out,
-                                      int64_t h, int64_t v, int dtype, int reduction_code,
-                                      void* grad_hidden, void* grad_weight, void* stream_) {
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
-  TLCE_REQUIRE(dtype == TLCE_DTYPE_BF16, "apply_grad_output: unsupported dtype code %d (bf16 only)",
-               dtype);
+template <typename T>
+int apply_grad_output_entry(const float* grad_hidden_f32, const float* grad_weight_f32,
+                            const int64_t* row_idx, const int64_t* row_count,
+                            const float* grad_output, const float* valid_count, int64_t m,
+                            int64_t n_out, int64_t h, int64_t v, int reduction_code,
+                            void* grad_hidden, void* grad_weight, hipStream_t stream) {
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0 && (h % 4) == 0, "apply_grad_output: bad shape");
   TLCE_REQUIRE(reduction_code == TLCE_REDUCTION_SUM || reduction_code == TLCE_REDUCTION_MEAN ||
                    reduction_code == TLCE_REDUCTION_NONE,
@@ -1072,9 +1079,8 @@ extern "C" int tlce_apply_grad_output(const float* grad_hidden_f32, const float*
   TLCE_REQUIRE((((uintptr_t)grad_hidden | (uintptr_t)grad_weight | (uintptr_t)grad_hidden_f32 |
                  (uintptr_t)grad_weight_f32) & 15) == 0,
                "apply_grad_output: gradients must be 16-byte aligned");
-  const int64_t es = dtype_bytes(dtype);
   if (row_idx != nullptr || m == 0) {
-    if (int rc = fill_zero(grad_hidden, n_out * h * es, stream)) return rc;
+    if (int rc = fill_zero(grad_hidden, n_out * h * (int64_t)sizeof(T), stream)) return rc;
   }
   ScaleCastArgs a;
   a.grad_output = grad_output; a.valid_count = valid_count; a.reduction = reduction_code;
@@ -1083,14 +1089,91 @@ extern "C" int tlce_apply_grad_output(const float* grad_hidden_f32, const float*
     TLCE_REQUIRE(grad_hidden_f32 != nullptr, "apply_grad_output: null pointer");
     a.in = grad_hidden_f32; a.row_idx = row_idx; a.rows = m; a.out = grad_hidden;
     a.m_dev = row_count;
-    if (int rc = launch_scale_cast(a, stream)) return rc;
+    if (int rc = launch_scale_cast<T>(a, stream)) return rc;
     a.m_dev = nullptr;
   }
   if (grad_weight != nullptr) {
     a.in = grad_weight_f32; a.row_idx = nullptr; a.rows = v; a.out = grad_weight;
-    if (int rc = launch_scale_cast(a, stream)) return rc;
+    if (int rc = launch_scale_cast<T>(a, stream)) return rc;
   }
   return 0;
+}
+
+}  // namespace
+
+extern "C" int tlce_forward_with_gradients(
+    const void* hidden, const void* weight, const int64_t* labels, const int64_t* row_idx,
+    const float* token_weights, const int64_t* row_count, int64_t m, int64_t n_out, int64_t h,
+    int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
+    float logit_multiplier,
+    float* losses, float* lse, float* valid_count, float* grad_hidden_f32, float* grad_weight_f32,
+    int64_t panel_bytes, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
+  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype),
+               "forward_with_gradients: needs bf16 inputs with h and v multiples of 64 "
+               "(h=%lld v=%lld dtype=%d)", (long long)h, (long long)v, dtype);
+  return forward_with_gradients_entry(hidden, weight, labels, row_idx, token_weights, row_count, m,
+                                      n_out, h, v, dtype, ignore_index, exclude_index,
+                                      logit_softcap, logit_multiplier, losses, lse, valid_count,
+                                      grad_hidden_f32, grad_weight_f32, panel_bytes, workspace,
+                                      workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tlce_apply_grad_output(const float* grad_hidden_f32, const float* grad_weight_f32,
+                                      const int64_t* row_idx, const int64_t* row_count,
+                                      const float* grad_output,
+                                      const float* valid_count, int64_t m, int64_t n_out,
+                                      int64_t h, int64_t v, int dtype, int reduction_code,
+                                      void* grad_hidden, void* grad_weight, void* stream) {
+  TLCE_REQUIRE(dtype == TLCE_DTYPE_BF16, "apply_grad_output: unsupported dtype code %d (bf16 only)",
+               dtype);
+  return apply_grad_output_entry<__bf16>(grad_hidden_f32, grad_weight_f32, row_idx, row_count,
+                                         grad_output, valid_count, m, n_out, h, v, reduction_code,
+                                         grad_hidden, grad_weight,
+                                         static_cast<hipStream_t>(stream));
+}
+
+// ------------------------------------- the same pair for float32 in planes ----
+extern "C" int tlce_f32_gradients_in_forward_supported(int64_t m, int64_t h, int64_t v) {
+  return (m >= 0 && h > 0 && v > 0 && f32_gradients_in_forward_supported(m, h, v)) ? 1 : 0;
+}
+
+extern "C" int64_t tlce_forward_with_gradients_f32_workspace_bytes(int64_t m, int64_t h, int64_t v,
+                                                                   int compute_weight_grad,
+                                                                   int64_t panel_bytes) {
+  if (!tlce_f32_gradients_in_forward_supported(m, h, v)) return -1;
+  return fused_layout(make_fused_plan(m, h, v, TLCE_DTYPE_F32, panel_bytes), m, h, TLCE_DTYPE_F32,
+                      compute_weight_grad != 0).total;
+}
+
+extern "C" int tlce_forward_with_gradients_f32(
+    const float* hidden, const float* weight, const int64_t* labels, const int64_t* row_idx,
+    const float* token_weights, const int64_t* row_count, int64_t m, int64_t n_out, int64_t h,
+    int64_t v, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
+    float logit_multiplier, float* losses, float* lse, float* valid_count, float* grad_hidden,
+    float* grad_weight, int64_t panel_bytes, void* workspace, int64_t workspace_bytes,
+    void* stream) {
+  if (int rc = validate_common(hidden, weight, m, h, v, TLCE_DTYPE_F32)) return rc;
+  TLCE_REQUIRE(f32_gradients_in_forward_supported(m, h, v),
+               "forward_with_gradients_f32: not taken for m=%lld h=%lld v=%lld",
+               (long long)m, (long long)h, (long long)v);
+  return forward_with_gradients_entry(hidden, weight, labels, row_idx, token_weights, row_count, m,
+                                      n_out, h, v, TLCE_DTYPE_F32, ignore_index, exclude_index,
+                                      logit_softcap, logit_multiplier, losses, lse, valid_count,
+                                      grad_hidden, grad_weight, panel_bytes, workspace,
+                                      workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tlce_apply_grad_output_f32(const float* grad_hidden_in, const float* grad_weight_in,
+                                          const int64_t* row_idx, const int64_t* row_count,
+                                          const float* grad_output, const float* valid_count,
+                                          int64_t m, int64_t n_out, int64_t h, int64_t v,
+                                          int reduction_code, float* grad_hidden,
+                                          float* grad_weight, void* stream) {
+  return apply_grad_output_entry<float>(grad_hidden_in, grad_weight_in, row_idx, row_count,
+                                        grad_output, valid_count, m, n_out, h, v, reduction_code,
+                                        grad_hidden, grad_weight,
+                                        static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tlce_grad_weight_from_panel(const void* hidden, const int64_t* row_idx,

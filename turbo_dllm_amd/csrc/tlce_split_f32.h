@@ -57,9 +57,10 @@ struct SplitPlan {
 //   vocabulary  1000: 8192 rows, H = 1024  1145 / 1359      2048: 1548 / 1466
 //   hidden  256: 2048 rows, V = 32000  1244 / 1023, 8192 rows  4607 / 4777;  128: 725 / 821
 //           512: 1024 rows, V = 16384   657 / 524
-inline bool split_f32_supported(int64_t m, int64_t h, int64_t v, int dtype) {
-  return dtype == TLCE_DTYPE_F32 && (h % 4) == 0 && h >= 512 && m > 384 && v >= 2048 &&
-         ceil_div(m, 256) * ceil_div(v, 256) >= 128;
+inline bool split_f32_supported(int64_t m, int64_t h, int64_t v, int dtype,
+                                int64_t more_than_rows = 384, int64_t min_tiles = 128) {
+  return dtype == TLCE_DTYPE_F32 && (h % 4) == 0 && h >= 512 && m > more_than_rows &&
+         v >= 2048 && ceil_div(m, 256) * ceil_div(v, 256) >= min_tiles;
 }
 
 inline SplitPlan make_split_plan(int64_t m, int64_t h, int64_t v, int64_t panel_bytes) {

@@ -1,5 +1,6 @@
 // Launch sequences of the float32 cross entropy on the bf16 matrix units
 // (tlce_split_f32.h); their contractions are the kernels of tlce_kernels.h on SplitF32Engine.
+#include "tlce_fused.h"
 #include "tlce_split_f32.h"
 
 namespace tlce {
@@ -11,6 +12,8 @@ TLCE_LAUNCHERS_GRAD_LOGITS(extern template, SplitF32Engine, false, true)
 TLCE_LAUNCHERS_GRAD_LOGITS(extern template, SplitF32Engine, true, true)
 extern template int launch_gemm<SplitF32Engine, true, false>(GemmArgs, int, int, hipStream_t);
 extern template int launch_gemm<SplitF32Engine, true, true>(GemmArgs, int, int, hipStream_t);
+TLCE_LAUNCHERS_EXP_GRADIENTS(extern template, SplitF32Engine)
+TLCE_FUSED_GRADIENTS(template, SplitF32Engine)
 
 // Eight columns per thread: 32 bytes in, 16 bytes per plane out.  Bound by memory.
 __global__ __launch_bounds__(256) void lce_split_planes_kernel(const float* __restrict__ in,

@@ -279,7 +279,9 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
     wants_grad = bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
     ctx.fused = (
         wants_grad and options.get_gradient_mode() == "forward"
-        and native.fused_gradients_supported(rows, weight_vf, bias, in_place or weight_dim_first)
+        and (native.fused_gradients_supported(rows, weight_vf, bias, in_place or weight_dim_first)
+             or native.f32_gradients_in_forward_supported(m, rows, weight_vf, bias,
+                                                          in_place or weight_dim_first))
     )
     can_wait = ctx.fused and bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
         m, rows.shape[1], weight_vf.shape[0], rows.dtype)
@@ -291,12 +293,15 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
         # all rows in one block: the grad_weight contraction waits for the upstream
         # gradient and is stored in the input dtype at once (no float32 [V, H] buffer)
         ctx.postponed = can_wait
-        losses, lse, valid_count, grad_rows32, grad_weight32 = native.forward_with_gradients(
+        if rows.dtype == torch.float32:
+            forward, wait = native.forward_with_gradients_f32, {}
+        else:
+            forward, wait = native.forward_with_gradients, {"postpone_weight_grad": ctx.postponed}
+        losses, lse, valid_count, grad_rows32, grad_weight32 = forward(
             rows, weight_vf, targets, ignore_index=ignore_index, exclude_index=exclude_index,
             logit_softcap=float(logit_softcap),
             compute_weight_grad=bool(ctx.needs_input_grad[1]), row_idx=row_idx, n_out=n,
-            row_count=row_count if mode == "device" else None,
-            postpone_weight_grad=ctx.postponed,
+            row_count=row_count if mode == "device" else None, **wait,
         )
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx,
                               row_count if mode == "device" else None,
@@ -350,10 +355,14 @@ def _device_backward(ctx, grad_output, frozen: bool):
 
     if ctx.fused:
         grad_rows32, grad_weight32, valid_count, row_idx, row_count, rows = ctx.saved_tensors
-        grad_hidden, grad_weight = native.apply_grad_output(
+        if ctx.grad_dtype == torch.float32:
+            apply, kind = native.apply_grad_output_f32, {}
+        else:
+            apply, kind = native.apply_grad_output, {"dtype": ctx.grad_dtype}
+        grad_hidden, grad_weight = apply(
             grad_rows32, None if ctx.postponed else grad_weight32, grad_output, valid_count,
-            reduction=ctx.reduction, dtype=ctx.grad_dtype, row_idx=row_idx, n_out=ctx.n_rows,
-            vocab=ctx.vocab, row_count=row_count,
+            reduction=ctx.reduction, row_idx=row_idx, n_out=ctx.n_rows, vocab=ctx.vocab,
+            row_count=row_count, **kind,
         )
         if ctx.postponed and not frozen:
             # grad_weight32 is the forward's workspace: its panel still holds every row
