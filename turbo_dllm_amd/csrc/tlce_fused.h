@@ -66,6 +66,8 @@ struct ExpPanelArgs {
   float* part_max;      // [n_vtiles, part_ld] tile maximum of z in base-2 units
   int part_ld;
   const int* run_flag;  // non-null: the launch does nothing unless *run_flag != 0
+  float* part_entry = nullptr;     // [n_vtiles, part_ld] sum over the tile of the entries,
+  float* part_rounded = nullptr;   // exact and rounded (kRounded)
   // Row count known only to the device (null: m is exact): m is then the block's
   // capacity, and the block holds rows [row0, row0 + m) of the counted rows.
   const int64_t* m_dev = nullptr;
@@ -74,7 +76,9 @@ struct ExpPanelArgs {
 
 // kPlain: the panel receives exp(z - c) itself, without the soft cap's derivative
 // (a forward value, the unnormalised softmax, not a logit gradient).
-template <class E, bool kSoftcap, bool kPlain = false>
+// kRounded: the sums of the entries before and after their rounding go out as well, so that
+// the factor common to a row's rounding errors can be taken out again.
+template <class E, bool kSoftcap, bool kPlain = false, bool kRounded = false>
 __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_panel_kernel(ExpPanelArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
@@ -117,6 +121,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
                     (p.exclude >= vbase && p.exclude < vbase + E::kTile);
   const int excluded = (int)p.exclude;
   float col_sum[E::kCols], col_max[E::kCols];
+  float col_entry[kRounded ? E::kCols : 1], col_rounded[kRounded ? E::kCols : 1];
   T* panel = static_cast<T*>(p.panel);
   const int pcol = vt * E::kTile;   // first panel column of this tile
 
@@ -134,7 +139,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
       const int tok = E::kPlanes > 1
                           ? (j % E::kStageCols) * E::kTokensPerIndex + eng.position_in_index()
                           : eng.col(j);
-      float s = 0.0f, mx = -INFINITY;
+      float s = 0.0f, mx = -INFINITY, entry = 0.0f, rounded = 0.0f;
 #pragma unroll
       for (int i = 0; i < E::kRows; i += 4) {
         float e4[4];
@@ -171,10 +176,21 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
                       part[2][pl], part[3][pl]);
         } else {
           store4<T>(reinterpret_cast<T*>(dst), e4[0], e4[1], e4[2], e4[3]);
+          if (kRounded) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              if (kSoftcap) entry += e4[q];
+              rounded += to_float<T>(from_float<T>(e4[q]));
+            }
+          }
         }
       }
       col_sum[j] = s;
       col_max[j] = mx;
+      if (kRounded) {
+        col_entry[j] = kSoftcap ? entry : s;
+        col_rounded[j] = rounded;
+      }
       if (j % E::kStageCols != E::kStageCols - 1) continue;
       __syncthreads();
       if constexpr (E::kPlanes > 1) {
@@ -231,17 +247,39 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
     p.part_sum[o] = sum;
     p.part_max[o] = mx;
   }
+  if (kRounded) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < E::kCols; ++j) {
+      sh_sum[slot * E::kTile + eng.col(j)] = col_entry[j];
+      sh_max[slot * E::kTile + eng.col(j)] = col_rounded[j];
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < E::kTile; c += E::kThreads) {
+      float entry = 0.0f, rounded = 0.0f;
+#pragma unroll
+      for (int sl = 0; sl < E::kShare; ++sl) {
+        entry += sh_sum[sl * E::kTile + c];
+        rounded += sh_max[sl * E::kTile + c];
+      }
+      const int64_t o = (int64_t)vt * p.part_ld + tt * E::kTile + c;
+      p.part_entry[o] = entry;
+      p.part_rounded[o] = rounded;
+    }
+  }
 }
 
-template <class E, bool kSoftcap, bool kPlain = false>
+template <class E, bool kSoftcap, bool kPlain = false, bool kRounded = false>
 int launch_exp_panel_variant(const ExpPanelArgs& a, hipStream_t stream) {
   static LdsOptIn lds;
   constexpr int kLdsBytes = E::kSmemBytes + E::kTile * (int)sizeof(float);   // stages + stash
-  if (int rc = enable_large_lds(lce_exp_logits_panel_kernel<E, kSoftcap, kPlain>, kLdsBytes, lds))
+  if (int rc = enable_large_lds(lce_exp_logits_panel_kernel<E, kSoftcap, kPlain, kRounded>,
+                                kLdsBytes, lds))
     return rc;
   const int grid = xcd_grid((int64_t)a.n_ttiles * a.n_vtiles);
   ScopedTimer timer(kClassExpPanel, stream);
-  lce_exp_logits_panel_kernel<E, kSoftcap, kPlain><<<grid, E::kThreads, kLdsBytes, stream>>>(a);
+  lce_exp_logits_panel_kernel<E, kSoftcap, kPlain, kRounded>
+      <<<grid, E::kThreads, kLdsBytes, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
@@ -284,6 +322,12 @@ struct FusedRowsArgs {
   int64_t ld;
   float* lse;                  // [m]
   float* losses;               // scattered, or null
+  float* probabilities = nullptr;   // [m] exp(-loss), or null
+  bool keep_label = false;     // the label's entry stays exp(z - c): the panel's contraction
+                               // is d lse / d hidden, without the label's term
+  const float* part_entry = nullptr;     // kRounded sums of the producer, or null: the row
+  const float* part_rounded = nullptr;   // factor makes up for the rounding of the row's sum,
+  float* row_rounded = nullptr;          // [m] which goes here
   float* row_scale;            // [m_pad]
   void* scaled_hidden;         // [m_pad, h] or [m_pad, 3, hp], or null (no grad_weight)
   float* ref_next;             // [m] reference of the second try
@@ -308,7 +352,15 @@ struct ReduceSlabsArgs {
   // the real rows of the block (dynamic_k_splits); the same inputs reproduce them here
   int n_htiles = 0, tile = 0, launched_splits = 0, k_steps = 0;
   int64_t slab_budget = 0;
+  // non-null: row r also gets sum_j fix_value[r, j] * weight[fix_id[r, j], :] (j < kTopkFix),
+  // before the row factor
+  const float* fix_value = nullptr;
+  const int* fix_id = nullptr;
+  const void* weight = nullptr;     // bf16 [.., h]
 };
+// Largest entries of a row whose rounding the top-k path makes up for: they are known exactly
+// and weigh most (a label or word of probability near 1 is most of the sum).
+constexpr int kTopkFix = 8;
 
 // out[row_idx[r], :] = dtype(g * in[r, :]) with g = grad_output[0] (/ valid_count[0]
 // for the mean): the upstream gradient applied to the float32 gradients the
@@ -747,6 +799,29 @@ int soft_embedding_fused_impl(const FusedPlan& p, const void* hidden, const void
 }
 
 // ---- frozen-head cross entropy with top-k: the gradient formed in the forward ----
+// Two ways.  Through exponentiated logits (topk_from_exp_impl): the pass over the head is
+// the cross entropy's, entries exp(z - label's logit)*cap' in bf16 and exact float32 maxima of
+// every 256-word tile; no float32 logits cross memory.  lce_topk_select_kernel finds the k
+// largest logits from them: the k-th largest tile maximum bounds the k-th largest logit from
+// below, so only tiles that reach it are read (about k of them), entries above the bound are
+// candidates, and the logits of the few that remain are computed again in float32, one dot
+// product each.  Rows that this cannot settle (more near-ties than it has room for, top
+// logits so far below the label's that their entries underflow) raise a flag, on which the
+// second way's panels and scan run for the block, lists only.
+//
+// What the rows lose by a reference other than their maximum (whose entry would be 1 exactly)
+// they get back twice: the row factor divides by the sum of the entries as rounded, so the
+// part of the rounding errors that is common to a row cancels, and the kTopkFix largest
+// entries' errors, which are known once their logits are, are added to the contraction's row.
+// d lse / d hidden against float64, the other way -> this (512 rows, H = 512, V = 32000, label
+// logits raised by 0 / 8 / 12): 3.41e-4, 1.24e-4, 7.0e-6 -> 3.33e-4, 1.21e-4, 7.7e-6; with a soft
+// cap of 30 (H = 1024, V = 50001) 4.0e-4, 8.7e-4, 1.3e-3 -> 3.8e-4, 2.2e-4, 2.5e-5.
+//
+// Measured on 8192 rows, H = 4096, V = 151936, k = 16, forward and backward: 18.5 -> 15.2 ms: the
+// pass over the head 8.1 -> 7.6, the scan's 2.1, the entries' 1.4 and their rescaling's 0.4 ->
+// 0.25 for the selection and 0.1 for the corrections.
+//
+// Through float32 logits (the rest of this comment), for few tiles per top-k entry:
 // The backward of tlce_ce_topk_* recomputes the logits to form the softmax panel
 // (3 contractions per step).  Here the forward, which stages float32 logits panels
 // anyway, also writes e = exp(z - reference) * cap' of every panel in bf16 into a
@@ -791,8 +866,45 @@ int launch_rescale_exp_rows(const RescaleExpArgs& a, int n_panels, hipStream_t s
 int launch_topk_row_scale(const TopkRowScaleArgs& a, hipStream_t stream);
 int launch_topk_apply(const TopkApplyArgs& a, hipStream_t stream);
 
+struct TopkSelectArgs {
+  const void* panel;       // bf16 [.., ld] exp(z - ref) * cap'
+  int64_t ld;
+  const float* part_max;   // [n_vtiles, part_ld] base-2 tile maxima of z
+  int part_ld, n_vtiles;
+  const float* ref;        // [m] the label's logit; ref_next where *redo
+  const float* ref_next;
+  const int* redo;
+  const void* hidden;      // [m, h]
+  const void* weight;      // [v, h]
+  int m, h, k;
+  float softcap, logit_scale;
+  float* top_values;       // [m, k]
+  int64_t* top_ids;        // [m, k]
+  int* unsettled;          // set when some row's list could not be found
+  // the largest entries (kTopkFix, at most k): their exact values less the rounded ones, and
+  // the row factor for a sum that holds the exact ones
+  float* fix_value;        // [m, kTopkFix]
+  int* fix_id;             // [m, kTopkFix]
+  const float* row_rounded;   // [m] sum of the row's rounded entries
+  float* row_scale;        // [m]
+};
+int launch_topk_select(const TopkSelectArgs& a, hipStream_t stream);
+
+// Tiles whose maxima a wave holds; the k-th largest of them is a useful bound while there
+// are some per list entry.
+constexpr int kTopkSelectTiles = 1024;
+// Below 2^25 logits the step is bound by the host's launches, of which there are more here
+// (ms, float32 logits / this: 300 rows, V = 16384 0.335 / 0.345; 1024, V = 20000 0.335 / 0.350;
+// 1024 rows, H = 2048, V = 33000 0.593 / 0.524; 4096, H = 1024, V = 32768, k = 64 1.38 / 0.92).
+inline bool topk_from_exp_supported(int64_t m, int64_t v, int top_k) {
+  const int64_t tiles = ceil_div(v, 256);
+  if (m * v < (1ll << 25)) return false;
+  return tiles <= kTopkSelectTiles && tiles >= std::max<int64_t>(64, 2 * top_k);
+}
+
 struct TopkFusedLayout {
-  int64_t forward, panel, ref_used, row_scale, slabs, k_tail, total;
+  int64_t forward, panel, ref_used, row_scale, slabs, k_tail, part_sum, part_max, part_entry,
+      part_rounded, target, ref, ref_next, row_rounded, fix_value, fix_id, flags, total;
 };
 
 // Rows are taken in blocks of the panel budget of the forward that leaves the gradients
@@ -818,8 +930,124 @@ inline TopkFusedLayout topk_fused_layout(const TopkPlan& t, const FusedPlan& p, 
   l.row_scale = off;  off += align256(p.block_rows * 4);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
   l.k_tail = off;     off += k_tail_bytes(p.v, h);
+  l.part_sum = off;   off += align256((int64_t)p.n_vtiles * p.block_rows * 4);
+  l.part_max = off;   off += align256((int64_t)p.n_vtiles * p.block_rows * 4);
+  l.part_entry = off; off += align256((int64_t)p.n_vtiles * p.block_rows * 4);
+  l.part_rounded = off; off += align256((int64_t)p.n_vtiles * p.block_rows * 4);
+  l.target = off;     off += align256(p.block_rows * 4);
+  l.ref = off;        off += align256(p.block_rows * 4);
+  l.ref_next = off;   off += align256(p.block_rows * 4);
+  l.row_rounded = off; off += align256(p.block_rows * 4);
+  l.fix_value = off;  off += align256(p.block_rows * kTopkFix * 4);
+  l.fix_id = off;     off += align256(p.block_rows * kTopkFix * 4);
+  l.flags = off;      off += 256;   // redo, unsettled, count of rows (unused)
   l.total = off;
   return l;
+}
+
+// unit[r, :] = row_scale[r] * (panel . weight)[r, :]
+template <class E>
+int topk_contraction(const TopkFusedLayout& l, const FusedPlan& p, const void* weight, int64_t m,
+                     int64_t h, int64_t v, float* unit_grad, char* ws, hipStream_t stream,
+                     bool fix = false) {
+  const int m_pad = (int)p.block_rows;
+  float* slabs = reinterpret_cast<float*>(ws + l.slabs);
+  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
+  GemmArgs g;
+  set_head_operand(g, weight, v, h, ws + l.k_tail);
+  g.b = ws + l.panel; g.ldb = p.vp; g.b_rows = m_pad;
+  g.k_per_split = 0;
+  g.ni = p.n_htiles; g.nj = m_pad / E::kTile;
+  g.c = slabs; g.ldc = h; g.c_rows = (int)m; g.c_cols = (int)h;
+  g.c_split_stride = p.block_rows * h;
+  g.mode = kStoreF32;
+  if (int rc = launch_gemm<E, true, false>(g, p.dh_ksplit, kClassGradHidden, stream)) return rc;
+  ReduceSlabsArgs rs;
+  rs.slabs = slabs; rs.n_splits = p.dh_ksplit; rs.split_stride = p.block_rows * h;
+  rs.row_scale = reinterpret_cast<const float*>(ws + l.row_scale);
+  rs.m = (int)m; rs.h = (int)h;
+  rs.out = unit_grad;
+  if (fix) {
+    rs.fix_value = reinterpret_cast<const float*>(ws + l.fix_value);
+    rs.fix_id = reinterpret_cast<const int*>(ws + l.fix_id);
+    rs.weight = weight;
+  }
+  return launch_reduce_slabs(rs, stream);
+}
+
+template <class E>
+int topk_from_exp_impl(const TopkPlan& t, const FusedPlan& p, const void* hidden,
+                       const void* weight, const int64_t* labels, int64_t m, int64_t h, int64_t v,
+                       int top_k, float multiplier, float softcap, float* losses,
+                       float* probabilities, float* top_values, int64_t* top_ids, float* lse,
+                       float* unit_grad, char* ws, hipStream_t stream) {
+  const TopkFusedLayout l = topk_fused_layout(t, p, h);
+  constexpr int64_t kNoIgnore = INT64_MIN;   // every row has a loss
+  float* target = reinterpret_cast<float*>(ws + l.target);
+  float* ref = reinterpret_cast<float*>(ws + l.ref);
+  float* ref_next = reinterpret_cast<float*>(ws + l.ref_next);
+  int* redo = reinterpret_cast<int*>(ws + l.flags);
+  int* unsettled = redo + 1;
+  if (int rc = fill_zero(redo, 16, stream)) return rc;
+  LabelLogitArgs la;
+  la.hidden = hidden; la.weight = weight; la.labels = labels;
+  la.m = (int)m; la.h = (int)h; la.v = (int)v;
+  la.ignore = kNoIgnore; la.exclude = -1; la.softcap = softcap; la.logit_scale = multiplier;
+  la.target = target; la.ref = ref; la.valid_count = reinterpret_cast<float*>(redo + 2);
+  if (int rc = launch_label_logit<typename E::T>(la, stream)) return rc;
+
+  ExpPanelArgs ea;
+  ea.hidden = hidden; ea.weight = weight;
+  ea.m = (int)m; ea.h = (int)h; ea.v = (int)v;
+  ea.exclude = -1; ea.softcap = softcap; ea.logit_scale = multiplier;
+  ea.n_ttiles = (int)(p.block_rows / E::kTile); ea.n_vtiles = p.n_vtiles;
+  ea.panel = ws + l.panel; ea.ld = p.vp;
+  ea.part_sum = reinterpret_cast<float*>(ws + l.part_sum);
+  ea.part_max = reinterpret_cast<float*>(ws + l.part_max);
+  ea.part_ld = (int)p.block_rows;
+  ea.part_entry = reinterpret_cast<float*>(ws + l.part_entry);
+  ea.part_rounded = reinterpret_cast<float*>(ws + l.part_rounded);
+  FusedRowsArgs ra;
+  ra.part_entry = ea.part_entry; ra.part_rounded = ea.part_rounded;
+  ra.row_rounded = reinterpret_cast<float*>(ws + l.row_rounded);
+  ra.hidden = hidden; ra.labels = labels; ra.target = target; ra.token_weights = nullptr;
+  ra.row_idx = nullptr; ra.loss_row0 = 0;
+  ra.part_sum = ea.part_sum; ra.part_max = ea.part_max;
+  ra.part_ld = ea.part_ld; ra.n_vtiles = p.n_vtiles;
+  ra.m = (int)m; ra.m_pad = (int)p.block_rows; ra.h = (int)h; ra.v = (int)v;
+  ra.ignore = kNoIgnore; ra.exclude = -1; ra.softcap = softcap; ra.logit_scale = multiplier;
+  ra.window = kRefWindow;
+  ra.panel = ea.panel; ra.ld = ea.ld;
+  ra.lse = lse; ra.losses = losses; ra.probabilities = probabilities; ra.keep_label = true;
+  ra.row_scale = reinterpret_cast<float*>(ws + l.row_scale); ra.scaled_hidden = nullptr;
+  ra.ref_next = ref_next; ra.redo = redo;
+  for (int attempt = 0; attempt < 2; ++attempt) {
+    ea.ref = ra.ref = attempt ? ref_next : ref;
+    ea.run_flag = ra.run_flag = attempt ? redo : nullptr;
+    if (softcap > 0.0f) {
+      if (int rc = launch_exp_panel_variant<E, true, false, true>(ea, stream)) return rc;
+    } else {
+      if (int rc = launch_exp_panel_variant<E, false, false, true>(ea, stream)) return rc;
+    }
+    if (int rc = launch_fused_rows<typename E::T>(ra, stream)) return rc;
+  }
+
+  TopkSelectArgs sa;
+  sa.panel = ea.panel; sa.ld = ea.ld;
+  sa.part_max = ea.part_max; sa.part_ld = ea.part_ld; sa.n_vtiles = p.n_vtiles;
+  sa.ref = ref; sa.ref_next = ref_next; sa.redo = redo;
+  sa.hidden = hidden; sa.weight = weight;
+  sa.m = (int)m; sa.h = (int)h; sa.k = top_k; sa.softcap = softcap; sa.logit_scale = multiplier;
+  sa.top_values = top_values; sa.top_ids = top_ids; sa.unsettled = unsettled;
+  sa.fix_value = reinterpret_cast<float*>(ws + l.fix_value);
+  sa.fix_id = reinterpret_cast<int*>(ws + l.fix_id);
+  sa.row_rounded = ra.row_rounded; sa.row_scale = ra.row_scale;
+  if (int rc = launch_topk_select(sa, stream)) return rc;
+  if (int rc = topk_forward_impl<E>(t, hidden, weight, labels, m, h, v, top_k, multiplier, softcap,
+                                    losses, probabilities, top_values, top_ids, lse,
+                                    ws + l.forward, stream, nullptr, unsettled))
+    return rc;
+  return topk_contraction<E>(l, p, weight, m, h, v, unit_grad, ws, stream, true);
 }
 
 template <class E>
@@ -830,12 +1058,15 @@ int topk_forward_with_gradient_impl(const TopkPlan& t, const FusedPlan& p, const
                                     float* top_values, int64_t* top_ids, float* lse,
                                     float* unit_grad, char* ws, hipStream_t stream) {
   using T = typename E::T;
+  if (topk_from_exp_supported(m, v, top_k))
+    return topk_from_exp_impl<E>(t, p, hidden, weight, labels, m, h, v, top_k, multiplier, softcap,
+                                 losses, probabilities, top_values, top_ids, lse, unit_grad, ws,
+                                 stream);
   const TopkFusedLayout l = topk_fused_layout(t, p, h);
   char* fws = ws + l.forward;
   T* panel = reinterpret_cast<T*>(ws + l.panel);
   float* ref_used = reinterpret_cast<float*>(ws + l.ref_used);
   float* row_scale = reinterpret_cast<float*>(ws + l.row_scale);
-  float* slabs = reinterpret_cast<float*>(ws + l.slabs);
   const int m_pad = (int)p.block_rows;
   TopkExpHook hook;
   hook.panel = panel; hook.ld = p.vp; hook.m_pad = m_pad; hook.ref_used = ref_used;
@@ -856,22 +1087,7 @@ int topk_forward_with_gradient_impl(const TopkPlan& t, const FusedPlan& p, const
   sa.run_sum = run_sum; sa.multiplier = multiplier; sa.m = (int)m; sa.m_pad = m_pad;
   sa.row_scale = row_scale;
   if (int rc = launch_topk_row_scale(sa, stream)) return rc;
-
-  if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
-  GemmArgs g;
-  set_head_operand(g, weight, v, h, ws + l.k_tail);
-  g.b = panel; g.ldb = p.vp; g.b_rows = m_pad;
-  g.k_per_split = 0;
-  g.ni = p.n_htiles; g.nj = m_pad / E::kTile;
-  g.c = slabs; g.ldc = h; g.c_rows = (int)m; g.c_cols = (int)h;
-  g.c_split_stride = p.block_rows * h;
-  g.mode = kStoreF32;
-  if (int rc = launch_gemm<E, true, false>(g, p.dh_ksplit, kClassGradHidden, stream)) return rc;
-  ReduceSlabsArgs rs;
-  rs.slabs = slabs; rs.n_splits = p.dh_ksplit; rs.split_stride = p.block_rows * h;
-  rs.row_scale = row_scale; rs.m = (int)m; rs.h = (int)h;
-  rs.out = unit_grad;
-  return launch_reduce_slabs(rs, stream);
+  return topk_contraction<E>(l, p, weight, m, h, v, unit_grad, ws, stream);
 }
 
 // ---- frozen-head KL: the gradient formed in the forward (3 contractions, not 6) ----
@@ -1157,7 +1373,9 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
 #define TLCE_LAUNCHERS_EXP_PANEL(X, E)                                                  \
   X int launch_kl_panel_emit<E>(const KlPanelArgs&, hipStream_t);                       \
   TLCE_LAUNCHERS_EXP_GRADIENTS(X, E)                                                    \
-  X int launch_exp_panel_variant<E, true, true>(const ExpPanelArgs&, hipStream_t);
+  X int launch_exp_panel_variant<E, true, true>(const ExpPanelArgs&, hipStream_t);      \
+  X int launch_exp_panel_variant<E, false, false, true>(const ExpPanelArgs&, hipStream_t); \
+  X int launch_exp_panel_variant<E, true, false, true>(const ExpPanelArgs&, hipStream_t);
 #define TLCE_FUSED_GRADIENTS(X, E)                                                               \
   X int fused_gradients_impl<E>(const FusedPlan&, const void*, const void*, const int64_t*,      \
                                 const int64_t*, int64_t, int64_t, int64_t, int, int64_t,         \

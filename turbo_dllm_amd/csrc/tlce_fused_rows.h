@@ -67,6 +67,8 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
   __shared__ float sh_sum[kFusedRowsWaves][kFusedRowsPerBlock];
   __shared__ float sh_max[kFusedRowsWaves][kFusedRowsPerBlock];
   __shared__ float sh_factor[kFusedRowsPerBlock];
+  __shared__ float sh_entry[kFusedRowsWaves][kFusedRowsPerBlock];
+  __shared__ float sh_rounded[kFusedRowsWaves][kFusedRowsPerBlock];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int row0 = blockIdx.x * kFusedRowsPerBlock;
@@ -83,6 +85,18 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
     }
     sh_sum[wave][lane] = sum;
     sh_max[wave][lane] = mx2;
+    if (p.part_rounded != nullptr) {
+      float entry = 0.0f, rounded = 0.0f;
+      if (r < p.m) {
+#pragma unroll 4
+        for (int t = wave; t < p.n_vtiles; t += kFusedRowsWaves) {
+          entry += p.part_entry[(int64_t)t * p.part_ld + r];
+          rounded += p.part_rounded[(int64_t)t * p.part_ld + r];
+        }
+      }
+      sh_entry[wave][lane] = entry;
+      sh_rounded[wave][lane] = rounded;
+    }
   }
   __syncthreads();
   if (wave == 0) {
@@ -105,15 +119,26 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
       const int64_t label = p.labels[r];
       const float lse = live ? c + logf(sum) : 0.0f;
       if (live) factor = w * p.logit_scale / sum;
+      if (p.part_rounded != nullptr) {
+        float entry = sh_entry[0][lane], rounded = sh_rounded[0][lane];
+#pragma unroll
+        for (int q = 1; q < kFusedRowsWaves; ++q) {
+          entry += sh_entry[q][lane];
+          rounded += sh_rounded[q][lane];
+        }
+        if (live && rounded > 0.0f) factor *= entry / rounded;
+        if (p.row_rounded != nullptr) p.row_rounded[r] = rounded;
+      }
       p.lse[r] = lse;
       if (p.losses != nullptr) {
         const int64_t o = (p.row_idx != nullptr) ? p.row_idx[r] : p.loss_row0 + r;
         p.losses[o] = live ? lse - target : 0.0f;
       }
+      if (p.probabilities != nullptr) p.probabilities[r] = live ? expf(target - lse) : 0.0f;
       p.ref_next[r] = (live && !in_window) ? mx : c;
       if (live && !in_window) atomicOr(p.redo, 1);
       // the label's entry: s * entry = (softmax - 1) * cap'
-      if (live && label >= 0 && label < p.v && label != p.exclude) {
+      if (!p.keep_label && live && label >= 0 && label < p.v && label != p.exclude) {
         float dcap = 1.0f;
         if (p.softcap > 0.0f) {
           const float t = target / p.softcap;
@@ -227,11 +252,31 @@ __global__ __launch_bounds__(256) void lce_reduce_scaled_slabs_kernel(ReduceSlab
   }
   const float s = p.row_scale[r];
   const float* src = p.slabs + (int64_t)r * p.h;
+  float fix[kTopkFix];
+  const __bf16* fix_row[kTopkFix];
+  if (p.fix_value != nullptr) {
+#pragma unroll
+    for (int j = 0; j < kTopkFix; ++j) {
+      fix[j] = p.fix_value[(int64_t)r * kTopkFix + j];
+      fix_row[j] = static_cast<const __bf16*>(p.weight) +
+                   (int64_t)p.fix_id[(int64_t)r * kTopkFix + j] * p.h;
+    }
+  }
   for (int k = threadIdx.x * 4; k < p.h; k += 256 * 4) {
     f32x4_t sum = *reinterpret_cast<const f32x4_t*>(src + k);
 #pragma unroll 8
     for (int q = 1; q < p.n_splits; ++q)
       sum += *reinterpret_cast<const f32x4_t*>(src + (int64_t)q * p.split_stride + k);
+    if (p.fix_value != nullptr) {
+      typedef __bf16 v4_t __attribute__((ext_vector_type(4)));
+      v4_t w[kTopkFix];
+#pragma unroll
+      for (int j = 0; j < kTopkFix; ++j) w[j] = *reinterpret_cast<const v4_t*>(fix_row[j] + k);
+#pragma unroll
+      for (int j = 0; j < kTopkFix; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] = fmaf(fix[j], to_float<__bf16>(w[j][e]), sum[e]);
+    }
     sum = sum * s;
     if (p.out_t != nullptr) {
       store4<__bf16>(static_cast<__bf16*>(p.out_t) + (int64_t)r * p.h + k, sum[0], sum[1], sum[2],
@@ -288,6 +333,248 @@ __global__ __launch_bounds__(256) void lce_kl_grad_from_exp_kernel(KlGradFromExp
     for (int i = 0; i < 8; ++i) out[i] = from_float<__bf16>(0.0f);
   }
   *reinterpret_cast<v8_t*>(e) = out;
+}
+
+// Orders LDS accesses of one wave's lanes (its LDS instructions complete in order).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One wave per row, eight rows per workgroup (neighbouring rows' tile maxima share the 64-byte
+// sectors they are read from); nothing is shared between the waves.  What bounds it is the
+// latency of each row's chain: maxima, about k tiles of entries (512 bytes each), a few dot
+// products of h.
+constexpr int kSelectRows = 8;
+constexpr int kSelectCap = 768;    // candidates; pruned beyond kSelectPrune (a tile adds 256)
+constexpr int kSelectPrune = 512;
+
+__global__ __launch_bounds__(64 * kSelectRows) void lce_topk_select_kernel(TopkSelectArgs p) {
+  __shared__ unsigned ids_all[kSelectRows][kSelectCap];
+  __shared__ unsigned short ent_all[kSelectRows][kSelectCap];   // bf16 bits of the entries
+  // the tiles to read, then (in their place) the candidates' logits
+  __shared__ float val_all[kSelectRows][kSelectPrune];
+  static_assert(kSelectPrune * sizeof(float) >= kTopkSelectTiles * sizeof(unsigned short), "");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = blockIdx.x * kSelectRows + wave;
+  if (r >= p.m) return;
+  unsigned* ids = ids_all[wave];
+  unsigned short* ent = ent_all[wave];
+  unsigned short* tiles = reinterpret_cast<unsigned short*>(val_all[wave]);
+  float* val = val_all[wave];
+  const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  const __bf16* hrow = static_cast<const __bf16*>(p.hidden) + (int64_t)r * p.h;
+  auto as_bf16 = [](unsigned bits) { return __uint_as_float(bits << 16); };
+
+  // the row's tile maxima as keys that order like the numbers (NaN lowest: no tile holds one)
+  constexpr int kKeys = kTopkSelectTiles / 64;
+  unsigned key[kKeys];
+  float row_max = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < kKeys; ++i) {
+    const int t = lane + 64 * i;
+    key[i] = 0;
+    if (t < p.n_vtiles) {
+      const float mx = p.part_max[(int64_t)t * p.part_ld + r];
+      const unsigned u = __float_as_uint(mx);
+      key[i] = (u & 0x80000000u) ? ~u : u | 0x80000000u;
+      row_max = fmaxf(row_max, mx);
+    }
+  }
+  row_max = wave_max(row_max);
+  // the k-th largest of them
+  unsigned kth = 0;
+  for (int bit = 31; bit >= 0; --bit) {
+    const unsigned trial = kth | (1u << bit);
+    int count = 0;
+#pragma unroll
+    for (int i = 0; i < kKeys; ++i) count += __popcll(__ballot(key[i] >= trial));
+    if (count >= p.k) kth = trial;
+  }
+  const float bound2 = __uint_as_float((kth & 0x80000000u) ? kth & 0x7fffffffu : ~kth);
+
+  // every one of the k largest logits has an entry of at least `least`: their logits are at
+  // least the bound, entries are rounded to bf16 (2^-9), and the logits of this pass and of
+  // the dot products differ by float32 roundings.  Under a soft cap entries carry cap', which
+  // lies between cap' at the bound and at the row's maximum.
+  const float ref2 = (*p.redo != 0 ? p.ref_next[r] : p.ref[r]) * TLCE_LOG2E;
+  const float slack2 = 0.02f + 1e-5f * fabsf(bound2);
+  float dcap = 1.0f;
+  if (p.softcap > 0.0f) {
+    const float a = bound2 * TLCE_LN2 / p.softcap, b = row_max * TLCE_LN2 / p.softcap;
+    dcap = fminf(1.0f - a * a, 1.0f - b * b);
+  }
+  const float down = dcap * exp2f(-slack2);
+  float least = exp2f(bound2 - ref2) * down;
+  // (entries stay normal numbers, and a factor near 0 would let everything in)
+  bool settled = bound2 - ref2 > -100.0f && bound2 - ref2 < 100.0f && dcap > 0.05f;
+
+  int count = 0;
+  // the k-th largest entry so far (entries are not negative: their bits order like them)
+  // raises `least`; what lies below it leaves the list
+  auto prune = [&]() {
+    wave_lds_order();
+    unsigned top = 0;
+    for (int bit = 14; bit >= 0; --bit) {
+      const unsigned trial = top | (1u << bit);
+      int n = 0;
+      for (int i = 0; i < count; i += 64)
+        n += __popcll(__ballot(i + lane < count && ent[i + lane] >= trial));
+      if (n >= p.k) top = trial;
+    }
+    least = fmaxf(least, as_bf16(top) * down);
+    int kept = 0;
+    for (int i = 0; i < count; i += 64) {
+      const bool in = i + lane < count;
+      const unsigned id = in ? ids[i + lane] : 0;
+      const unsigned e = in ? ent[i + lane] : 0;
+      const bool keep = in && as_bf16(e) >= least;
+      const unsigned long long mask = __ballot(keep);
+      wave_lds_order();
+      if (keep) {
+        const int at = kept + __popcll(mask & below);
+        ids[at] = id;
+        ent[at] = (unsigned short)e;
+      }
+      kept += __popcll(mask);
+      wave_lds_order();
+    }
+    count = kept;
+  };
+  if (settled) {
+    int n_tiles = 0;
+#pragma unroll
+    for (int i = 0; i < kKeys; ++i) {
+      const unsigned u = (key[i] & 0x80000000u) ? key[i] & 0x7fffffffu : ~key[i];
+      const bool hit = key[i] != 0 && __uint_as_float(u) >= bound2 - slack2;
+      const unsigned long long mask = __ballot(hit);
+      if (hit) tiles[n_tiles + __popcll(mask & below)] = (unsigned short)(lane + 64 * i);
+      n_tiles += __popcll(mask);
+    }
+    wave_lds_order();
+    const __bf16* row = static_cast<const __bf16*>(p.panel) + (int64_t)r * p.ld;
+    constexpr int kAhead = 8;   // tiles in flight
+    for (int t0 = 0; t0 < n_tiles && settled; t0 += kAhead) {
+      uint2 quad[kAhead];
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j)
+        quad[j] = *reinterpret_cast<const uint2*>(
+            row + (int64_t)tiles[min(t0 + j, n_tiles - 1)] * 256 + lane * 4);
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) {
+        if (t0 + j >= n_tiles) break;
+        const unsigned first = (unsigned)tiles[t0 + j] * 256 + lane * 4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const unsigned half = q < 2 ? quad[j].x : quad[j].y;
+          const unsigned bits = (q & 1) ? half >> 16 : half & 0xffffu;
+          const bool in = as_bf16(bits) >= least;
+          const unsigned long long mask = __ballot(in);
+          if (in) {
+            const int at = count + __popcll(mask & below);
+            ids[at] = first + q;
+            ent[at] = (unsigned short)bits;
+          }
+          count += __popcll(mask);
+        }
+        if (count > kSelectPrune) {
+          prune();
+          if (count > kSelectPrune) {
+            settled = false;
+            break;
+          }
+        }
+      }
+    }
+    if (settled) prune();
+    settled = settled && count >= p.k && count <= min(3 * p.k + 96, kSelectPrune);
+  }
+  // (no correction until one is known; slots beyond k stay like this)
+  if (lane < kTopkFix) {
+    p.fix_value[(int64_t)r * kTopkFix + lane] = 0.0f;
+    p.fix_id[(int64_t)r * kTopkFix + lane] = 0;
+  }
+  if (!settled) {
+    // a row of zeros (padding): all logits are 0, the list is the first k words
+    float any = 0.0f;
+    for (int k = lane; k < p.h; k += 64) any = fmaxf(any, fabsf(to_float<__bf16>(hrow[k])));
+    if (wave_max(any) == 0.0f && row_max == 0.0f) {
+      for (int j = lane; j < p.k; j += 64) {
+        p.top_values[(int64_t)r * p.k + j] = 0.0f;
+        p.top_ids[(int64_t)r * p.k + j] = j;
+      }
+    } else if (lane == 0) {
+      atomicOr(p.unsettled, 1);
+    }
+    return;
+  }
+
+  // the candidates' logits, four dot products at a time (each as wave_dot adds it up)
+  bool numbers = true;
+  typedef __bf16 v8_t __attribute__((ext_vector_type(8)));
+  for (int c = 0; c < count; c += 4) {
+    const __bf16* w[4];
+    float dot[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      w[j] = static_cast<const __bf16*>(p.weight) + (int64_t)ids[min(c + j, count - 1)] * p.h;
+      dot[j] = 0.0f;
+    }
+#pragma unroll 2
+    for (int k = lane * 8; k < p.h; k += 64 * 8) {
+      const v8_t a = *reinterpret_cast<const v8_t*>(hrow + k);
+      v8_t b[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[j] = *reinterpret_cast<const v8_t*>(w[j] + k);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          dot[j] = fmaf(to_float<__bf16>(a[e]), to_float<__bf16>(b[j][e]), dot[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float z = wave_sum(dot[j]) * p.logit_scale;
+      if (p.softcap > 0.0f) z = p.softcap * tanhf(z / p.softcap);
+      if (lane == 0 && c + j < count) val[c + j] = z;
+      numbers = numbers && z == z;
+    }
+  }
+  if (!numbers) {
+    if (lane == 0) atomicOr(p.unsettled, 1);
+    return;
+  }
+  wave_lds_order();
+  // each by its rank: larger first, then the smaller id
+  float fixed = 0.0f;
+  for (int i = lane; i < count; i += 64) {
+    const float z = val[i];
+    const unsigned id = ids[i];
+    int rank = 0;
+    for (int j = 0; j < count; ++j) {
+      const float other = val[j];
+      rank += (other > z || (other == z && ids[j] < id)) ? 1 : 0;
+    }
+    if (rank < p.k) {
+      p.top_values[(int64_t)r * p.k + rank] = z;
+      p.top_ids[(int64_t)r * p.k + rank] = id;
+    }
+    if (rank < min(p.k, kTopkFix)) {
+      float cap = 1.0f;
+      if (p.softcap > 0.0f) {
+        const float t = z / p.softcap;
+        cap = 1.0f - t * t;
+      }
+      const float fix = exp2f(z * TLCE_LOG2E - ref2) * cap - as_bf16(ent[i]);
+      p.fix_value[(int64_t)r * kTopkFix + rank] = fix;
+      p.fix_id[(int64_t)r * kTopkFix + rank] = (int)id;
+      fixed += fix;
+    }
+  }
+  fixed = wave_sum(fixed);
+  const float rounded = p.row_rounded[r];
+  if (lane == 0 && rounded > 0.0f && rounded + fixed > 0.0f)
+    p.row_scale[r] *= rounded / (rounded + fixed);
 }
 
 // One row and 2048 columns per workgroup, 8 columns per thread.

@@ -887,7 +887,10 @@ int topk_forward_impl(const TopkPlan& t, const void* hidden, const void* weight,
                       const int64_t* labels, int64_t m, int64_t h, int64_t v, int top_k,
                       float multiplier, float softcap, float* losses, float* probabilities,
                       float* top_values, int64_t* top_ids, float* lse, char* ws,
-                      hipStream_t stream, const TopkExpHook* hook = nullptr) {
+                      hipStream_t stream, const TopkExpHook* hook = nullptr,
+                      const int* run_flag = nullptr) {
+  // run_flag: only the lists, and only if *run_flag != 0 (losses, probabilities and lse
+  // have been written from another pass over the logits)
   using T = typename E::T;
   const Plan& p = t.plan;
   float* run_max = reinterpret_cast<float*>(ws + t.run_max);
@@ -902,7 +905,7 @@ int topk_forward_impl(const TopkPlan& t, const void* hidden, const void* weight,
     la.m = (int)m; la.h = (int)h; la.v = (int)v;
     la.softcap = softcap; la.logit_scale = multiplier;
     la.v0 = (int)v0; la.n_ttiles = p.n_ttiles; la.n_ptiles = (int)(width / p.tile);
-    la.panel = panel; la.ld = t.vcf;
+    la.panel = panel; la.ld = t.vcf; la.run_flag = run_flag;
     if (softcap > 0.0f) {
       if (int rc = launch_logits_panel_variant<E, true>(la, stream)) return rc;
     } else {
@@ -912,6 +915,7 @@ int topk_forward_impl(const TopkPlan& t, const void* hidden, const void* weight,
     sa.panel = panel; sa.ld = t.vcf; sa.m = (int)m; sa.v0 = v0; sa.width = (int)valid;
     sa.stored = (int)width; sa.k = top_k; sa.first = pi == 0;
     sa.run_max = run_max; sa.run_sum = run_sum; sa.top_values = top_values; sa.top_ids = top_ids;
+    sa.run_flag = run_flag;
     if (int rc = launch_topk_scan(sa, stream)) return rc;
     if (hook != nullptr) {
       ExpFromLogitsArgs xa;
@@ -922,6 +926,7 @@ int topk_forward_impl(const TopkPlan& t, const void* hidden, const void* weight,
       if (int rc = launch_exp_from_logits(xa, stream)) return rc;
     }
   }
+  if (run_flag != nullptr) return 0;
   TopkFinishArgs fa;
   fa.hidden = hidden; fa.weight = weight; fa.labels = labels; fa.m = (int)m; fa.h = (int)h;
   fa.softcap = softcap; fa.logit_scale = multiplier;
@@ -1060,7 +1065,7 @@ int soft_embedding_impl(const Plan& fp, const Plan& bp, const SoftEmbeddingLayou
   X int topk_forward_impl<E>(const TopkPlan&, const void*, const void*, const int64_t*,         \
                              int64_t, int64_t, int64_t, int, float, float, float*, float*,      \
                              float*, int64_t*, float*, char*, hipStream_t,                      \
-                             const TopkExpHook*);                                               \
+                             const TopkExpHook*, const int*);                                   \
   X int topk_backward_impl<E>(const TopkPlan&, const void*, const void*, const int64_t*,        \
                               const float*, const int64_t*, const float*, const float*,         \
                               int64_t, int64_t, int64_t, int, int, float, float, void*, char*,  \

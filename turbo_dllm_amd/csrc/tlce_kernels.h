@@ -1026,12 +1026,14 @@ struct LogitsPanelArgs {
   int n_ttiles, n_ptiles;
   float* panel;         // [mp, ld] float32; columns past the vocabulary get -inf
   int64_t ld;
+  const int* run_flag = nullptr;   // non-null: the launch does nothing unless *run_flag != 0
 };
 
 template <class E, bool kSoftcap>
 __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_logits_panel_kernel(LogitsPanelArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
+  if (p.run_flag != nullptr && *p.run_flag == 0) return;
   int tt, pv;
   if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_ptiles, (int64_t)E::kTile * p.h * sizeof(T), &tt, &pv))
     return;
@@ -1119,6 +1121,7 @@ struct TopkScanArgs {
   float* run_sum;
   float* top_values;    // [m, k]
   int64_t* top_ids;     // [m, k]
+  const int* run_flag = nullptr;   // non-null: the launch does nothing unless *run_flag != 0
 };
 
 // One wave per row: lse, the label's logit as a direct dot product, loss and

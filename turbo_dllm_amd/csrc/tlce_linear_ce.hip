@@ -129,6 +129,13 @@ int launch_rescale_exp_rows(const RescaleExpArgs& a, int n_panels, hipStream_t s
   return 0;
 }
 
+int launch_topk_select(const TopkSelectArgs& a, hipStream_t stream) {
+  ScopedTimer timer(kClassOther, stream);
+  lce_topk_select_kernel<<<(int)ceil_div(a.m, kSelectRows), 64 * kSelectRows, 0, stream>>>(a);
+  TLCE_LAUNCH_CHECK();
+  return 0;
+}
+
 int launch_topk_row_scale(const TopkRowScaleArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassOther, stream);
   lce_topk_row_scale_kernel<<<(int)ceil_div(a.m_pad, 256), 256, 0, stream>>>(a);

@@ -180,6 +180,7 @@ __global__ __launch_bounds__(kTopkScanThreads, 6) void lce_topk_scan_kernel(Topk
   __shared__ float wave_kth[kWaves];
   __shared__ int wave_total[kWaves];
   __shared__ __align__(16) float tmax[kThreads];
+  if (p.run_flag != nullptr && *p.run_flag == 0) return;
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
   const int row = blockIdx.x;
