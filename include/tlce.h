@@ -590,6 +590,36 @@ int tlce_apply_grad_output(const float* grad_hidden_f32, const float* grad_weigh
                            int64_t h, int64_t v, int dtype, int reduction_code,
                            void* grad_hidden, void* grad_weight, void* stream);
 
+/* tlce_forward_with_gradients and what follows it in fewer launches (the library's own
+ * autograd functions take these).  The forward also reduces the losses into loss[0] (their
+ * sum; over valid_count[0] for the mean; loss may be NULL for TLCE_REDUCTION_NONE; losses is
+ * needed for either) and, with row_idx, leaves row_of[n_out] (int32): the row of an output
+ * row, -1 where there is none.  dtype: bf16, or float32 where
+ * tlce_f32_gradients_in_forward_supported (workspace: the size its own entry point tells).
+ *
+ * tlce_finish_gradients (bf16) replaces tlce_apply_grad_output and
+ * tlce_grad_weight_from_panel: one pass over the output rows, then the contraction that
+ * has waited when `hidden`, the forward's rows, is given with the forward's workspace, or
+ * the scaled grad_weight_f32 when that is.  May be called again on the same workspace. */
+int tlce_forward_with_gradients_reduced(const void* hidden, const void* weight,
+                                        const int64_t* labels, const int64_t* row_idx,
+                                        const float* token_weights, const int64_t* row_count,
+                                        int64_t m, int64_t n_out, int64_t h, int64_t v, int dtype,
+                                        int64_t ignore_index, int64_t exclude_index,
+                                        float logit_softcap, float logit_multiplier,
+                                        int reduction_code, float* losses, float* loss,
+                                        float* lse, float* valid_count, float* grad_hidden_f32,
+                                        float* grad_weight_f32, int* row_of,
+                                        int64_t panel_bytes, void* workspace,
+                                        int64_t workspace_bytes, void* stream);
+
+int tlce_finish_gradients(const float* grad_hidden_f32, const float* grad_weight_f32,
+                          const int* row_of, const int64_t* row_count, const float* grad_output,
+                          const float* valid_count, int64_t m, int64_t n_out, int64_t h,
+                          int64_t v, int reduction_code, void* grad_hidden, void* grad_weight,
+                          const void* hidden, int64_t panel_bytes, void* forward_workspace,
+                          int64_t workspace_bytes, void* stream);
+
 /* The pair for float32 operands whose products run on the bf16 matrix units
  * (tlce_f32_gradients_in_forward_supported: more than 128 rows, h a multiple of 4
  * and at least 512, 96 or more tiles of 256 x 256, 1 GiB or less of planes, six

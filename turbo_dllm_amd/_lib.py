@@ -122,6 +122,28 @@ SIGNATURES = {
             c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
         ],
     ),
+    "tlce_forward_with_gradients_reduced": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,   # hidden weight labels row_idx weights
+            c_void_p,                                           # row_count
+            c_int64, c_int64, c_int64, c_int64, c_int,          # m n_out h v dtype
+            c_int64, c_int64, c_float, c_float, c_int,          # ignore exclude softcap multiplier reduction
+            c_void_p, c_void_p, c_void_p, c_void_p,             # losses loss lse valid_count
+            c_void_p, c_void_p, c_void_p,                       # grad_hidden_f32 grad_weight_f32 row_of
+            c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
+        ],
+    ),
+    "tlce_finish_gradients": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_void_p, c_void_p,             # dh32 dw32 row_of row_count
+            c_void_p, c_void_p,                                 # grad_output valid_count
+            c_int64, c_int64, c_int64, c_int64, c_int,          # m n_out h v reduction
+            c_void_p, c_void_p, c_void_p,                       # grad_hidden grad_weight hidden
+            c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
+        ],
+    ),
     "tlce_f32_gradients_in_forward_supported": (c_int, [c_int64, c_int64, c_int64]),
     "tlce_forward_with_gradients_f32_workspace_bytes": (
         c_int64, [c_int64, c_int64, c_int64, c_int, c_int64]

@@ -477,6 +477,147 @@ def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
         hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
 
 
+def gradients_in_forward_supported(m: int, hidden: torch.Tensor, weight: torch.Tensor,
+                                   bias: torch.Tensor | None, weight_dim_first: bool) -> bool:
+    """Whether ``forward_with_gradients_reduced`` takes ``m`` rows of these operands."""
+    return (fused_gradients_supported(hidden, weight, bias, weight_dim_first)
+            or f32_gradients_in_forward_supported(m, hidden, weight, bias, weight_dim_first))
+
+
+def forward_with_gradients_reduced(
+    hidden: torch.Tensor,
+    weight: torch.Tensor,
+    labels: torch.Tensor,
+    *,
+    reduction: str,
+    ignore_index: int,
+    exclude_index: int,
+    logit_softcap: float,
+    compute_weight_grad: bool,
+    postpone_weight_grad: bool,
+    token_weights: torch.Tensor | None = None,
+    logit_multiplier: float = 1.0,
+    row_idx: torch.Tensor | None = None,
+    n_out: int | None = None,
+    row_count: torch.Tensor | None = None,
+):
+    """``forward_with_gradients`` (and ``_f32``) in fewer launches, with the loss reduced on
+    the way: ``(loss, valid_count, grad_hidden_f32, grad_weight_f32 or workspace, row_of)``.
+
+    ``loss`` is ``[n_out]`` for reduction "none", else one number (over the count of rows
+    with a loss for "mean").  ``row_of`` (int32 ``[n_out]``, when ``row_idx`` is given) is the
+    inverse of ``row_idx``, -1 elsewhere: ``finish_gradients`` takes it."""
+    device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
+    reduction_code = _reduction_code(reduction)
+    m, h = hidden.shape
+    v = weight.shape[0]
+    if not gradients_in_forward_supported(m, hidden, weight, None, False):
+        raise RuntimeError("forward_with_gradients_reduced does not take these operands "
+                           "(gradients_in_forward_supported)")
+    hidden = _dense(hidden)
+    weight = _dense(weight)
+    if labels.dtype != torch.long or not labels.is_contiguous() or labels.numel() != m:
+        raise RuntimeError("labels must be contiguous int64 with one entry per row")
+    if row_idx is not None and row_idx.numel() != m:
+        raise RuntimeError("row_idx must have one entry per row")
+    if token_weights is not None and (
+            token_weights.numel() != m or token_weights.dtype != torch.float32
+            or not token_weights.is_contiguous()):
+        raise RuntimeError("token_weights must be contiguous float32 with one entry per row")
+    n_out = m if n_out is None else int(n_out)
+    lib = _lib.library()
+    code = _dtype_code(hidden)
+    f32 = hidden.dtype == torch.float32
+    postpone = bool(postpone_weight_grad and compute_weight_grad)
+    if postpone and not weight_grad_can_wait(m, h, v, hidden.dtype):
+        raise RuntimeError("the weight gradient can be postponed only when all rows fit "
+                           "one block of the forward (weight_grad_can_wait)")
+    panel = get_panel_bytes()
+    reduced = reduction_code != _lib.REDUCTION_NONE
+    with torch.cuda.device(device):
+        losses = torch.empty(n_out, dtype=torch.float32, device=device)
+        lse = torch.empty(m, dtype=torch.float32, device=device)
+        valid_count = torch.empty(1, dtype=torch.float32, device=device)
+        loss = torch.empty((), dtype=torch.float32, device=device) if reduced else losses
+        row_of = (torch.empty(n_out, dtype=torch.int32, device=device)
+                  if row_idx is not None else None)
+        grad_hidden32 = torch.empty((m, h), dtype=torch.float32, device=device)
+        grad_weight32 = (torch.empty((v, h), dtype=torch.float32, device=device)
+                         if compute_weight_grad and not postpone else None)
+        if f32:
+            size = lib.tlce_forward_with_gradients_f32_workspace_bytes(
+                m, h, v, int(compute_weight_grad), panel)
+        else:
+            size = lib.tlce_forward_with_gradients_workspace_bytes(
+                m, h, v, code, int(compute_weight_grad), panel)
+        ws = _workspace(size, device)
+        _lib.check(
+            lib.tlce_forward_with_gradients_reduced(
+                hidden.data_ptr(), weight.data_ptr(), labels.data_ptr(), _ptr(row_idx),
+                _ptr(token_weights), _ptr(row_count), m, n_out, h, v, code,
+                int(ignore_index), int(exclude_index), float(logit_softcap),
+                float(logit_multiplier), reduction_code,
+                losses.data_ptr(), loss.data_ptr(), lse.data_ptr(), valid_count.data_ptr(),
+                grad_hidden32.data_ptr(), _ptr(grad_weight32), _ptr(row_of),
+                panel, ws.data_ptr(), ws.numel(), _stream(device),
+            ),
+            "tlce_forward_with_gradients_reduced",
+        )
+    return loss, valid_count, grad_hidden32, (ws if postpone else grad_weight32), row_of
+
+
+def finish_gradients(
+    grad_hidden32: torch.Tensor,
+    grad_weight32: torch.Tensor | None,
+    grad_output: torch.Tensor,
+    valid_count: torch.Tensor,
+    *,
+    reduction: str,
+    n_out: int,
+    vocab: int,
+    row_of: torch.Tensor | None,
+    row_count: torch.Tensor | None,
+    rows: torch.Tensor | None,
+    panel_bytes: int,
+) -> tuple[torch.Tensor, torch.Tensor | None]:
+    """The bf16 gradients of what ``forward_with_gradients_reduced`` left, times the upstream
+    gradient.  ``rows``: the forward's hidden rows when grad_weight was postponed
+    (``grad_weight32`` is then its workspace)."""
+    device = _require_device(grad_hidden32, grad_weight32, grad_output, valid_count, row_of,
+                             row_count, rows)
+    reduction_code = _reduction_code(reduction)
+    m, h = grad_hidden32.shape
+    v = int(vocab)
+    grad_output = _upstream_gradient(grad_output, reduction_code, n_out)
+    if grad_hidden32.dtype != torch.float32 or not grad_hidden32.is_contiguous():
+        raise RuntimeError("grad_hidden32 must be a contiguous float32 [m, h] tensor")
+    if row_of is not None and (row_of.dtype != torch.int32 or row_of.numel() != n_out):
+        raise RuntimeError("row_of must be int32 with one entry per output row")
+    waited = rows is not None
+    if waited and (rows.shape != grad_hidden32.shape or not rows.is_contiguous()
+                   or grad_weight32 is None or grad_weight32.dtype != torch.uint8):
+        raise RuntimeError("a postponed grad_weight needs the forward's rows and workspace")
+    if not waited and grad_weight32 is not None and (
+            grad_weight32.dtype != torch.float32 or tuple(grad_weight32.shape) != (v, h)
+            or not grad_weight32.is_contiguous()):
+        raise RuntimeError("grad_weight32 must be a contiguous float32 [v, h] tensor")
+    with torch.cuda.device(device):
+        grad_hidden = torch.empty((n_out, h), dtype=torch.bfloat16, device=device)
+        grad_weight = (torch.empty((v, h), dtype=torch.bfloat16, device=device)
+                       if grad_weight32 is not None else None)
+        _lib.check(
+            _lib.library().tlce_finish_gradients(
+                _ptr(grad_hidden32), None if waited else _ptr(grad_weight32), _ptr(row_of),
+                _ptr(row_count), grad_output.data_ptr(), _ptr(valid_count), m, n_out, h, v,
+                reduction_code, _ptr(grad_hidden), _ptr(grad_weight), _ptr(rows),
+                int(panel_bytes), grad_weight32.data_ptr() if waited else None,
+                grad_weight32.numel() if waited else 0, _stream(device),
+            ),
+            "tlce_finish_gradients",
+        )
+    return grad_hidden, grad_weight
+
+
 def f32_gradients_in_forward_supported(m: int, hidden: torch.Tensor, weight: torch.Tensor,
                                        bias: torch.Tensor | None,
                                        weight_dim_first: bool) -> bool:

@@ -298,8 +298,14 @@ struct LabelLogitArgs {
   float softcap, logit_scale;
   float* target;        // [m] cap(scale * h . w[label]); 0 when the label has no logit
   float* ref;           // [m] reference logit; +inf for rows without loss
-  float* valid_count;   // [1] += rows with a label other than `ignore`
+  float* valid_count;   // [1] rows with a label other than `ignore`
   const int64_t* m_dev = nullptr;   // device row count (null: m is exact)
+  // what the sequence needs cleared before it, in the same launch
+  int* flags = nullptr;             // [n_flags] = 0
+  int n_flags = 0;
+  float* losses = nullptr;          // [n_out] = 0
+  int* row_of = nullptr;            // [n_out] = -1
+  int64_t n_out = 0;
 };
 
 struct FusedRowsArgs {
@@ -310,6 +316,7 @@ struct FusedRowsArgs {
   const float* token_weights;  // [m] or null
   const int64_t* row_idx;      // [m] or null: where the row's loss goes
   int64_t loss_row0;           // row_idx == null: index of the block's first row in `losses`
+  int* row_of = nullptr;       // with row_idx: row_of[row_idx[r]] = index of row r of the call
   const float* part_sum;
   const float* part_max;
   int part_ld, n_vtiles;
@@ -357,6 +364,12 @@ struct ReduceSlabsArgs {
   const float* fix_value = nullptr;
   const int* fix_id = nullptr;
   const void* weight = nullptr;     // bf16 [.., h]
+  // non-null: one more workgroup adds up the losses (over valid_count[0] for the mean)
+  float* loss = nullptr;
+  const float* losses = nullptr;    // [n_losses]
+  int64_t n_losses = 0;
+  const float* valid_count = nullptr;
+  bool mean = false;
 };
 // Largest entries of a row whose rounding the top-k path makes up for: they are known exactly
 // and weigh most (a label or word of probability near 1 is most of the sum).
@@ -391,6 +404,25 @@ struct ScaleRowsArgs {
   const int64_t* m_dev = nullptr;   // device row count (null: m is exact)
   const int64_t* row_idx = nullptr; // output row of row r (null: r)
 };
+
+// The backward's pass over rows when the forward has left row_of: one workgroup per output
+// row writes its gradient (lce_scale_cast_rows_kernel) or zeros and, when grad_weight has
+// waited, the row of its operand (lce_scale_rows_kernel).
+struct FinishRowsArgs {
+  const float* grad_hidden32;  // [m, h]
+  const int* row_of;           // [n_out] row of an output row, -1: none (null: the same row)
+  const float* grad_output;    // [1]; reduction none: [n_out]
+  const float* valid_count;    // [1], read for the mean reduction only
+  int reduction;
+  int64_t n_out;
+  int m, m_pad, h;
+  const int64_t* m_dev;        // device row count (null: m is exact)
+  void* grad_hidden;           // bf16 [n_out, h]
+  const void* hidden = nullptr;       // [m, h], with what follows, or null
+  const float* row_scale = nullptr;   // [m]
+  void* scaled = nullptr;             // bf16 [m_pad, h], zero rows from the row count on
+};
+int launch_finish_rows(const FinishRowsArgs& a, hipStream_t stream);
 
 // row_scale[r] = scale / sum over the vocabulary tiles of part_sum[tile][r] (0 for rows
 // from m up to m_pad): the normaliser of rows whose panel holds exp(z - c).
@@ -538,6 +570,10 @@ struct FusedOptions {
   float logit_scale = 1.0f;
   const float* token_weights = nullptr;   // [m] per-row loss weights or null
   const int64_t* row_count = nullptr;     // device int64: the real number of rows (m: capacity)
+  int64_t n_out = 0;                      // entries of losses (cleared when row_idx is given)
+  int* row_of = nullptr;                  // [n_out], with row_idx: LabelLogitArgs, FusedRowsArgs
+  float* loss = nullptr;                  // [1]: the losses' sum, or their mean
+  bool mean = false;
 };
 
 template <class E>
@@ -585,8 +621,11 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     weight_t = ws + l.weight_planes;
   }
 
-  if (int rc = fill_zero(redo, (int64_t)p.n_blocks * 4, stream)) return rc;
   LabelLogitArgs la;
+  la.flags = redo; la.n_flags = p.n_blocks;
+  if (row_idx != nullptr) {
+    la.losses = losses; la.row_of = opt.row_of; la.n_out = opt.n_out;
+  }
   la.hidden = hidden; la.weight = weight; la.labels = labels;
   la.m = (int)m; la.h = (int)h; la.v = (int)v;
   la.ignore = ignore; la.exclude = exclude; la.softcap = softcap; la.logit_scale = opt.logit_scale;
@@ -615,6 +654,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     ra.target = target + r0;
     ra.token_weights = opt.token_weights ? opt.token_weights + r0 : nullptr;
     ra.row_idx = row_idx ? row_idx + r0 : nullptr; ra.loss_row0 = r0;
+    ra.row_of = row_idx ? opt.row_of : nullptr;
     ra.part_sum = part_sum; ra.part_max = part_max;
     ra.part_ld = (int)p.block_rows; ra.n_vtiles = p.n_vtiles;
     ra.m = (int)rows; ra.m_pad = (int)rows_p; ra.h = (int)h; ra.v = (int)v; ra.hp = (int)hp;
@@ -674,6 +714,10 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     rs.row_scale = row_scale; rs.m = (int)rows; rs.h = (int)h;
     rs.out = grad_hidden32 + r0 * h;
     rs.m_dev = m_dev; rs.row0 = r0;
+    if (r0 + rows >= m) {
+      rs.loss = opt.loss; rs.losses = losses; rs.n_losses = row_idx != nullptr ? opt.n_out : m;
+      rs.valid_count = valid_count; rs.mean = opt.mean;
+    }
     if (int rc = launch_reduce_slabs(rs, stream)) return rc;
 
     if (weight_grad) {
@@ -702,20 +746,9 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
 // since (the forward was called without a grad_weight buffer, as for a frozen head,
 // on a workspace sized for one).
 template <class E>
-int deferred_grad_weight_impl(const FusedPlan& p, const void* hidden, int64_t m, int64_t h,
-                              int64_t v, int dtype, const float* grad_output,
-                              const float* valid_count, int reduction, const int64_t* m_dev,
-                              const int64_t* row_idx, void* grad_weight, char* ws,
-                              hipStream_t stream) {
+int deferred_contraction(const FusedPlan& p, const FusedLayout& l, int64_t m, int64_t h, int64_t v,
+                         const int64_t* m_dev, void* grad_weight, char* ws, hipStream_t stream) {
   using T = typename E::T;
-  const FusedLayout l = fused_layout(p, m, h, dtype, true);
-  const int64_t rows_p = round_up(m, E::kTile);
-  ScaleRowsArgs sa;
-  sa.hidden = hidden; sa.row_scale = reinterpret_cast<const float*>(ws + l.row_scale);
-  sa.grad_output = grad_output; sa.valid_count = valid_count; sa.reduction = reduction;
-  sa.m = (int)m; sa.m_pad = (int)rows_p; sa.h = (int)h;
-  sa.out = ws + l.scaled_hidden; sa.m_dev = m_dev; sa.row_idx = row_idx;
-  if (int rc = launch_scale_rows(sa, stream)) return rc;
   GemmArgs dw;
   dw.a = ws + l.scaled_hidden; dw.lda = h; dw.a_rows = (int)h;
   dw.b = ws + l.panel; dw.ldb = p.vp; dw.b_rows = (int)p.vp;
@@ -727,6 +760,23 @@ int deferred_grad_weight_impl(const FusedPlan& p, const void* hidden, int64_t m,
   dw.mode = kStoreT;
   dw.m_dev = m_dev; dw.m_role = kKFollows; dw.m_round = 64;
   return launch_gemm<E, true, true>(dw, 1, kClassGradWeight, stream);
+}
+
+template <class E>
+int deferred_grad_weight_impl(const FusedPlan& p, const void* hidden, int64_t m, int64_t h,
+                              int64_t v, int dtype, const float* grad_output,
+                              const float* valid_count, int reduction, const int64_t* m_dev,
+                              const int64_t* row_idx, void* grad_weight, char* ws,
+                              hipStream_t stream) {
+  const FusedLayout l = fused_layout(p, m, h, dtype, true);
+  const int64_t rows_p = round_up(m, E::kTile);
+  ScaleRowsArgs sa;
+  sa.hidden = hidden; sa.row_scale = reinterpret_cast<const float*>(ws + l.row_scale);
+  sa.grad_output = grad_output; sa.valid_count = valid_count; sa.reduction = reduction;
+  sa.m = (int)m; sa.m_pad = (int)rows_p; sa.h = (int)h;
+  sa.out = ws + l.scaled_hidden; sa.m_dev = m_dev; sa.row_idx = row_idx;
+  if (int rc = launch_scale_rows(sa, stream)) return rc;
+  return deferred_contraction<E>(p, l, m, h, v, m_dev, grad_weight, ws, stream);
 }
 
 // Soft embedding under a soft cap in two contractions instead of three
@@ -988,8 +1038,8 @@ int topk_from_exp_impl(const TopkPlan& t, const FusedPlan& p, const void* hidden
   float* ref_next = reinterpret_cast<float*>(ws + l.ref_next);
   int* redo = reinterpret_cast<int*>(ws + l.flags);
   int* unsettled = redo + 1;
-  if (int rc = fill_zero(redo, 16, stream)) return rc;
   LabelLogitArgs la;
+  la.flags = redo; la.n_flags = 2;
   la.hidden = hidden; la.weight = weight; la.labels = labels;
   la.m = (int)m; la.h = (int)h; la.v = (int)v;
   la.ignore = kNoIgnore; la.exclude = -1; la.softcap = softcap; la.logit_scale = multiplier;
@@ -1398,6 +1448,8 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
                                          const void*, const void*, int64_t, int64_t, int64_t,    \
                                          int64_t, int, float, float*, float*, float*, float*,    \
                                          char*, hipStream_t);                                    \
+  X int deferred_contraction<E>(const FusedPlan&, const FusedLayout&, int64_t, int64_t, int64_t, \
+                                const int64_t*, void*, char*, hipStream_t);                      \
   X int deferred_grad_weight_impl<E>(const FusedPlan&, const void*, int64_t, int64_t, int64_t,   \
                                      int, const float*, const float*, int, const int64_t*,       \
                                      const int64_t*, void*, char*, hipStream_t);

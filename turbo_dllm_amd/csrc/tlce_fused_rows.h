@@ -8,17 +8,43 @@
 
 namespace tlce {
 
-// One wave per row, 16 rows per workgroup (one atomic per workgroup for the count
-// of rows with a loss).
+// One wave per row, 16 rows per workgroup; behind those, one workgroup that counts the rows
+// with a loss and clears the flags, and workgroups that clear the losses and the map of rows.
+// Those were launches of their own, as were the sum of the losses (now in the slab reduction)
+// and the backward's two passes over rows and the clearing before them
+// (lce_finish_rows_kernel): 5 us of host time each, which is what bounds small steps (64 rows
+// over V = 32000 252 -> 224 us, 1036 rows 343 -> 322).
+constexpr int kClearPerBlock = 4096;
+
 template <typename T>
 __global__ __launch_bounds__(256) void lce_label_logit_kernel(LabelLogitArgs p) {
-  __shared__ int block_valid;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  if (threadIdx.x == 0) block_valid = 0;
-  __syncthreads();
+  const int extra = (int)blockIdx.x - (p.m + 15) / 16;
   p.m = effective_rows(p.m, p.m_dev);
-  int wave_valid = 0;
+  if (extra == 0) {
+    __shared__ int sh_valid[4];
+    for (int i = threadIdx.x; i < p.n_flags; i += 256) p.flags[i] = 0;
+    int valid = 0;
+#pragma unroll 8
+    for (int r = threadIdx.x; r < p.m; r += 256) valid += p.labels[r] != p.ignore ? 1 : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) valid += __shfl_xor(valid, o, 64);
+    if (lane == 0) sh_valid[wave] = valid;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      p.valid_count[0] = (float)(sh_valid[0] + sh_valid[1] + sh_valid[2] + sh_valid[3]);
+    return;
+  }
+  if (extra > 0) {
+    const int64_t first = (int64_t)(extra - 1) * kClearPerBlock;
+    const int64_t last = min(first + kClearPerBlock, p.n_out);
+    for (int64_t i = first + threadIdx.x; i < last; i += 256) {
+      if (p.losses != nullptr) p.losses[i] = 0.0f;
+      if (p.row_of != nullptr) p.row_of[i] = -1;
+    }
+    return;
+  }
   for (int i = 0; i < 4; ++i) {
     const int r = blockIdx.x * 16 + wave * 4 + i;
     if (r >= p.m) continue;
@@ -39,11 +65,7 @@ __global__ __launch_bounds__(256) void lce_label_logit_kernel(LabelLogitArgs p) 
       p.target[r] = (here && label != p.exclude) ? z : 0.0f;
       p.ref[r] = valid ? z : INFINITY;
     }
-    wave_valid += valid ? 1 : 0;
   }
-  if (lane == 0 && wave_valid != 0) atomicAdd(&block_valid, wave_valid);
-  __syncthreads();
-  if (threadIdx.x == 0 && block_valid != 0) atomicAdd(p.valid_count, (float)block_valid);
 }
 
 // 64 rows per workgroup of 16 waves, the rows across the lanes (coalesced: partials are
@@ -130,10 +152,9 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
         if (p.row_rounded != nullptr) p.row_rounded[r] = rounded;
       }
       p.lse[r] = lse;
-      if (p.losses != nullptr) {
-        const int64_t o = (p.row_idx != nullptr) ? p.row_idx[r] : p.loss_row0 + r;
-        p.losses[o] = live ? lse - target : 0.0f;
-      }
+      const int64_t o = (p.row_idx != nullptr) ? p.row_idx[r] : p.loss_row0 + r;
+      if (p.losses != nullptr) p.losses[o] = live ? lse - target : 0.0f;
+      if (p.row_of != nullptr) p.row_of[o] = (int)(p.loss_row0 + r);
       if (p.probabilities != nullptr) p.probabilities[r] = live ? expf(target - lse) : 0.0f;
       p.ref_next[r] = (live && !in_window) ? mx : c;
       if (live && !in_window) atomicOr(p.redo, 1);
@@ -206,6 +227,51 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
   }
 }
 
+__global__ __launch_bounds__(256) void lce_finish_rows_kernel(FinishRowsArgs p) {
+  typedef __bf16 v8_t __attribute__((ext_vector_type(8)));
+  const int m = effective_rows(p.m, p.m_dev);
+  const int64_t o = blockIdx.x;
+  const v8_t zero = {};
+  if (o >= p.n_out) {   // rows of the operand past the row count
+    const int64_t r = (p.m_dev != nullptr ? 0 : p.m) + (o - p.n_out);
+    if (r < m || r >= p.m_pad) return;
+    v8_t* out = reinterpret_cast<v8_t*>(static_cast<__bf16*>(p.scaled) + r * p.h);
+    for (int k = threadIdx.x; k < p.h / 8; k += 256) out[k] = zero;
+    return;
+  }
+  const int64_t r = p.row_of != nullptr ? p.row_of[o] : o;
+  v8_t* dst = reinterpret_cast<v8_t*>(static_cast<__bf16*>(p.grad_hidden) + o * p.h);
+  if (r < 0 || r >= m) {
+    for (int k = threadIdx.x; k < p.h / 8; k += 256) dst[k] = zero;
+    return;
+  }
+  float g = p.grad_output[p.reduction == TLCE_REDUCTION_NONE ? o : 0];
+  if (p.reduction == TLCE_REDUCTION_MEAN) {
+    // no row with a loss: every gradient entry is zero and stays zero
+    const float count = p.valid_count[0];
+    g = count > 0.0f ? g / count : 0.0f;
+  }
+  const float* src = p.grad_hidden32 + r * p.h;
+  const bool operand = p.hidden != nullptr;
+  const float factor = operand ? g * p.row_scale[r] : 0.0f;
+  const __bf16* hrow = static_cast<const __bf16*>(p.hidden) + r * p.h;
+  __bf16* scaled = static_cast<__bf16*>(p.scaled) + r * p.h;
+  for (int k = threadIdx.x * 8; k < p.h; k += 256 * 8) {
+    const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(src + k);
+    const f32x4_t x1 = *reinterpret_cast<const f32x4_t*>(src + k + 4);
+    v8_t y;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = from_float<__bf16>((e < 4 ? x0[e] : x1[e - 4]) * g);
+    dst[k / 8] = y;
+    if (operand) {
+      const v8_t x = *reinterpret_cast<const v8_t*>(hrow + k);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = from_float<__bf16>(to_float<__bf16>(x[e]) * factor);
+      *reinterpret_cast<v8_t*>(scaled + k) = y;
+    }
+  }
+}
+
 // One wave per row, 16 rows per workgroup.
 template <typename T>
 __global__ __launch_bounds__(256) void lce_scale_rows_kernel(ScaleRowsArgs p) {
@@ -242,8 +308,29 @@ __global__ __launch_bounds__(256) void lce_scale_rows_kernel(ScaleRowsArgs p) {
   }
 }
 
+// Sum of n floats by one workgroup of 256 threads, in an order that depends on n alone.
+__device__ __forceinline__ float block_sum(const float* x, int64_t n) {
+  __shared__ float part[4];
+  float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+  for (int64_t i = threadIdx.x; i < n; i += 1024) {
+    s0 += x[i];
+    if (i + 256 < n) s1 += x[i + 256];
+    if (i + 512 < n) s2 += x[i + 512];
+    if (i + 768 < n) s3 += x[i + 768];
+  }
+  const float s = wave_sum((s0 + s1) + (s2 + s3));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+  __syncthreads();
+  return (part[0] + part[1]) + (part[2] + part[3]);
+}
+
 __global__ __launch_bounds__(256) void lce_reduce_scaled_slabs_kernel(ReduceSlabsArgs p) {
   const int r = blockIdx.x;
+  if (p.loss != nullptr && r == (int)gridDim.x - 1) {   // behind the rows
+    const float sum = block_sum(p.losses, p.n_losses);
+    if (threadIdx.x == 0) p.loss[0] = p.mean ? sum / p.valid_count[0] : sum;
+    return;
+  }
   if (p.m_dev != nullptr) {
     const int rows = effective_block_rows(p.m, p.m_dev, p.row0);
     if (r >= rows) return;

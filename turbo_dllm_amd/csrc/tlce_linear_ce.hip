@@ -84,7 +84,9 @@ int launch_sum(const float* x, int64_t n, float* out, hipStream_t stream) {
 template <typename T>
 int launch_label_logit(const LabelLogitArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassCombine, stream);
-  lce_label_logit_kernel<T><<<(int)ceil_div(a.m, 16), 256, 0, stream>>>(a);
+  const int64_t clear =
+      a.losses != nullptr || a.row_of != nullptr ? ceil_div(a.n_out, kClearPerBlock) : 0;
+  lce_label_logit_kernel<T><<<(int)(ceil_div(a.m, 16) + 1 + clear), 256, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
@@ -94,6 +96,14 @@ int launch_fused_rows(const FusedRowsArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassCombine, stream);
   lce_fused_rows_kernel<T>
       <<<(int)ceil_div(a.m_pad, kFusedRowsPerBlock), 64 * kFusedRowsWaves, 0, stream>>>(a);
+  TLCE_LAUNCH_CHECK();
+  return 0;
+}
+
+int launch_finish_rows(const FinishRowsArgs& a, hipStream_t stream) {
+  ScopedTimer timer(kClassOther, stream);
+  const int64_t pad = a.scaled == nullptr ? 0 : a.m_dev != nullptr ? a.m_pad : a.m_pad - a.m;
+  lce_finish_rows_kernel<<<(unsigned)(a.n_out + pad), 256, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
@@ -166,7 +176,7 @@ int launch_soft_rows(const SoftRowsArgs& a, hipStream_t stream) {
 
 int launch_reduce_slabs(const ReduceSlabsArgs& a, hipStream_t stream) {
   ScopedTimer timer(kClassOther, stream);
-  lce_reduce_scaled_slabs_kernel<<<a.m, 256, 0, stream>>>(a);
+  lce_reduce_scaled_slabs_kernel<<<a.m + (a.loss != nullptr ? 1 : 0), 256, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
@@ -1011,7 +1021,8 @@ int forward_with_gradients_entry(
     int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
     float logit_multiplier,
     float* losses, float* lse, float* valid_count, float* grad_hidden_f32, float* grad_weight_f32,
-    int64_t panel_bytes, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+    int64_t panel_bytes, void* workspace, int64_t workspace_bytes, hipStream_t stream,
+    float* loss = nullptr, bool mean = false, int* row_of = nullptr) {
   TLCE_REQUIRE(valid_count != nullptr, "forward_with_gradients: valid_count is null");
   TLCE_REQUIRE(logit_multiplier > 0.0f,
                "forward_with_gradients: the logit multiplier must be positive");
@@ -1035,15 +1046,22 @@ int forward_with_gradients_entry(
     TLCE_REQUIRE(((uintptr_t)workspace & 255) == 0,
                  "forward_with_gradients: workspace must be 256-byte aligned");
   }
-  if (int rc = fill_zero(valid_count, 4, stream)) return rc;
-  if (losses != nullptr && (row_idx != nullptr || m == 0)) {
-    if (int rc = fill_zero(losses, n_out * 4, stream)) return rc;
-  }
   if (m == 0) {
+    if (int rc = fill_zero(valid_count, 4, stream)) return rc;
+    if (losses != nullptr) {
+      if (int rc = fill_zero(losses, n_out * 4, stream)) return rc;
+    }
+    if (loss != nullptr) {
+      ReduceSlabsArgs rs = {};
+      rs.loss = loss; rs.losses = losses; rs.n_losses = n_out;
+      rs.valid_count = valid_count; rs.mean = mean;
+      if (int rc = launch_reduce_slabs(rs, stream)) return rc;
+    }
     if (grad_weight_f32 != nullptr) return fill_zero(grad_weight_f32, v * h * 4, stream);
     return 0;
   }
   FusedOptions opt;
+  opt.n_out = n_out; opt.row_of = row_of; opt.loss = loss; opt.mean = mean;
   opt.logit_scale = logit_multiplier;
   opt.token_weights = token_weights;
   opt.row_count = row_count;
@@ -1138,6 +1156,103 @@ extern "C" int tlce_apply_grad_output(const float* grad_hidden_f32, const float*
                                          grad_output, valid_count, m, n_out, h, v, reduction_code,
                                          grad_hidden, grad_weight,
                                          static_cast<hipStream_t>(stream));
+}
+
+// ------------------------------------ the pair with fewer launches ----
+extern "C" int tlce_forward_with_gradients_reduced(
+    const void* hidden, const void* weight, const int64_t* labels, const int64_t* row_idx,
+    const float* token_weights, const int64_t* row_count, int64_t m, int64_t n_out, int64_t h,
+    int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
+    float logit_multiplier, int reduction_code, float* losses, float* loss, float* lse,
+    float* valid_count, float* grad_hidden_f32, float* grad_weight_f32, int* row_of,
+    int64_t panel_bytes, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
+  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype) ||
+                   (dtype == TLCE_DTYPE_F32 && f32_gradients_in_forward_supported(m, h, v)),
+               "forward_with_gradients_reduced: not taken for m=%lld h=%lld v=%lld dtype=%d",
+               (long long)m, (long long)h, (long long)v, dtype);
+  TLCE_REQUIRE(reduction_code >= TLCE_REDUCTION_NONE && reduction_code <= TLCE_REDUCTION_MEAN,
+               "forward_with_gradients_reduced: bad reduction code %d", reduction_code);
+  const bool reduced = reduction_code != TLCE_REDUCTION_NONE;
+  TLCE_REQUIRE(losses != nullptr || n_out == 0,
+               "forward_with_gradients_reduced: losses is null");
+  TLCE_REQUIRE(loss != nullptr || !reduced, "forward_with_gradients_reduced: loss is null");
+  return forward_with_gradients_entry(
+      hidden, weight, labels, row_idx, token_weights, row_count, m, n_out, h, v, dtype,
+      ignore_index, exclude_index, logit_softcap, logit_multiplier, losses, lse, valid_count,
+      grad_hidden_f32, grad_weight_f32, panel_bytes, workspace, workspace_bytes,
+      static_cast<hipStream_t>(stream), reduced ? loss : nullptr,
+      reduction_code == TLCE_REDUCTION_MEAN, row_of);
+}
+
+extern "C" int tlce_finish_gradients(const float* grad_hidden_f32, const float* grad_weight_f32,
+                                     const int* row_of, const int64_t* row_count,
+                                     const float* grad_output, const float* valid_count, int64_t m,
+                                     int64_t n_out, int64_t h, int64_t v, int reduction_code,
+                                     void* grad_hidden, void* grad_weight, const void* hidden,
+                                     int64_t panel_bytes, void* forward_workspace,
+                                     int64_t workspace_bytes, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  TLCE_REQUIRE(m >= 0 && h > 0 && v > 0 && fused_gradients_supported(h, v, TLCE_DTYPE_BF16),
+               "finish_gradients: needs h and v multiples of 64");
+  TLCE_REQUIRE(reduction_code >= TLCE_REDUCTION_NONE && reduction_code <= TLCE_REDUCTION_MEAN,
+               "finish_gradients: unknown reduction code %d", reduction_code);
+  if (m == 0) {
+    TLCE_REQUIRE(grad_hidden != nullptr || n_out == 0, "finish_gradients: grad_hidden is null");
+    if (int rc = fill_zero(grad_hidden, n_out * h * 2, stream)) return rc;
+    return grad_weight != nullptr ? fill_zero(grad_weight, v * h * 2, stream) : 0;
+  }
+  const bool waited = hidden != nullptr;   // grad_weight is to be contracted here
+  TLCE_REQUIRE(!waited || grad_weight_f32 == nullptr,
+               "finish_gradients: grad_weight either has waited or was accumulated");
+  TLCE_REQUIRE((grad_weight != nullptr) == (waited || grad_weight_f32 != nullptr),
+               "finish_gradients: grad_weight and its source go together");
+  TLCE_REQUIRE(reduction_code != TLCE_REDUCTION_NONE || grad_weight_f32 == nullptr,
+               "finish_gradients: with one upstream gradient per row (reduction none) the "
+               "grad_weight contraction has to wait for it");
+  TLCE_REQUIRE(n_out >= m, "finish_gradients: n_out=%lld < m=%lld", (long long)n_out,
+               (long long)m);
+  TLCE_REQUIRE(row_of != nullptr || n_out == m || m == 0,
+               "finish_gradients: n_out != m without row_of");
+  TLCE_REQUIRE(row_count == nullptr || row_of != nullptr,
+               "finish_gradients: a device-side row count needs row_of");
+  TLCE_REQUIRE(grad_hidden != nullptr || n_out == 0, "finish_gradients: grad_hidden is null");
+  TLCE_REQUIRE(grad_output != nullptr, "finish_gradients: grad_output is null");
+  TLCE_REQUIRE(valid_count != nullptr || reduction_code != TLCE_REDUCTION_MEAN,
+               "finish_gradients: the mean reduction needs valid_count");
+  TLCE_REQUIRE((((uintptr_t)grad_hidden | (uintptr_t)grad_weight | (uintptr_t)grad_hidden_f32 |
+                 (uintptr_t)grad_weight_f32 | (uintptr_t)hidden) & 15) == 0,
+               "finish_gradients: operands must be 16-byte aligned");
+  TLCE_REQUIRE(grad_hidden_f32 != nullptr, "finish_gradients: null pointer");
+  FinishRowsArgs fa;
+  fa.grad_hidden32 = grad_hidden_f32; fa.row_of = row_of;
+  fa.grad_output = grad_output; fa.valid_count = valid_count; fa.reduction = reduction_code;
+  fa.n_out = n_out; fa.m = (int)m; fa.m_pad = (int)round_up(m, 256); fa.h = (int)h;
+  fa.m_dev = row_count; fa.grad_hidden = grad_hidden;
+  if (!waited) {
+    if (int rc = launch_finish_rows(fa, stream)) return rc;
+    if (grad_weight == nullptr) return 0;
+    ScaleCastArgs a;
+    a.grad_output = grad_output; a.valid_count = valid_count; a.reduction = reduction_code;
+    a.h = (int)h;
+    a.in = grad_weight_f32; a.row_idx = nullptr; a.rows = v; a.out = grad_weight;
+    return launch_scale_cast<__bf16>(a, stream);
+  }
+  const FusedPlan p = make_fused_plan(m, h, v, TLCE_DTYPE_BF16, panel_bytes);
+  TLCE_REQUIRE(p.n_blocks == 1, "finish_gradients: the forward took %d blocks of rows; the "
+               "contraction can wait for one block only", p.n_blocks);
+  const FusedLayout l = fused_layout(p, m, h, TLCE_DTYPE_BF16, true);
+  TLCE_REQUIRE(forward_workspace != nullptr && workspace_bytes >= l.total,
+               "finish_gradients: this is not the forward's workspace (%lld < %lld)",
+               (long long)workspace_bytes, (long long)l.total);
+  TLCE_REQUIRE(((uintptr_t)forward_workspace & 255) == 0,
+               "finish_gradients: workspace must be 256-byte aligned");
+  char* ws = static_cast<char*>(forward_workspace);
+  fa.hidden = hidden; fa.row_scale = reinterpret_cast<const float*>(ws + l.row_scale);
+  fa.scaled = ws + l.scaled_hidden;
+  if (int rc = launch_finish_rows(fa, stream)) return rc;
+  return deferred_contraction<MfmaDirect4Engine<__bf16>>(p, l, m, h, v, row_count, grad_weight, ws,
+                                                         stream);
 }
 
 // ------------------------------------- the same pair for float32 in planes ----

@@ -69,27 +69,23 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         ctx.fused = (
             bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
             and get_gradient_mode() == "forward"
-            and (native.fused_gradients_supported(rows, weight, bias, False)
-                 or native.f32_gradients_in_forward_supported(m, rows, weight, bias, False))
+            and native.gradients_in_forward_supported(m, rows, weight, bias, False)
         )
         if ctx.fused:
             rows = rows[:m]
             ctx.postponed = bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
                 m, rows.shape[1], weight.shape[0], rows.dtype)
-            if rows.dtype == torch.float32:
-                forward, wait = native.forward_with_gradients_f32, {}
-            else:
-                forward = native.forward_with_gradients
-                wait = {"postpone_weight_grad": ctx.postponed}
-            losses, _, valid_count, grad_rows32, grad_weight32 = forward(
-                rows, weight, targets[:m], ignore_index=-100, exclude_index=exclude_index,
-                logit_softcap=logit_softcap, compute_weight_grad=bool(ctx.needs_input_grad[1]),
-                token_weights=None if token_weights is None else token_weights[:m],
-                logit_multiplier=multiplier,
-                row_idx=row_idx, n_out=n, row_count=row_count if mode == "device" else None,
-                **wait,
-            )
-            ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx,
+            losses, valid_count, grad_rows32, grad_weight32, row_of = (
+                native.forward_with_gradients_reduced(
+                    rows, weight, targets[:m], reduction="none", ignore_index=-100,
+                    exclude_index=exclude_index, logit_softcap=logit_softcap,
+                    compute_weight_grad=bool(ctx.needs_input_grad[1]),
+                    postpone_weight_grad=ctx.postponed,
+                    token_weights=None if token_weights is None else token_weights[:m],
+                    logit_multiplier=multiplier, row_idx=row_idx, n_out=n,
+                    row_count=row_count if mode == "device" else None,
+                ))
+            ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                                   row_count if mode == "device" else None,
                                   rows if ctx.postponed else None)
             ctx.panel_bytes = native.get_panel_bytes()
@@ -116,20 +112,18 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         from . import chunked_linear_ce_native as native
 
         if ctx.fused:
-            grad_rows32, grad_weight32, valid_count, row_idx, row_count, rows = ctx.saved_tensors
+            grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows = (
+                ctx.saved_tensors)
             if ctx.grad_dtype == torch.float32:
-                apply, kind = native.apply_grad_output_f32, {}
+                grad_hidden, grad_weight = native.apply_grad_output_f32(
+                    grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum",
+                    row_idx=row_idx, n_out=ctx.n_rows, vocab=ctx.vocab, row_count=row_count,
+                )
             else:
-                apply, kind = native.apply_grad_output, {"dtype": ctx.grad_dtype}
-            grad_hidden, grad_weight = apply(
-                grad_rows32, None if ctx.postponed else grad_weight32, grad_output, valid_count,
-                reduction="sum", row_idx=row_idx, n_out=ctx.n_rows, vocab=ctx.vocab,
-                row_count=row_count, **kind,
-            )
-            if ctx.postponed:
-                grad_weight = native.grad_weight_from_panel(
-                    rows, grad_weight32, grad_output, valid_count, reduction="sum",
-                    vocab=ctx.vocab, panel_bytes=ctx.panel_bytes, row_count=row_count,
+                grad_hidden, grad_weight = native.finish_gradients(
+                    grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum",
+                    n_out=ctx.n_rows, vocab=ctx.vocab, row_of=row_of, row_count=row_count,
+                    rows=rows, panel_bytes=ctx.panel_bytes,
                 )
             return (grad_hidden.reshape(ctx.hidden_shape), grad_weight, None) + (None,) * 6
         rows, weight, bias, targets, token_weights, lse, row_idx, row_count = ctx.saved_tensors
@@ -416,9 +410,8 @@ def dflash_token_loss(
             targets = gather_rows(target_token_ids.reshape(-1).contiguous(), valid_indices)
             if (device_path and get_gradient_mode() == "forward"
                     and (hidden.requires_grad or lm_head.weight.requires_grad)
-                    and (native.fused_gradients_supported(hidden, lm_head.weight, None, False)
-                         or native.f32_gradients_in_forward_supported(
-                             hidden.shape[0], hidden, lm_head.weight, None, False))):
+                    and native.gradients_in_forward_supported(
+                        hidden.shape[0], hidden, lm_head.weight, None, False)):
                 # The whole reduction is linear in the token losses,
                 #   loss = sum_r token_loss_r * w_r / ((count_{b(r)} + 1e-5) * B),
                 # and its per-row factors depend on the inputs only, so the gradients can

@@ -279,9 +279,8 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
     wants_grad = bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
     ctx.fused = (
         wants_grad and options.get_gradient_mode() == "forward"
-        and (native.fused_gradients_supported(rows, weight_vf, bias, in_place or weight_dim_first)
-             or native.f32_gradients_in_forward_supported(m, rows, weight_vf, bias,
-                                                          in_place or weight_dim_first))
+        and native.gradients_in_forward_supported(m, rows, weight_vf, bias,
+                                                  in_place or weight_dim_first)
     )
     can_wait = ctx.fused and bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
         m, rows.shape[1], weight_vf.shape[0], rows.dtype)
@@ -293,17 +292,15 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
         # all rows in one block: the grad_weight contraction waits for the upstream
         # gradient and is stored in the input dtype at once (no float32 [V, H] buffer)
         ctx.postponed = can_wait
-        if rows.dtype == torch.float32:
-            forward, wait = native.forward_with_gradients_f32, {}
-        else:
-            forward, wait = native.forward_with_gradients, {"postpone_weight_grad": ctx.postponed}
-        losses, lse, valid_count, grad_rows32, grad_weight32 = forward(
-            rows, weight_vf, targets, ignore_index=ignore_index, exclude_index=exclude_index,
-            logit_softcap=float(logit_softcap),
-            compute_weight_grad=bool(ctx.needs_input_grad[1]), row_idx=row_idx, n_out=n,
-            row_count=row_count if mode == "device" else None, **wait,
-        )
-        ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx,
+        loss, valid_count, grad_rows32, grad_weight32, row_of = (
+            native.forward_with_gradients_reduced(
+                rows, weight_vf, targets, reduction=reduction, ignore_index=ignore_index,
+                exclude_index=exclude_index, logit_softcap=float(logit_softcap),
+                compute_weight_grad=bool(ctx.needs_input_grad[1]),
+                postpone_weight_grad=ctx.postponed, row_idx=row_idx, n_out=n,
+                row_count=row_count if mode == "device" else None,
+            ))
+        ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                               row_count if mode == "device" else None,
                               rows if ctx.postponed else None)
         ctx.panel_bytes = native.get_panel_bytes()
@@ -312,11 +309,7 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
         ctx.reduction = reduction
         ctx.grad_dtype = hidden.dtype
         ctx.vocab = weight_vf.shape[0]
-        if reduction == "none":
-            return losses.reshape(labels.shape)
-        if reduction == "sum":
-            return losses.sum()
-        return losses.sum() / valid_count.squeeze(0)
+        return loss.reshape(labels.shape) if reduction == "none" else loss
     if row_count is None:
         losses, lse, valid_count = native.forward(
             rows, weight_vf, bias, targets,
@@ -354,22 +347,20 @@ def _device_backward(ctx, grad_output, frozen: bool):
     from . import chunked_linear_ce_native as native
 
     if ctx.fused:
-        grad_rows32, grad_weight32, valid_count, row_idx, row_count, rows = ctx.saved_tensors
+        grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows = (
+            ctx.saved_tensors)
         if ctx.grad_dtype == torch.float32:
-            apply, kind = native.apply_grad_output_f32, {}
+            grad_hidden, grad_weight = native.apply_grad_output_f32(
+                grad_rows32, grad_weight32, grad_output, valid_count, reduction=ctx.reduction,
+                row_idx=row_idx, n_out=ctx.n_rows, vocab=ctx.vocab, row_count=row_count,
+            )
         else:
-            apply, kind = native.apply_grad_output, {"dtype": ctx.grad_dtype}
-        grad_hidden, grad_weight = apply(
-            grad_rows32, None if ctx.postponed else grad_weight32, grad_output, valid_count,
-            reduction=ctx.reduction, row_idx=row_idx, n_out=ctx.n_rows, vocab=ctx.vocab,
-            row_count=row_count, **kind,
-        )
-        if ctx.postponed and not frozen:
-            # grad_weight32 is the forward's workspace: its panel still holds every row
-            grad_weight = native.grad_weight_from_panel(
-                rows, grad_weight32, grad_output, valid_count, reduction=ctx.reduction,
-                vocab=ctx.vocab, panel_bytes=ctx.panel_bytes, row_count=row_count,
-                row_idx=row_idx, n_out=ctx.n_rows,
+            # a postponed grad_weight: grad_weight32 is the forward's workspace, whose panel
+            # still holds every row
+            grad_hidden, grad_weight = native.finish_gradients(
+                grad_rows32, grad_weight32, grad_output, valid_count, reduction=ctx.reduction,
+                n_out=ctx.n_rows, vocab=ctx.vocab, row_of=row_of, row_count=row_count, rows=rows,
+                panel_bytes=ctx.panel_bytes,
             )
         return (grad_hidden.reshape(ctx.hidden_shape), None if frozen else grad_weight,
                 None) + (None,) * 9
