@@ -594,7 +594,11 @@ int tlce_apply_grad_output(const float* grad_hidden_f32, const float* grad_weigh
  * autograd functions take these).  The forward also reduces the losses into loss[0] (their
  * sum; over valid_count[0] for the mean; loss may be NULL for TLCE_REDUCTION_NONE; losses is
  * needed for either) and, with row_idx, leaves row_of[n_out] (int32): the row of an output
- * row, -1 where there is none.  dtype: bf16, or float32 where
+ * row, -1 where there is none.  rows_copy (bf16 [m, h], may be NULL): for rows that were
+ * not compacted; receives the hidden rows with zeros in place of those whose label is
+ * ignore_index, and is read instead of hidden, so that nothing such a row holds reaches a
+ * gradient; row_of [m], needed with it, is -1 for those rows, so that their upstream
+ * gradients do not either.  dtype: bf16, or float32 where
  * tlce_f32_gradients_in_forward_supported (workspace: the size its own entry point tells).
  *
  * tlce_finish_gradients (bf16) replaces tlce_apply_grad_output and
@@ -610,7 +614,7 @@ int tlce_forward_with_gradients_reduced(const void* hidden, const void* weight,
                                         int reduction_code, float* losses, float* loss,
                                         float* lse, float* valid_count, float* grad_hidden_f32,
                                         float* grad_weight_f32, int* row_of,
-                                        int64_t panel_bytes, void* workspace,
+                                        void* rows_copy, int64_t panel_bytes, void* workspace,
                                         int64_t workspace_bytes, void* stream);
 
 int tlce_finish_gradients(const float* grad_hidden_f32, const float* grad_weight_f32,

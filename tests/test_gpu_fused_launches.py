@@ -65,3 +65,50 @@ def test_joined_launches(gpu_device, n, kept, reduction, postpone, device_count)
             assert bool(loss.isnan()) and bool(want.isnan())
         else:
             assert abs(float(loss) - float(want)) <= n * 2.0 ** -24 * abs(float(want))
+
+
+@pytest.mark.parametrize("n,kept", [(1, 0), (1, 1), (37, 20), (256, 1), (256, 255), (256, 256)])
+@pytest.mark.parametrize("reduction,trainable", [("mean", True), ("none", True), ("none", False)])
+def test_rows_of_one_tile_are_not_compacted(gpu_device, n, kept, reduction, trainable):
+    """Against the same call on the compacted rows; whatever ignored rows and their upstream
+    gradients hold stays out of the results.  (Both calls make the same products; sums over the
+    rows meet zeros in between: bit for bit.)"""
+    from turbo_dllm_amd.tiled_linear_cross_entropy import tiled_linear_cross_entropy
+    print("[case]", n, kept, reduction, trainable, flush=True)
+    h, v = 192, 1600
+    gen = torch.Generator().manual_seed(n + kept)
+    hidden = torch.randn(n, h, generator=gen).bfloat16()
+    weight = (torch.randn(v, h, generator=gen) * 0.1).bfloat16().to(gpu_device)
+    labels = torch.randint(0, v, (n,), generator=gen)
+    gone = torch.randperm(n, generator=gen)[kept:]
+    labels[gone] = -100
+    hidden[gone] = float("nan")
+    up = torch.rand(n, generator=gen) + 0.5
+    up[gone] = float("inf")
+    keep = (labels != -100).nonzero().flatten()
+
+    def step(x, y, go, mode):
+        x = x.to(gpu_device).requires_grad_()
+        w = weight.clone().requires_grad_(trainable)
+        with torch.no_grad():
+            alone = tiled_linear_cross_entropy(x, w, y.to(gpu_device), reduction="none")
+        loss = tiled_linear_cross_entropy(x, w, y.to(gpu_device), reduction=reduction,
+                                          compaction=mode)
+        loss.backward(go.to(gpu_device) if reduction == "none" else torch.ones_like(loss))
+        return alone, loss.detach(), x.grad, w.grad
+
+    alone, loss, dx, dw = step(hidden, labels, up, "sync")
+    rows = keep.to(gpu_device)
+    assert not alone.isnan().any() and bool((alone[gone.to(gpu_device)] == 0).all())
+    assert bool((dx[gone.to(gpu_device)] == 0).all())
+    if kept == 0:
+        assert bool(loss.isnan().all()) == (reduction == "mean") and bool((dx == 0).all())
+        assert not trainable or bool((dw == 0).all())
+        return
+    _, want, want_dx, want_dw = step(hidden[keep], labels[keep], up[keep], "none")
+    assert torch.equal(loss[rows] if reduction == "none" else loss, want) or (
+        reduction == "mean" and abs(float(loss - want)) <= n * 2.0 ** -24 * float(want))
+    assert torch.equal(dx[rows], want_dx)
+    # grad_weight's sum over rows is taken 32 at a time, in other places of the groups
+    if trainable:
+        assert float((dw.double() - want_dw.double()).norm()) <= 4e-3 * float(want_dw.double().norm())

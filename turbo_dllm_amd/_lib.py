@@ -130,7 +130,7 @@ SIGNATURES = {
             c_int64, c_int64, c_int64, c_int64, c_int,          # m n_out h v dtype
             c_int64, c_int64, c_float, c_float, c_int,          # ignore exclude softcap multiplier reduction
             c_void_p, c_void_p, c_void_p, c_void_p,             # losses loss lse valid_count
-            c_void_p, c_void_p, c_void_p,                       # grad_hidden_f32 grad_weight_f32 row_of
+            c_void_p, c_void_p, c_void_p, c_void_p,             # dh32 dw32 row_of rows_copy
             c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
         ],
     ),

@@ -477,6 +477,11 @@ def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
         hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
 
 
+# Rows of one token tile: leaving some out saves no work, so they are not compacted (scan,
+# count read back, gather: a third of the time of such a step).
+ONE_TILE_ROWS = 256
+
+
 def gradients_in_forward_supported(m: int, hidden: torch.Tensor, weight: torch.Tensor,
                                    bias: torch.Tensor | None, weight_dim_first: bool) -> bool:
     """Whether ``forward_with_gradients_reduced`` takes ``m`` rows of these operands."""
@@ -500,14 +505,18 @@ def forward_with_gradients_reduced(
     row_idx: torch.Tensor | None = None,
     n_out: int | None = None,
     row_count: torch.Tensor | None = None,
+    rows_copy: torch.Tensor | None = None,
 ):
     """``forward_with_gradients`` (and ``_f32``) in fewer launches, with the loss reduced on
     the way: ``(loss, valid_count, grad_hidden_f32, grad_weight_f32 or workspace, row_of)``.
 
     ``loss`` is ``[n_out]`` for reduction "none", else one number (over the count of rows
-    with a loss for "mean").  ``row_of`` (int32 ``[n_out]``, when ``row_idx`` is given) is the
-    inverse of ``row_idx``, -1 elsewhere: ``finish_gradients`` takes it."""
-    device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count)
+    with a loss for "mean").  ``row_of`` (int32 ``[n_out]``, when ``row_idx`` or ``rows_copy``
+    is given) holds the row of an output row, -1 where that has none or one without a loss:
+    ``finish_gradients`` takes it.  ``rows_copy`` (bf16,
+    shaped like ``hidden``, for rows that were not compacted) receives the rows, zeros in place
+    of ignored ones, and is what the gradients are formed from."""
+    device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count, rows_copy)
     reduction_code = _reduction_code(reduction)
     m, h = hidden.shape
     v = weight.shape[0]
@@ -524,6 +533,9 @@ def forward_with_gradients_reduced(
             token_weights.numel() != m or token_weights.dtype != torch.float32
             or not token_weights.is_contiguous()):
         raise RuntimeError("token_weights must be contiguous float32 with one entry per row")
+    if rows_copy is not None and (rows_copy.shape != hidden.shape or not rows_copy.is_contiguous()
+                                  or rows_copy.dtype != torch.bfloat16):
+        raise RuntimeError("rows_copy must be contiguous bf16, shaped like the rows")
     n_out = m if n_out is None else int(n_out)
     lib = _lib.library()
     code = _dtype_code(hidden)
@@ -540,7 +552,7 @@ def forward_with_gradients_reduced(
         valid_count = torch.empty(1, dtype=torch.float32, device=device)
         loss = torch.empty((), dtype=torch.float32, device=device) if reduced else losses
         row_of = (torch.empty(n_out, dtype=torch.int32, device=device)
-                  if row_idx is not None else None)
+                  if row_idx is not None or rows_copy is not None else None)
         grad_hidden32 = torch.empty((m, h), dtype=torch.float32, device=device)
         grad_weight32 = (torch.empty((v, h), dtype=torch.float32, device=device)
                          if compute_weight_grad and not postpone else None)
@@ -558,7 +570,7 @@ def forward_with_gradients_reduced(
                 int(ignore_index), int(exclude_index), float(logit_softcap),
                 float(logit_multiplier), reduction_code,
                 losses.data_ptr(), loss.data_ptr(), lse.data_ptr(), valid_count.data_ptr(),
-                grad_hidden32.data_ptr(), _ptr(grad_weight32), _ptr(row_of),
+                grad_hidden32.data_ptr(), _ptr(grad_weight32), _ptr(row_of), _ptr(rows_copy),
                 panel, ws.data_ptr(), ws.numel(), _stream(device),
             ),
             "tlce_forward_with_gradients_reduced",

@@ -306,6 +306,10 @@ struct LabelLogitArgs {
   float* losses = nullptr;          // [n_out] = 0
   int* row_of = nullptr;            // [n_out] = -1
   int64_t n_out = 0;
+  // non-null (bf16): [m, h] receives the rows, zeros in place of rows without a loss (whose
+  // values, NaN among them, must reach no sum over rows)
+  void* rows_copy = nullptr;
+  int* row_map = nullptr;           // with rows_copy: [m] the row's own index, -1 without a loss
 };
 
 struct FusedRowsArgs {
@@ -411,6 +415,8 @@ struct ScaleRowsArgs {
 struct FinishRowsArgs {
   const float* grad_hidden32;  // [m, h]
   const int* row_of;           // [n_out] row of an output row, -1: none (null: the same row)
+  bool holes = false;          // row_of is the identity but for its -1s: rows were not compacted,
+                               // and the operand has zero rows in those places
   const float* grad_output;    // [1]; reduction none: [n_out]
   const float* valid_count;    // [1], read for the mean reduction only
   int reduction;
@@ -574,6 +580,7 @@ struct FusedOptions {
   int* row_of = nullptr;                  // [n_out], with row_idx: LabelLogitArgs, FusedRowsArgs
   float* loss = nullptr;                  // [1]: the losses' sum, or their mean
   bool mean = false;
+  void* rows_copy = nullptr;              // bf16 [m, h]: LabelLogitArgs
 };
 
 template <class E>
@@ -630,7 +637,15 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
   la.m = (int)m; la.h = (int)h; la.v = (int)v;
   la.ignore = ignore; la.exclude = exclude; la.softcap = softcap; la.logit_scale = opt.logit_scale;
   la.target = target; la.ref = ref; la.valid_count = valid_count; la.m_dev = m_dev;
+  la.rows_copy = opt.rows_copy;
+  la.row_map = opt.rows_copy != nullptr ? opt.row_of : nullptr;
   if (int rc = launch_label_logit<In>(la, stream)) return rc;
+  if constexpr (kPlanes == 1) {
+    if (opt.rows_copy != nullptr) {   // everything below reads the copy
+      hidden_in = static_cast<const In*>(opt.rows_copy);
+      hidden_t = hidden_in;
+    }
+  }
 
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;

@@ -64,6 +64,16 @@ __global__ __launch_bounds__(256) void lce_label_logit_kernel(LabelLogitArgs p) 
       // real column's logit serves
       p.target[r] = (here && label != p.exclude) ? z : 0.0f;
       p.ref[r] = valid ? z : INFINITY;
+      if (p.row_map != nullptr) p.row_map[r] = valid ? r : -1;
+    }
+    if (sizeof(T) == 2 && p.rows_copy != nullptr) {
+      typedef T v8_t __attribute__((ext_vector_type(8)));
+      const v8_t zero = {};
+      const T* from = static_cast<const T*>(p.hidden) + (int64_t)r * p.h;
+      T* to = static_cast<T*>(p.rows_copy) + (int64_t)r * p.h;
+      for (int k = lane * 8; k < p.h; k += 64 * 8)
+        *reinterpret_cast<v8_t*>(to + k) =
+            valid ? *reinterpret_cast<const v8_t*>(from + k) : zero;
     }
   }
 }
@@ -243,6 +253,10 @@ __global__ __launch_bounds__(256) void lce_finish_rows_kernel(FinishRowsArgs p) 
   v8_t* dst = reinterpret_cast<v8_t*>(static_cast<__bf16*>(p.grad_hidden) + o * p.h);
   if (r < 0 || r >= m) {
     for (int k = threadIdx.x; k < p.h / 8; k += 256) dst[k] = zero;
+    if (p.holes && p.scaled != nullptr) {
+      v8_t* out = reinterpret_cast<v8_t*>(static_cast<__bf16*>(p.scaled) + o * p.h);
+      for (int k = threadIdx.x; k < p.h / 8; k += 256) out[k] = zero;
+    }
     return;
   }
   float g = p.grad_output[p.reduction == TLCE_REDUCTION_NONE ? o : 0];

@@ -1022,7 +1022,7 @@ int forward_with_gradients_entry(
     float logit_multiplier,
     float* losses, float* lse, float* valid_count, float* grad_hidden_f32, float* grad_weight_f32,
     int64_t panel_bytes, void* workspace, int64_t workspace_bytes, hipStream_t stream,
-    float* loss = nullptr, bool mean = false, int* row_of = nullptr) {
+    float* loss = nullptr, bool mean = false, int* row_of = nullptr, void* rows_copy = nullptr) {
   TLCE_REQUIRE(valid_count != nullptr, "forward_with_gradients: valid_count is null");
   TLCE_REQUIRE(logit_multiplier > 0.0f,
                "forward_with_gradients: the logit multiplier must be positive");
@@ -1062,6 +1062,7 @@ int forward_with_gradients_entry(
   }
   FusedOptions opt;
   opt.n_out = n_out; opt.row_of = row_of; opt.loss = loss; opt.mean = mean;
+  opt.rows_copy = rows_copy;
   opt.logit_scale = logit_multiplier;
   opt.token_weights = token_weights;
   opt.row_count = row_count;
@@ -1165,8 +1166,14 @@ extern "C" int tlce_forward_with_gradients_reduced(
     int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
     float logit_multiplier, int reduction_code, float* losses, float* loss, float* lse,
     float* valid_count, float* grad_hidden_f32, float* grad_weight_f32, int* row_of,
-    int64_t panel_bytes, void* workspace, int64_t workspace_bytes, void* stream) {
+    void* rows_copy, int64_t panel_bytes, void* workspace, int64_t workspace_bytes,
+    void* stream) {
   if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
+  TLCE_REQUIRE(rows_copy == nullptr ||
+                   (dtype == TLCE_DTYPE_BF16 && ((uintptr_t)rows_copy & 15) == 0 &&
+                    row_of != nullptr && row_idx == nullptr),
+               "forward_with_gradients_reduced: rows_copy is bf16, 16-byte aligned, for rows "
+               "that were not compacted, and needs row_of");
   TLCE_REQUIRE(fused_gradients_supported(h, v, dtype) ||
                    (dtype == TLCE_DTYPE_F32 && f32_gradients_in_forward_supported(m, h, v)),
                "forward_with_gradients_reduced: not taken for m=%lld h=%lld v=%lld dtype=%d",
@@ -1182,7 +1189,7 @@ extern "C" int tlce_forward_with_gradients_reduced(
       ignore_index, exclude_index, logit_softcap, logit_multiplier, losses, lse, valid_count,
       grad_hidden_f32, grad_weight_f32, panel_bytes, workspace, workspace_bytes,
       static_cast<hipStream_t>(stream), reduced ? loss : nullptr,
-      reduction_code == TLCE_REDUCTION_MEAN, row_of);
+      reduction_code == TLCE_REDUCTION_MEAN, row_of, rows_copy);
 }
 
 extern "C" int tlce_finish_gradients(const float* grad_hidden_f32, const float* grad_weight_f32,
@@ -1229,6 +1236,7 @@ extern "C" int tlce_finish_gradients(const float* grad_hidden_f32, const float* 
   fa.grad_output = grad_output; fa.valid_count = valid_count; fa.reduction = reduction_code;
   fa.n_out = n_out; fa.m = (int)m; fa.m_pad = (int)round_up(m, 256); fa.h = (int)h;
   fa.m_dev = row_count; fa.grad_hidden = grad_hidden;
+  fa.holes = row_of != nullptr && n_out == m && row_count == nullptr;
   if (!waited) {
     if (int rc = launch_finish_rows(fa, stream)) return rc;
     if (grad_weight == nullptr) return 0;

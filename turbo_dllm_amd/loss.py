@@ -62,13 +62,19 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         weight = weight.contiguous()
         n = hidden_flat.shape[0]
 
+        wants_grad = bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
+        rows_copy = None
+        if (mode == "sync" and 0 < n <= native.ONE_TILE_ROWS and wants_grad
+                and get_gradient_mode() == "forward"
+                and native.fused_gradients_supported(hidden_flat, weight, bias, False)):
+            mode = "none"
+            rows_copy = torch.empty_like(hidden_flat)
         rows, targets, token_weights, row_idx, row_count, m = native.compact_loss_rows(
             hidden_flat, labels_flat, weights_flat, -100, mode)
         # gradients while the logits exist (3 contractions instead of 4), where the
         # library takes the operands and the row count is known to the host
         ctx.fused = (
-            bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
-            and get_gradient_mode() == "forward"
+            wants_grad and get_gradient_mode() == "forward"
             and native.gradients_in_forward_supported(m, rows, weight, bias, False)
         )
         if ctx.fused:
@@ -83,8 +89,10 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
                     postpone_weight_grad=ctx.postponed,
                     token_weights=None if token_weights is None else token_weights[:m],
                     logit_multiplier=multiplier, row_idx=row_idx, n_out=n,
-                    row_count=row_count if mode == "device" else None,
+                    row_count=row_count if mode == "device" else None, rows_copy=rows_copy,
                 ))
+            if rows_copy is not None:
+                rows = rows_copy
             ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                                   row_count if mode == "device" else None,
                                   rows if ctx.postponed else None)

@@ -256,6 +256,19 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
     if bias is not None:
         bias = bias.contiguous()
 
+    wants_grad = bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
+    rows_copy = None
+    if mode == "sync" and 0 < n <= native.ONE_TILE_ROWS and hidden.dtype != torch.float32:
+        if not wants_grad and not ctx.needs_input_grad[2]:
+            # (ignored rows touch nothing but their own statistics)
+            mode = "none" if hidden_flat.shape[1] % 8 == 0 else mode
+        elif (options.get_gradient_mode() == "forward"
+              and native.fused_gradients_supported(hidden_flat, weight_vf, bias,
+                                                   in_place or weight_dim_first)
+              and native.weight_grad_can_wait(n, hidden_flat.shape[1], weight_vf.shape[0],
+                                              hidden.dtype)):
+            mode = "none"
+            rows_copy = torch.empty_like(hidden_flat)
     if in_place and mode == "sync":
         # the entry points that take a device-side row count read a [V, H] head only:
         # compact with the count read back, as the reference's call sites do
@@ -276,7 +289,6 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
     # any reduction; grad_weight needs the upstream gradient inside its contraction,
     # so with per-token losses (reduction "none") it must be the postponed contraction,
     # which exists when all rows form one block.
-    wants_grad = bool(ctx.needs_input_grad[0] or ctx.needs_input_grad[1])
     ctx.fused = (
         wants_grad and options.get_gradient_mode() == "forward"
         and native.gradients_in_forward_supported(m, rows, weight_vf, bias,
@@ -298,8 +310,10 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
                 exclude_index=exclude_index, logit_softcap=float(logit_softcap),
                 compute_weight_grad=bool(ctx.needs_input_grad[1]),
                 postpone_weight_grad=ctx.postponed, row_idx=row_idx, n_out=n,
-                row_count=row_count if mode == "device" else None,
+                row_count=row_count if mode == "device" else None, rows_copy=rows_copy,
             ))
+        if rows_copy is not None:
+            rows = rows_copy
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                               row_count if mode == "device" else None,
                               rows if ctx.postponed else None)
