@@ -118,6 +118,17 @@ int tlce_gather_loss_rows(const void* hidden_src, const int64_t* labels_src,
                           int64_t ignore_index, void* hidden_dst,
                           int64_t* labels_dst, float* weights_dst, void* stream);
 
+/* tlce_gather_loss_rows for the drafter's loss: row r of the outputs belongs to sample
+ * s = row_idx[r] / segment_length, and gets the factor
+ *     weights[row_idx[r]] / ((denominators[s] + 1e-5) * n_segments)
+ * its token loss has in the mean over samples (denominators: float32 [n_segments]). */
+int tlce_gather_sample_rows(const void* hidden_src, const int64_t* labels_src,
+                            const float* weights_src, const float* denominators,
+                            int64_t segment_length, int64_t n_segments, const int64_t* row_idx,
+                            const int64_t* row_count, int64_t capacity, int64_t padded_rows,
+                            int64_t row_bytes, int64_t ignore_index, void* hidden_dst,
+                            int64_t* labels_dst, float* factors_dst, void* stream);
+
 /* Zero-fills `bytes` bytes at dst with a kernel (safe inside graph capture). */
 int tlce_fill_zero(void* dst, int64_t bytes, void* stream);
 
@@ -592,7 +603,8 @@ int tlce_apply_grad_output(const float* grad_hidden_f32, const float* grad_weigh
 
 /* tlce_forward_with_gradients and what follows it in fewer launches (the library's own
  * autograd functions take these).  The forward also reduces the losses into loss[0] (their
- * sum; over valid_count[0] for the mean; loss may be NULL for TLCE_REDUCTION_NONE; losses is
+ * sum, with token_weights their weighted sum; over valid_count[0] for the mean, which takes
+ * no token_weights; loss may be NULL for TLCE_REDUCTION_NONE; losses is
  * needed for either) and, with row_idx, leaves row_of[n_out] (int32): the row of an output
  * row, -1 where there is none.  rows_copy (bf16 [m, h], may be NULL): for rows that were
  * not compacted; receives the hidden rows with zeros in place of those whose label is

@@ -112,3 +112,29 @@ def test_rows_of_one_tile_are_not_compacted(gpu_device, n, kept, reduction, trai
     # grad_weight's sum over rows is taken 32 at a time, in other places of the groups
     if trainable:
         assert float((dw.double() - want_dw.double()).norm()) <= 4e-3 * float(want_dw.double().norm())
+
+
+@pytest.mark.parametrize("b,t,kept,dtype", [
+    (1, 5, 5, torch.bfloat16), (3, 300, 1, torch.bfloat16), (4, 257, 300, torch.bfloat16),
+    (7, 65, 64, torch.float32),
+])
+def test_gathered_sample_rows(gpu_device, b, t, kept, dtype):
+    """Rows, targets and per-row factors of a batch in one launch: bit for bit what the
+    separate operations make, and padded to 64 rows with zeros and ignored labels."""
+    gen = torch.Generator().manual_seed(b * t)
+    hidden = torch.randn(b * t, 96, generator=gen).to(dtype).to(gpu_device)
+    labels = torch.randint(0, 1000, (b, t), generator=gen).to(gpu_device)
+    weights = torch.rand(b, t, generator=gen).to(gpu_device)
+    counts = torch.rand(b, generator=gen).to(gpu_device) * 9
+    mask = torch.zeros(b * t, dtype=torch.bool)
+    mask[torch.randperm(b * t, generator=gen)[:kept]] = True
+    mask = mask.to(gpu_device)
+    row_idx, count = native.compact_mask_device(mask)
+    rows, targets, factors = native.gather_sample_rows(hidden, labels, weights, counts, t, row_idx,
+                                                       count, kept)
+    at = mask.nonzero().flatten()
+    want = weights.flatten()[at] / ((counts[at // t] + 1.0e-5) * b)
+    assert torch.equal(rows[:kept], hidden[at]) and torch.equal(targets[:kept], labels.flatten()[at])
+    assert torch.equal(factors[:kept], want)
+    assert len(rows) == -(-kept // 64) * 64
+    assert bool((rows[kept:] == 0).all()) and bool((targets[kept:] == -100).all())

@@ -45,6 +45,15 @@ SIGNATURES = {
             c_void_p, c_void_p, c_void_p, c_void_p,             # hidden_dst labels_dst weights_dst stream
         ],
     ),
+    "tlce_gather_sample_rows": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_void_p, c_void_p,             # hidden labels weights denominators
+            c_int64, c_int64, c_void_p, c_void_p,               # segment_length n_segments row_idx count
+            c_int64, c_int64, c_int64, c_int64,                 # capacity padded_rows row_bytes ignore
+            c_void_p, c_void_p, c_void_p, c_void_p,             # hidden_dst labels_dst factors_dst stream
+        ],
+    ),
     "tlce_forward_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int]),
     "tlce_forward": (
         c_int,

@@ -264,6 +264,46 @@ def gather_loss_rows(
     return rows, targets, w
 
 
+def gather_sample_rows(
+    hidden: torch.Tensor,
+    labels: torch.Tensor,
+    weights: torch.Tensor,
+    denominators: torch.Tensor,
+    segment_length: int,
+    row_idx: torch.Tensor,
+    row_count: torch.Tensor,
+    capacity: int,
+) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """``gather_loss_rows`` for the first ``capacity`` (read back, at least 1) positions in
+    ``row_idx`` of a ``[samples, segment_length]`` batch, with ``weights / ((denominators of
+    the sample + 1e-5) * samples)`` in place of the weights."""
+    device = _require_device(hidden, labels, weights, denominators, row_idx, row_count)
+    hidden = hidden.contiguous()
+    labels = labels.reshape(-1).to(torch.long).contiguous()
+    weights = weights.reshape(-1).to(torch.float32).contiguous()
+    denominators = denominators.reshape(-1).to(torch.float32).contiguous()
+    n, h = hidden.shape
+    n_segments = denominators.numel()
+    if (labels.numel() != n or weights.numel() != n or not 0 < capacity <= n
+            or row_idx.numel() < capacity or segment_length * n_segments != n):
+        raise RuntimeError("gather_sample_rows: lengths differ")
+    padded = (capacity + 63) // 64 * 64
+    with torch.cuda.device(device):
+        rows = torch.empty((padded, h), dtype=hidden.dtype, device=device)
+        targets = torch.empty(padded, dtype=torch.long, device=device)
+        factors = torch.empty(padded, dtype=torch.float32, device=device)
+        _lib.check(
+            _lib.library().tlce_gather_sample_rows(
+                hidden.data_ptr(), labels.data_ptr(), weights.data_ptr(), denominators.data_ptr(),
+                int(segment_length), n_segments, row_idx.data_ptr(), row_count.data_ptr(),
+                capacity, padded, h * hidden.element_size(), -100,
+                rows.data_ptr(), targets.data_ptr(), factors.data_ptr(), _stream(device),
+            ),
+            "tlce_gather_sample_rows",
+        )
+    return rows, targets, factors
+
+
 def compact_loss_rows(
     hidden: torch.Tensor,
     labels: torch.Tensor,
@@ -510,8 +550,8 @@ def forward_with_gradients_reduced(
     """``forward_with_gradients`` (and ``_f32``) in fewer launches, with the loss reduced on
     the way: ``(loss, valid_count, grad_hidden_f32, grad_weight_f32 or workspace, row_of)``.
 
-    ``loss`` is ``[n_out]`` for reduction "none", else one number (over the count of rows
-    with a loss for "mean").  ``row_of`` (int32 ``[n_out]``, when ``row_idx`` or ``rows_copy``
+    ``loss`` is ``[n_out]`` for reduction "none", else one number: the losses' sum (with
+    ``token_weights`` the weighted one), over the count of rows with a loss for "mean".  ``row_of`` (int32 ``[n_out]``, when ``row_idx`` or ``rows_copy``
     is given) holds the row of an output row, -1 where that has none or one without a loss:
     ``finish_gradients`` takes it.  ``rows_copy`` (bf16,
     shaped like ``hidden``, for rows that were not compacted) receives the rows, zeros in place

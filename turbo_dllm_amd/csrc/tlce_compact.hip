@@ -182,7 +182,8 @@ __global__ __launch_bounds__(256) void gather_loss_rows_kernel(
     const float* __restrict__ weights_src, const int64_t* __restrict__ row_idx,
     const int64_t* __restrict__ row_count, int64_t capacity, int64_t padded_rows,
     int vecs_per_row, int64_t ignore, V* __restrict__ hidden_dst,
-    int64_t* __restrict__ labels_dst, float* __restrict__ weights_dst) {
+    int64_t* __restrict__ labels_dst, float* __restrict__ weights_dst,
+    const float* __restrict__ denominators, int64_t segment_length, float segments) {
   // row_idx holds `capacity` entries: a count outside [0, capacity] is clamped, as
   // every consumer of the count clamps it
   const int64_t count = min(max(*row_count, (int64_t)0), capacity);
@@ -195,7 +196,12 @@ __global__ __launch_bounds__(256) void gather_loss_rows_kernel(
       for (int c = threadIdx.x; c < vecs_per_row; c += 256) dst[c] = src[c];
       if (threadIdx.x == 0) {
         labels_dst[r] = labels_src[s];
-        if (weights_dst != nullptr) weights_dst[r] = weights_src[s];
+        if (weights_dst != nullptr) {
+          const float w = weights_src[s];
+          weights_dst[r] = denominators == nullptr
+                               ? w
+                               : w / ((denominators[s / segment_length] + 1.0e-5f) * segments);
+        }
       }
     } else {
       V z;
@@ -330,13 +336,12 @@ extern "C" int tlce_scatter_rows(const void* src, const int64_t* row_idx, int64_
   return move_rows<false>(src, row_idx, m, row_bytes, dst, static_cast<hipStream_t>(stream));
 }
 
-extern "C" int tlce_gather_loss_rows(const void* hidden_src, const int64_t* labels_src,
-                                     const float* weights_src, const int64_t* row_idx,
-                                     const int64_t* row_count, int64_t capacity,
-                                     int64_t padded_rows, int64_t row_bytes,
-                                     int64_t ignore_index, void* hidden_dst,
-                                     int64_t* labels_dst, float* weights_dst, void* stream_) {
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
+static int gather_loss_rows(const void* hidden_src, const int64_t* labels_src,
+                            const float* weights_src, const int64_t* row_idx,
+                            const int64_t* row_count, int64_t capacity, int64_t padded_rows,
+                            int64_t row_bytes, int64_t ignore_index, void* hidden_dst,
+                            int64_t* labels_dst, float* weights_dst, const float* denominators,
+                            int64_t segment_length, float segments, hipStream_t stream) {
   TLCE_REQUIRE(capacity >= 0 && padded_rows >= capacity && row_bytes > 0,
                "gather_loss_rows: bad sizes");
   if (capacity == 0) return 0;
@@ -352,7 +357,7 @@ extern "C" int tlce_gather_loss_rows(const void* hidden_src, const int64_t* labe
   gather_loss_rows_kernel<V><<<grid, 256, 0, stream>>>(                                     \
       static_cast<const V*>(hidden_src), labels_src, weights_src, row_idx, row_count,       \
       capacity, padded_rows, (int)vpr, ignore_index, static_cast<V*>(hidden_dst), labels_dst,         \
-      weights_dst)
+      weights_dst, denominators, segment_length, segments)
   switch (vb) {
     case 16: TLCE_GATHER(uint4); break;
     case 8: TLCE_GATHER(uint2); break;
@@ -363,4 +368,30 @@ extern "C" int tlce_gather_loss_rows(const void* hidden_src, const int64_t* labe
 #undef TLCE_GATHER
   TLCE_LAUNCH_CHECK();
   return 0;
+}
+
+extern "C" int tlce_gather_loss_rows(const void* hidden_src, const int64_t* labels_src,
+                                     const float* weights_src, const int64_t* row_idx,
+                                     const int64_t* row_count, int64_t capacity,
+                                     int64_t padded_rows, int64_t row_bytes,
+                                     int64_t ignore_index, void* hidden_dst,
+                                     int64_t* labels_dst, float* weights_dst, void* stream) {
+  return gather_loss_rows(hidden_src, labels_src, weights_src, row_idx, row_count, capacity,
+                          padded_rows, row_bytes, ignore_index, hidden_dst, labels_dst,
+                          weights_dst, nullptr, 1, 1.0f, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tlce_gather_sample_rows(const void* hidden_src, const int64_t* labels_src,
+                                       const float* weights_src, const float* denominators,
+                                       int64_t segment_length, int64_t n_segments,
+                                       const int64_t* row_idx, const int64_t* row_count,
+                                       int64_t capacity, int64_t padded_rows, int64_t row_bytes,
+                                       int64_t ignore_index, void* hidden_dst,
+                                       int64_t* labels_dst, float* factors_dst, void* stream) {
+  TLCE_REQUIRE(weights_src && denominators && factors_dst && segment_length > 0 && n_segments > 0,
+               "gather_sample_rows: null pointer or bad sizes");
+  return gather_loss_rows(hidden_src, labels_src, weights_src, row_idx, row_count, capacity,
+                          padded_rows, row_bytes, ignore_index, hidden_dst, labels_dst,
+                          factors_dst, denominators, segment_length, (float)n_segments,
+                          static_cast<hipStream_t>(stream));
 }

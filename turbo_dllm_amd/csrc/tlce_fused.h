@@ -372,6 +372,8 @@ struct ReduceSlabsArgs {
   float* loss = nullptr;
   const float* losses = nullptr;    // [n_losses]
   int64_t n_losses = 0;
+  const float* loss_weights = nullptr;   // non-null: sum_r loss_weights[r] * losses[loss_idx[r]]
+  const int64_t* loss_idx = nullptr;     // over n_losses rows (null: r), those on the device
   const float* valid_count = nullptr;
   bool mean = false;
 };
@@ -732,6 +734,9 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     if (r0 + rows >= m) {
       rs.loss = opt.loss; rs.losses = losses; rs.n_losses = row_idx != nullptr ? opt.n_out : m;
       rs.valid_count = valid_count; rs.mean = opt.mean;
+      if (opt.loss != nullptr && opt.token_weights != nullptr) {
+        rs.loss_weights = opt.token_weights; rs.loss_idx = row_idx; rs.n_losses = m;
+      }
     }
     if (int rc = launch_reduce_slabs(rs, stream)) return rc;
 

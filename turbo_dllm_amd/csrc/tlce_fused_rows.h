@@ -322,15 +322,16 @@ __global__ __launch_bounds__(256) void lce_scale_rows_kernel(ScaleRowsArgs p) {
   }
 }
 
-// Sum of n floats by one workgroup of 256 threads, in an order that depends on n alone.
-__device__ __forceinline__ float block_sum(const float* x, int64_t n) {
+// Sum of n numbers by one workgroup of 256 threads, in an order that depends on n alone.
+template <class At>
+__device__ __forceinline__ float block_sum(int64_t n, At&& at) {
   __shared__ float part[4];
   float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
   for (int64_t i = threadIdx.x; i < n; i += 1024) {
-    s0 += x[i];
-    if (i + 256 < n) s1 += x[i + 256];
-    if (i + 512 < n) s2 += x[i + 512];
-    if (i + 768 < n) s3 += x[i + 768];
+    s0 += at(i);
+    if (i + 256 < n) s1 += at(i + 256);
+    if (i + 512 < n) s2 += at(i + 512);
+    if (i + 768 < n) s3 += at(i + 768);
   }
   const float s = wave_sum((s0 + s1) + (s2 + s3));
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
@@ -341,7 +342,14 @@ __device__ __forceinline__ float block_sum(const float* x, int64_t n) {
 __global__ __launch_bounds__(256) void lce_reduce_scaled_slabs_kernel(ReduceSlabsArgs p) {
   const int r = blockIdx.x;
   if (p.loss != nullptr && r == (int)gridDim.x - 1) {   // behind the rows
-    const float sum = block_sum(p.losses, p.n_losses);
+    float sum;
+    if (p.loss_weights == nullptr) {
+      sum = block_sum(p.n_losses, [&](int64_t i) { return p.losses[i]; });
+    } else {
+      sum = block_sum(effective_rows((int)p.n_losses, p.m_dev), [&](int64_t i) {
+        return p.loss_weights[i] * p.losses[p.loss_idx != nullptr ? p.loss_idx[i] : i];
+      });
+    }
     if (threadIdx.x == 0) p.loss[0] = p.mean ? sum / p.valid_count[0] : sum;
     return;
   }

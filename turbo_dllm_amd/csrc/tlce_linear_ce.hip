@@ -1181,6 +1181,8 @@ extern "C" int tlce_forward_with_gradients_reduced(
   TLCE_REQUIRE(reduction_code >= TLCE_REDUCTION_NONE && reduction_code <= TLCE_REDUCTION_MEAN,
                "forward_with_gradients_reduced: bad reduction code %d", reduction_code);
   const bool reduced = reduction_code != TLCE_REDUCTION_NONE;
+  TLCE_REQUIRE(token_weights == nullptr || reduction_code != TLCE_REDUCTION_MEAN,
+               "forward_with_gradients_reduced: the mean takes no token weights");
   TLCE_REQUIRE(losses != nullptr || n_out == 0,
                "forward_with_gradients_reduced: losses is null");
   TLCE_REQUIRE(loss != nullptr || !reduced, "forward_with_gradients_reduced: loss is null");

@@ -81,13 +81,12 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             rows = rows[:m]
             ctx.postponed = bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
                 m, rows.shape[1], weight.shape[0], rows.dtype)
-            losses, valid_count, grad_rows32, grad_weight32, row_of = (
+            loss, valid_count, grad_rows32, grad_weight32, row_of = (
                 native.forward_with_gradients_reduced(
-                    rows, weight, targets[:m], reduction="none", ignore_index=-100,
+                    rows, weight, targets[:m], reduction="sum", ignore_index=-100,
                     exclude_index=exclude_index, logit_softcap=logit_softcap,
                     compute_weight_grad=bool(ctx.needs_input_grad[1]),
-                    postpone_weight_grad=ctx.postponed,
-                    token_weights=None if token_weights is None else token_weights[:m],
+                    postpone_weight_grad=ctx.postponed, token_weights=token_weights[:m],
                     logit_multiplier=multiplier, row_idx=row_idx, n_out=n,
                     row_count=row_count if mode == "device" else None, rows_copy=rows_copy,
                 ))
@@ -100,8 +99,7 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             ctx.hidden_shape = hidden.shape
             ctx.n_rows, ctx.m = n, m
             ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]
-            # losses holds the unweighted token losses at their positions, zeros elsewhere
-            return torch.dot(losses, weights_flat)
+            return loss
         _, lse, _, weighted_sum = native.masked_loss_forward(
             rows, weight, bias, targets, token_weights, m=m, row_idx=row_idx,
             row_count=row_count, n_out=n, ignore_index=-100, exclude_index=exclude_index,
@@ -120,19 +118,7 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         from . import chunked_linear_ce_native as native
 
         if ctx.fused:
-            grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows = (
-                ctx.saved_tensors)
-            if ctx.grad_dtype == torch.float32:
-                grad_hidden, grad_weight = native.apply_grad_output_f32(
-                    grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum",
-                    row_idx=row_idx, n_out=ctx.n_rows, vocab=ctx.vocab, row_count=row_count,
-                )
-            else:
-                grad_hidden, grad_weight = native.finish_gradients(
-                    grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum",
-                    n_out=ctx.n_rows, vocab=ctx.vocab, row_of=row_of, row_count=row_count,
-                    rows=rows, panel_bytes=ctx.panel_bytes,
-                )
+            grad_hidden, grad_weight = _gradients_of_weighted_sum(ctx, grad_output)
             return (grad_hidden.reshape(ctx.hidden_shape), grad_weight, None) + (None,) * 6
         rows, weight, bias, targets, token_weights, lse, row_idx, row_count = ctx.saved_tensors
         with native.panel_budget(ctx.panel_bytes):
@@ -148,6 +134,60 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             grad_weight if ctx.needs_input_grad[1] else None,
             grad_bias if (bias is not None and ctx.needs_input_grad[2]) else None,
         ) + (None,) * 6
+
+
+def _gradients_of_weighted_sum(ctx, grad_output):
+    """Gradients of a weighted loss sum whose forward left them."""
+    from . import chunked_linear_ce_native as native
+
+    grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows = ctx.saved_tensors
+    if ctx.grad_dtype == torch.float32:
+        return native.apply_grad_output_f32(
+            grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum",
+            row_idx=row_idx, n_out=ctx.n_rows, vocab=ctx.vocab, row_count=row_count,
+        )
+    return native.finish_gradients(
+        grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum", n_out=ctx.n_rows,
+        vocab=ctx.vocab, row_of=row_of, row_count=row_count, rows=rows,
+        panel_bytes=ctx.panel_bytes,
+    )
+
+
+class _FusedSampleLoss(torch.autograd.Function):
+    """mean over samples of sum_r w_r * token_loss_r / (count + 1e-5), over the ``m`` rows
+    ``row_idx`` of a [samples, length] batch.  The reduction is linear in the token losses and
+    its per-row factors depend on the inputs only, so the gradients are formed while the logits
+    exist (three contractions instead of four; two instead of three with a frozen head) and the
+    upstream gradient is a scalar.  Rows, targets and factors are gathered in one launch."""
+
+    @staticmethod
+    def forward(ctx, hidden, weight, labels, weights, denominators, segment_length, row_idx,
+                row_count, m, logit_softcap):  # type: ignore[override]
+        from . import chunked_linear_ce_native as native
+
+        weight = weight.contiguous()
+        rows, targets, factors = native.gather_sample_rows(
+            hidden, labels, weights, denominators, segment_length, row_idx, row_count, m)
+        rows = rows[:m]
+        wait = bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
+            m, rows.shape[1], weight.shape[0], rows.dtype)
+        loss, valid_count, grad_rows32, grad_weight32, row_of = (
+            native.forward_with_gradients_reduced(
+                rows, weight, targets[:m], reduction="sum", ignore_index=-100, exclude_index=-1,
+                logit_softcap=logit_softcap, compute_weight_grad=bool(ctx.needs_input_grad[1]),
+                postpone_weight_grad=wait, token_weights=factors[:m], row_idx=row_idx[:m],
+                n_out=hidden.shape[0],
+            ))
+        ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx[:m], row_of, None,
+                              rows if wait else None)
+        ctx.panel_bytes = native.get_panel_bytes()   # the backward may run on another thread
+        ctx.n_rows = hidden.shape[0]
+        ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]
+        return loss
+
+    @staticmethod
+    def backward(ctx, grad_output):  # type: ignore[override]
+        return (*_gradients_of_weighted_sum(ctx, grad_output),) + (None,) * 8
 
 
 class _FusedTokenLosses(torch.autograd.Function):
@@ -386,7 +426,9 @@ def dflash_token_loss(
     if device_path:
         from . import chunked_linear_ce_native as native
 
-        valid_indices, n_valid = native.compact_mask(supervised_mask)
+        valid_indices, row_count = native.compact_mask_device(supervised_mask)
+        n_valid = int(row_count.item())
+        all_indices, valid_indices = valid_indices, valid_indices[:n_valid]
     else:
         valid_indices = torch.nonzero(supervised_mask.reshape(-1), as_tuple=False).flatten()
         n_valid = valid_indices.numel()
@@ -399,6 +441,16 @@ def dflash_token_loss(
         # numerators are all zero: only the dependence on the parameters remains
         zero = zero_loss_with_module_parameters(hidden_states, lm_head)
         numerators = zero.reshape(1).expand(batch_size) * 1.0
+    elif (device_path and loss_kind == "paper_ce" and get_gradient_mode() == "forward"
+            and torch.is_grad_enabled()
+            and (hidden_states.requires_grad or lm_head.weight.requires_grad)
+            and native.gradients_in_forward_supported(n_valid, hidden_flat, lm_head.weight, None,
+                                                      False)):
+        loss = _FusedSampleLoss.apply(
+            hidden_flat, lm_head.weight, target_token_ids, position_weights, denominators,
+            tokens_per_sample, all_indices, row_count, n_valid,
+            0.0 if logit_softcap is None else float(logit_softcap))
+        return loss * float(loss_scale)
     else:
         hidden = gather_rows(hidden_flat, valid_indices)
         weights = gather_rows(position_weights.reshape(-1).contiguous(),
@@ -416,21 +468,6 @@ def dflash_token_loss(
                                           teacher_head.weight, logit_softcap=logit_softcap)
         else:
             targets = gather_rows(target_token_ids.reshape(-1).contiguous(), valid_indices)
-            if (device_path and get_gradient_mode() == "forward"
-                    and (hidden.requires_grad or lm_head.weight.requires_grad)
-                    and native.gradients_in_forward_supported(
-                        hidden.shape[0], hidden, lm_head.weight, None, False)):
-                # The whole reduction is linear in the token losses,
-                #   loss = sum_r token_loss_r * w_r / ((count_{b(r)} + 1e-5) * B),
-                # and its per-row factors depend on the inputs only, so the gradients can
-                # be formed while the logits exist (three contractions instead of four; two
-                # instead of three with a frozen head) and the upstream gradient is a scalar.
-                sample = torch.div(valid_indices, tokens_per_sample, rounding_mode="floor")
-                row_factors = weights / ((denominators[sample] + 1.0e-5) * batch_size)
-                loss = _FusedMaskedTokenLoss.apply(
-                    hidden, lm_head.weight, None, targets, row_factors, 1.0, -1,
-                    0.0 if logit_softcap is None else float(logit_softcap), "none")
-                return loss * float(loss_scale)
             # the rows are compacted and every one of them bears loss
             token_loss = tiled_linear_cross_entropy(
                 hidden, lm_head.weight, targets, reduction="none", dtype=hidden.dtype,
