@@ -816,10 +816,33 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_ke
   eng.mainloop_set(static_cast<const T*>(p.weight), p.h, vbase, p.v,
                    static_cast<const T*>(p.hidden), p.h, tt * E::kTile, p.m, 0, p.h, acc, smem);
 
+  T* panel = static_cast<T*>(p.panel);
+  const T* panel_in = p.panel_in != nullptr ? static_cast<const T*>(p.panel_in) : panel;
+  const int64_t ld_in = p.panel_in != nullptr ? p.ld_in : p.ld;
+  const int prow = pv * E::kTile;   // first panel column of this tile
+  constexpr bool kCanStage = E::kHasKMajor && sizeof(T) == 2;
+  if constexpr (kCanStage && !kNoTeacher) {
+    // The teacher's tile goes to LDS (free after the main loop) without passing registers,
+    // all 32 pieces of a wave in flight while the maxima below are found: 16-byte chunk c of
+    // token t in slot c ^ (t & 31), each lane fetching what its slot holds.  (Through
+    // registers, four at a time, the tile waited for memory eight times in a row: the emitting
+    // draft pass over 8192 rows, H = 4096, V = 151936 took 9.2 ms, now 8.5.)
+    const char* tile_in =
+        reinterpret_cast<const char*>(panel_in + (int64_t)tt * E::kTile * ld_in + prow);
+    const unsigned lds0 = (unsigned)(uintptr_t)smem;
+#pragma unroll 4
+    for (int it = 0; it < (E::kTile * 32) / E::kThreads; ++it) {
+      const int first = (it * E::kThreads + (int)(threadIdx.x & ~63u)) >> 5;   // of two tokens
+      const int tok = first + ((threadIdx.x & 63) >> 5);
+      const int ch = (threadIdx.x & 31) ^ (tok & 31);
+      E::load_to_lds(__builtin_amdgcn_readfirstlane(lds0 + (unsigned)first * 512),
+                     (unsigned)(tok * ld_in * (int)sizeof(T) + ch * 16), tile_in);
+    }
+  }
   const float inv_cap = kSoftcap ? 1.0f / p.softcap : 0.0f;
   if (!grad) {
-    // maxima of the capped draft logits per owned column (base-2 units) for the
-    // tile's softmax partial; the capped values replace the raw accumulators
+    // maxima of the capped draft logits per owned column (base-2 units) for the tile's
+    // softmax partial; under a cap the capped values replace the raw accumulators
 #pragma unroll
     for (int i = 0; i < E::kRows; ++i) {
       const bool vok = vbase + eng.row(i) < p.v;
@@ -828,7 +851,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_ke
         float z = E::get(acc, j, i);
         if (kSoftcap) z = p.softcap * tanh_of<E::kPrecise>(z * inv_cap);
         z = vok ? z * TLCE_LOG2E : -INFINITY;
-        E::set(acc, j, i, z);
+        if (kSoftcap) E::set(acc, j, i, z);
         tile_max[j] = fmaxf(tile_max[j], z);
       }
     }
@@ -849,11 +872,6 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_ke
       }
     }
   }
-  T* panel = static_cast<T*>(p.panel);
-  const T* panel_in = p.panel_in != nullptr ? static_cast<const T*>(p.panel_in) : panel;
-  const int64_t ld_in = p.panel_in != nullptr ? p.ld_in : p.ld;
-  const int prow = pv * E::kTile;   // first panel column of this tile
-  constexpr bool kCanStage = E::kHasKMajor && sizeof(T) == 2;
 
   // one group of 4 consecutive vocabulary rows of owned column j: t[] in,
   // gradient out (kKlGrad) or the loss partial updated (kKlLoss)
@@ -874,7 +892,9 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_ke
         const float v = (exp2_of<E::kPrecise>(lp2) - t[u]) * scale[j] * dcap;
         g[u] = vok ? v : 0.0f;
       } else {
-        // z already is the capped draft logit in base-2 units (-inf past the vocabulary)
+        // the capped draft logit in base-2 units (-inf past the vocabulary): already there
+        // under a cap
+        if (!kSoftcap) z = vok ? z * TLCE_LOG2E : -INFINITY;
         // selects, not branches: the lanes of a wave disagree on tv > 0
         const float tv = kNoTeacher ? 0.0f : t[u] * tscale[j];
         const float e = exp2_of<E::kPrecise>(z - tile_max[j]);
@@ -891,18 +911,9 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_ke
   };
 
   if constexpr (kCanStage) {
-    // the tile of the panel goes through LDS in whole 512-byte token rows
-    // (16-byte chunk c of token t in slot c ^ (t & 31)), both ways
+    // the tile of the panel goes through LDS in whole 512-byte token rows, both ways
     if constexpr (!kNoTeacher) {
-#pragma unroll 4
-      for (int it = 0; it < (E::kTile * 32) / E::kThreads; ++it) {
-        const int c = it * E::kThreads + threadIdx.x;
-        const int tok = c >> 5;
-        const int ch = c & 31;
-        *reinterpret_cast<uint4*>(smem + tok * 512 + ((ch ^ (tok & 31)) * 16)) =
-            *reinterpret_cast<const uint4*>(panel_in + ((int64_t)tt * E::kTile + tok) * ld_in +
-                                            prow + ch * 8);
-      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
     }
 #pragma unroll
