@@ -28,6 +28,9 @@ LIBRARY_PATH = PACKAGE_DIR / LIBRARY_NAME
 # whose kernels take the longest to compile.
 _SPLIT_ENGINES = {"direct_bf16": "MfmaDirect4Engine<__bf16>",
                   "direct_f16": "MfmaDirect4Engine<_Float16>",
+                  # the same over hidden sizes that are no multiple of 64: logits only
+                  "column_tail_bf16": "ColumnTailEngine<__bf16>",
+                  "column_tail_f16": "ColumnTailEngine<_Float16>",
                   # float32 operands as three bf16 planes: cross entropies only
                   "split_f32": "SplitF32Engine"}
 _WHOLE_ENGINES = {"staged_bf16": "MfmaEngine<__bf16>", "staged_f16": "MfmaEngine<_Float16>",
@@ -38,14 +41,15 @@ _PARTS = {2: "grad_logits", 7: "grad_logits_cap", 8: "grad_logits_bias", 9: "gra
           10: "forward_dim_first", 11: "grad_logits_dim_first", 12: "exp_panel"}
 # the forward that leaves the gradients (part 12 and its launch sequence) exists for bf16 only
 _FUSED_ENGINES = ("direct_bf16",)
-_SPLIT_F32_PARTS = (1, 2, 3, 7, 8, 9, 12)   # its launch sequences are tlce_split_f32.hip
+_SOME_PARTS = {"split_f32": (1, 2, 3, 7, 8, 9, 12),   # its launch sequences: tlce_split_f32.hip
+               "column_tail_bf16": (1, 2, 7, 8, 9), "column_tail_f16": (1, 2, 7, 8, 9)}
 UNITS = (
     [(f"engine_{tag}_{name}", "tlce_engine_unit.hip",
       (f"-DTLCE_UNIT_ENGINE={engine}", f"-DTLCE_UNIT_PART={part}")
       + (("-DTLCE_UNIT_FUSED=1",) if tag in _FUSED_ENGINES else ())
       + (("-DTLCE_UNIT_PLANES=1",) if tag == "split_f32" else ()))
      for tag, engine in _SPLIT_ENGINES.items() for part, name in _PARTS.items()
-     if (part in _SPLIT_F32_PARTS if tag == "split_f32"
+     if (part in _SOME_PARTS[tag] if tag in _SOME_PARTS
          else part != 12 or tag in _FUSED_ENGINES)]
     + [(f"engine_{tag}", "tlce_engine_unit.hip",
         (f"-DTLCE_UNIT_ENGINE={engine}", "-DTLCE_UNIT_PART=0"))

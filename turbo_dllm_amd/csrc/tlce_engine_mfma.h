@@ -390,6 +390,8 @@ struct Operand {
   int rows;       // valid rows / columns of the matrix; accesses beyond are clamped
   // K-major: K rows from k_full on (a multiple of 64; the matrix has fewer than 64 more)
   // are read from `tail`, a [64, ld] copy of them with zero rows after the last.
+  // K-contiguous first operand of the engine that has column tails: the columns after the
+  // last whole 64 are read from `tail`, a [rows, 64] copy with zero columns after the last.
   const T* tail = nullptr;
   int k_full = 0x7fffffff;
 };
@@ -417,7 +419,7 @@ template <> struct DirectMfma<_Float16> {
   }
 };
 
-template <typename T_, int kPlanes_>
+template <typename T_, int kPlanes_, bool kColumnTail = false>
 struct DirectToLdsEngine : DirectTileLayout<T_> {
   using Base = DirectTileLayout<T_>;
   using T = T_;
@@ -428,6 +430,7 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
   static constexpr unsigned kPassPlaneA = kPlanes == 1 ? 0u : 0x001102u;
   static constexpr unsigned kPassPlaneB = kPlanes == 1 ? 0u : 0x010120u;
   static_assert(kPlanes == 1 || kPlanes == 3, "matrices as they are, or float32 in three planes");
+  static_assert(!kColumnTail || kPlanes == 1, "planes are padded to whole K tiles");
   static constexpr bool kPrecise = kPlanes > 1;              // float32 in, float32 epilogues
   using Op = DirectMfma<T_>;
   using V8 = typename MfmaOp<T_>::V8;
@@ -494,12 +497,14 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
     const char* next;       // base address of the next K tile to request
     int64_t step;           // bytes between consecutive K tiles
     const char* last;       // K-major: base address of the last K tile (the operand's tail
-                            // when the K range ends inside a 64-row slab)
+                            // when the K range ends inside a 64-row slab); column tails:
+                            // the tail's first row of this tile
+    unsigned last_off[kColumnTail ? kLoads : 1];   // column tails: `off` of the last K tile
     const char* begin;      // base address of the first K tile in plane 0
     int64_t plane;          // bytes from one plane to the next
   };
 
-  template <bool kKMajor>
+  template <bool kKMajor, bool kTail = false>
   __device__ __forceinline__ Loader make_loader(const Operand<T>& x, int k_begin, int nk,
                                                 unsigned lds_op) const {
     Loader ld;
@@ -516,6 +521,15 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
       ld.next = reinterpret_cast<const char*>(x.ptr + (int64_t)x.row0 * x.ld * kPlanes + k_begin);
       ld.step = kBK * 2;
       ld.last = nullptr;
+      if constexpr (kTail) {
+        ld.last = reinterpret_cast<const char*>(x.tail + (int64_t)x.row0 * kBK);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+          const int r = wave * 64 + j * 8 + (lane >> 3);
+          const int chunk = (lane & 7) ^ ((r >> 1) & 7);
+          ld.last_off[j] = (unsigned)((min(x.row0 + r, x.rows - 1) - x.row0) * kBK * 2 + chunk * 16);
+        }
+      }
     } else {
       // this wave fills K rows [16w, 16w+16) of the slab, two rows per instruction
       const int last_chunk = x.rows / 8 - 1 - x.row0 / 8;   // relative to the tile
@@ -589,7 +603,9 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // acc = A-tile * B-tile^T over K in [k_begin, k_end), a multiple of 64 wide and not empty
+  // acc = A-tile * B-tile^T over K in [k_begin, k_end), not empty and a multiple of 64 wide
+  // (with column tails, of K-contiguous operands: 65 wide at least and no such multiple, and
+  // the rows of B hold zeros up to the next one)
   // (the first 64 MFMAs take a zero constant as their addend, which saves zeroing 256
   // accumulator registers per tile).
   // K-contiguous operand: tile rows row0 .. row0+256 of x (rows clamped to
@@ -601,9 +617,11 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
                                               int k_begin, int k_end, Acc& acc,
                                               char* smem) const {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
-    const int pass_tiles = (k_end - k_begin) / kBK;   // K tiles of one pass
+    static_assert(!kColumnTail || (!kAKMajor && !kBKMajor), "column tails: K-contiguous operands");
+    // K tiles of one pass
+    const int pass_tiles = (k_end - k_begin) / kBK + (kColumnTail ? 1 : 0);
     const int nk = pass_tiles * kPasses;
-    Loader la = make_loader<kAKMajor>(A, k_begin, nk, lds0);
+    Loader la = make_loader<kAKMajor, kColumnTail>(A, k_begin, nk, lds0);
     Loader lb = make_loader<kBKMajor>(B, k_begin, nk, lds0 + kOperandBytes);
     // The place of a K tile among the passes, advanced one tile at a time.
     struct Place { int pass, tile; };
@@ -626,7 +644,13 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
     }
     // the loaders move on to K tile `k`, the next one
     auto advance = [&](int k) {
-      if constexpr (kPlanes == 1) {
+      if constexpr (kColumnTail) {
+        const bool at_last = k == nk - 1;
+        la.next = at_last ? la.last : la.next + la.step;
+        lb.next += lb.step;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) la.off[j] = at_last ? la.last_off[j] : la.off[j];
+      } else if constexpr (kPlanes == 1) {
         la.next = kAKMajor && k == nk - 1 ? la.last : la.next + la.step;
         lb.next = kBKMajor && k == nk - 1 ? lb.last : lb.next + lb.step;
       } else {
@@ -670,7 +694,8 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
     const unsigned touch_lds =
         __builtin_amdgcn_readfirstlane(lds0 + 2 * kStageBytes + (unsigned)wave * 256);
     // (a tail is small and in L2 already; the tile before it is touched again)
-    const bool ragged = touch_b ? kBKMajor && k_end > B.k_full : kAKMajor && k_end > A.k_full;
+    const bool ragged = touch_b ? kBKMajor && k_end > B.k_full
+                                : kColumnTail || (kAKMajor && k_end > A.k_full);
     const int touch_last = __builtin_amdgcn_readfirstlane(nk - 1 - (ragged ? 1 : 0));
     const unsigned touch_planes =
         __builtin_amdgcn_readfirstlane(touch_b ? kPassPlaneB : kPassPlaneA);
@@ -796,6 +821,18 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
 // 16-bit matrices as they are stored.
 template <typename T_>
 struct MfmaDirect4Engine : DirectToLdsEngine<T_, 1> {};
+
+// The same for logits over hidden sizes that are no multiple of 64 (a multiple of 8, above 64):
+// the last K tile of the first operand, the head, comes from a zero-padded copy of its last
+// columns, and the second, the rows, is a copy padded with zeros to whole K tiles.  An engine
+// of its own: the choice of the last tile's addresses costs the other up to 1.5 %.
+template <typename T_>
+struct ColumnTailEngine : DirectToLdsEngine<T_, 1, true> {};
+template <class E> constexpr bool kReadsColumnTails = false;
+template <typename T> constexpr bool kReadsColumnTails<ColumnTailEngine<T>> = true;
+// The engine that does so for engine E.
+template <class E> struct ColumnTailOf { using type = E; };
+template <typename T> struct ColumnTailOf<MfmaDirect4Engine<T>> { using type = ColumnTailEngine<T>; };
 
 // Float32 matrices in three bf16 planes (tlce_split_f32.h): an operand's row holds its
 // planes one after the other, so `ld` is the distance of two planes and a third of the

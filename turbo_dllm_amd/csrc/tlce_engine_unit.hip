@@ -92,6 +92,12 @@ TLCE_LAUNCHERS_EXP_GRADIENTS(template, UnitEngine)
 #endif
 #endif
 #if TLCE_UNIT_PART == 6
+using UnitTailEngine = ColumnTailOf<UnitEngine>::type;   // built in units of its own
+TLCE_LAUNCHERS_FORWARD(extern template, UnitTailEngine)
+TLCE_LAUNCHERS_GRAD_LOGITS(extern template, UnitTailEngine, false, false)
+TLCE_LAUNCHERS_GRAD_LOGITS(extern template, UnitTailEngine, true, false)
+TLCE_LAUNCHERS_GRAD_LOGITS(extern template, UnitTailEngine, false, true)
+TLCE_LAUNCHERS_GRAD_LOGITS(extern template, UnitTailEngine, true, true)
 TLCE_ENGINE_ENTRY_POINTS(template, UnitEngine)
 #ifdef TLCE_UNIT_FUSED
 TLCE_FUSED_ENTRY_POINTS(template, UnitEngine)

@@ -81,6 +81,8 @@ struct Plan {
   int64_t v;    // vocabulary rows
   int engine;   // 3 = float32 MFMA, 2 = direct-to-LDS MFMA, 1 = register-staged MFMA, 0 = generic
   bool kmajor;  // gradient contractions read K-major operands in place
+  int64_t column_tail;  // not 0: the logits contractions read copies of the operands
+                        // (launch_column_tails), hidden's with rows of this length
   int tile;
   int bk;
   int64_t mp, vp;
@@ -99,15 +101,29 @@ inline int engine_class(int64_t h, int dtype) {
 }
 
 inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_grad,
-               int64_t panel_bytes, int max_engine = 3) {
+               int64_t panel_bytes, int max_engine = 3, bool column_tail = false) {
   Plan p;
   p.v = v;
+  p.column_tail = 0;
   // 16-bit inputs: 2: four-wave direct-to-LDS MFMA (h % 64 == 0), 1: register-staged MFMA
   // (h % 8 == 0); float32: 3: float32 MFMA (h % 4 == 0); 0: generic float32-FMA tiles
   p.engine = std::min(engine_class(h, dtype), max_engine);
   // a float32 vocabulary that one generic tile holds would leave most of a 128x128 tile
   // and of its matrix instructions empty (both take about 10 us there)
   if (p.engine == 3 && v < 64) p.engine = 0;
+  // Hidden sizes that are multiples of 8 but not of 64: the direct engine takes the last K tile
+  // of the head from a zero-padded copy of its last columns and hidden from a padded copy
+  // (callers with scratch for them).  Forward / both directions in us, staged -> direct:
+  //   4096 rows, H = 2040, V = 65536   1203 -> 1001 / 5100 -> 3688  (H = 2048: 820 / 2550,
+  //                                    from three contractions and aligned rows of the head)
+  //   300 rows, H = 1000, V = 16384    89 -> 83 / 291 -> 253
+  //   70 rows, H = 5000, V = 32000     242 -> 188 / 995 -> 636
+  // Short rows are mostly tail and the copies' launch is part of small calls: forward at
+  // H = 72, 4096 rows, V = 32000 108 -> 117; H = 136, 2048 rows, V = 1024 72 -> 77.
+  if (column_tail && p.engine == 1 && h >= 256 && m > 64 && m * v >= (1ll << 21)) {
+    p.engine = 2;
+    p.column_tail = round_up(h, 64);
+  }
   // The direct and the float32 engine read weight, hidden and the logit-gradient panel
   // in their stored form for the gradient contractions (no transposed copies).  The
   // direct one takes whole 64-row K slabs: of a last, incomplete slab of weight or
@@ -174,8 +190,14 @@ inline bool dim_first_in_place(int64_t h, int64_t v, int dtype) {
   return engine_class(h, dtype) == 2 && (v % 64) == 0;
 }
 
+// Bytes of what launch_column_tails writes: the copy of weight's last columns [vp, 64], then
+// that of hidden [mp, column_tail].
+inline int64_t column_tail_bytes(const Plan& p) {
+  return p.column_tail != 0 ? (p.vp * 64 + p.mp * p.column_tail) * 2 : 0;
+}
+
 struct ForwardLayout {
-  int64_t part_max, part_sum, weighted, total;
+  int64_t part_max, part_sum, weighted, tails, total;
 };
 // dynamic_rows: the partials must fit whatever plan the kernels derive from a
 // device-side row count <= m (at most kTargetWorkgroups tiles, or one split of
@@ -189,12 +211,13 @@ inline ForwardLayout forward_layout(const Plan& p, bool dynamic_rows = false,
   l.part_max = 0;
   l.part_sum = part;
   l.weighted = 2 * part;
-  l.total = 2 * part + (weighted ? align256(p.mp * 4) : 0);
+  l.tails = 2 * part + (weighted ? align256(p.mp * 4) : 0);
+  l.total = l.tails + column_tail_bytes(p);
   return l;
 }
 
 struct BackwardLayout {
-  int64_t scale, acc32, wt, ht, g, gt, total;
+  int64_t scale, acc32, wt, ht, g, gt, tails, total;
 };
 // Bytes of the zero-padded copy of a 16-bit [rows, h] matrix's last K slab that a
 // direct-engine contraction over its rows needs (none: all slabs are whole).
@@ -216,6 +239,7 @@ inline BackwardLayout backward_layout(const Plan& p, int64_t m, int64_t h, int d
   if (weight_grad) off += direct ? k_tail_bytes(m, h) : p.kmajor ? 0 : align256(h * p.mp * es);
   l.g = off;     off += align256(p.mp * p.vc * es);
   l.gt = off;    off += (weight_grad && !p.kmajor) ? align256(p.vc * p.mp * es) : 0;
+  l.tails = off; off += column_tail_bytes(p);
   l.total = off;
   return l;
 }
@@ -372,6 +396,11 @@ int launch_transpose(const T* in, int64_t ld_in, int64_t rows, int64_t cols, T* 
 // beside the C ABI.
 int fill_zero(void* dst, int64_t bytes, hipStream_t stream);
 int launch_k_tail(const void* matrix, int64_t rows, int64_t h, void* tail, hipStream_t stream);
+// Copies of 16-bit weight [v, h] and hidden [m, h] (h a multiple of 8 but not of 64):
+// weight_tail [v, 64] holds the columns after the last whole 64 and then zeros, hidden_copy
+// [m, h rounded up to 64] the rows followed by zeros.
+int launch_column_tails(const void* weight, int64_t v, const void* hidden, int64_t m, int64_t h,
+                        void* weight_tail, void* hidden_copy, hipStream_t stream);
 int launch_token_scale(const ScaleArgs& sa, hipStream_t stream);
 int launch_kl_finish(float* losses, const float* loss_part, const float* tsum_part, int n_tiles,
                      int64_t part_ld, const float* lse, int64_t m, hipStream_t stream);
@@ -422,6 +451,12 @@ int forward_impl(const Plan& p, const void* hidden, const void* weight, const fl
   const ForwardLayout l = forward_layout(p, dynamic, opt.weighted_sum != nullptr);
   ForwardArgs fa;
   fa.hidden = hidden; fa.weight = weight; fa.bias = bias;
+  if (p.column_tail != 0) {
+    char* hidden_copy = ws + l.tails + p.vp * 64 * 2;
+    if (int rc = launch_column_tails(weight, v, hidden, m, h, ws + l.tails, hidden_copy, stream))
+      return rc;
+    fa.weight_tail = ws + l.tails; fa.hidden = hidden_copy;
+  }
   fa.m = (int)m; fa.h = (int)h; fa.v = (int)v;
   fa.exclude = exclude - shard.vocab_start; fa.softcap = softcap;
   fa.logit_scale = opt.logit_scale; fa.m_dev = opt.row_count;
@@ -432,7 +467,10 @@ int forward_impl(const Plan& p, const void* hidden, const void* weight, const fl
   if (opt.weight_dim_first) {
     if (int rc = launch_forward_dim_first<E>(p, fa, stream)) return rc;
   } else {
-    if (int rc = launch_forward<E>(p, fa, stream)) return rc;
+    using Tail = typename ColumnTailOf<E>::type;
+    if (int rc = p.column_tail != 0 ? launch_forward<Tail>(p, fa, stream)
+                                    : launch_forward<E>(p, fa, stream))
+      return rc;
   }
 
   CombineArgs ca;
@@ -622,9 +660,16 @@ int backward_impl(const Plan& p, const void* hidden, const void* weight, const f
   if (grad_bias != nullptr) {
     if (int rc = fill_zero(grad_bias, v * 4, stream)) return rc;
   }
+  char* hidden_copy = ws + l.tails + p.vp * 64 * 2;   // p.column_tail
+  if (p.column_tail != 0) {
+    if (int rc = launch_column_tails(weight, v, hidden, m, h, ws + l.tails, hidden_copy, stream))
+      return rc;
+  }
   auto produce = [&](int64_t v0, int64_t width, void* g, void* gt) -> int {
     GradLogitsArgs ga;
-    ga.hidden = hidden; ga.weight = weight; ga.bias = bias; ga.labels = labels;
+    ga.hidden = p.column_tail != 0 ? hidden_copy : hidden;
+    ga.weight_tail = p.column_tail != 0 ? ws + l.tails : nullptr;
+    ga.weight = weight; ga.bias = bias; ga.labels = labels;
     ga.lse = lse; ga.scale = scale;
     ga.m = (int)m; ga.h = (int)h; ga.v = (int)v;
     ga.ignore = ignore; ga.exclude = exclude - vocab_start; ga.softcap = softcap;
@@ -637,7 +682,9 @@ int backward_impl(const Plan& p, const void* hidden, const void* weight, const f
     ga.g = g; ga.ldg = p.vc; ga.gt = gt; ga.ldgt = p.mp;
     ga.grad_bias = (bias != nullptr) ? grad_bias : nullptr;
     if (opt.weight_dim_first) return launch_grad_logits_dim_first<E>(ga, stream);
-    return launch_grad_logits<E>(ga, stream);
+    using Tail = typename ColumnTailOf<E>::type;
+    return p.column_tail != 0 ? launch_grad_logits<Tail>(ga, stream)
+                              : launch_grad_logits<E>(ga, stream);
   };
   return panel_contractions<E>(p, l, hidden, weight, row_idx, m, n_out, h, v, dtype, grad_hidden,
                                grad_weight, ws, stream, produce, nullptr, opt.row_count,

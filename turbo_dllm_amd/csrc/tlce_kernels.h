@@ -27,6 +27,7 @@ struct ForwardArgs {
   const void* weight;   // [v, h], or [h, v] for the kernels instantiated with kWDimFirst
   const float* bias;    // [v] or null
   int m, h, v;
+  const void* weight_tail = nullptr;   // column tails (logits_mainloop)
   int64_t exclude;
   float softcap;
   float logit_scale = 1.0f;   // logits = cap(logit_scale * hidden . weight^T + bias); > 0
@@ -39,6 +40,23 @@ struct ForwardArgs {
   // exactly as the host plan would have set them for it.
   const int64_t* m_dev = nullptr;
 };
+
+// The contraction of a logits^T tile.  Column tails: `weight_tail` and `hidden` are the
+// copies that launch_column_tails makes.
+template <class E, class Args>
+__device__ __forceinline__ void logits_mainloop(const E& eng, const Args& p, int vbase, int row0,
+                                                typename E::Acc& acc, char* smem) {
+  using T = typename E::T;
+  const T* weight = static_cast<const T*>(p.weight);
+  const T* hidden = static_cast<const T*>(p.hidden);
+  if constexpr (kReadsColumnTails<E>) {
+    const Operand<T> a = {weight, p.h, vbase, p.v, static_cast<const T*>(p.weight_tail)};
+    const Operand<T> b = {hidden, (p.h + 63) / 64 * 64, row0, p.m};
+    eng.template mainloop_ex<false, false>(a, b, 0, p.h, acc, smem);
+  } else {
+    eng.mainloop_set(weight, p.h, vbase, p.v, hidden, p.h, row0, p.m, 0, p.h, acc, smem);
+  }
+}
 
 // kWDimFirst (engines with K-major operands only): the head is stored [h, v]
 // (fused_linear_ce.cpp:104 `weight_dim_first`) and read in place as a K-major
@@ -88,8 +106,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_forward_sta
       const Operand<T> b = {hidden, p.h, tt * E::kTile, p.m};
       eng.template mainloop_ex<true, false>(a, b, 0, p.h, acc, smem);
     } else {
-      eng.mainloop_set(weight, p.h, vt * E::kTile, p.v, hidden, p.h, tt * E::kTile, p.m, 0, p.h,
-                       acc, smem);
+      logits_mainloop(eng, p, vt * E::kTile, tt * E::kTile, acc, smem);
     }
     const int vbase = vt * E::kTile;
     // Only the last vocabulary tile (rows past v) and the tile that holds the
@@ -391,6 +408,7 @@ struct GradLogitsArgs {
   const float* lse;
   const float* scale;
   int m, h, v;
+  const void* weight_tail = nullptr;   // column tails (logits_mainloop)
   int64_t ignore, exclude;
   float softcap;
   int64_t label_offset;  // global id of weight row 0 (vocabulary shards), else 0
@@ -492,7 +510,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
     const Operand<T> b = {hidden, p.h, tt * E::kTile, p.m};
     eng.template mainloop_ex<true, false>(a, b, 0, p.h, acc, smem);
   } else {
-    eng.mainloop_set(weight, p.h, vbase, p.v, hidden, p.h, tt * E::kTile, p.m, 0, p.h, acc, smem);
+    logits_mainloop(eng, p, vbase, tt * E::kTile, acc, smem);
   }
 
   // the bias add applies the logit multiplier itself (z = multiplier * dot + bias)

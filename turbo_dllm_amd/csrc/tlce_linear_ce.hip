@@ -51,6 +51,17 @@ int launch_k_tail(const void* matrix, int64_t rows, int64_t h, void* tail, hipSt
   return 0;
 }
 
+int launch_column_tails(const void* weight, int64_t v, const void* hidden, int64_t m, int64_t h,
+                        void* weight_tail, void* hidden_copy, hipStream_t stream) {
+  ScopedTimer timer(kClassTranspose, stream);
+  const int64_t pieces = v * 8 + m * (round_up(h, 64) / 8);
+  lce_column_tail_kernel<<<(unsigned)ceil_div(pieces, 256), 256, 0, stream>>>(
+      static_cast<const uint4*>(weight), v, static_cast<const uint4*>(hidden), m, (int)(h / 8),
+      static_cast<uint4*>(weight_tail), static_cast<uint4*>(hidden_copy));
+  TLCE_LAUNCH_CHECK();
+  return 0;
+}
+
 int launch_token_scale(const ScaleArgs& sa, hipStream_t stream) {
   ScopedTimer timer(kClassOther, stream);
   lce_token_scale_kernel<<<(int)ceil_div(sa.mp, 256), 256, 0, stream>>>(sa);
@@ -247,7 +258,7 @@ extern "C" int tlce_query_plan(int64_t m, int64_t h, int64_t v, int dtype, int c
                                int64_t* forward_vocab_splits, int64_t* panel_columns,
                                int64_t* n_panels, int64_t* grad_hidden_k_splits) {
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0, "query_plan: bad shape");
-  const Plan p = make_plan(m, h, v, dtype, compute_weight_grad != 0, panel_bytes);
+  const Plan p = make_plan(m, h, v, dtype, compute_weight_grad != 0, panel_bytes, 3, true);
   if (engine) *engine = p.engine;
   if (tile) *tile = p.tile;
   if (forward_vocab_splits) *forward_vocab_splits = p.nsplit;
@@ -260,17 +271,18 @@ extern "C" int tlce_query_plan(int64_t m, int64_t h, int64_t v, int dtype, int c
 namespace {
 
 int64_t forward_workspace(int64_t m, int64_t h, int64_t v, int dtype, bool dynamic_rows,
-                          bool weighted, bool no_split = false) {
-  if (!no_split && split_forward_taken(m, h, v, dtype, dynamic_rows))
+                          bool weighted, bool no_copies = false) {
+  if (!no_copies && split_forward_taken(m, h, v, dtype, dynamic_rows))
     return split_forward_layout(make_split_plan(m, h, v, 0), dynamic_rows, weighted).total;
-  return forward_layout(make_plan(m, h, v, dtype, false, 0), dynamic_rows, weighted).total;
+  return forward_layout(make_plan(m, h, v, dtype, false, 0, 3, !no_copies), dynamic_rows, weighted)
+      .total;
 }
 
 int64_t backward_workspace(int64_t m, int64_t h, int64_t v, int dtype, bool weight_grad,
                            int64_t panel_bytes) {
   if (split_f32_supported(m, h, v, dtype))
     return split_backward_layout(make_split_plan(m, h, v, panel_bytes), h).total;
-  const Plan p = make_plan(m, h, v, dtype, weight_grad, panel_bytes);
+  const Plan p = make_plan(m, h, v, dtype, weight_grad, panel_bytes, 3, true);
   return backward_layout(p, m, h, dtype, weight_grad).total;
 }
 
@@ -283,14 +295,14 @@ extern "C" int64_t tlce_forward_workspace_bytes(int64_t m, int64_t h, int64_t v,
 
 namespace {
 
-// no_split: float32 stays on the float32 engine (callers without room for planes)
+// no_copies: for callers without room for copies of operands (float32 planes, last columns)
 int forward_entry(const void* hidden, const void* weight, const float* bias,
                   const int64_t* labels, const int64_t* row_idx, int64_t m, int64_t n_out,
                   int64_t h, int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index,
                   float logit_softcap, float* losses, float* lse, float* valid_count,
                   const ShardStats& shard, void* workspace, int64_t workspace_bytes,
                   hipStream_t stream, const RowOptions& opt = RowOptions{},
-                  bool no_split = false) {
+                  bool no_copies = false) {
   const bool local = shard.local_max != nullptr;
   const bool fused = opt.weighted_sum != nullptr;   // the masked-token loss entry point
   if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
@@ -315,15 +327,15 @@ int forward_entry(const void* hidden, const void* weight, const float* bias,
   TLCE_REQUIRE(labels && workspace && (local || ((losses || fused) && lse)),
                "forward: null pointer");
   const bool dynamic = opt.row_count != nullptr;
-  const int64_t need = forward_workspace(m, h, v, dtype, dynamic, fused, no_split);
+  const int64_t need = forward_workspace(m, h, v, dtype, dynamic, fused, no_copies);
   TLCE_REQUIRE(workspace_bytes >= need, "forward: workspace too small (%lld < %lld)",
                (long long)workspace_bytes, (long long)need);
   TLCE_REQUIRE(((uintptr_t)workspace & 255) == 0, "forward: workspace must be 256-byte aligned");
-  if (!no_split && split_forward_taken(m, h, v, dtype, dynamic))
+  if (!no_copies && split_forward_taken(m, h, v, dtype, dynamic))
     return split_forward(make_split_plan(m, h, v, 0), hidden, weight, bias, labels, row_idx, m, h,
                          v, ignore_index, exclude_index, logit_softcap, losses, lse, valid_count,
                          shard, static_cast<char*>(workspace), stream, opt);
-  const Plan p = make_plan(m, h, v, dtype, false, 0);
+  const Plan p = make_plan(m, h, v, dtype, false, 0, 3, !no_copies);
   TLCE_DISPATCH(p, dtype,
                 forward_impl<E>(p, hidden, weight, bias, labels, row_idx, m, h, v, ignore_index,
                                 exclude_index, logit_softcap, losses, lse, valid_count, shard,
@@ -491,7 +503,7 @@ int backward_entry(const void* hidden, const void* weight, const float* bias,
                           ignore_index, exclude_index, logit_softcap, vocab_start, grad_hidden,
                           grad_weight, (bias != nullptr) ? grad_bias : nullptr,
                           static_cast<char*>(workspace), stream, opt);
-  const Plan p = make_plan(m, h, v, dtype, grad_weight != nullptr, panel_bytes);
+  const Plan p = make_plan(m, h, v, dtype, grad_weight != nullptr, panel_bytes, 3, true);
   TLCE_DISPATCH(p, dtype,
                 backward_impl<E>(p, hidden, weight, bias, labels, row_idx, lse, valid_count,
                                  grad_output, m, n_out, h, v, dtype, reduction_code, ignore_index,
@@ -606,8 +618,8 @@ extern "C" int tlce_masked_loss_backward(const void* hidden, const void* weight,
 extern "C" int64_t tlce_soft_embedding_workspace_bytes(int64_t m, int64_t h, int64_t v, int dtype,
                                                        int64_t panel_bytes) {
   if (m < 0 || h <= 0 || v <= 0) return -1;
-  const Plan fp = make_plan(m, h, v, dtype, false, 0);
-  const Plan bp = make_plan(m, h, v, dtype, false, panel_bytes);
+  const Plan fp = make_plan(m, h, v, dtype, false, 0, 3, true);
+  const Plan bp = make_plan(m, h, v, dtype, false, panel_bytes, 3, true);
   int64_t need = soft_embedding_layout(fp, bp, m, h, dtype).total;
   // the soft cap is not known here: enough for either sequence
   if (fused_gradients_supported(h, v, dtype)) {
@@ -645,8 +657,8 @@ extern "C" int tlce_soft_embedding(const void* hidden, const void* weight, int64
         p, hidden, weight, m, h, v, dtype, logit_softcap, embedding_scale, out,
         static_cast<char*>(workspace), stream);
   }
-  const Plan fp = make_plan(m, h, v, dtype, false, 0);
-  const Plan bp = make_plan(m, h, v, dtype, false, panel_bytes);
+  const Plan fp = make_plan(m, h, v, dtype, false, 0, 3, true);
+  const Plan bp = make_plan(m, h, v, dtype, false, panel_bytes, 3, true);
   const SoftEmbeddingLayout l = soft_embedding_layout(fp, bp, m, h, dtype);
   TLCE_REQUIRE(workspace_bytes >= l.total, "soft_embedding: workspace too small (%lld < %lld)",
                (long long)workspace_bytes, (long long)l.total);

@@ -394,6 +394,27 @@ __global__ __launch_bounds__(kTopkScanThreads, 6) void lce_topk_scan_kernel(Topk
   }
 }
 
+// launch_column_tails; the matrices are [*, 8 h8] elements, eight of them per thread.
+__global__ __launch_bounds__(256) void lce_column_tail_kernel(const uint4* __restrict__ weight,
+                                                              int64_t v,
+                                                              const uint4* __restrict__ hidden,
+                                                              int64_t m, int h8,
+                                                              uint4* __restrict__ weight_tail,
+                                                              uint4* __restrict__ hidden_copy) {
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+  if (i < v * 8) {
+    const int c = h8 / 8 * 8 + (int)(i & 7);
+    weight_tail[i] = c < h8 ? weight[(i >> 3) * h8 + c] : zero;
+    return;
+  }
+  i -= v * 8;
+  const int ld8 = (h8 + 7) / 8 * 8;
+  const int64_t r = i / ld8;
+  const int c = (int)(i - r * ld8);
+  if (r < m) hidden_copy[i] = c < h8 ? hidden[r * h8 + c] : zero;
+}
+
 // The first `valid16` 16-byte pieces of src, then zeros (the zero-padded copy of a
 // matrix's last rows).
 __global__ __launch_bounds__(256) void lce_k_tail_kernel(const uint4* __restrict__ src,
