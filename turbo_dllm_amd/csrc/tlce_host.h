@@ -330,12 +330,12 @@ template <class E, bool kSoftcap, bool kBias, bool kWDimFirst = false>
 int launch_grad_logits_variant(const GradLogitsArgs& a, hipStream_t stream) {
   static LdsOptIn lds;
   if (int rc = enable_large_lds(lce_grad_logits_panel_kernel<E, kSoftcap, kBias, kWDimFirst>,
-                                E::kSmemBytes, lds))
+                                (kGradLogitsLdsBytes<E, kBias>), lds))
     return rc;
   const int grid = xcd_grid((int64_t)a.n_ttiles * a.n_ptiles);
   ScopedTimer timer(kClassGradLogits, stream);
   lce_grad_logits_panel_kernel<E, kSoftcap, kBias, kWDimFirst>
-      <<<grid, E::kThreads, E::kSmemBytes, stream>>>(a);
+      <<<grid, E::kThreads, (kGradLogitsLdsBytes<E, kBias>), stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
