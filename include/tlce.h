@@ -575,6 +575,11 @@ int tlce_segment_weighted_sum(const float* values, const float* weights,
  * HIP graph that serves any mask. */
 int tlce_fused_gradients_supported(int64_t h, int64_t v, int dtype);
 
+/* Without grad_weight_f32 (a frozen head) tlce_forward_with_gradients_reduced and
+ * tlce_finish_gradients also take, and the workspace query below answers for, vocabularies
+ * that are no multiple of 64, from 2^34 multiply-adds a contraction on. */
+int tlce_frozen_gradients_supported(int64_t m, int64_t h, int64_t v, int dtype);
+
 int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
                           int64_t panel_bytes, int64_t* block_rows, int* n_blocks,
                           int* grad_hidden_k_splits);

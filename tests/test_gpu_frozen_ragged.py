@@ -1,0 +1,138 @@
+"""Cross entropies under a frozen head whose vocabulary is no multiple of 64: the gradient is
+formed in the forward, and what the label's entry loses to bf16 is added back in float32.
+
+An entry rounded to bf16 is off by 2^-7 / sqrt(12) * sqrt(3 / (8 ln 2)) = 1.66e-3 relative
+(root mean square, mantissas spread evenly over a binade).  With the label's entry exact only
+the result's own rounding is left, 1.66e-3 in the 2-norm; a path that rounds the entry as well
+is at sqrt(2) * 1.66e-3 = 2.35e-3.  Held to the middle of the two, 2.0e-3."""
+
+import pytest
+import torch
+
+from turbo_dllm_amd import _lib, options
+from turbo_dllm_amd.loss import dflash_token_loss, masked_token_loss
+from turbo_dllm_amd.tiled_linear_cross_entropy import tiled_linear_cross_entropy
+
+ONE_ROUNDING = 2.0e-3
+
+
+def operands(dev, m, h, v, logit=8.0, ignored=0.0):
+    gen = torch.Generator().manual_seed(m + v)
+    weight = (torch.randn(v, h, generator=gen) * 0.03).bfloat16().to(dev)
+    labels = torch.randint(0, v - 1, (m,), generator=gen)
+    labels[0] = v - 2     # a word of the incomplete last slab
+    hidden = torch.randn(m, h, generator=gen).to(dev)
+    hidden = hidden + weight[labels.to(dev)].float() * (logit / (0.03 ** 2 * h))
+    labels[torch.rand(m, generator=gen) < ignored] = -100
+    return hidden.bfloat16(), weight, labels.to(dev), (torch.rand(m, generator=gen) + 0.5).to(dev)
+
+
+def exact(hidden, weight, labels, factors, softcap=0.0, exclude=-1, multiplier=1.0):
+    """Losses and sum over rows of factor * d loss / d hidden, in float64."""
+    w = weight.double()
+    losses, grads = [], []
+    for lo in range(0, hidden.shape[0], 512):
+        x = hidden[lo:lo + 512].double().requires_grad_()
+        z = x @ w.t() * multiplier
+        if softcap:
+            z = softcap * torch.tanh(z / softcap)
+        if exclude >= 0:
+            z = z.index_fill(1, torch.tensor([exclude], device=z.device), float("-inf"))
+        part = torch.nn.functional.cross_entropy(z, labels[lo:lo + 512], reduction="none",
+                                                 ignore_index=-100)
+        (part * factors[lo:lo + 512]).sum().backward()
+        losses.append(part.detach())
+        grads.append(x.grad)
+    return torch.cat(losses), torch.cat(grads)
+
+
+def off(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+CASES = [
+    # one word over and one short of whole slabs and tiles, a row over whole token tiles
+    dict(m=2305, h=256, v=32001),
+    dict(m=2100, h=512, v=16447, kw=dict(logit_softcap=30.0)),
+    dict(m=1700, h=512, v=32003, kw=dict(exclude_index=32002), ignored=0.3),
+    # several blocks of rows, the last of them small
+    dict(m=1290, h=448, v=33279, panel=33280 * 2 * 512),
+    # labels so far below the largest logit that the block is produced a second time
+    dict(m=1030, h=576, v=32065, far=True),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["sync", "device", "none"])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c['m']}x{c['h']}x{c['v']}")
+def test_against_float64(gpu_device, case, reduction, mode):
+    m, h, v, kw = case["m"], case["h"], case["v"], case.get("kw", {})
+    print("[case]", case, reduction, mode, flush=True)
+    hidden, weight, labels, up = operands(gpu_device, m, h, v, ignored=case.get("ignored", 0.0))
+    if case.get("far"):
+        # the third row's label is no longer the word it was drawn towards, by about 90 nats
+        hidden[2] = (weight[labels[1]].float() * (90.0 / (0.03 ** 2 * h))).bfloat16()
+    live = labels != -100
+    factors = {"mean": live / live.sum(), "sum": live.float(), "none": up}[reduction].double()
+    losses, grad = exact(hidden, weight, labels, factors, kw.get("logit_softcap", 0.0),
+                         kw.get("exclude_index", -1))
+    x = hidden.clone().requires_grad_()
+    with options.panel_budget(case.get("panel", 0)), _lib.kernel_profile() as prof:
+        got = tiled_linear_cross_entropy(x, weight, labels, reduction=reduction,
+                                         dtype=torch.bfloat16, compaction=mode, **kw)
+        ((got * up).sum() if reduction == "none" else got).backward()
+    assert prof.launches["exp_logits_panel"] > 0 and prof.launches["forward_stats"] == 0
+    want = {"mean": losses.sum() / live.sum(), "sum": losses.sum(), "none": losses}[reduction]
+    assert off(got.detach(), want) < 1e-5
+    assert off(x.grad, grad) < ONE_ROUNDING
+    assert not x.grad[~live].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["masked", "drafter"])
+def test_loss_methods(gpu_device, kind):
+    m, h, v = 2112, 512, 16447
+    hidden, weight, labels, up = operands(gpu_device, m, h, v)
+    head = torch.nn.Linear(h, v, bias=False, device="meta")
+    head.weight = torch.nn.Parameter(weight, requires_grad=False)
+    with _lib.kernel_profile() as prof:
+        if kind == "masked":
+            x = hidden.clone().requires_grad_()
+            loss = masked_token_loss(x, labels, up, head, valid_token_count=float(m),
+                                     exclude_mask_token=False, output_multiplier=0.5)
+            want, grad = exact(hidden, weight, labels, up.double() / m, multiplier=0.5)
+            want = (want * up).sum() / m
+        else:
+            x = hidden.reshape(4, -1, h).clone().requires_grad_()
+            shape = x.shape[:2]
+            counts = torch.full((4,), float(shape[1]), device=gpu_device)
+            loss = dflash_token_loss(
+                x, labels.reshape(shape), torch.ones(shape, dtype=torch.bool, device=gpu_device),
+                up.reshape(shape), head, loss_kind="paper_ce", normalization_count=counts)
+            factors = up.double() / (shape[1] + 1e-5) / 4
+            want, grad = exact(hidden, weight, labels, factors)
+            want = (want * factors).sum()
+        loss.backward()
+    assert prof.launches["exp_logits_panel"] > 0 and prof.launches["forward_stats"] == 0
+    assert off(loss.detach(), want) < 1e-5
+    assert off(x.grad.reshape(m, h), grad) < ONE_ROUNDING
+
+
+def test_where_the_path_is_taken():
+    lib = _lib.library()
+    taken = lib.tlce_frozen_gradients_supported
+    bf16 = _lib.DTYPE_BF16
+    assert taken(2100, 256, 32001, bf16) == 1 and taken(1 << 20, 4096, 262143, bf16) == 1
+    assert taken(2097, 256, 32001, bf16) == 0           # just under 2^34 multiply-adds
+    assert taken(1, 256, 32000, bf16) == 1              # whole slabs: any size, as before
+    assert taken(8192, 1000, 32003, bf16) == 0
+    assert taken(8192, 1024, 32003, _lib.DTYPE_F16) == 0
+    assert taken(8192, 1024, 32003, _lib.DTYPE_F32) == 0
+    size = lib.tlce_forward_with_gradients_workspace_bytes
+    assert size(8192, 1024, 32003, bf16, 0, 0) > 0
+    assert size(8192, 1024, 32003, bf16, 1, 0) == -1 and size(64, 64, 32003, bf16, 0, 0) == -1
+    fake = 4096     # never dereferenced: refused first
+    rc = lib.tlce_finish_gradients(fake, fake, None, None, fake, fake, 8, 8, 64, 32003, 1,
+                                   fake, fake, None, 0, None, 0, None)
+    assert rc != 0 and "multiples of 64" in _lib.last_error()

@@ -113,6 +113,7 @@ SIGNATURES = {
         ],
     ),
     "tlce_fused_gradients_supported": (c_int, [c_int64, c_int64, c_int]),
+    "tlce_frozen_gradients_supported": (c_int, [c_int64, c_int64, c_int64, c_int]),
     "tlce_query_fused_plan": (
         c_int, [c_int64, c_int64, c_int64, c_int, c_int64, c_void_p, c_void_p, c_void_p]
     ),

@@ -507,14 +507,17 @@ def fused_gradients_supported(hidden: torch.Tensor, weight: torch.Tensor,
     """Whether ``forward_with_gradients`` takes these operands: bf16 inputs on the
     GPU, head stored [V, H], no bias, H and V multiples of 64.  (f16's exponent
     range cannot hold exp(logit - reference) and its row sums.)"""
+    return _bf16_head(hidden, weight, bias, weight_dim_first) and bool(
+        _lib.library().tlce_fused_gradients_supported(
+            hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
+
+
+def _bf16_head(hidden, weight, bias, weight_dim_first) -> bool:
     if bias is not None or weight_dim_first or not hidden.is_cuda:
         return False
     if hidden.dtype != torch.bfloat16 or weight.dtype != hidden.dtype:
         return False
-    if hidden.dim() != 2 or weight.dim() != 2 or weight.shape[1] != hidden.shape[1]:
-        return False
-    return bool(_lib.library().tlce_fused_gradients_supported(
-        hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
+    return hidden.dim() == 2 and weight.dim() == 2 and weight.shape[1] == hidden.shape[1]
 
 
 # Rows of one token tile: leaving some out saves no work, so they are not compacted (scan,
@@ -523,8 +526,13 @@ ONE_TILE_ROWS = 256
 
 
 def gradients_in_forward_supported(m: int, hidden: torch.Tensor, weight: torch.Tensor,
-                                   bias: torch.Tensor | None, weight_dim_first: bool) -> bool:
-    """Whether ``forward_with_gradients_reduced`` takes ``m`` rows of these operands."""
+                                   bias: torch.Tensor | None, weight_dim_first: bool,
+                                   trainable: bool) -> bool:
+    """Whether ``forward_with_gradients_reduced`` takes ``m`` rows of these operands, with a
+    gradient of the head or (``trainable`` false: any vocabulary, from a size on) without."""
+    if not trainable and _bf16_head(hidden, weight, bias, weight_dim_first):
+        return bool(_lib.library().tlce_frozen_gradients_supported(
+            m, hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
     return (fused_gradients_supported(hidden, weight, bias, weight_dim_first)
             or f32_gradients_in_forward_supported(m, hidden, weight, bias, weight_dim_first))
 
@@ -560,7 +568,7 @@ def forward_with_gradients_reduced(
     reduction_code = _reduction_code(reduction)
     m, h = hidden.shape
     v = weight.shape[0]
-    if not gradients_in_forward_supported(m, hidden, weight, None, False):
+    if not gradients_in_forward_supported(m, hidden, weight, None, False, compute_weight_grad):
         raise RuntimeError("forward_with_gradients_reduced does not take these operands "
                            "(gradients_in_forward_supported)")
     hidden = _dense(hidden)

@@ -339,6 +339,7 @@ struct FusedRowsArgs {
   const float* part_entry = nullptr;     // kRounded sums of the producer, or null: the row
   const float* part_rounded = nullptr;   // factor makes up for the rounding of the row's sum,
   float* row_rounded = nullptr;          // [m] which goes here
+  float* label_rest = nullptr;           // [m] what the label's entry lost when it was rounded
   float* row_scale;            // [m_pad]
   void* scaled_hidden;         // [m_pad, h] or [m_pad, 3, hp], or null (no grad_weight)
   float* ref_next;             // [m] reference of the second try
@@ -367,6 +368,8 @@ struct ReduceSlabsArgs {
   // before the row factor
   const float* fix_value = nullptr;
   const int* fix_id = nullptr;
+  const float* label_rest = nullptr;     // and label_rest[r] * weight[labels[r], :]
+  const int64_t* labels = nullptr;       // (read where label_rest[r] != 0)
   const void* weight = nullptr;     // bf16 [.., h]
   // non-null: one more workgroup adds up the losses (over valid_count[0] for the mean)
   float* loss = nullptr;
@@ -464,17 +467,33 @@ struct FusedPlan {
 // Float32 entries are three bf16 planes.
 inline int panel_entry_bytes(int dtype) { return dtype == TLCE_DTYPE_F32 ? 6 : 2; }
 
-// Cross entropies and soft embeddings whose panel entries are formed in the forward:
-// vocabularies of whole 64-row slabs.  Others keep the sequences that recompute the
-// logits, which are more exact: their logit gradients are rounded with the upstream factor
-// in them, and grad_weight contracts the hidden rows as they are, not a rounded product of
-// them with a row factor.  2-norm errors against float64, recomputed / in the forward,
-// 1500 rows, H = 1024, V = 32003: grad_weight 2.42e-3 / 2.83e-3, grad_hidden under a frozen
-// head 2.21e-3 / 2.36e-3 (reduction "sum" 2.07e-3 / 2.36e-3), soft embeddings 2.25e-3 /
+// Cross entropies with a gradient of the head, and soft embeddings, whose panel entries are
+// formed in the forward: vocabularies of whole 64-row slabs.  Others keep the sequences that
+// recompute the logits, which are more exact: grad_weight contracts the hidden rows as they
+// are, not a rounded product of them with a row factor, and probabilities are rounded when they
+// are normalised.  2-norm errors against float64, recomputed / in the forward,
+// 1500 rows, H = 1024, V = 32003: grad_weight 2.42e-3 / 2.83e-3, soft embeddings 2.25e-3 /
 // 2.25e-3 (H = 3840, V = 40001, a soft cap of 30: 2.25e-3 / 2.31e-3).  A step of 2741 rows over
 // H = 2048 takes 1.32 ms recomputed (1.55 from transposed copies) and took 1.04 in the forward.
 inline bool fused_gradients_supported(int64_t h, int64_t v, int dtype) {
   return dtype == TLCE_DTYPE_BF16 && engine_class(h, dtype) == 2 && (v % 64) == 0;
+}
+
+// Cross entropies under a frozen head: any vocabulary.  grad_hidden is the more exact of the
+// two sequences since what the label's entry loses to its rounding is added back in float32
+// (lce_reduce_scaled_slabs_kernel), and two contractions replace three.  Recomputed / in the
+// forward, us a step and 2-norm errors of grad_hidden against float64 (reductions mean to none):
+//    600 rows, H = 1024, V = 32003    258 .. 278 / 206 .. 235   2.1e-3 .. 2.4e-3 / 1.66e-3
+//   1500 rows, H = 1024, V = 32003    354 .. 382 / 260 .. 268   2.1e-3 .. 2.4e-3 / 1.66e-3
+//   2741 rows, H = 2048, V = 32003   1021 .. 1036 / 727 .. 743  2.1e-3 .. 2.4e-3 / 1.66e-3
+//   1610 rows, H = 4096, V = 151935        4950 / 3400
+// Below 2^34 multiply-adds a contraction a step is bound by its launches (300 rows, H = 1024,
+// V = 32003: 217 to 241 recomputed) and keeps its sequence.
+constexpr int64_t kFrozenRaggedMinMacs = 1ll << 34;
+inline bool frozen_gradients_supported(int64_t m, int64_t h, int64_t v, int dtype) {
+  return fused_gradients_supported(h, v, dtype) ||
+         (dtype == TLCE_DTYPE_BF16 && engine_class(h, dtype) == 2 &&
+          (double)m * h * v >= (double)kFrozenRaggedMinMacs);
 }
 
 // KL and CE with top-k take any vocabulary: the contraction over it reads the rows of an
@@ -512,7 +531,7 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
 
 struct FusedLayout {
   int64_t panel, part_sum, part_max, target, ref, ref_next, row_scale, scaled_hidden, slabs,
-      redo, hidden_planes, weight_planes, total;
+      redo, hidden_planes, weight_planes, label_rest, k_tail, total;
 };
 
 inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dtype,
@@ -538,6 +557,10 @@ inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dt
   if (planes) off += align256(mp * hp * es);
   l.weight_planes = off;
   if (planes) off += align256(p.vp * hp * es);
+  l.label_rest = off;
+  if (!planes) off += align256(p.block_rows * 4);
+  l.k_tail = off;
+  if (!planes && !weight_grad) off += k_tail_bytes(p.v, h);
   l.total = off;
   return l;
 }
@@ -647,7 +670,10 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
       hidden_in = static_cast<const In*>(opt.rows_copy);
       hidden_t = hidden_in;
     }
+    // (a vocabulary of incomplete slabs: frozen heads only)
+    if (int rc = prepare_k_tail(weight, v, h, ws + l.k_tail, stream)) return rc;
   }
+  float* label_rest = kPlanes == 1 ? reinterpret_cast<float*>(ws + l.label_rest) : nullptr;
 
   for (int block = 0; block < p.n_blocks; ++block) {
     const int64_t r0 = (int64_t)block * p.block_rows;
@@ -683,6 +709,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     ra.row_scale = row_scale; ra.scaled_hidden = scaled_hidden;
     ra.ref_next = ref_next; ra.redo = redo + block;
     ra.m_dev = m_dev; ra.row0 = r0;
+    ra.label_rest = label_rest;
 
     for (int attempt = 0; attempt < 2; ++attempt) {
       ea.ref = attempt ? ref_next : ref + r0;
@@ -701,8 +728,12 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     // grad_hidden of the block: A = weight as stored or its planes (K-major, K = vocabulary),
     // B = panel
     GemmArgs dh;
-    dh.a = weight_t; dh.lda = hp; dh.a_rows = (int)hp;
-    dh.k = (int)round_up(v, 64);   // (planes have zero rows up to there)
+    if constexpr (kPlanes == 1) {
+      set_head_operand(dh, weight, v, h, ws + l.k_tail);
+    } else {
+      dh.a = weight_t; dh.lda = hp; dh.a_rows = (int)hp;
+      dh.k = (int)round_up(v, 64);   // (planes have zero rows up to there)
+    }
     dh.b = panel; dh.ldb = p.vp; dh.b_rows = (int)rows_p;
     dh.k_per_split = 0;
     dh.ni = p.n_htiles; dh.nj = n_ttiles;
@@ -731,6 +762,9 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
     rs.row_scale = row_scale; rs.m = (int)rows; rs.h = (int)h;
     rs.out = grad_hidden32 + r0 * h;
     rs.m_dev = m_dev; rs.row0 = r0;
+    if (label_rest != nullptr) {
+      rs.label_rest = label_rest; rs.labels = labels + r0; rs.weight = weight;
+    }
     if (r0 + rows >= m) {
       rs.loss = opt.loss; rs.losses = losses; rs.n_losses = row_idx != nullptr ? opt.n_out : m;
       rs.valid_count = valid_count; rs.mean = opt.mean;

@@ -168,6 +168,7 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
       if (p.probabilities != nullptr) p.probabilities[r] = live ? expf(target - lse) : 0.0f;
       p.ref_next[r] = (live && !in_window) ? mx : c;
       if (live && !in_window) atomicOr(p.redo, 1);
+      float rest = 0.0f;
       // the label's entry: s * entry = (softmax - 1) * cap'
       if (!p.keep_label && live && label >= 0 && label < p.v && label != p.exclude) {
         float dcap = 1.0f;
@@ -183,9 +184,12 @@ __global__ __launch_bounds__(64 * kFusedRowsWaves) void lce_fused_rows_kernel(Fu
 #pragma unroll
           for (int pl = 0; pl < 3; ++pl) at[pl * p.ld] = from_float<__bf16>(part[pl]);
         } else {
-          static_cast<T*>(p.panel)[(int64_t)r * p.ld + label] = from_float<T>(entry);
+          const T rounded = from_float<T>(entry);
+          static_cast<T*>(p.panel)[(int64_t)r * p.ld + label] = rounded;
+          rest = entry - to_float<T>(rounded);
         }
       }
+      if (p.label_rest != nullptr) p.label_rest[r] = rest;
     }
     if (r < p.m_pad) p.row_scale[r] = factor;
     sh_factor[lane] = factor;
@@ -361,6 +365,14 @@ __global__ __launch_bounds__(256) void lce_reduce_scaled_slabs_kernel(ReduceSlab
   }
   const float s = p.row_scale[r];
   const float* src = p.slabs + (int64_t)r * p.h;
+  // The label's entry, the softmax minus one, is nearly all of a row's gradient until the model
+  // is certain, and so is its rounding to bf16: added back in float32, one row of the head read.
+  float rest = 0.0f;
+  const __bf16* label_row = nullptr;
+  if (p.label_rest != nullptr) {
+    rest = p.label_rest[r];
+    label_row = static_cast<const __bf16*>(p.weight) + (rest != 0.0f ? p.labels[r] : 0) * p.h;
+  }
   float fix[kTopkFix];
   const __bf16* fix_row[kTopkFix];
   if (p.fix_value != nullptr) {
@@ -371,13 +383,19 @@ __global__ __launch_bounds__(256) void lce_reduce_scaled_slabs_kernel(ReduceSlab
                    (int64_t)p.fix_id[(int64_t)r * kTopkFix + j] * p.h;
     }
   }
+  typedef __bf16 v4_t __attribute__((ext_vector_type(4)));
   for (int k = threadIdx.x * 4; k < p.h; k += 256 * 4) {
+    v4_t lw = {};
+    if (label_row != nullptr) lw = *reinterpret_cast<const v4_t*>(label_row + k);
     f32x4_t sum = *reinterpret_cast<const f32x4_t*>(src + k);
 #pragma unroll 8
     for (int q = 1; q < p.n_splits; ++q)
       sum += *reinterpret_cast<const f32x4_t*>(src + (int64_t)q * p.split_stride + k);
+    if (rest != 0.0f) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] = fmaf(rest, to_float<__bf16>(lw[e]), sum[e]);
+    }
     if (p.fix_value != nullptr) {
-      typedef __bf16 v4_t __attribute__((ext_vector_type(4)));
       v4_t w[kTopkFix];
 #pragma unroll
       for (int j = 0; j < kTopkFix; ++j) w[j] = *reinterpret_cast<const v4_t*>(fix_row[j] + k);

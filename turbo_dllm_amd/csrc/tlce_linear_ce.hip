@@ -1004,6 +1004,10 @@ extern "C" int tlce_fused_gradients_supported(int64_t h, int64_t v, int dtype) {
   return (h > 0 && v > 0 && fused_gradients_supported(h, v, dtype)) ? 1 : 0;
 }
 
+extern "C" int tlce_frozen_gradients_supported(int64_t m, int64_t h, int64_t v, int dtype) {
+  return (m >= 0 && h > 0 && v > 0 && frozen_gradients_supported(m, h, v, dtype)) ? 1 : 0;
+}
+
 extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
                                      int64_t panel_bytes, int64_t* block_rows, int* n_blocks,
                                      int* grad_hidden_k_splits) {
@@ -1020,7 +1024,10 @@ extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
 extern "C" int64_t tlce_forward_with_gradients_workspace_bytes(int64_t m, int64_t h, int64_t v,
                                                                int dtype, int compute_weight_grad,
                                                                int64_t panel_bytes) {
-  if (m < 0 || h <= 0 || v <= 0 || !fused_gradients_supported(h, v, dtype)) return -1;
+  if (m < 0 || h <= 0 || v <= 0) return -1;
+  if (compute_weight_grad != 0 ? !fused_gradients_supported(h, v, dtype)
+                               : !frozen_gradients_supported(m, h, v, dtype))
+    return -1;
   return fused_layout(make_fused_plan(m, h, v, dtype, panel_bytes), m, h, dtype,
                       compute_weight_grad != 0).total;
 }
@@ -1186,7 +1193,8 @@ extern "C" int tlce_forward_with_gradients_reduced(
                     row_of != nullptr && row_idx == nullptr),
                "forward_with_gradients_reduced: rows_copy is bf16, 16-byte aligned, for rows "
                "that were not compacted, and needs row_of");
-  TLCE_REQUIRE(fused_gradients_supported(h, v, dtype) ||
+  TLCE_REQUIRE((grad_weight_f32 != nullptr ? fused_gradients_supported(h, v, dtype)
+                                           : frozen_gradients_supported(m, h, v, dtype)) ||
                    (dtype == TLCE_DTYPE_F32 && f32_gradients_in_forward_supported(m, h, v)),
                "forward_with_gradients_reduced: not taken for m=%lld h=%lld v=%lld dtype=%d",
                (long long)m, (long long)h, (long long)v, dtype);
@@ -1214,8 +1222,10 @@ extern "C" int tlce_finish_gradients(const float* grad_hidden_f32, const float* 
                                      int64_t panel_bytes, void* forward_workspace,
                                      int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
-  TLCE_REQUIRE(m >= 0 && h > 0 && v > 0 && fused_gradients_supported(h, v, TLCE_DTYPE_BF16),
-               "finish_gradients: needs h and v multiples of 64");
+  TLCE_REQUIRE(m >= 0 && h > 0 && v > 0 &&
+                   (grad_weight != nullptr ? fused_gradients_supported(h, v, TLCE_DTYPE_BF16)
+                                           : (h % 64) == 0),
+               "finish_gradients: needs h, and with grad_weight v, multiples of 64");
   TLCE_REQUIRE(reduction_code >= TLCE_REDUCTION_NONE && reduction_code <= TLCE_REDUCTION_MEAN,
                "finish_gradients: unknown reduction code %d", reduction_code);
   if (m == 0) {

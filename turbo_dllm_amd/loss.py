@@ -75,7 +75,8 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         # library takes the operands and the row count is known to the host
         ctx.fused = (
             wants_grad and get_gradient_mode() == "forward"
-            and native.gradients_in_forward_supported(m, rows, weight, bias, False)
+            and native.gradients_in_forward_supported(m, rows, weight, bias, False,
+                                                      bool(ctx.needs_input_grad[1]))
         )
         if ctx.fused:
             rows = rows[:m]
@@ -445,7 +446,7 @@ def dflash_token_loss(
             and torch.is_grad_enabled()
             and (hidden_states.requires_grad or lm_head.weight.requires_grad)
             and native.gradients_in_forward_supported(n_valid, hidden_flat, lm_head.weight, None,
-                                                      False)):
+                                                      False, lm_head.weight.requires_grad)):
         loss = _FusedSampleLoss.apply(
             hidden_flat, lm_head.weight, target_token_ids, position_weights, denominators,
             tokens_per_sample, all_indices, row_count, n_valid,

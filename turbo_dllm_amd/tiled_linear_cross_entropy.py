@@ -292,7 +292,8 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
     ctx.fused = (
         wants_grad and options.get_gradient_mode() == "forward"
         and native.gradients_in_forward_supported(m, rows, weight_vf, bias,
-                                                  in_place or weight_dim_first)
+                                                  in_place or weight_dim_first,
+                                                  bool(ctx.needs_input_grad[1]))
     )
     can_wait = ctx.fused and bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
         m, rows.shape[1], weight_vf.shape[0], rows.dtype)
