@@ -583,16 +583,14 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
   };
 
   // kBiasInLds: the logits of four consecutive rows of owned column j
+  constexpr bool kAddBias = kBias && kBiasInLds<E>;
   auto logits_of = [&](int j, int i, float (&z)[4]) {
-    if constexpr (kBias && kBiasInLds<E>) {
+    if constexpr (kAddBias) {
       const float4 b = *reinterpret_cast<const float4*>(bias_stash + eng.row(i));
       z[0] = fmaf(E::read(acc, j, i), p.logit_scale, b.x);
       z[1] = fmaf(E::read(acc, j, i + 1), p.logit_scale, b.y);
       z[2] = fmaf(E::read(acc, j, i + 2), p.logit_scale, b.z);
       z[3] = fmaf(E::read(acc, j, i + 3), p.logit_scale, b.w);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) z[q] = E::get(acc, j, i + q);
     }
   };
   // row_sum over the 16 lanes that hold the same rows: each exchange halves the rows a lane
@@ -648,7 +646,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
           for (int q = 0; q < 4; ++q) {
             const int row = eng.row(i + q);
             const bool vok = !kEdge || ((vbase + row < p.v) && (vbase + row != excluded));
-            const float g = grad_of(z[q], j, row, vok, edge_tag, onehot_tag);
+            const float g = grad_of(kAddBias ? z[q] : E::get(acc, j, i + q), j, row, vok, edge_tag, onehot_tag);
             if (kBias) row_sum[i + q] += g;
             split_planes(g, part[q]);
           }
@@ -711,7 +709,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
           for (int q = 0; q < 4; ++q) {
             const int row = eng.row(i + q);
             const bool vok = !kEdge || ((vbase + row < p.v) && (vbase + row != excluded));
-            g4[q] = grad_of(z[q], j, row, vok, edge_tag, onehot_tag);
+            g4[q] = grad_of(kAddBias ? z[q] : E::get(acc, j, i + q), j, row, vok, edge_tag, onehot_tag);
             if (kBias) row_sum[i + q] += g4[q];
           }
           const int vq = eng.row(i) >> 2;
