@@ -580,6 +580,11 @@ int tlce_fused_gradients_supported(int64_t h, int64_t v, int dtype);
  * that are no multiple of 64, from 2^34 multiply-adds a contraction on. */
 int tlce_frozen_gradients_supported(int64_t m, int64_t h, int64_t v, int dtype);
 
+/* Whether the rows make one block, so that grad_weight can be contracted in the backward
+ * (tlce_finish_gradients with `hidden`).  Vocabularies that are no multiple of 64: from 2^37
+ * multiply-adds on, and the backward needs the forward's `labels` (int64 [m]). */
+int tlce_weight_grad_can_wait(int64_t m, int64_t h, int64_t v, int dtype, int64_t panel_bytes);
+
 int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
                           int64_t panel_bytes, int64_t* block_rows, int* n_blocks,
                           int* grad_hidden_k_splits);
@@ -638,7 +643,7 @@ int tlce_finish_gradients(const float* grad_hidden_f32, const float* grad_weight
                           const int* row_of, const int64_t* row_count, const float* grad_output,
                           const float* valid_count, int64_t m, int64_t n_out, int64_t h,
                           int64_t v, int reduction_code, void* grad_hidden, void* grad_weight,
-                          const void* hidden, int64_t panel_bytes, void* forward_workspace,
+                          const void* hidden, const int64_t* labels, int64_t panel_bytes, void* forward_workspace,
                           int64_t workspace_bytes, void* stream);
 
 /* The pair for float32 operands whose products run on the bf16 matrix units

@@ -1,5 +1,5 @@
-"""Cross entropies under a frozen head whose vocabulary is no multiple of 64: the gradient is
-formed in the forward, and what the label's entry loses to bf16 is added back in float32.
+"""Cross entropies over vocabularies that are no multiple of 64: the gradients are formed in
+the forward, and what the label's entry loses to bf16 is added back in float32.
 
 An entry rounded to bf16 is off by 2^-7 / sqrt(12) * sqrt(3 / (8 ln 2)) = 1.66e-3 relative
 (root mean square, mantissas spread evenly over a binade).  With the label's entry exact only
@@ -119,6 +119,80 @@ def test_loss_methods(gpu_device, kind):
     assert off(x.grad.reshape(m, h), grad) < ONE_ROUNDING
 
 
+# from 2^37 multiply-adds on
+TRAINABLE = [
+    dict(m=2305, h=1920, v=32001),
+    dict(m=4200, h=2048, v=16447, kw=dict(logit_softcap=30.0)),
+    dict(m=3200, h=2112, v=32003, kw=dict(exclude_index=32002), ignored=0.3),
+    dict(m=2100, h=2112, v=32065, far=True),
+]
+
+
+def exact_grad_weight(hidden, weight, labels, factors, softcap=0.0, exclude=-1):
+    w = weight.double()
+    out = torch.zeros_like(w)
+    for lo in range(0, hidden.shape[0], 512):
+        x, y, f = hidden[lo:lo + 512].double(), labels[lo:lo + 512], factors[lo:lo + 512]
+        z = (x @ w.t()).requires_grad_()
+        capped = softcap * torch.tanh(z / softcap) if softcap else z
+        if exclude >= 0:
+            capped = capped.index_fill(1, torch.tensor([exclude], device=z.device), float("-inf"))
+        (torch.nn.functional.cross_entropy(capped, y, reduction="none", ignore_index=-100)
+         * f).sum().backward()
+        out += z.grad.t().contiguous() @ x
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["sync", "device", "none"])
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+@pytest.mark.parametrize("case", TRAINABLE,
+                         ids=lambda c: f"{c['m']}x{c['h']}x{c['v']}")
+def test_trainable_heads_against_float64(gpu_device, case, reduction, mode):
+    m, h, v, kw = case["m"], case["h"], case["v"], case.get("kw", {})
+    print("[case]", case, reduction, mode, flush=True)
+    hidden, weight, labels, up = operands(gpu_device, m, h, v, ignored=case.get("ignored", 0.0))
+    if case.get("far"):
+        hidden[2] = (weight[labels[1]].float() * (90.0 / (0.03 ** 2 * h))).bfloat16()
+    live = labels != -100
+    factors = {"mean": live / live.sum(), "sum": live.float(), "none": up}[reduction].double()
+    cap, exclude = kw.get("logit_softcap", 0.0), kw.get("exclude_index", -1)
+    losses, grad = exact(hidden, weight, labels, factors, cap, exclude)
+    x, w = hidden.clone().requires_grad_(), weight.clone().requires_grad_()
+    with _lib.kernel_profile() as prof:
+        got = tiled_linear_cross_entropy(x, w, labels, reduction=reduction,
+                                         dtype=torch.bfloat16, compaction=mode, **kw)
+        total = (got * up).sum() if reduction == "none" else got
+        total.backward(retain_graph=True)
+    assert prof.launches["exp_logits_panel"] > 0 and prof.launches["forward_stats"] == 0
+    assert off(x.grad, grad) < ONE_ROUNDING
+    assert off(w.grad, exact_grad_weight(hidden, weight, labels, factors, cap, exclude)) < ONE_ROUNDING
+    first, w.grad = w.grad, None
+    total.backward()      # again on the same workspace
+    assert torch.equal(first, w.grad)
+
+
+@pytest.mark.gpu
+def test_a_word_with_more_rows_than_are_kept(gpu_device):
+    """Half of the rows have one label: a wave's list of a tile's rows (256) overflows, and the
+    later rows keep the rounding of their operands (three roundings at most: 2.87e-3)."""
+    m, h, v = 8192, 1088, 16447
+    hidden, weight, labels, _ = operands(gpu_device, m, h, v)
+    labels[::2] = 16440
+    factors = torch.full((m,), 1.0, dtype=torch.float64, device=gpu_device)
+    grads = []
+    for _ in range(2):
+        w = weight.clone().requires_grad_()
+        tiled_linear_cross_entropy(hidden.clone().requires_grad_(), w, labels, reduction="sum",
+                                   dtype=torch.bfloat16).backward()
+        grads.append(w.grad)
+    assert torch.equal(*grads)
+    want = exact_grad_weight(hidden, weight, labels, factors)
+    assert off(grads[0], want) < 2.87e-3
+    others = torch.arange(v, device=gpu_device) < 16384    # tiles whose rows all fit
+    assert off(grads[0][others], want[others]) < ONE_ROUNDING
+
+
 def test_where_the_path_is_taken():
     lib = _lib.library()
     taken = lib.tlce_frozen_gradients_supported
@@ -131,8 +205,16 @@ def test_where_the_path_is_taken():
     assert taken(8192, 1024, 32003, _lib.DTYPE_F32) == 0
     size = lib.tlce_forward_with_gradients_workspace_bytes
     assert size(8192, 1024, 32003, bf16, 0, 0) > 0
-    assert size(8192, 1024, 32003, bf16, 1, 0) == -1 and size(64, 64, 32003, bf16, 0, 0) == -1
+    assert size(64, 64, 32003, bf16, 0, 0) == -1
+    # a trainable head: in one block of rows
+    wait = lib.tlce_weight_grad_can_wait
+    assert wait(8192, 1024, 32003, bf16, 0) == 1 and wait(8192, 1024, 32003, bf16, 1 << 28) == 0
+    assert wait(2048, 1024, 32003, bf16, 0) == 0 and wait(2048, 1024, 32000, bf16, 0) == 1
+    assert size(8192, 1024, 32003, bf16, 1, 0) > 0
+    assert size(8192, 1024, 32003, bf16, 1, 1 << 28) == -1
+    assert wait(64, 64, 32003, bf16, 0) == 0 and wait(8192, 1024, 32003, _lib.DTYPE_F16, 0) == 0
     fake = 4096     # never dereferenced: refused first
-    rc = lib.tlce_finish_gradients(fake, fake, None, None, fake, fake, 8, 8, 64, 32003, 1,
-                                   fake, fake, None, 0, None, 0, None)
-    assert rc != 0 and "multiples of 64" in _lib.last_error()
+    for dw32, hidden, labels in ((fake, None, None), (None, fake, None), (fake, None, fake)):
+        rc = lib.tlce_finish_gradients(fake, dw32, None, None, fake, fake, 8, 8, 64, 32003, 1,
+                                       fake, fake, hidden, labels, 0, None, 0, None)
+        assert rc != 0 and "multiples of 64" in _lib.last_error()

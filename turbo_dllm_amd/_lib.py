@@ -114,6 +114,7 @@ SIGNATURES = {
     ),
     "tlce_fused_gradients_supported": (c_int, [c_int64, c_int64, c_int]),
     "tlce_frozen_gradients_supported": (c_int, [c_int64, c_int64, c_int64, c_int]),
+    "tlce_weight_grad_can_wait": (c_int, [c_int64, c_int64, c_int64, c_int, c_int64]),
     "tlce_query_fused_plan": (
         c_int, [c_int64, c_int64, c_int64, c_int, c_int64, c_void_p, c_void_p, c_void_p]
     ),
@@ -150,7 +151,7 @@ SIGNATURES = {
             c_void_p, c_void_p, c_void_p, c_void_p,             # dh32 dw32 row_of row_count
             c_void_p, c_void_p,                                 # grad_output valid_count
             c_int64, c_int64, c_int64, c_int64, c_int,          # m n_out h v reduction
-            c_void_p, c_void_p, c_void_p,                       # grad_hidden grad_weight hidden
+            c_void_p, c_void_p, c_void_p, c_void_p,             # grad_hidden grad_weight hidden labels
             c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
         ],
     ),

@@ -529,10 +529,14 @@ def gradients_in_forward_supported(m: int, hidden: torch.Tensor, weight: torch.T
                                    bias: torch.Tensor | None, weight_dim_first: bool,
                                    trainable: bool) -> bool:
     """Whether ``forward_with_gradients_reduced`` takes ``m`` rows of these operands, with a
-    gradient of the head or (``trainable`` false: any vocabulary, from a size on) without."""
+    gradient of the head or without.  Vocabularies that are no multiple of 64 are taken from a
+    size on, for a ``trainable`` head in one block of rows (``weight_grad_can_wait``)."""
     if not trainable and _bf16_head(hidden, weight, bias, weight_dim_first):
         return bool(_lib.library().tlce_frozen_gradients_supported(
             m, hidden.shape[1], weight.shape[0], _dtype_code(hidden)))
+    if _bf16_head(hidden, weight, bias, weight_dim_first) and weight_grad_can_wait(
+            m, hidden.shape[1], weight.shape[0], hidden.dtype):
+        return True
     return (fused_gradients_supported(hidden, weight, bias, weight_dim_first)
             or f32_gradients_in_forward_supported(m, hidden, weight, bias, weight_dim_first))
 
@@ -639,10 +643,12 @@ def finish_gradients(
     row_count: torch.Tensor | None,
     rows: torch.Tensor | None,
     panel_bytes: int,
+    labels: torch.Tensor | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor | None]:
     """The bf16 gradients of what ``forward_with_gradients_reduced`` left, times the upstream
     gradient.  ``rows``: the forward's hidden rows when grad_weight was postponed
-    (``grad_weight32`` is then its workspace)."""
+    (``grad_weight32`` is then its workspace); ``labels``: their labels, needed for
+    vocabularies that are no multiple of 64."""
     device = _require_device(grad_hidden32, grad_weight32, grad_output, valid_count, row_of,
                              row_count, rows)
     reduction_code = _reduction_code(reduction)
@@ -654,6 +660,9 @@ def finish_gradients(
     if row_of is not None and (row_of.dtype != torch.int32 or row_of.numel() != n_out):
         raise RuntimeError("row_of must be int32 with one entry per output row")
     waited = rows is not None
+    if labels is not None and (labels.dtype != torch.long or not labels.is_contiguous()
+                               or labels.numel() != m or labels.device != grad_hidden32.device):
+        raise RuntimeError("labels must be contiguous int64 with one entry per row")
     if waited and (rows.shape != grad_hidden32.shape or not rows.is_contiguous()
                    or grad_weight32 is None or grad_weight32.dtype != torch.uint8):
         raise RuntimeError("a postponed grad_weight needs the forward's rows and workspace")
@@ -669,7 +678,7 @@ def finish_gradients(
             _lib.library().tlce_finish_gradients(
                 _ptr(grad_hidden32), None if waited else _ptr(grad_weight32), _ptr(row_of),
                 _ptr(row_count), grad_output.data_ptr(), _ptr(valid_count), m, n_out, h, v,
-                reduction_code, _ptr(grad_hidden), _ptr(grad_weight), _ptr(rows),
+                reduction_code, _ptr(grad_hidden), _ptr(grad_weight), _ptr(rows), _ptr(labels),
                 int(panel_bytes), grad_weight32.data_ptr() if waited else None,
                 grad_weight32.numel() if waited else 0, _stream(device),
             ),
@@ -822,10 +831,8 @@ def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
     """Whether ``forward_with_gradients`` takes ``m`` rows as one block under the
     panel budget in force, so that its grad_weight contraction can be postponed to
     the backward (``grad_weight_from_panel``)."""
-    if dtype != torch.bfloat16 or not _lib.library().tlce_fused_gradients_supported(
-            h, v, _lib.DTYPE_BF16):
-        return False
-    return _lib.query_fused_plan(m, h, v, _lib.DTYPE_BF16, get_panel_bytes())["n_blocks"] == 1
+    return dtype == torch.bfloat16 and bool(_lib.library().tlce_weight_grad_can_wait(
+        m, h, v, _lib.DTYPE_BF16, get_panel_bytes()))
 
 
 def _upstream_gradient(grad_output: torch.Tensor, reduction_code: int, n_out: int) -> torch.Tensor:

@@ -432,6 +432,7 @@ struct FinishRowsArgs {
   const void* hidden = nullptr;       // [m, h], with what follows, or null
   const float* row_scale = nullptr;   // [m]
   void* scaled = nullptr;             // bf16 [m_pad, h], zero rows from the row count on
+  float* row_factor = nullptr;        // [m] what the rows of `scaled` are multiplied by
 };
 int launch_finish_rows(const FinishRowsArgs& a, hipStream_t stream);
 
@@ -468,10 +469,10 @@ struct FusedPlan {
 inline int panel_entry_bytes(int dtype) { return dtype == TLCE_DTYPE_F32 ? 6 : 2; }
 
 // Cross entropies with a gradient of the head, and soft embeddings, whose panel entries are
-// formed in the forward: vocabularies of whole 64-row slabs.  Others keep the sequences that
-// recompute the logits, which are more exact: grad_weight contracts the hidden rows as they
-// are, not a rounded product of them with a row factor, and probabilities are rounded when they
-// are normalised.  2-norm errors against float64, recomputed / in the forward,
+// formed in the forward: vocabularies of whole 64-row slabs.  Others (but see
+// weight_grad_can_wait) keep the sequences that recompute the logits, which are more exact:
+// grad_weight contracts the hidden rows as they are, not a rounded product of them with a row
+// factor, and probabilities are rounded when they are normalised.  2-norm errors against float64, recomputed / in the forward,
 // 1500 rows, H = 1024, V = 32003: grad_weight 2.42e-3 / 2.83e-3, soft embeddings 2.25e-3 /
 // 2.25e-3 (H = 3840, V = 40001, a soft cap of 30: 2.25e-3 / 2.31e-3).  A step of 2741 rows over
 // H = 2048 takes 1.32 ms recomputed (1.55 from transposed copies) and took 1.04 in the forward.
@@ -487,8 +488,10 @@ inline bool fused_gradients_supported(int64_t h, int64_t v, int dtype) {
 //   1500 rows, H = 1024, V = 32003    354 .. 382 / 260 .. 268   2.1e-3 .. 2.4e-3 / 1.66e-3
 //   2741 rows, H = 2048, V = 32003   1021 .. 1036 / 727 .. 743  2.1e-3 .. 2.4e-3 / 1.66e-3
 //   1610 rows, H = 4096, V = 151935        4950 / 3400
-// Below 2^34 multiply-adds a contraction a step is bound by its launches (300 rows, H = 1024,
-// V = 32003: 217 to 241 recomputed) and keeps its sequence.
+// Steps below 2^34 multiply-adds a contraction are bound by their launches, of which either
+// sequence has about as many (300 rows, H = 1024, V = 32003: 240 / 217, with grad_weight
+// 272 / 238), and keep the results of the recomputing one bit for bit
+// (tests/test_gpu_gradient_routes.py).
 constexpr int64_t kFrozenRaggedMinMacs = 1ll << 34;
 inline bool frozen_gradients_supported(int64_t m, int64_t h, int64_t v, int dtype) {
   return fused_gradients_supported(h, v, dtype) ||
@@ -529,9 +532,33 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
   return p;
 }
 
+// Whether all rows make one block, so that the grad_weight contraction can wait for the
+// upstream gradient.  Vocabularies that are no multiple of 64: adding back what the label's
+// entry and its row of hidden states lose when they are rounded, in the float32 tile
+// (store_tile_t_with_labels); several blocks, whose sums stay in float32 memory until the last
+// pass, recompute.  Recomputed / in the forward, us a step and 2-norm errors of grad_weight
+// against float64:
+//    2741 rows, H = 2048, V = 32003    1343 / 1131   2.32e-3 / 1.66e-3
+//                        Zipf labels   1332 / 1169   1.82e-3 / 1.76e-3 (words of hundreds of rows)
+//    8192 rows, H = 1024, V = 50257    2951 / 2340, Zipf 3001 / 2356
+//    1610 rows, H = 4096, V = 151935   6731 / 5427, Zipf 6824 / 5653
+//   32768 rows, H = 512, V = 16447, Zipf  3080 / 2225   1.72e-3 / 1.72e-3
+// A tile of frequent words ends up to 150 us after the others (kLabelRowsPerWave rows in each
+// wave's list, eight at a time), which the contraction saved has to outweigh: 16384 rows,
+// H = 512, V = 16447 with Zipf labels (2^37 multiply-adds) 1296 / 1289, 5000 rows 505 / 624.
+constexpr int64_t kWaitRaggedMinMacs = 1ll << 37;
+inline bool weight_grad_can_wait(int64_t m, int64_t h, int64_t v, int dtype,
+                                 int64_t panel_bytes) {
+  if (!fused_gradients_supported(h, v, dtype) &&
+      !(frozen_gradients_supported(m, h, v, dtype) &&
+        (double)m * h * v >= (double)kWaitRaggedMinMacs))
+    return false;
+  return make_fused_plan(m, h, v, dtype, panel_bytes).n_blocks == 1;
+}
+
 struct FusedLayout {
   int64_t panel, part_sum, part_max, target, ref, ref_next, row_scale, scaled_hidden, slabs,
-      redo, hidden_planes, weight_planes, label_rest, k_tail, total;
+      redo, hidden_planes, weight_planes, label_rest, row_factor, k_tail, total;
 };
 
 inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dtype,
@@ -549,6 +576,11 @@ inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dt
   l.ref = off;        off += align256(mp * 4);
   l.ref_next = off;   off += align256(p.block_rows * 4);
   l.row_scale = off;  off += align256(p.block_rows * 4);
+  // (up to here the same with and without weight_grad)
+  l.label_rest = off;
+  if (!planes) off += align256(p.block_rows * 4);
+  l.row_factor = off;
+  if (!planes) off += align256(p.block_rows * 4);
   l.scaled_hidden = off;
   if (weight_grad) off += align256(p.block_rows * hp * es);
   l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
@@ -557,10 +589,8 @@ inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dt
   if (planes) off += align256(mp * hp * es);
   l.weight_planes = off;
   if (planes) off += align256(p.vp * hp * es);
-  l.label_rest = off;
-  if (!planes) off += align256(p.block_rows * 4);
   l.k_tail = off;
-  if (!planes && !weight_grad) off += k_tail_bytes(p.v, h);
+  if (!planes) off += k_tail_bytes(p.v, h);
   l.total = off;
   return l;
 }
@@ -801,7 +831,8 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
 // on a workspace sized for one).
 template <class E>
 int deferred_contraction(const FusedPlan& p, const FusedLayout& l, int64_t m, int64_t h, int64_t v,
-                         const int64_t* m_dev, void* grad_weight, char* ws, hipStream_t stream) {
+                         const int64_t* m_dev, void* grad_weight, char* ws, hipStream_t stream,
+                         const void* hidden = nullptr, const int64_t* labels = nullptr) {
   using T = typename E::T;
   GemmArgs dw;
   dw.a = ws + l.scaled_hidden; dw.lda = h; dw.a_rows = (int)h;
@@ -813,6 +844,12 @@ int deferred_contraction(const FusedPlan& p, const FusedLayout& l, int64_t m, in
   dw.c_split_stride = 0;
   dw.mode = kStoreT;
   dw.m_dev = m_dev; dw.m_role = kKFollows; dw.m_round = 64;
+  if (v % 64 != 0) {
+    dw.labels = labels; dw.rows = hidden; dw.n_rows = (int)m;
+    dw.label_rest = reinterpret_cast<const float*>(ws + l.label_rest);
+    dw.row_factor = reinterpret_cast<const float*>(ws + l.row_factor);
+    return launch_gemm<E, true, true, true>(dw, 1, kClassGradWeight, stream);
+  }
   return launch_gemm<E, true, true>(dw, 1, kClassGradWeight, stream);
 }
 
@@ -1503,7 +1540,8 @@ int soft_embedding_emit_impl(const FusedPlan& p, const void* hidden, const void*
                                          int64_t, int, float, float*, float*, float*, float*,    \
                                          char*, hipStream_t);                                    \
   X int deferred_contraction<E>(const FusedPlan&, const FusedLayout&, int64_t, int64_t, int64_t, \
-                                const int64_t*, void*, char*, hipStream_t);                      \
+                                const int64_t*, void*, char*, hipStream_t, const void*,          \
+                                const int64_t*);                                                 \
   X int deferred_grad_weight_impl<E>(const FusedPlan&, const void*, int64_t, int64_t, int64_t,   \
                                      int, const float*, const float*, int, const int64_t*,       \
                                      const int64_t*, void*, char*, hipStream_t);

@@ -272,6 +272,7 @@ __global__ __launch_bounds__(256) void lce_finish_rows_kernel(FinishRowsArgs p) 
   const float* src = p.grad_hidden32 + r * p.h;
   const bool operand = p.hidden != nullptr;
   const float factor = operand ? g * p.row_scale[r] : 0.0f;
+  if (operand && p.row_factor != nullptr && threadIdx.x == 0) p.row_factor[r] = factor;
   const __bf16* hrow = static_cast<const __bf16*>(p.hidden) + r * p.h;
   __bf16* scaled = static_cast<__bf16*>(p.scaled) + r * p.h;
   for (int k = threadIdx.x * 8; k < p.h; k += 256 * 8) {

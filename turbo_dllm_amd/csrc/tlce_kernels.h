@@ -1329,6 +1329,13 @@ struct GemmArgs {
   int a_k_full = 0x7fffffff;
   const void* b_tail = nullptr;
   int b_k_full = 0x7fffffff;
+  // kLabels: A = bf16(row_factor * rows), B = a panel of gradients whose entry at labels[r] was
+  // rounded and lost label_rest[r] by it; n_rows of them (K without its padding)
+  const int64_t* labels = nullptr;
+  const float* label_rest = nullptr;
+  const float* row_factor = nullptr;
+  const void* rows = nullptr;        // [n_rows, lda]
+  int n_rows = 0;
 };
 
 // K splits and slab stride the grad_hidden contraction uses for a device-side
@@ -1481,7 +1488,138 @@ __device__ __forceinline__ void store_tile_t_by_rows(const E& eng, const typenam
   }
 }
 
-template <class E, bool kAKMajor, bool kBKMajor>
+// Rows of an output tile's words: the rows r with labels[r] in [row0, row0 + tile), in
+// ascending order, a quarter of all rows per wave, in LDS beyond the engine's stages.
+struct LabelRow {
+  int row, word;   // word: within the tile
+};
+constexpr int kLabelRowsPerWave = 256;   // (later ones keep the rounding of 16-bit operands)
+constexpr int kLabelLdsBytes = 16 + 4 * kLabelRowsPerWave * (int)sizeof(LabelRow);
+
+template <class E>
+__device__ __forceinline__ void find_label_rows(const GemmArgs& p, int row0, char* lds) {
+  static_assert(E::kThreads == 256, "four waves");
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  LabelRow* list = reinterpret_cast<LabelRow*>(lds + 16) + wave * kLabelRowsPerWave;
+  const int per = (p.n_rows + 3) / 4;
+  const int begin = min(wave * per, p.n_rows), end = min(begin + per, p.n_rows);
+  constexpr int kAhead = 8;
+  int found = 0;
+  for (int r0 = begin; r0 < end; r0 += 64 * kAhead) {
+    int64_t y[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int r = r0 + u * 64 + lane;
+      y[u] = r < end ? p.labels[r] - row0 : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const bool mine = y[u] >= 0 && y[u] < E::kTile && row0 + y[u] < p.c_rows;
+      const unsigned long long mask = __ballot(mine);
+      const int at = found + __popcll(mask & ((1ull << lane) - 1));
+      if (mine && at < kLabelRowsPerWave) list[at] = {r0 + u * 64 + lane, (int)y[u]};
+      found += __popcll(mask);
+    }
+  }
+  if (lane == 0) reinterpret_cast<int*>(lds)[wave] = min(found, kLabelRowsPerWave);
+}
+
+// The float32 tile leaves in 16 bits through LDS, in two halves (store_tile_f32_by_rows), and
+// the words of find_label_rows' rows receive in between what their label entries lost to the
+// 16-bit operands: (entry + rest) * factor * hidden instead of entry * bf16(factor * hidden).
+// A word belongs to one wave, which takes its rows in order: the sums are reproducible.
+// Bound by the latency of the rows' loads, eight rows in flight; a tile has about
+// n_rows * 256 / v of them (22 for 2741 rows over 32003 words).
+template <class E>
+__device__ __forceinline__ void store_tile_t_with_labels(const E& eng, const typename E::Acc& acc,
+                                                         char* smem, const char* lds,
+                                                         const GemmArgs& p, int row0, int col0) {
+  using T = typename E::T;
+  typedef T v4_t __attribute__((ext_vector_type(4)));
+  constexpr int kPerIndex = E::kTokensPerIndex;
+  constexpr int kHalf = E::kCols / 2;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int col = col0 + lane * 4;
+  const bool col_ok = col < p.c_cols;
+  const int at_col = col_ok ? col : 0;
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    if (half) __syncthreads();   // the first half has been read out
+#pragma unroll
+    for (int jj = 0; jj < kHalf; ++jj) {
+      const int j = kHalf * half + jj;
+      const int s_row = jj * kPerIndex + eng.position_in_index();
+#pragma unroll
+      for (int i4 = 0; i4 < E::kRows; i4 += 4) {
+        const int chunk = eng.row(i4) >> 2;
+        const f32x4_t quad = {E::get(acc, j, i4), E::get(acc, j, i4 + 1), E::get(acc, j, i4 + 2),
+                              E::get(acc, j, i4 + 3)};
+        *reinterpret_cast<f32x4_t*>(smem + s_row * 1024 + ((chunk ^ (s_row & 63)) * 16)) = quad;
+      }
+    }
+    __syncthreads();
+    for (int w = 0; w < 4; ++w) {
+      const LabelRow* list = reinterpret_cast<const LabelRow*>(lds + 16) + w * kLabelRowsPerWave;
+      const int n = reinterpret_cast<const int*>(lds)[w];
+      for (int base = 0; base < n; base += 64) {
+        const LabelRow e = list[min(base + lane, n - 1)];
+        // owned index and position of the word (E::token_of_index)
+        const int j = (e.word >> 4) & 7, t = (e.word >> 7) * 16 + (e.word & 15);
+        const bool mine = base + lane < n && (j >= kHalf) == (half != 0) && (e.word & 3) == wave;
+        unsigned long long mask = __ballot(mine);
+        const int my_row = (j - kHalf * half) * kPerIndex + t;
+        while (mask != 0) {
+          constexpr int kAtOnce = 8;   // rows whose loads are in flight together
+          int s_row[kAtOnce];
+          float entry[kAtOnce], exact[kAtOnce];
+          v4_t x[kAtOnce], a[kAtOnce];
+          int l = 0;
+#pragma unroll
+          for (int u = 0; u < kAtOnce; ++u) {
+            const bool some = mask != 0;   // (else the last row again, times zero)
+            l = some ? __ffsll((long long)mask) - 1 : l;
+            mask &= mask - 1;              // (0 stays 0)
+            s_row[u] = __builtin_amdgcn_readlane(my_row, l);
+            const int64_t r = __builtin_amdgcn_readlane(e.row, l);
+            const int word = __builtin_amdgcn_readlane(e.word, l);
+            const float b = to_float<T>(static_cast<const T*>(p.b)[r * p.ldb + row0 + word]);
+            entry[u] = some ? b : 0.0f;
+            exact[u] = some ? (b + p.label_rest[r]) * p.row_factor[r] : 0.0f;
+            x[u] = *reinterpret_cast<const v4_t*>(static_cast<const T*>(p.rows) + r * p.lda + at_col);
+            a[u] = *reinterpret_cast<const v4_t*>(static_cast<const T*>(p.a) + r * p.lda + at_col);
+          }
+          f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int u = 0; u < kAtOnce; ++u) {
+            f32x4_t* at = reinterpret_cast<f32x4_t*>(smem + s_row[u] * 1024 +
+                                                     ((lane ^ (s_row[u] & 63)) * 16));
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              sum[q] += fmaf(exact[u], to_float<T>(x[u][q]), -(entry[u] * to_float<T>(a[u][q])));
+            if (u + 1 < kAtOnce && s_row[u + 1 < kAtOnce ? u + 1 : u] == s_row[u]) continue;
+            *at += sum;
+            sum = {0.0f, 0.0f, 0.0f, 0.0f};
+          }
+        }
+      }
+    }
+    __syncthreads();
+    constexpr int kMine = kHalf * kPerIndex * 64 / E::kThreads;   // 16-byte pieces per thread
+#pragma unroll 8
+    for (int it = 0; it < kMine; ++it) {
+      const int s_row = it * 4 + wave;
+      const int out_row = row0 + E::token_of_index(kHalf * half + s_row / kPerIndex,
+                                                   s_row % kPerIndex);
+      const f32x4_t val =
+          *reinterpret_cast<const f32x4_t*>(smem + s_row * 1024 + ((lane ^ (s_row & 63)) * 16));
+      if (out_row < p.c_rows && col_ok)
+        store4<T>(static_cast<T*>(p.c) + (int64_t)out_row * p.ldc + col, val[0], val[1], val[2],
+                  val[3]);
+    }
+  }
+}
+
+template <class E, bool kAKMajor, bool kBKMajor, bool kLabels = false>
 __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_kernel(GemmArgs p) {
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
@@ -1495,6 +1633,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
       p.k_per_split = ((p.k + E::kBK - 1) / E::kBK + n_splits - 1) / n_splits * E::kBK;
     } else if (p.m_role == kKFollows) {
       const int rows = effective_block_rows(p.k, p.m_dev, p.m_dev_offset);
+      if (kLabels) p.n_rows = effective_block_rows(p.n_rows, p.m_dev, p.m_dev_offset);
       p.k = (rows + p.m_round - 1) / p.m_round * p.m_round;
       // nothing to add to an accumulator that already holds earlier blocks of rows
       if (p.k == 0 && p.mode == kAddF32) return;
@@ -1531,6 +1670,8 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
   p.c = static_cast<char*>(p.c) +
         (int64_t)split * p.c_split_stride * (p.mode == kStoreT ? sizeof(T) : sizeof(float));
 
+  // (visible to every wave after the barriers of the main loop or of the store)
+  if constexpr (kLabels) find_label_rows<E>(p, tj * E::kTile, smem + E::kSmemBytes);
   E eng;
   typename E::Acc acc;
   if (k_begin >= k_end) {
@@ -1552,7 +1693,9 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
     // and its outputs (workspace slabs, rows of grad_weight) are 16-byte aligned:
     // whole output rows leave through LDS (the main loop has ended on a barrier).
     const int row0 = tj * E::kTile, col0 = ti * E::kTile;
-    if (p.mode == kStoreT) {
+    if constexpr (kLabels) {
+      store_tile_t_with_labels<E>(eng, acc, smem, smem + E::kSmemBytes, p, row0, col0);
+    } else if (p.mode == kStoreT) {
       store_tile_t_by_rows<E>(eng, acc, smem, static_cast<T*>(p.c), p.ldc, row0, col0, p.c_rows,
                               p.c_cols);
     } else if (p.mode == kStoreF32) {

@@ -1008,6 +1008,11 @@ extern "C" int tlce_frozen_gradients_supported(int64_t m, int64_t h, int64_t v, 
   return (m >= 0 && h > 0 && v > 0 && frozen_gradients_supported(m, h, v, dtype)) ? 1 : 0;
 }
 
+extern "C" int tlce_weight_grad_can_wait(int64_t m, int64_t h, int64_t v, int dtype,
+                                         int64_t panel_bytes) {
+  return (m >= 0 && h > 0 && v > 0 && weight_grad_can_wait(m, h, v, dtype, panel_bytes)) ? 1 : 0;
+}
+
 extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
                                      int64_t panel_bytes, int64_t* block_rows, int* n_blocks,
                                      int* grad_hidden_k_splits) {
@@ -1025,8 +1030,9 @@ extern "C" int64_t tlce_forward_with_gradients_workspace_bytes(int64_t m, int64_
                                                                int dtype, int compute_weight_grad,
                                                                int64_t panel_bytes) {
   if (m < 0 || h <= 0 || v <= 0) return -1;
-  if (compute_weight_grad != 0 ? !fused_gradients_supported(h, v, dtype)
-                               : !frozen_gradients_supported(m, h, v, dtype))
+  if (!frozen_gradients_supported(m, h, v, dtype) ||
+      (compute_weight_grad != 0 && !fused_gradients_supported(h, v, dtype) &&
+       !weight_grad_can_wait(m, h, v, dtype, panel_bytes)))
     return -1;
   return fused_layout(make_fused_plan(m, h, v, dtype, panel_bytes), m, h, dtype,
                       compute_weight_grad != 0).total;
@@ -1219,13 +1225,13 @@ extern "C" int tlce_finish_gradients(const float* grad_hidden_f32, const float* 
                                      const float* grad_output, const float* valid_count, int64_t m,
                                      int64_t n_out, int64_t h, int64_t v, int reduction_code,
                                      void* grad_hidden, void* grad_weight, const void* hidden,
-                                     int64_t panel_bytes, void* forward_workspace,
+                                     const int64_t* labels, int64_t panel_bytes, void* forward_workspace,
                                      int64_t workspace_bytes, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   TLCE_REQUIRE(m >= 0 && h > 0 && v > 0 &&
-                   (grad_weight != nullptr ? fused_gradients_supported(h, v, TLCE_DTYPE_BF16)
-                                           : (h % 64) == 0),
-               "finish_gradients: needs h, and with grad_weight v, multiples of 64");
+                   (grad_weight == nullptr || (hidden != nullptr && labels != nullptr)
+                        ? (h % 64) == 0 : fused_gradients_supported(h, v, TLCE_DTYPE_BF16)),
+               "finish_gradients: needs h, and for grad_weight without labels v, multiples of 64");
   TLCE_REQUIRE(reduction_code >= TLCE_REDUCTION_NONE && reduction_code <= TLCE_REDUCTION_MEAN,
                "finish_gradients: unknown reduction code %d", reduction_code);
   if (m == 0) {
@@ -1282,9 +1288,10 @@ extern "C" int tlce_finish_gradients(const float* grad_hidden_f32, const float* 
   char* ws = static_cast<char*>(forward_workspace);
   fa.hidden = hidden; fa.row_scale = reinterpret_cast<const float*>(ws + l.row_scale);
   fa.scaled = ws + l.scaled_hidden;
+  if (v % 64 != 0) fa.row_factor = reinterpret_cast<float*>(ws + l.row_factor);
   if (int rc = launch_finish_rows(fa, stream)) return rc;
   return deferred_contraction<MfmaDirect4Engine<__bf16>>(p, l, m, h, v, row_count, grad_weight, ws,
-                                                         stream);
+                                                         stream, hidden, labels);
 }
 
 // ------------------------------------- the same pair for float32 in planes ----

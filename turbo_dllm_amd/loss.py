@@ -95,7 +95,7 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
                 rows = rows_copy
             ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                                   row_count if mode == "device" else None,
-                                  rows if ctx.postponed else None)
+                                  *((rows, targets[:m]) if ctx.postponed else (None, None)))
             ctx.panel_bytes = native.get_panel_bytes()
             ctx.hidden_shape = hidden.shape
             ctx.n_rows, ctx.m = n, m
@@ -141,7 +141,8 @@ def _gradients_of_weighted_sum(ctx, grad_output):
     """Gradients of a weighted loss sum whose forward left them."""
     from . import chunked_linear_ce_native as native
 
-    grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows = ctx.saved_tensors
+    grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows, targets = (
+        ctx.saved_tensors)
     if ctx.grad_dtype == torch.float32:
         return native.apply_grad_output_f32(
             grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum",
@@ -150,7 +151,7 @@ def _gradients_of_weighted_sum(ctx, grad_output):
     return native.finish_gradients(
         grad_rows32, grad_weight32, grad_output, valid_count, reduction="sum", n_out=ctx.n_rows,
         vocab=ctx.vocab, row_of=row_of, row_count=row_count, rows=rows,
-        panel_bytes=ctx.panel_bytes,
+        panel_bytes=ctx.panel_bytes, labels=targets,
     )
 
 
@@ -180,7 +181,7 @@ class _FusedSampleLoss(torch.autograd.Function):
                 n_out=hidden.shape[0],
             ))
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx[:m], row_of, None,
-                              rows if wait else None)
+                              *((rows, targets[:m]) if wait else (None, None)))
         ctx.panel_bytes = native.get_panel_bytes()   # the backward may run on another thread
         ctx.n_rows = hidden.shape[0]
         ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]

@@ -317,7 +317,7 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
             rows = rows_copy
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                               row_count if mode == "device" else None,
-                              rows if ctx.postponed else None)
+                              *((rows, targets) if ctx.postponed else (None, None)))
         ctx.panel_bytes = native.get_panel_bytes()
         ctx.hidden_shape = hidden.shape
         ctx.n_rows, ctx.m = n, m
@@ -362,7 +362,7 @@ def _device_backward(ctx, grad_output, frozen: bool):
     from . import chunked_linear_ce_native as native
 
     if ctx.fused:
-        grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows = (
+        grad_rows32, grad_weight32, valid_count, row_idx, row_of, row_count, rows, targets = (
             ctx.saved_tensors)
         if ctx.grad_dtype == torch.float32:
             grad_hidden, grad_weight = native.apply_grad_output_f32(
@@ -375,7 +375,7 @@ def _device_backward(ctx, grad_output, frozen: bool):
             grad_hidden, grad_weight = native.finish_gradients(
                 grad_rows32, grad_weight32, grad_output, valid_count, reduction=ctx.reduction,
                 n_out=ctx.n_rows, vocab=ctx.vocab, row_of=row_of, row_count=row_count, rows=rows,
-                panel_bytes=ctx.panel_bytes,
+                panel_bytes=ctx.panel_bytes, labels=targets,
             )
         return (grad_hidden.reshape(ctx.hidden_shape), None if frozen else grad_weight,
                 None) + (None,) * 9
