@@ -193,6 +193,21 @@ def test_a_word_with_more_rows_than_are_kept(gpu_device):
     assert off(grads[0][others], want[others]) < ONE_ROUNDING
 
 
+@pytest.mark.gpu
+def test_labels_of_whole_slabs_may_change_before_the_backward(gpu_device):
+    hidden, weight, labels, _ = operands(gpu_device, 700, 256, 3008)
+    grads = []
+    for change in (False, True):
+        y = labels.clone()
+        x, w = hidden.clone().requires_grad_(), weight.clone().requires_grad_()
+        loss = tiled_linear_cross_entropy(x, w, y, reduction="mean", dtype=torch.bfloat16)
+        if change:
+            y.fill_(-100)
+        loss.backward()
+        grads.append((x.grad, w.grad))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
+
+
 def test_where_the_path_is_taken():
     lib = _lib.library()
     taken = lib.tlce_frozen_gradients_supported

@@ -835,6 +835,13 @@ def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
         m, h, v, _lib.DTYPE_BF16, get_panel_bytes()))
 
 
+def labels_for_backward(labels: torch.Tensor, weight: torch.Tensor,
+                        postponed: bool) -> torch.Tensor | None:
+    """The labels where ``finish_gradients`` reads them again; elsewhere the caller may change
+    them between forward and backward."""
+    return labels if postponed and weight.shape[0] % 64 != 0 else None
+
+
 def _upstream_gradient(grad_output: torch.Tensor, reduction_code: int, n_out: int) -> torch.Tensor:
     """The upstream gradient as the library reads it: float32, one element for a
     scalar reduction, one per output row for reduction "none"."""

@@ -95,7 +95,8 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
                 rows = rows_copy
             ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                                   row_count if mode == "device" else None,
-                                  *((rows, targets[:m]) if ctx.postponed else (None, None)))
+                                  rows if ctx.postponed else None,
+                                  native.labels_for_backward(targets[:m], weight, ctx.postponed))
             ctx.panel_bytes = native.get_panel_bytes()
             ctx.hidden_shape = hidden.shape
             ctx.n_rows, ctx.m = n, m
@@ -181,7 +182,8 @@ class _FusedSampleLoss(torch.autograd.Function):
                 n_out=hidden.shape[0],
             ))
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx[:m], row_of, None,
-                              *((rows, targets[:m]) if wait else (None, None)))
+                              rows if wait else None,
+                              native.labels_for_backward(targets[:m], weight, wait))
         ctx.panel_bytes = native.get_panel_bytes()   # the backward may run on another thread
         ctx.n_rows = hidden.shape[0]
         ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]

@@ -317,7 +317,8 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
             rows = rows_copy
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                               row_count if mode == "device" else None,
-                              *((rows, targets) if ctx.postponed else (None, None)))
+                              rows if ctx.postponed else None,
+                              native.labels_for_backward(targets, weight_vf, ctx.postponed))
         ctx.panel_bytes = native.get_panel_bytes()
         ctx.hidden_shape = hidden.shape
         ctx.n_rows, ctx.m = n, m
