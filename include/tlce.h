@@ -294,6 +294,39 @@ int tlce_masked_loss_backward(const void* hidden, const void* weight, const floa
                               int64_t panel_bytes,
                               void* workspace, int64_t workspace_bytes, void* stream);
 
+/* ---- products kept for the backward --------------------------------------
+ * tlce_masked_loss_forward / _backward (and, with weight_dim_first, the [h, v] head's) whose
+ * forward leaves hidden . weight^T in float32 for the first tiles of the vocabulary, so that the
+ * backward forms their logit gradients without contracting them again: the same gradients, bit
+ * for bit.  16-bit operands on the direct engine, no bias.
+ *   tlce_kept_logits_bytes: the size `kept` should have within `budget` bytes (0: these operands
+ *     keep none, -1: bad shape); whole tiles of 256 x 256, 4 m v bytes and the edges' padding for
+ *     all of them.  Both calls must be given the same m, h, v, dtype, kept and kept_bytes. */
+int64_t tlce_kept_logits_bytes(int64_t m, int64_t h, int64_t v, int dtype, int has_bias,
+                               int64_t budget);
+
+int tlce_forward_keeping_logits(const void* hidden, const void* weight, const int64_t* labels,
+                                const float* token_weights, const int64_t* row_idx,
+                                const int64_t* row_count, int64_t m, int64_t n_out, int64_t h,
+                                int64_t v, int dtype, int64_t ignore_index,
+                                int64_t exclude_index, float logit_softcap,
+                                float logit_multiplier, int weight_dim_first, float* losses,
+                                float* lse, float* valid_count, float* weighted_sum, void* kept,
+                                int64_t kept_bytes, void* workspace, int64_t workspace_bytes,
+                                void* stream);
+
+int tlce_backward_from_kept_logits(const void* hidden, const void* weight, const int64_t* labels,
+                                   const float* token_weights, const int64_t* row_idx,
+                                   const int64_t* row_count, const float* lse,
+                                   const float* valid_count, const float* grad_output, int64_t m,
+                                   int64_t n_out, int64_t h, int64_t v, int dtype,
+                                   int reduction_code, int64_t ignore_index,
+                                   int64_t exclude_index, float logit_softcap,
+                                   float logit_multiplier, int weight_dim_first,
+                                   void* grad_hidden, void* grad_weight, const void* kept,
+                                   int64_t kept_bytes, int64_t panel_bytes, void* workspace,
+                                   int64_t workspace_bytes, void* stream);
+
 /* ---- vocabulary shards ---------------------------------------------------
  * Replace vocab_parallel_ce_forward_local / vocab_parallel_ce_backward_local
  * (fused_linear_ce.cpp:209-265; fused_vocab_parallel_ce_forward_cuda and

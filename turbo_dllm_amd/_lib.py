@@ -220,6 +220,29 @@ SIGNATURES = {
             c_void_p, c_int64, c_void_p,                        # workspace bytes stream
         ],
     ),
+    "tlce_kept_logits_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int, c_int, c_int64]),
+    "tlce_forward_keeping_logits": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_void_p, c_void_p,             # hidden weight labels token_weights
+            c_void_p, c_void_p,                                 # row_idx row_count
+            c_int64, c_int64, c_int64, c_int64, c_int,          # m n_out h v dtype
+            c_int64, c_int64, c_float, c_float, c_int,          # ignore exclude softcap multiplier dim_first
+            c_void_p, c_void_p, c_void_p, c_void_p,             # losses lse valid_count weighted_sum
+            c_void_p, c_int64, c_void_p, c_int64, c_void_p,     # kept bytes workspace bytes stream
+        ],
+    ),
+    "tlce_backward_from_kept_logits": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_void_p, c_void_p,             # hidden weight labels token_weights
+            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,   # row_idx row_count lse valid_count grad_output
+            c_int64, c_int64, c_int64, c_int64, c_int,          # m n_out h v dtype
+            c_int, c_int64, c_int64, c_float, c_float, c_int,   # reduction ignore exclude softcap multiplier dim_first
+            c_void_p, c_void_p, c_void_p, c_int64,              # grad_hidden grad_weight kept bytes
+            c_int64, c_void_p, c_int64, c_void_p,               # panel_bytes workspace bytes stream
+        ],
+    ),
     "tlce_masked_loss_backward": (
         c_int,
         [

@@ -20,7 +20,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _lib, options
 
 _DTYPE_CODES = {
     torch.float32: _lib.DTYPE_F32,
@@ -1055,6 +1055,44 @@ def backward_frozen_weight(
     )
 
 
+# ------------------------------------------------- logits kept for the backward --
+# Held between forward and backward without asking how much memory there is: the recomputing
+# backward's own default panel.  Beyond that an eighth of what is free, so that what the backward
+# allocates next finds room, and a twenty-fourth of the device (12 GiB of 288).  Which tiles are
+# kept changes no result, so the answer may differ from call to call.
+_KEEP_UNASKED_BYTES = 1 << 30
+
+
+def kept_logits_buffer(m: int, hidden: torch.Tensor, vocab: int,
+                       bias: torch.Tensor | None) -> torch.Tensor | None:
+    """Where the forward of a recomputing cross entropy over ``m`` rows leaves its logits for
+    the backward (``masked_loss_forward(kept=...)``), or None when it is to recompute all of
+    them: operands or sizes that gain nothing, the gradient mode "recompute", a call that is
+    being captured, whose graph would hold the buffer.  A panel budget bounds it as well."""
+    if m == 0 or options.get_gradient_mode() != "forward" or hidden.dtype not in _DTYPE_CODES:
+        return None
+    lib = _lib.library()
+    h, code, has_bias = hidden.shape[1], _dtype_code(hidden), int(bias is not None)
+    budget = get_panel_bytes() or (1 << 62)
+    nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, budget)
+    if nbytes <= 0 or torch.cuda.is_current_stream_capturing():
+        return None
+    device = hidden.device
+    if nbytes > _KEEP_UNASKED_BYTES:
+        free, total = torch.cuda.mem_get_info(device)
+        stats = torch.cuda.memory_stats_as_nested_dict(device)
+        cached = (stats["reserved_bytes"]["all"]["current"]
+                  - stats["allocated_bytes"]["all"]["current"]) if stats else 0
+        room = max(min((free + cached) // 8, total // 24), _KEEP_UNASKED_BYTES)
+        nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, min(nbytes, room))
+        if nbytes <= 0:
+            return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 # ---------------------------------------------------------- masked-token loss --
 def masked_loss_forward(
     hidden: torch.Tensor,
@@ -1073,6 +1111,8 @@ def masked_loss_forward(
     logit_multiplier: float = 1.0,
     want_losses: bool = True,
     want_sum: bool = True,
+    kept: torch.Tensor | None = None,
+    weight_dim_first: bool = False,
 ) -> tuple[torch.Tensor | None, torch.Tensor, torch.Tensor, torch.Tensor | None]:
     """The forward with the loss method's arithmetic folded in
     (distributed_block_diffusion_loss, nemotron/model.py:2084-2151): logits
@@ -1085,10 +1125,16 @@ def masked_loss_forward(
     ``hidden`` must then hold ``round_up(m, 64)`` rows (``gather_loss_rows``
     provides them).  Returns ``(losses [n_out] | None, lse [m], valid_count [1],
     weighted_sum [1] | None)``, all float32.
+
+    ``kept`` (``kept_logits_buffer``; no bias): receives the logits of the first vocabulary
+    tiles, for a ``masked_loss_backward`` with the same buffer.  ``weight_dim_first`` (with
+    ``kept``): ``weight`` is a [D, V] head that is read in place (``dim_first_in_place``).
     """
-    device = _require_device(hidden, weight, bias, labels, token_weights, row_idx, row_count)
-    if hidden.dim() != 2 or weight.dim() != 2 or weight.shape[1] != hidden.shape[1]:
+    device = _require_device(hidden, weight, bias, labels, token_weights, row_idx, row_count, kept)
+    if (hidden.dim() != 2 or weight.dim() != 2
+            or weight.shape[0 if weight_dim_first else 1] != hidden.shape[1]):
         raise RuntimeError("masked loss expects hidden [N, D] and weight [V, D]")
+    _check_kept(kept, bias, weight_dim_first)
     if weight.dtype != hidden.dtype:
         raise RuntimeError("native linear CE expects hidden and weight of one dtype")
     if not (want_losses or want_sum):
@@ -1097,7 +1143,7 @@ def masked_loss_forward(
     weight = _dense(weight)
     labels = labels.reshape(-1).to(torch.long).contiguous()
     h = hidden.shape[1]
-    v = weight.shape[0]
+    v = weight.shape[1 if weight_dim_first else 0]
     m = hidden.shape[0] if m is None else int(m)
     need_rows = (m + 63) // 64 * 64 if row_count is not None else m
     if hidden.shape[0] < need_rows or labels.numel() < m:
@@ -1119,6 +1165,19 @@ def masked_loss_forward(
             lib.tlce_masked_loss_forward_workspace_bytes(m, h, v, code, int(row_count is not None)),
             device,
         )
+        if kept is not None:
+            _lib.check(
+                lib.tlce_forward_keeping_logits(
+                    _ptr(hidden), _ptr(weight), _ptr(labels), _ptr(token_weights),
+                    _ptr(row_idx), _ptr(row_count), m, n_out, h, v, code,
+                    int(ignore_index), int(exclude_index), float(logit_softcap),
+                    float(logit_multiplier), int(weight_dim_first),
+                    _ptr(losses), _ptr(lse), valid_count.data_ptr(), _ptr(weighted_sum),
+                    kept.data_ptr(), kept.numel(), ws.data_ptr(), ws.numel(), _stream(device),
+                ),
+                "tlce_forward_keeping_logits",
+            )
+            return losses, lse, valid_count, weighted_sum
         _lib.check(
             lib.tlce_masked_loss_forward(
                 _ptr(hidden), _ptr(weight), _ptr(bias32), _ptr(labels), _ptr(token_weights),
@@ -1131,6 +1190,14 @@ def masked_loss_forward(
             "tlce_masked_loss_forward",
         )
     return losses, lse, valid_count, weighted_sum
+
+
+def _check_kept(kept, bias, weight_dim_first):
+    if kept is None:
+        if weight_dim_first:
+            raise RuntimeError("masked loss reads a [D, V] head only with kept logits")
+    elif bias is not None or kept.dtype != torch.uint8 or not kept.is_contiguous():
+        raise RuntimeError("kept logits: a buffer of kept_logits_buffer, and no bias")
 
 
 def masked_loss_backward(
@@ -1153,25 +1220,30 @@ def masked_loss_backward(
     logit_softcap: float,
     logit_multiplier: float = 1.0,
     compute_weight_grad: bool = True,
+    kept: torch.Tensor | None = None,
+    weight_dim_first: bool = False,
 ) -> tuple[torch.Tensor, torch.Tensor | None, torch.Tensor | None]:
-    """Gradients of ``masked_loss_forward``.  ``reduction="sum"`` with
+    """Gradients of ``masked_loss_forward`` (with the same ``kept`` and ``weight_dim_first``;
+    grad_weight is then in the head's layout).  ``reduction="sum"`` with
     ``grad_output`` [1] is the gradient of ``weighted_sum``; "none" / "mean" take
     the gradient of the per-token losses / of their mean, as ``backward`` does,
     with ``token_weights`` applied on top.  Returns ``(grad_hidden [n_out, H],
     grad_weight | None, grad_bias | None)`` in the input dtypes."""
     device = _require_device(hidden, weight, bias, labels, token_weights, lse, valid_count,
-                             grad_output, row_idx, row_count)
+                             grad_output, row_idx, row_count, kept)
+    _check_kept(kept, bias, weight_dim_first)
     hidden = _dense(hidden)
     weight = _dense(weight)
     labels = labels.reshape(-1).to(torch.long).contiguous()
     h = hidden.shape[1]
-    v = weight.shape[0]
+    v = weight.shape[1 if weight_dim_first else 0]
     m = hidden.shape[0] if m is None else int(m)
     # the C ABI cannot see tensor lengths: the same row checks as the forward
     need_rows = (m + 63) // 64 * 64 if row_count is not None else m
     if hidden.shape[0] < need_rows or labels.numel() < m or lse.numel() < m:
         raise RuntimeError("masked loss: hidden / labels / lse hold fewer rows than m")
-    if weight.dim() != 2 or weight.shape[1] != h or weight.dtype != hidden.dtype:
+    if (weight.dim() != 2 or weight.shape[0 if weight_dim_first else 1] != h
+            or weight.dtype != hidden.dtype):
         raise RuntimeError("masked loss expects weight [V, D] in the dtype of hidden")
     n_out = m if n_out is None else int(n_out)
     code = _dtype_code(hidden)
@@ -1190,7 +1262,8 @@ def masked_loss_backward(
     with torch.cuda.device(device):
         grad_hidden = torch.empty((n_out, h), dtype=hidden.dtype, device=device)
         grad_weight = (
-            torch.empty((v, h), dtype=weight.dtype, device=device) if compute_weight_grad else None
+            torch.empty(weight.shape, dtype=weight.dtype, device=device)
+            if compute_weight_grad else None
         )
         grad_bias32 = (
             torch.empty(v, dtype=torch.float32, device=device) if bias is not None else None
@@ -1201,6 +1274,20 @@ def masked_loss_backward(
             ),
             device,
         )
+        if kept is not None:
+            _lib.check(
+                lib.tlce_backward_from_kept_logits(
+                    _ptr(hidden), _ptr(weight), _ptr(labels), _ptr(token_weights),
+                    _ptr(row_idx), _ptr(row_count), _ptr(lse), _ptr(valid_count),
+                    _ptr(grad_output), m, n_out, h, v, code, reduction_code,
+                    int(ignore_index), int(exclude_index), float(logit_softcap),
+                    float(logit_multiplier), int(weight_dim_first),
+                    _ptr(grad_hidden), _ptr(grad_weight), kept.data_ptr(), kept.numel(),
+                    get_panel_bytes(), ws.data_ptr(), ws.numel(), _stream(device),
+                ),
+                "tlce_backward_from_kept_logits",
+            )
+            return grad_hidden, grad_weight, None
         _lib.check(
             lib.tlce_masked_loss_backward(
                 _ptr(hidden), _ptr(weight), _ptr(bias32), _ptr(labels), _ptr(token_weights),

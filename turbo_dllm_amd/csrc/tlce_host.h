@@ -195,12 +195,42 @@ struct RowOptions {
   // the head and its gradient are stored [h, v] (weight_dim_first of the reference's
   // extension, fused_linear_ce.cpp:104,121) and are read / written in place
   bool weight_dim_first = false;
+  KeptLogits kept;                        // written by the forward, read by the backward
 };
 
 // A [h, v] head is taken in place by the engine with K-major operand loaders, for
 // vocabularies made of whole 64-row K slabs.
 inline bool dim_first_in_place(int64_t h, int64_t v, int dtype) {
   return engine_class(h, dtype) == 2 && (v % 64) == 0;
+}
+
+// How many of the first vocabulary tiles' products a recomputing cross entropy's forward keeps
+// for its backward within `budget` bytes (0: none).  A kept logit costs 4 bytes written beside
+// the statistics, which passes under the contraction, and 4 read in the place of 2 h operations.
+// Forward and backward with a trainable head in us, recomputed / kept, bf16:
+//   8192 rows, H =  768, V =  65537   3033 /  3275      1000, H =  768, V =  50001    438 /  419
+//   8192 rows, H = 1024, V = 151937   8243 /  8116      2741, H = 1024, V =  32003    708 /  678
+//   4096 rows, H = 1280, V =  50001   1731 /  1592      8192, H = 1536, V = 151937  11669 / 10744
+//   2741 rows, H = 2048, V =  32003   1288 /  1130       500, H = 2048, V =  32003    366 /  327
+//    300 rows, H = 3072, V =  65537    864 /   691      4096, H = 4096, V = 151937  14407 / 11856
+//   4096 rows, H = 2040, V =  65536   3581 /  3058      16384, H = 4096, V = 151936 55836 / 45655
+constexpr int64_t kKeptTileBytes = (int64_t)kKeptTileFloats * 4;
+constexpr int64_t kKeepMinHidden = 1024;
+inline int64_t kept_vocab_tiles(int64_t m, int64_t h, int64_t v, int dtype, bool bias,
+                                int64_t budget) {
+  if (m <= 0 || bias || dtype == TLCE_DTYPE_F32 || h < kKeepMinHidden) return 0;
+  const Plan p = make_plan(m, h, v, dtype, false, 0, 3, kBackwardTails);
+  const Plan f = make_plan(m, h, v, dtype, false, 0, 3, kForwardTails);
+  if (p.engine != 2 || f.engine != 2) return 0;
+  return std::max<int64_t>(0, std::min<int64_t>(p.n_vtiles, budget / (kKeptTileBytes * p.n_ttiles)));
+}
+inline KeptLogits kept_logits(const Plan& p, void* tiles, int64_t bytes) {
+  KeptLogits k;
+  k.tiles = static_cast<float*>(tiles);
+  k.t_tiles = p.n_ttiles;
+  if (tiles != nullptr && p.n_ttiles > 0)
+    k.v_tiles = (int)std::min<int64_t>(p.n_vtiles, bytes / (kKeptTileBytes * p.n_ttiles));
+  return k;
 }
 
 // Bytes of what launch_column_tails writes: the copy of weight's last columns [vp, 64], then
@@ -367,6 +397,18 @@ int launch_grad_logits_dim_first(const GradLogitsArgs& a, hipStream_t stream) {
   }
 }
 
+template <typename T>
+int launch_grad_from_kept(const GradLogitsArgs& a, const KeptLogits& kept, hipStream_t stream) {
+  const int64_t grid = (int64_t)kept.t_tiles * a.n_ptiles * 4;   // quarters of tiles
+  ScopedTimer timer(kClassGradLogits, stream);
+  if (a.softcap > 0.0f)
+    lce_grad_from_kept_kernel<T, true><<<(int)grid, 256, 0, stream>>>(a, kept);
+  else
+    lce_grad_from_kept_kernel<T, false><<<(int)grid, 256, 0, stream>>>(a, kept);
+  TLCE_LAUNCH_CHECK();
+  return 0;
+}
+
 template <class E>
 int launch_grad_logits(const GradLogitsArgs& a, hipStream_t stream) {
   const bool softcap = a.softcap > 0.0f, bias = a.bias != nullptr;
@@ -479,6 +521,7 @@ int forward_impl(const Plan& p, const void* hidden, const void* weight, const fl
   fa.part_max = reinterpret_cast<float*>(ws + l.part_max);
   fa.part_sum = reinterpret_cast<float*>(ws + l.part_sum);
   fa.part_ld = (int)p.mp;
+  fa.kept = opt.kept;
   if (opt.weight_dim_first) {
     if (int rc = launch_forward_dim_first<E>(p, fa, stream)) return rc;
   } else {
@@ -662,6 +705,7 @@ int backward_impl(const Plan& p, const void* hidden, const void* weight, const f
                   float softcap, int64_t vocab_start, void* grad_hidden, void* grad_weight,
                   float* grad_bias, char* ws, hipStream_t stream,
                   float probabilities_scale, const RowOptions& opt) {
+  using T = typename E::T;
   const BackwardLayout l = backward_layout(p, m, h, dtype, grad_weight != nullptr);
   float* scale = reinterpret_cast<float*>(ws + l.scale);
   ScaleArgs sa;
@@ -697,6 +741,18 @@ int backward_impl(const Plan& p, const void* hidden, const void* weight, const f
     ga.n_ttiles = p.n_ttiles; ga.n_ptiles = (int)(width / p.tile);
     ga.g = g; ga.ldg = p.vc; ga.gt = gt; ga.ldgt = p.mp;
     ga.grad_bias = (bias != nullptr) ? grad_bias : nullptr;
+    if constexpr (kKeepsLogits<E>) {
+      const int kept = (int)std::min<int64_t>(ga.n_ptiles, opt.kept.v_tiles - v0 / p.tile);
+      if (kept > 0) {   // the panel's first tiles
+        GradLogitsArgs ka = ga;
+        ka.n_ptiles = kept;
+        if (int rc = launch_grad_from_kept<T>(ka, opt.kept, stream)) return rc;
+        if (kept == ga.n_ptiles) return 0;
+        ga.v0 += kept * p.tile;
+        ga.n_ptiles -= kept;
+        ga.g = static_cast<T*>(ga.g) + kept * p.tile;
+      }
+    }
     if (opt.weight_dim_first) return launch_grad_logits_dim_first<E>(ga, stream);
     using Tail = typename ColumnTailOf<E>::type;
     return p.column_tail != 0 ? launch_grad_logits<Tail>(ga, stream)

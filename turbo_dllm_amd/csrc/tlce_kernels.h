@@ -22,6 +22,39 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 // (fused_linear_ce_cuda.cu:156-224): bias add, tanh soft cap, excluded column
 // skipped, but as an online single pass instead of two passes over stored
 // logits.
+// Raw products hidden . weight^T that a forward leaves for its backward, so that the tiles need
+// no second contraction: float32, as they came out of the accumulators and in their order, so
+// that every wave instruction moves 1 KiB without a gap (a tile takes kKeptTileFloats floats,
+// whole ones at the edges too): [vocabulary tile < v_tiles][token tile < t_tiles][owned column
+// index][block of 16 rows][thread] of 16 bytes each.
+struct KeptLogits {
+  float* tiles = nullptr;
+  int v_tiles = 0;      // vocabulary tiles that are kept, the first of them
+  int t_tiles = 0;      // token tiles of the call
+};
+constexpr int kKeptTileFloats = 256 * 256;
+
+// The engines whose accumulators the kept layout is: 16-bit operands, direct to LDS.
+template <class E>
+constexpr bool kKeepsLogits = E::kHasKMajor && sizeof(typename E::T) == 2 && E::kPlanes == 1;
+
+template <class E>
+__device__ __forceinline__ void keep_logits(const typename E::Acc& acc, const KeptLogits& kept,
+                                            int vt, int tt) {
+  float* dst = kept.tiles + ((int64_t)vt * kept.t_tiles + tt) * kKeptTileFloats + threadIdx.x * 4;
+#pragma unroll
+  for (int j = 0; j < E::kCols; ++j) {
+#pragma unroll
+    for (int i = 0; i < E::kRows; i += 4) {
+      const f32x4_t quad = {E::read(acc, j, i), E::read(acc, j, i + 1), E::read(acc, j, i + 2),
+                            E::read(acc, j, i + 3)};
+      __builtin_nontemporal_store(
+          quad, reinterpret_cast<f32x4_t*>(dst + (j * (E::kRows / 4) + i / 4) * E::kThreads * 4));
+    }
+    __builtin_amdgcn_sched_barrier(0);   // (all 256 accumulators are not read at once)
+  }
+}
+
 struct ForwardArgs {
   const void* hidden;   // [m, h]
   const void* weight;   // [v, h], or [h, v] for the kernels instantiated with kWDimFirst
@@ -39,6 +72,7 @@ struct ForwardArgs {
   // capacity; token tiles, vocabulary splits and part_ld follow the real count
   // exactly as the host plan would have set them for it.
   const int64_t* m_dev = nullptr;
+  KeptLogits kept;      // where the first vocabulary tiles' products stay for the backward
 };
 
 // The contraction of a logits^T tile.  Column tails: `weight_tail` and `hidden` are the
@@ -107,6 +141,9 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_forward_sta
       eng.template mainloop_ex<true, false>(a, b, 0, p.h, acc, smem);
     } else {
       logits_mainloop(eng, p, vt * E::kTile, tt * E::kTile, acc, smem);
+    }
+    if constexpr (kKeepsLogits<E>) {
+      if (vt < p.kept.v_tiles) keep_logits<E>(acc, p.kept, vt, tt);
     }
     const int vbase = vt * E::kTile;
     // Only the last vocabulary tile (rows past v) and the tile that holds the
@@ -469,6 +506,30 @@ __device__ __forceinline__ void split_planes(float x, float (&part)[3]) {
   part[2] = (x - part[0]) - part[1];
 }
 
+// One raw logit -> its entry of the logit gradient (or, without `label` and cap_grad, of the
+// softmax).  inv_cap and log2e_scaled carry the logit multiplier.
+template <bool kPrecise, bool kSoftcap>
+struct LogitGradient {
+  float inv_cap, softcap, log2e_scaled;
+  bool cap_grad;
+  __device__ __forceinline__ float operator()(float z, float lse2, bool label, float scale) const {
+    float dcap = 1.0f;
+    float g;
+    if (kSoftcap) {
+      const float t = tanh_of<kPrecise>(z * inv_cap);
+      z = softcap * t;
+      dcap = 1.0f - t * t;
+      g = exp2_of<kPrecise>(fmaf(z, TLCE_LOG2E, -lse2));
+    } else {
+      g = exp2_of<kPrecise>(fmaf(z, log2e_scaled, -lse2));
+    }
+    if (label) g -= 1.0f;
+    g *= scale;
+    if (kSoftcap && cap_grad) g *= dcap;
+    return g;
+  }
+};
+
 // The bias of the tile's words waits in LDS beyond the engine's stages, is added where a
 // logit is used, and its gradient's row sums meet in a transposing reduction (30 exchanges and
 // two atomics a wave instead of 128 and 32).  Added to all accumulators first, the 256 results
@@ -556,26 +617,15 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
   const bool onehot = __syncthreads_or(label_here ? 1 : 0) != 0;
 
   const int excluded = (int)p.exclude;
+  const LogitGradient<E::kPrecise, kSoftcap> logit_gradient = {inv_cap, p.softcap, log2e_scaled,
+                                                               p.cap_grad != 0};
   // one logit -> its entry of g (kEdge: the tile holds rows past v or the
   // excluded column; kOnehot: some lane of the workgroup owns a label of the tile)
   auto grad_of = [&](float z, int j, int row, bool vok, auto edge_tag, auto onehot_tag) -> float {
     constexpr bool kEdge = decltype(edge_tag)::value;
     constexpr bool kOnehot = decltype(onehot_tag)::value;
-    float dcap = 1.0f;
-    float g;
-    if (kSoftcap) {
-      const float t = tanh_of<E::kPrecise>(z * inv_cap);   // inv_cap includes logit_scale
-      z = p.softcap * t;
-      dcap = 1.0f - t * t;
-      g = exp2_of<E::kPrecise>(fmaf(z, TLCE_LOG2E, -lse2[j]));
-    } else {
-      g = exp2_of<E::kPrecise>(fmaf(z, log2e_scaled, -lse2[j]));
-    }
-    if (kOnehot && row == label_row[j]) g -= 1.0f;
-    g *= scale[j];
-    if (kSoftcap && p.cap_grad) g *= dcap;
-    if (kEdge) g = vok ? g : 0.0f;
-    return g;
+    const float g = logit_gradient(z, lse2[j], kOnehot && row == label_row[j], scale[j]);
+    return kEdge ? (vok ? g : 0.0f) : g;
   };
   auto add_grad_bias = [&](int row, float row_sum) {
     const int v = vbase + row;
@@ -787,6 +837,90 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
           gt_out[(int64_t)(prow + eng.row(i)) * p.ldgt + r] = from_float<T>(E::get(acc, j, i));
       }
     }
+  }
+}
+
+// The panel of logit gradients from kept products instead of a contraction: the same entries,
+// bit for bit.  One workgroup per quarter of a tile (64 tokens, all of its 256 words): 64 KiB in,
+// a transposition through 32 KiB of LDS, 64 rows of 512 bytes out; a CU holds several, so that
+// one's loads pass under another's stores.  Bound by memory: 6 bytes a logit.  In the place of
+// the recomputing panels, a step of 16384 per-token losses of a trainable head, H = 4096,
+// V = 151936, takes 47.0 ms instead of 58.9, of 2741 rows, H = 2048, V = 32003 1.160 instead
+// of 1.339; the statistics' contraction, which writes the products, 15.2 instead of 14.5 and
+// 0.33 instead of 0.31.
+template <typename T, bool kSoftcap>
+__global__ __launch_bounds__(256) void lce_grad_from_kept_kernel(GradLogitsArgs p, KeptLogits kept) {
+  using E = DirectTileLayout<T>;
+  constexpr int kStage = E::kStageCols;
+  constexpr int kParts = E::kCols / kStage;                  // workgroups per tile
+  constexpr int kTokens = kStage * E::kTokensPerIndex;       // 64
+  __shared__ __align__(16) char stage[kTokens * 512];
+  if (p.m_dev != nullptr) {
+    p.m = effective_rows(p.m, p.m_dev);
+    p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
+  }
+  // neighbouring workgroups write neighbouring columns (the same columns of many rows, 64 KiB
+  // apart in the panels of 16384 rows, share a few memory channels: 3.3 ms a step instead of 2.5,
+  // which is 6 TB/s)
+  const int pv = (int)blockIdx.x % p.n_ptiles, part = (int)blockIdx.x / p.n_ptiles;
+  const int tt = part / kParts, j0 = (part % kParts) * kStage;
+  if (tt >= p.n_ttiles) return;
+  const int vbase = p.v0 + pv * E::kTile;
+  const float* src = kept.tiles +
+                     ((int64_t)(vbase / E::kTile) * kept.t_tiles + tt) * kKeptTileFloats +
+                     (int64_t)j0 * (E::kRows / 4) * E::kThreads * 4 + threadIdx.x * 4;
+  f32x4_t z[kStage][E::kRows / 4];
+#pragma unroll
+  for (int jj = 0; jj < kStage; ++jj)
+#pragma unroll
+    for (int q = 0; q < E::kRows / 4; ++q)
+      z[jj][q] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_t*>(
+          src + (jj * (E::kRows / 4) + q) * E::kThreads * 4));
+
+  E eng;
+  const float inv_cap = kSoftcap ? p.logit_scale / p.softcap : 0.0f;
+  const LogitGradient<E::kPrecise, kSoftcap> gradient = {inv_cap, p.softcap,
+                                                         TLCE_LOG2E * p.logit_scale,
+                                                         p.cap_grad != 0};
+  const bool edge = (vbase + E::kTile > p.v) ||
+                    (p.exclude >= vbase && p.exclude < vbase + E::kTile);
+  const int excluded = (int)p.exclude;
+#pragma unroll
+  for (int jj = 0; jj < kStage; ++jj) {
+    const int r = tt * E::kTile + eng.col(j0 + jj);
+    const int rc = min(r, p.m - 1);
+    const int64_t y = p.labels[rc];
+    const bool live = (r < p.m) && y != p.ignore;
+    const int64_t rel = y - p.label_offset - vbase;
+    const int label_row = live && rel >= 0 && rel < E::kTile ? (int)rel : -1;
+    const float lse2 = p.lse[rc] * TLCE_LOG2E;
+    const float scale = live ? p.scale[rc] : 0.0f;
+    const int slot = jj * E::kTokensPerIndex + eng.position_in_index();
+#pragma unroll
+    for (int q = 0; q < E::kRows / 4; ++q) {
+      float g[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = eng.row(q * 4 + u);
+        g[u] = gradient(z[jj][q][u], lse2, row == label_row, scale);
+        if (edge) g[u] = (vbase + row < p.v) && (vbase + row != excluded) ? g[u] : 0.0f;
+      }
+      const int vq = eng.row(q * 4) >> 2;
+      store4<T>(reinterpret_cast<T*>(stage + slot * 512 + (((vq >> 1) ^ (slot & 31)) * 16) +
+                                     (vq & 1) * 8),
+                g[0], g[1], g[2], g[3]);
+    }
+  }
+  __syncthreads();
+  T* out = static_cast<T*>(p.g) + (int64_t)tt * E::kTile * p.ldg + pv * E::kTile;
+#pragma unroll
+  for (int it = 0; it < kTokens * 32 / E::kThreads; ++it) {
+    const int c = it * E::kThreads + threadIdx.x;
+    const int slot = c >> 5, ch = c & 31;
+    const int t = E::token_of_index(j0 + slot / E::kTokensPerIndex, slot % E::kTokensPerIndex);
+    const uint4 val =
+        *reinterpret_cast<const uint4*>(stage + slot * 512 + ((ch ^ (slot & 31)) * 16));
+    stream_store16(out + (int64_t)t * p.ldg + ch * 8, val);
   }
 }
 

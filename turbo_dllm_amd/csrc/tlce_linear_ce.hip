@@ -636,6 +636,74 @@ extern "C" int tlce_masked_loss_backward(const void* hidden, const void* weight,
                         workspace_bytes, static_cast<hipStream_t>(stream), opt);
 }
 
+// ------------------------------------------- products kept for the backward --
+namespace {
+
+int with_kept(RowOptions& opt, void* kept, int64_t kept_bytes, int64_t m, int64_t h, int64_t v,
+              int dtype, const float* bias) {
+  if (kept == nullptr || m == 0) return 0;
+  TLCE_REQUIRE(((uintptr_t)kept & 15) == 0, "kept logits must be 16-byte aligned");
+  TLCE_REQUIRE(kept_bytes > 0 && kept_vocab_tiles(m, h, v, dtype, bias != nullptr, kept_bytes) > 0,
+               "these operands' logits cannot be kept in %lld bytes (tlce_kept_logits_bytes)",
+               (long long)kept_bytes);
+  opt.kept = kept_logits(make_plan(m, h, v, dtype, false, 0, 3, kBackwardTails), kept, kept_bytes);
+  return 0;
+}
+
+}  // namespace
+
+extern "C" int64_t tlce_kept_logits_bytes(int64_t m, int64_t h, int64_t v, int dtype, int has_bias,
+                                          int64_t budget) {
+  if (m < 0 || h <= 0 || v <= 0) return -1;
+  return kept_vocab_tiles(m, h, v, dtype, has_bias != 0, budget) * kKeptTileBytes *
+         ceil_div(std::max<int64_t>(m, 1), 256);
+}
+
+extern "C" int tlce_forward_keeping_logits(
+    const void* hidden, const void* weight, const int64_t* labels, const float* token_weights,
+    const int64_t* row_idx, const int64_t* row_count, int64_t m, int64_t n_out, int64_t h,
+    int64_t v, int dtype, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
+    float logit_multiplier, int weight_dim_first, float* losses, float* lse, float* valid_count,
+    float* weighted_sum, void* kept, int64_t kept_bytes, void* workspace, int64_t workspace_bytes,
+    void* stream) {
+  TLCE_REQUIRE(weighted_sum != nullptr || losses != nullptr || n_out == 0,
+               "forward_keeping_logits: neither weighted_sum nor losses given");
+  RowOptions opt;
+  opt.logit_scale = logit_multiplier;
+  opt.token_weights = token_weights;
+  opt.row_count = row_count;
+  opt.weighted_sum = weighted_sum;
+  opt.weight_dim_first = weight_dim_first != 0;
+  if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
+  if (int rc = with_kept(opt, kept, kept_bytes, m, h, v, dtype, nullptr)) return rc;
+  return forward_entry(hidden, weight, nullptr, labels, row_idx, m, n_out, h, v, dtype,
+                       ignore_index, exclude_index, logit_softcap, losses, lse, valid_count,
+                       ShardStats{}, workspace, workspace_bytes, static_cast<hipStream_t>(stream),
+                       opt);
+}
+
+extern "C" int tlce_backward_from_kept_logits(
+    const void* hidden, const void* weight, const int64_t* labels, const float* token_weights,
+    const int64_t* row_idx, const int64_t* row_count, const float* lse, const float* valid_count,
+    const float* grad_output, int64_t m, int64_t n_out, int64_t h, int64_t v, int dtype,
+    int reduction_code, int64_t ignore_index, int64_t exclude_index, float logit_softcap,
+    float logit_multiplier, int weight_dim_first, void* grad_hidden, void* grad_weight,
+    const void* kept, int64_t kept_bytes, int64_t panel_bytes, void* workspace,
+    int64_t workspace_bytes, void* stream) {
+  RowOptions opt;
+  opt.logit_scale = logit_multiplier;
+  opt.token_weights = token_weights;
+  opt.row_count = row_count;
+  opt.weight_dim_first = weight_dim_first != 0;
+  if (int rc = validate_common(hidden, weight, m, h, v, dtype)) return rc;
+  if (int rc = with_kept(opt, const_cast<void*>(kept), kept_bytes, m, h, v, dtype, nullptr))
+    return rc;
+  return backward_entry(hidden, weight, nullptr, labels, row_idx, lse, valid_count, grad_output, m,
+                        n_out, h, v, dtype, reduction_code, 0, ignore_index, exclude_index,
+                        logit_softcap, grad_hidden, grad_weight, nullptr, panel_bytes, workspace,
+                        workspace_bytes, static_cast<hipStream_t>(stream), opt);
+}
+
 // ---------------------------------------------------------- soft embedding --
 
 extern "C" int64_t tlce_soft_embedding_workspace_bytes(int64_t m, int64_t h, int64_t v, int dtype,

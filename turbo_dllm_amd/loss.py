@@ -101,13 +101,17 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             ctx.n_rows, ctx.m = n, m
             ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]
             return loss
+        kept = None
+        if mode != "device" and (wants_grad or ctx.needs_input_grad[2]):
+            kept = native.kept_logits_buffer(m, rows, weight.shape[0], bias)
         _, lse, _, weighted_sum = native.masked_loss_forward(
             rows, weight, bias, targets, token_weights, m=m, row_idx=row_idx,
             row_count=row_count, n_out=n, ignore_index=-100, exclude_index=exclude_index,
             logit_softcap=logit_softcap, logit_multiplier=multiplier,
-            want_losses=False, want_sum=True,
+            want_losses=False, want_sum=True, kept=kept,
         )
-        ctx.save_for_backward(rows, weight, bias, targets, token_weights, lse, row_idx, row_count)
+        ctx.save_for_backward(rows, weight, bias, targets, token_weights, lse, row_idx, row_count,
+                              kept)
         ctx.hidden_shape = hidden.shape
         ctx.n_rows, ctx.m = n, m
         ctx.multiplier, ctx.exclude_index, ctx.logit_softcap = multiplier, exclude_index, logit_softcap
@@ -121,14 +125,15 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         if ctx.fused:
             grad_hidden, grad_weight = _gradients_of_weighted_sum(ctx, grad_output)
             return (grad_hidden.reshape(ctx.hidden_shape), grad_weight, None) + (None,) * 6
-        rows, weight, bias, targets, token_weights, lse, row_idx, row_count = ctx.saved_tensors
+        rows, weight, bias, targets, token_weights, lse, row_idx, row_count, kept = (
+            ctx.saved_tensors)
         with native.panel_budget(ctx.panel_bytes):
             grad_hidden, grad_weight, grad_bias = native.masked_loss_backward(
                 rows, weight, bias, targets, token_weights, lse, None, grad_output,
                 reduction="sum", m=ctx.m, row_idx=row_idx, row_count=row_count, n_out=ctx.n_rows,
                 ignore_index=-100, exclude_index=ctx.exclude_index,
                 logit_softcap=ctx.logit_softcap, logit_multiplier=ctx.multiplier,
-                compute_weight_grad=ctx.needs_input_grad[1],
+                compute_weight_grad=ctx.needs_input_grad[1], kept=kept,
             )
         return (
             grad_hidden.reshape(ctx.hidden_shape),
@@ -202,12 +207,15 @@ class _FusedTokenLosses(torch.autograd.Function):
         rows = hidden.reshape(-1, hidden.shape[-1]).contiguous()
         targets = labels.reshape(-1).to(torch.long).contiguous()
         weight = weight.contiguous()
+        kept = None
+        if any(ctx.needs_input_grad[:3]):
+            kept = native.kept_logits_buffer(rows.shape[0], rows, weight.shape[0], bias)
         losses, lse, valid_count, _ = native.masked_loss_forward(
             rows, weight, bias, targets, None, ignore_index=-100, exclude_index=-1,
             logit_softcap=logit_softcap, logit_multiplier=multiplier,
-            want_losses=True, want_sum=False,
+            want_losses=True, want_sum=False, kept=kept,
         )
-        ctx.save_for_backward(rows, weight, bias, targets, lse, valid_count)
+        ctx.save_for_backward(rows, weight, bias, targets, lse, valid_count, kept)
         ctx.hidden_shape = hidden.shape
         ctx.multiplier, ctx.logit_softcap = multiplier, logit_softcap
         ctx.panel_bytes = native.get_panel_bytes()
@@ -217,13 +225,13 @@ class _FusedTokenLosses(torch.autograd.Function):
     def backward(ctx, grad_output):  # type: ignore[override]
         from . import chunked_linear_ce_native as native
 
-        rows, weight, bias, targets, lse, valid_count = ctx.saved_tensors
+        rows, weight, bias, targets, lse, valid_count, kept = ctx.saved_tensors
         with native.panel_budget(ctx.panel_bytes):
             grad_hidden, grad_weight, grad_bias = native.masked_loss_backward(
                 rows, weight, bias, targets, None, lse, valid_count, grad_output,
                 reduction="none", ignore_index=-100, exclude_index=-1,
                 logit_softcap=ctx.logit_softcap, logit_multiplier=ctx.multiplier,
-                compute_weight_grad=ctx.needs_input_grad[1],
+                compute_weight_grad=ctx.needs_input_grad[1], kept=kept,
             )
         return (
             grad_hidden.reshape(ctx.hidden_shape),

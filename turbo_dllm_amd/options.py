@@ -51,7 +51,9 @@ _panel_bytes = contextvars.ContextVar("tlce_panel_bytes", default=0)
 #               take this path with a frozen head, and with a trainable head
 #               when all rows fit one block: grad_weight needs the per-row
 #               upstream gradients inside its contraction, which then runs in
-#               the backward;
+#               the backward.  Other 16-bit calls keep the logits of as many
+#               vocabulary tiles as there is room for between forward and backward
+#               (native.kept_logits_buffer) and recompute the rest;
 #   "recompute" by a backward that recomputes the logits in vocabulary panels, as
 #               the reference's backward does block by block
 #               (fused_linear_ce_cuda.cu:618-791).

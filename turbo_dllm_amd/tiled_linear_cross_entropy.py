@@ -337,7 +337,13 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
         ctx.grad_dtype = hidden.dtype
         ctx.vocab = weight_vf.shape[0]
         return loss.reshape(labels.shape) if reduction == "none" else loss
-    if row_count is None:
+    # The logits of as many vocabulary tiles as there is room for stay until the backward, which
+    # contracts the others again (not of rows counted on the device: the buffer would be sized
+    # for all of them)
+    kept = None
+    if mode != "device" and (wants_grad or ctx.needs_input_grad[2]):
+        kept = native.kept_logits_buffer(m, rows, weight_vf.shape[1 if in_place else 0], bias)
+    if row_count is None and kept is None:
         losses, lse, valid_count = native.forward(
             rows, weight_vf, bias, targets,
             row_block_size=0, ignore_index=ignore_index, exclude_index=exclude_index,
@@ -348,9 +354,11 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
         losses, lse, valid_count, _ = native.masked_loss_forward(
             rows, weight_vf, bias, targets, None, m=m, row_idx=row_idx, row_count=row_count,
             n_out=n, ignore_index=ignore_index, exclude_index=exclude_index,
-            logit_softcap=float(logit_softcap), want_losses=True, want_sum=False,
+            logit_softcap=float(logit_softcap), want_losses=True, want_sum=False, kept=kept,
+            weight_dim_first=in_place,
         )
-    ctx.save_for_backward(rows, weight_vf, bias, targets, lse, valid_count, row_idx, row_count)
+    ctx.save_for_backward(rows, weight_vf, bias, targets, lse, valid_count, row_idx, row_count,
+                          kept)
     ctx.hidden_shape = hidden.shape
     ctx.n_rows, ctx.m = n, m
     ctx.reduction = reduction
@@ -391,9 +399,9 @@ def _device_backward(ctx, grad_output, frozen: bool):
             )
         return (grad_hidden.reshape(ctx.hidden_shape), None if frozen else grad_weight,
                 None) + (None,) * 9
-    rows, weight_vf, bias, targets, lse, valid_count, row_idx, row_count = ctx.saved_tensors
+    rows, weight_vf, bias, targets, lse, valid_count, row_idx, row_count, kept = ctx.saved_tensors
     with native.panel_budget(ctx.panel_bytes):
-        if row_count is None:
+        if row_count is None and kept is None:
             call = native.backward_frozen_weight if frozen else native.backward
             grad_hidden, grad_weight, grad_bias = call(
                 rows, weight_vf, bias, targets, lse, valid_count, grad_output,
@@ -407,7 +415,8 @@ def _device_backward(ctx, grad_output, frozen: bool):
                 rows, weight_vf, bias, targets, None, lse, valid_count, grad_output,
                 reduction=ctx.reduction, m=ctx.m, row_idx=row_idx, row_count=row_count,
                 n_out=ctx.n_rows, ignore_index=ctx.ignore_index, exclude_index=ctx.exclude_index,
-                logit_softcap=ctx.logit_softcap, compute_weight_grad=not frozen,
+                logit_softcap=ctx.logit_softcap, compute_weight_grad=not frozen, kept=kept,
+                weight_dim_first=ctx.in_place,
             )
     if not frozen and ctx.weight_dim_first and not ctx.in_place:
         grad_weight = grad_weight.t().contiguous()
