@@ -565,22 +565,26 @@ def main() -> int:
         if fused:
             # as the autograd functions do: one block of rows -> the grad_weight contraction
             # waits for the upstream gradient and is stored in bf16 at once
-            postpone = native.weight_grad_can_wait(m_rows, h, v, hidden.dtype)
+            panel = (native.reduced_loss_panel_bytes(m_rows, h, v, hidden.dtype)
+                     if on_device is None else options.get_panel_bytes())
+            postpone = native.weight_grad_can_wait(m_rows, h, v, hidden.dtype, panel)
             with _lib.kernel_profile() as prof:
                 _, valid, grad_hidden32, kept, row_of = native.forward_with_gradients_reduced(
                     rows[:m_rows], weight.detach(), targets[:m_rows], reduction="mean",
                     ignore_index=-100, exclude_index=-1, logit_softcap=softcap,
                     compute_weight_grad=True, postpone_weight_grad=postpone, row_idx=row_idx,
-                    n_out=n, row_count=on_device)
+                    n_out=n, row_count=on_device, panel_bytes=panel)
                 native.finish_gradients(
                     grad_hidden32, kept, go, valid, reduction="mean", n_out=n, vocab=v,
                     row_of=row_of, row_count=on_device,
                     rows=rows[:m_rows] if postpone else None,
-                    panel_bytes=options.get_panel_bytes())
+                    panel_bytes=panel)
             del grad_hidden32, kept
         elif count is not None:
+            keep = (native.kept_logits_buffer(m_rows, rows, v, None)
+                    if args.gradients == "forward" and on_device is None else None)
             kw = dict(m=m_rows, row_idx=row_idx, row_count=count, n_out=n, ignore_index=-100,
-                      exclude_index=-1, logit_softcap=softcap)
+                      exclude_index=-1, logit_softcap=softcap, kept=keep)
             with _lib.kernel_profile() as prof:
                 _, lse, valid, _ = native.masked_loss_forward(
                     rows, weight.detach(), None, targets, None, want_losses=True, want_sum=False,
@@ -634,7 +638,7 @@ def main() -> int:
     plan_rows = m if args.compaction_mode == "sync" else n
     if fused:
         plan = {"engine": "mfma_direct", "tile": 256,
-                **_lib.query_fused_plan(plan_rows, h, v, _lib.DTYPE_BF16, options.get_panel_bytes())}
+                **_lib.query_fused_plan(plan_rows, h, v, _lib.DTYPE_BF16, panel)}
     else:
         plan = _lib.query_plan(plan_rows, h, v, _lib.DTYPE_BF16, True, options.get_panel_bytes())
     traffic, traffic_note = measured_traffic(wl.name, dominant)

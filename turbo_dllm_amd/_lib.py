@@ -117,6 +117,7 @@ SIGNATURES = {
     "tlce_query_fused_plan": (
         c_int, [c_int64, c_int64, c_int64, c_int, c_int64, c_void_p, c_void_p, c_void_p]
     ),
+    "tlce_reduced_loss_panel_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int]),
     "tlce_forward_with_gradients_workspace_bytes": (
         c_int64, [c_int64, c_int64, c_int64, c_int, c_int, c_int64]
     ),

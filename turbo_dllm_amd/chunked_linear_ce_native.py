@@ -559,6 +559,7 @@ def forward_with_gradients_reduced(
     n_out: int | None = None,
     row_count: torch.Tensor | None = None,
     rows_copy: torch.Tensor | None = None,
+    panel_bytes: int | None = None,
 ):
     """``forward_with_gradients``, of float32 operands as well, in fewer launches and with the
     loss reduced on the way:
@@ -569,7 +570,8 @@ def forward_with_gradients_reduced(
     ``row_of`` (int32 ``[n_out]``, when ``row_idx`` or ``rows_copy`` is given) holds the row of
     an output row, -1 where that has none or one without a loss: ``finish_gradients`` takes it.
     ``rows_copy`` (bf16, shaped like ``hidden``, for rows that were not compacted) receives the
-    rows, zeros in place of ignored ones, and is what the gradients are formed from."""
+    rows, zeros in place of ignored ones, and is what the gradients are formed from.
+    ``panel_bytes`` (``reduced_loss_panel_bytes``) takes the place of the panel budget in force."""
     device = _require_device(hidden, weight, labels, row_idx, token_weights, row_count, rows_copy)
     reduction_code = _reduction_code(reduction)
     m, h = hidden.shape
@@ -595,10 +597,10 @@ def forward_with_gradients_reduced(
     code = _dtype_code(hidden)
     f32 = hidden.dtype == torch.float32
     postpone = bool(postpone_weight_grad and compute_weight_grad)
-    if postpone and not weight_grad_can_wait(m, h, v, hidden.dtype):
+    panel = get_panel_bytes() if panel_bytes is None else int(panel_bytes)
+    if postpone and not weight_grad_can_wait(m, h, v, hidden.dtype, panel):
         raise RuntimeError("the weight gradient can be postponed only when all rows fit "
                            "one block of the forward (weight_grad_can_wait)")
-    panel = get_panel_bytes()
     reduced = reduction_code != _lib.REDUCTION_NONE
     with torch.cuda.device(device):
         losses = torch.empty(n_out, dtype=torch.float32, device=device)
@@ -787,14 +789,26 @@ def forward_with_gradients(
     return losses, lse, valid_count, grad_hidden32, (ws if postpone else grad_weight32)
 
 
-def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype) -> bool:
+def reduced_loss_panel_bytes(m: int, h: int, v: int, dtype: torch.dtype) -> int:
+    """The panel budget for ``m`` rows, whose count the host knows, of a trainable head under a
+    loss reduced to one number: the one in force, or, where none is and it costs no memory at
+    the step's peak, one that takes them as one block."""
+    panel = get_panel_bytes()
+    if panel or dtype != torch.bfloat16:
+        return panel
+    return _lib.library().tlce_reduced_loss_panel_bytes(m, h, v, _lib.DTYPE_BF16)
+
+
+def weight_grad_can_wait(m: int, h: int, v: int, dtype: torch.dtype,
+                         panel_bytes: int | None = None) -> bool:
     """Whether ``forward_with_gradients`` takes ``m`` rows as one block under the
-    panel budget in force, so that its grad_weight contraction can be postponed to
+    panel budget in force (or ``panel_bytes``), so that its grad_weight contraction can be postponed to
     the backward (``grad_weight_from_panel``)."""
     if dtype != torch.bfloat16 or not _lib.library().tlce_fused_gradients_supported(
             h, v, _lib.DTYPE_BF16):
         return False
-    return _lib.query_fused_plan(m, h, v, _lib.DTYPE_BF16, get_panel_bytes())["n_blocks"] == 1
+    panel = get_panel_bytes() if panel_bytes is None else panel_bytes
+    return _lib.query_fused_plan(m, h, v, _lib.DTYPE_BF16, panel)["n_blocks"] == 1
 
 
 def _upstream_gradient(grad_output: torch.Tensor, reduction_code: int, n_out: int) -> torch.Tensor:

@@ -539,6 +539,23 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
   return p;
 }
 
+// Panel budget (0: the default) of a call with a trainable head whose loss is reduced to one
+// number.  In one block the panel waits for the backward, in several the float32 [v, h] sum does,
+// which every block but the first reads and writes and a last pass rounds.  One block is taken
+// beyond the default as well where the step's peak stays what it is: the panel and the 16-bit
+// gradient in the backward against a default panel and the float32 sum in the forward, i.e. up to
+// the default and one 16-bit gradient.  Several blocks / one, ms a step and GB at its peak:
+//   8212 rows, H = 3840, V = 262144, cap 30   39.7 / 38.8   6.5 / 6.6
+//   6000 rows, H = 4096, V = 262144           33.8 / 28.2   6.5 / 5.5    (16 and 8 token tiles)
+//  10000 rows, H = 4096, V = 151936           29.8 / 27.4   5.2 / 4.7    (32 and 8)
+//  16384 rows, H = 4096, V = 151936           45.0 / 43.8   5.3 / 6.6    (not taken)
+inline int64_t reduced_loss_panel_bytes(int64_t m, int64_t h, int64_t v) {
+  const int64_t vp = round_up(v, 256);
+  const int64_t all = round_up(std::max<int64_t>(m, 1), 256) * vp * 2;
+  const int64_t limit = kDefaultFusedPanelBytes + 2 * v * h;
+  return all > kDefaultFusedPanelBytes && all <= limit ? all : 0;
+}
+
 struct FusedLayout {
   int64_t panel, part_sum, part_max, target, ref, ref_next, row_scale, scaled_hidden, slabs,
       redo, hidden_planes, weight_planes, label_rest, k_tail, loss_parts, total;

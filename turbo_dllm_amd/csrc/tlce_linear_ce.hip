@@ -1112,6 +1112,11 @@ extern "C" int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
   return 0;
 }
 
+extern "C" int64_t tlce_reduced_loss_panel_bytes(int64_t m, int64_t h, int64_t v, int dtype) {
+  if (m < 0 || h <= 0 || v <= 0 || !fused_gradients_supported(h, v, dtype)) return 0;
+  return reduced_loss_panel_bytes(m, h, v);
+}
+
 extern "C" int64_t tlce_forward_with_gradients_workspace_bytes(int64_t m, int64_t h, int64_t v,
                                                                int dtype, int compute_weight_grad,
                                                                int64_t panel_bytes) {

@@ -80,8 +80,12 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         )
         if ctx.fused:
             rows = rows[:m]
+            ctx.panel_bytes = native.get_panel_bytes()   # the backward may run on another thread
+            if ctx.needs_input_grad[1] and mode != "device":
+                ctx.panel_bytes = native.reduced_loss_panel_bytes(m, rows.shape[1],
+                                                                  weight.shape[0], rows.dtype)
             ctx.postponed = bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
-                m, rows.shape[1], weight.shape[0], rows.dtype)
+                m, rows.shape[1], weight.shape[0], rows.dtype, ctx.panel_bytes)
             loss, valid_count, grad_rows32, grad_weight32, row_of = (
                 native.forward_with_gradients_reduced(
                     rows, weight, targets[:m], reduction="sum", ignore_index=-100,
@@ -90,13 +94,13 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
                     postpone_weight_grad=ctx.postponed, token_weights=token_weights[:m],
                     logit_multiplier=multiplier, row_idx=row_idx, n_out=n,
                     row_count=row_count if mode == "device" else None, rows_copy=rows_copy,
+                    panel_bytes=ctx.panel_bytes,
                 ))
             if rows_copy is not None:
                 rows = rows_copy
             ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                                   row_count if mode == "device" else None,
                                   rows if ctx.postponed else None)
-            ctx.panel_bytes = native.get_panel_bytes()
             ctx.hidden_shape = hidden.shape
             ctx.n_rows, ctx.m = n, m
             ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]
@@ -175,18 +179,21 @@ class _FusedSampleLoss(torch.autograd.Function):
         rows, targets, factors = native.gather_sample_rows(
             hidden, labels, weights, denominators, segment_length, row_idx, row_count, m)
         rows = rows[:m]
+        ctx.panel_bytes = native.get_panel_bytes()   # the backward may run on another thread
+        if ctx.needs_input_grad[1]:
+            ctx.panel_bytes = native.reduced_loss_panel_bytes(m, rows.shape[1], weight.shape[0],
+                                                              rows.dtype)
         wait = bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
-            m, rows.shape[1], weight.shape[0], rows.dtype)
+            m, rows.shape[1], weight.shape[0], rows.dtype, ctx.panel_bytes)
         loss, valid_count, grad_rows32, grad_weight32, row_of = (
             native.forward_with_gradients_reduced(
                 rows, weight, targets[:m], reduction="sum", ignore_index=-100, exclude_index=-1,
                 logit_softcap=logit_softcap, compute_weight_grad=bool(ctx.needs_input_grad[1]),
                 postpone_weight_grad=wait, token_weights=factors[:m], row_idx=row_idx[:m],
-                n_out=hidden.shape[0],
+                n_out=hidden.shape[0], panel_bytes=ctx.panel_bytes,
             ))
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx[:m], row_of, None,
                               rows if wait else None)
-        ctx.panel_bytes = native.get_panel_bytes()   # the backward may run on another thread
         ctx.n_rows = hidden.shape[0]
         ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]
         return loss

@@ -307,8 +307,14 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
                                                   in_place or weight_dim_first,
                                                   bool(ctx.needs_input_grad[1]))
     )
+    # the backward may run on an autograd worker thread, which does not see this
+    # thread's context: the panel budget in force now travels with the node
+    ctx.panel_bytes = native.get_panel_bytes()
+    if ctx.fused and ctx.needs_input_grad[1] and reduction != "none" and mode != "device":
+        ctx.panel_bytes = native.reduced_loss_panel_bytes(m, rows.shape[1], weight_vf.shape[0],
+                                                          rows.dtype)
     can_wait = ctx.fused and bool(ctx.needs_input_grad[1]) and native.weight_grad_can_wait(
-        m, rows.shape[1], weight_vf.shape[0], rows.dtype)
+        m, rows.shape[1], weight_vf.shape[0], rows.dtype, ctx.panel_bytes)
     if reduction == "none" and bool(ctx.needs_input_grad[1]) and not can_wait:
         ctx.fused = False
     if ctx.fused:
@@ -324,13 +330,13 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
                 compute_weight_grad=bool(ctx.needs_input_grad[1]),
                 postpone_weight_grad=ctx.postponed, row_idx=row_idx, n_out=n,
                 row_count=row_count if mode == "device" else None, rows_copy=rows_copy,
+                panel_bytes=ctx.panel_bytes,
             ))
         if rows_copy is not None:
             rows = rows_copy
         ctx.save_for_backward(grad_rows32, grad_weight32, valid_count, row_idx, row_of,
                               row_count if mode == "device" else None,
                               rows if ctx.postponed else None)
-        ctx.panel_bytes = native.get_panel_bytes()
         ctx.hidden_shape = hidden.shape
         ctx.n_rows, ctx.m = n, m
         ctx.reduction = reduction
@@ -368,9 +374,6 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
     ctx.weight_dim_first = weight_dim_first
     ctx.in_place = in_place
     ctx.logit_softcap = float(logit_softcap)
-    # the backward may run on an autograd worker thread, which does not see this
-    # thread's context: the panel budget in force now travels with the node
-    ctx.panel_bytes = native.get_panel_bytes()
     if reduction == "none":
         return losses.reshape(labels.shape)
     if reduction == "sum":
