@@ -1,0 +1,50 @@
+"""Last token tiles of at most 64 and at most 128 rows, which run narrower than 256 (engine
+``NarrowEngine``): one to four K steps, rows around both widths, alone and after a whole tile, a
+vocabulary that ends inside a tile and inside a K slab.  Per-token losses are those of the same rows
+in a tile of 256, bit for bit (the sums run in the same order); gradients within the operator's
+2e-2 relative max-norm of the float32 oracle."""
+
+import pytest
+import torch
+
+import linear_ce_oracle as oracle
+from turbo_dllm_amd.tiled_linear_cross_entropy import tiled_linear_cross_entropy
+
+pytestmark = pytest.mark.gpu
+
+
+def step(hidden, weight, labels, reduction, trainable, **keywords):
+    x = hidden.clone().requires_grad_()
+    w = weight.clone().requires_grad_(trainable)
+    loss = tiled_linear_cross_entropy(x, w, labels, reduction=reduction, dtype=x.dtype, **keywords)
+    loss.sum().backward()
+    return loss.detach(), x.grad, w.grad
+
+
+@pytest.mark.parametrize("rows", [1, 16, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("before", [0, 256])
+@pytest.mark.parametrize("h,v,keywords", [
+    (64, 320, {}),
+    (128, 448, dict(logit_softcap=20.0)),
+    (192, 1088, dict(exclude_index=300)),
+    (256, 4096, {}),
+    (320, 515, {}),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_last_tiles(gpu_device, rows, before, h, v, keywords, dtype):
+    m, wide = before + rows, before + 200
+    print("[case]", m, h, v, keywords, dtype, flush=True)
+    gen = torch.Generator().manual_seed(m + h + v)
+    hidden = torch.randn(wide, h, generator=gen).to(dtype)
+    weight = (torch.randn(v, h, generator=gen) * 0.05).to(dtype)
+    labels = torch.randint(0, 300, (wide,), generator=gen)
+    on_gpu = [t.to(gpu_device) for t in (hidden, weight, labels)]
+    losses, _, _ = step(on_gpu[0][:m], on_gpu[1], on_gpu[2][:m], "none", False, **keywords)
+    in_wide, _, _ = step(*on_gpu, "none", False, **keywords)
+    assert torch.equal(losses, in_wide[:m])
+    _, grad_hidden, grad_weight = step(on_gpu[0][:m], on_gpu[1], on_gpu[2][:m], "mean", True,
+                                       **keywords)
+    want_hidden, want_weight, _ = oracle.dense_linear_ce_grads(
+        hidden[:m], weight, labels[:m], dtype=torch.float32, **keywords)
+    assert oracle.relative_max_error(grad_hidden, want_hidden) <= 2e-2
+    assert oracle.relative_max_error(grad_weight, want_weight) <= 2e-2

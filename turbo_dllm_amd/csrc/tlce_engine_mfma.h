@@ -49,6 +49,7 @@ struct MfmaTileLayout {
   using V8 = typename Op::V8;
 
   static constexpr int kTile = 256;     // BM == BN
+  static constexpr int kTileB = kTile;
   static constexpr int kWavesN = 4;     // waves along B rows
   static constexpr int kThreads = 2 * kWavesN * 64;
   static constexpr int kTM = 4;         // 32-row blocks per wave along A rows
@@ -249,20 +250,22 @@ struct MfmaEngine : MfmaTileLayout<T_> {
 // K = 8*(l/16) .. +8  (one 16-byte chunk).
 typedef float acc4_t __attribute__((ext_vector_type(4)));
 
-template <typename T_>
+template <typename T_, int kTN_ = 8>
 struct DirectTileLayout {
   using T = T_;
   static constexpr int kTile = 256;
   static constexpr int kThreads = 256;
   static constexpr int kTM = 8;                  // 16-row blocks per wave along A rows
-  static constexpr int kTN = 8;                  // 16-row blocks per wave along B rows
+  static constexpr int kTN = kTN_;               // 16-row blocks per wave along B rows
+  static constexpr int kTileB = 32 * kTN;        // the tile's B rows (256, or fewer: narrow tiles)
+  static constexpr int kWaveB = 16 * kTN;        // B rows of a wave
   static constexpr int kCols = kTN;              // tile columns owned per thread
   static constexpr int kRows = kTM * 4;          // tile rows held per owned column
   static constexpr int kShare = 8;               // threads that hold the same column
   static constexpr int kStageCols = 2;           // owned columns per quarter of the tile
   static constexpr int kWavesPerSimd = 1;
   static constexpr bool kPrecise = false;
-  static constexpr bool kReadsWhereUsed = true;   // has read()
+  static constexpr bool kReadsWhereUsed = kTN == 8;   // read() in place of get()
 
   struct Acc { acc4_t c[kTM][kTN]; };
 
@@ -275,11 +278,11 @@ struct DirectTileLayout {
     wn = wave & 1;
   }
   __device__ __forceinline__ void forget_lane_invariants() { asm volatile("" : "+v"(lane)); }
-  __device__ __forceinline__ int col(int j) const { return wn * 128 + j * 16 + (lane & 15); }
+  __device__ __forceinline__ int col(int j) const { return wn * kWaveB + j * 16 + (lane & 15); }
   // The tile columns that have owned index j in some thread: number t of them.
   static constexpr int kTokensPerIndex = 32;
   static __device__ __forceinline__ int token_of_index(int j, int t) {
-    return (t >> 4) * 128 + j * 16 + (t & 15);
+    return (t >> 4) * kWaveB + j * 16 + (t & 15);
   }
   // Position of this lane's column among those with the same owned index.
   __device__ __forceinline__ int position_in_index() const { return wn * 16 + (lane & 15); }
@@ -409,6 +412,9 @@ template <> struct DirectMfma<__bf16> {
   static __device__ __forceinline__ void mma_set(bf16x8_t a, bf16x8_t b, acc4_t& c) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
   }
+  static __device__ __forceinline__ acc4_t mma_builtin(bf16x8_t a, bf16x8_t b, acc4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
 };
 template <> struct DirectMfma<_Float16> {
   static __device__ __forceinline__ void mma(f16x8_t a, f16x8_t b, acc4_t& c) {
@@ -417,11 +423,14 @@ template <> struct DirectMfma<_Float16> {
   static __device__ __forceinline__ void mma_set(f16x8_t a, f16x8_t b, acc4_t& c) {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(c) : "v"(a), "v"(b));
   }
+  static __device__ __forceinline__ acc4_t mma_builtin(f16x8_t a, f16x8_t b, acc4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
 };
 
-template <typename T_, int kPlanes_, bool kColumnTail = false>
-struct DirectToLdsEngine : DirectTileLayout<T_> {
-  using Base = DirectTileLayout<T_>;
+template <typename T_, int kPlanes_, bool kColumnTail = false, int kTN_ = 8>
+struct DirectToLdsEngine : DirectTileLayout<T_, kTN_> {
+  using Base = DirectTileLayout<T_, kTN_>;
   using T = T_;
   // The K loop's passes over the planes of the operands (kPlanes == 1: one over the
   // matrices themselves).  Plane of A and of B in pass s: nibble s of these.
@@ -446,8 +455,14 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
   static constexpr int kOperandBytes = kTile * kBK * 2;      // 32768
   static constexpr int kStageBytes = 2 * kOperandBytes;      // 65536
   static constexpr int kTouchBytes = 4 * 256;                // where the L2 touches land
-  static constexpr int kSmemBytes = 2 * kStageBytes + kTouchBytes;
+  static constexpr bool kNarrow = kTN_ < 8;
+  static constexpr int kNarrowStages = 3;
+  static constexpr int kNarrowStageBytes = (kTile + Base::kTileB) * kBK * 2;
+  static constexpr int kSmemBytes =
+      kNarrow ? kNarrowStages * kNarrowStageBytes : 2 * kStageBytes + kTouchBytes;
+  static_assert(!kNarrow || (kPlanes == 1 && !kColumnTail), "narrow tiles: matrices as they are");
   static constexpr int kLoads = 8;                           // per wave, operand and K tile
+  static constexpr int kLoadsB = kNarrow ? kTN_ : kLoads;    // of a K-contiguous second operand
   static constexpr int kTouchAhead = 2;                      // K tiles
   static constexpr int kLoadsAfterBarrier = 12;              // of the 16 of both operands
   static constexpr bool kHasKMajor = true;
@@ -504,20 +519,21 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
     int64_t plane;          // bytes from one plane to the next
   };
 
-  template <bool kKMajor, bool kTail = false>
+  template <bool kKMajor, bool kTail = false, int kN = kLoads>
   __device__ __forceinline__ Loader make_loader(const Operand<T>& x, int k_begin, int nk,
                                                 unsigned lds_op) const {
     Loader ld;
     if (!kKMajor) {
-      // this wave fills tile rows [64w, 64w+64), eight rows per instruction
+      // this wave fills tile rows [64w, 64w+64) (of kN loads: [8 kN w, ...)), eight rows per
+      // instruction
 #pragma unroll
-      for (int j = 0; j < kLoads; ++j) {
-        const int r = wave * 64 + j * 8 + (lane >> 3);
+      for (int j = 0; j < kN; ++j) {
+        const int r = wave * (8 * kN) + j * 8 + (lane >> 3);
         const int chunk = (lane & 7) ^ ((r >> 1) & 7);
         const int rr = min(x.row0 + r, x.rows - 1) - x.row0;
         ld.off[j] = (unsigned)((int64_t)rr * x.ld * kPlanes * 2 + chunk * 16);
       }
-      ld.fill = __builtin_amdgcn_readfirstlane(lds_op + (unsigned)(wave * 64 * 128));
+      ld.fill = __builtin_amdgcn_readfirstlane(lds_op + (unsigned)(wave * 8 * kN * 128));
       ld.next = reinterpret_cast<const char*>(x.ptr + (int64_t)x.row0 * x.ld * kPlanes + k_begin);
       ld.step = kBK * 2;
       ld.last = nullptr;
@@ -557,10 +573,10 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
 
   // Fragment addressing of one operand for this lane: LDS byte offset within the
   // operand stage of block 0, K slice 0.
-  template <bool kKMajor>
+  template <bool kKMajor, int kWaveRows = 128>
   __device__ __forceinline__ int reader_base(int wave_block) const {
     if (!kKMajor) {
-      return (wave_block * 128 + (lane & 15)) * 128 +
+      return (wave_block * kWaveRows + (lane & 15)) * 128 +
              (((lane >> 4) ^ ((lane >> 1) & 7)) * 16);
     } else {
       const int g = lane >> 4;           // 16-lane group
@@ -616,6 +632,119 @@ struct DirectToLdsEngine : DirectTileLayout<T_> {
   __device__ __forceinline__ void mainloop_ex(const Operand<T>& A, const Operand<T>& B,
                                               int k_begin, int k_end, Acc& acc,
                                               char* smem) const {
+    if constexpr (kNarrow) {
+      static_assert(!kBKMajor, "narrow tiles: a K-contiguous second operand");
+      narrow_loop<kAKMajor>(A, B, k_begin, k_end, acc, smem);
+    } else {
+      wide_loop<kAKMajor, kBKMajor>(A, B, k_begin, k_end, acc, smem);
+    }
+  }
+
+  // Narrow tiles: 64 or 128 rows of B.  The last token tile of a call holds what is left over
+  // 256, and a short call holds nothing else: 64 rows in a tile of 256 do four times the
+  // operations.  A K tile is short here (32 or 64 MFMAs a wave), so what bounds it is the
+  // operands' way: three stages, of which two are on the way while one is contracted, and the
+  // fragments of the next slice are read between the MFMAs of this one.  The sums are the wide
+  // loop's, in its order.  The MFMAs are the builtin's: few accumulators stay where they are
+  // without help, and the compiler sees to their hazards.  Without the reads in between (left to
+  // the compiler: two fragments, a wait, eight MFMAs) a tile took as long as a wide one.
+  // 64 rows, H = 1024, V = 32000: exponentiated logits 29 -> 16 us, grad_hidden 24 -> 16; a step of
+  // 64 rows over H = 4096, V = 151936 1050 -> 919 us (of 128 rows 1130 -> 1009), where its bytes
+  // take 790.  After whole tiles less is gained, as the neighbours share the head's strips: 1036
+  // rows of the small head 91 -> 85 us of exponentiated logits, 1610 rows over V = 151936 1646 ->
+  // 1605, 8212 rows over H = 1024, V = 65536 2.90 -> 2.84 ms a step.
+  template <bool kAKMajor>
+  __device__ __forceinline__ void narrow_loop(const Operand<T>& A, const Operand<T>& B,
+                                              int k_begin, int k_end, Acc& acc,
+                                              char* smem) const {
+    const unsigned lds0 = (unsigned)(uintptr_t)smem;
+    const int nk = (k_end - k_begin) / kBK;
+    Loader la = make_loader<kAKMajor>(A, k_begin, nk, lds0);
+    Loader lb = make_loader<false, false, kLoadsB>(B, k_begin, nk, lds0 + kOperandBytes);
+    const int ra = reader_base<kAKMajor>(wm);
+    const int rb = reader_base<false, Base::kWaveB>(wn);
+    auto advance = [&](int k) {
+      la.next = kAKMajor && k == nk - 1 ? la.last : la.next + la.step;
+      lb.next += lb.step;
+    };
+    // load number q of the K tile the loaders stand at
+    constexpr int kTileLoads = kLoads + kLoadsB;
+    auto issue_one = [&](unsigned s_off, int q) {
+      if (q < kLoads) load_to_lds(la.fill + s_off + q * 1024, la.off[q], la.next);
+      else load_to_lds(lb.fill + s_off + (q - kLoads) * 1024, lb.off[q - kLoads], lb.next);
+    };
+    auto issue = [&](int stage) {
+#pragma unroll
+      for (int q = 0; q < kTileLoads; ++q) issue_one((unsigned)(stage * kNarrowStageBytes), q);
+    };
+    // fragment number r of a slice: those of B, which every group needs, first
+    constexpr int kFrags = kTN + kTM;
+    V8 fa[2][kTM], fb[2][kTN];
+    auto read_one = [&](const char* stage, int s, int r) {
+      if (r < kTN) fb[s][r] = read_frag<false>(stage + kOperandBytes, rb, s, r);
+      else fa[s][r - kTN] = read_frag<kAKMajor>(stage, ra, s, r - kTN);
+    };
+    unsigned cur = 0;   // LDS offset of the current K tile's stage
+    // left: how many K tiles follow (0, 1, 2, or 3 for "three or more")
+    auto step = [&](int k, auto left_tag) {
+      constexpr int kLeft = decltype(left_tag)::value;
+      const unsigned nxt = cur == 2 * kNarrowStageBytes ? 0 : cur + kNarrowStageBytes;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        if (s == 1 && kLeft >= 1) {
+          // K tile k + 1 is complete and visible from here on, and the current stage free
+          asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kLeft >= 2 ? kTileLoads : 0) : "memory");
+          __syncthreads();
+          if (kLeft >= 3) advance(k + 3);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < kTM; ++q) {
+#pragma unroll
+          for (int t = 0; t < kTN; ++t)
+            acc.c[q][t] = Op::mma_builtin(fa[s][q], fb[s][t], acc.c[q][t]);
+#pragma unroll
+          for (int r = 2 * q; r < 2 * q + 2; ++r) {
+            if (r < kFrags && s == 0) read_one(smem + cur, 1, r);
+            if (r < kFrags && s == 1 && kLeft >= 1) read_one(smem + nxt, 0, r);
+            if (r < kTileLoads && s == 1 && kLeft >= 3) issue_one(cur, r);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      cur = nxt;
+    };
+    issue(0);
+    if (nk > 1) {
+      advance(1);
+      issue(1);
+    }
+    if (nk > 2) {
+      advance(2);
+      issue(2);
+    }
+    Base::zero(acc);
+    if (nk > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * kTileLoads) : "memory");
+    else if (nk == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kTileLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kFrags; ++r) read_one(smem, 0, r);
+    using Left0 = std::integral_constant<int, 0>;
+    using Left1 = std::integral_constant<int, 1>;
+    using Left2 = std::integral_constant<int, 2>;
+    using Left3 = std::integral_constant<int, 3>;
+    int k = 0;
+    for (; k + 3 < nk; ++k) step(k, Left3{});
+    if (k + 3 == nk) step(k++, Left2{});
+    if (k + 2 == nk) step(k++, Left1{});
+    step(k, Left0{});
+    __syncthreads();
+  }
+
+  template <bool kAKMajor, bool kBKMajor>
+  __device__ __forceinline__ void wide_loop(const Operand<T>& A, const Operand<T>& B, int k_begin,
+                                            int k_end, Acc& acc, char* smem) const {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
     static_assert(!kColumnTail || (!kAKMajor && !kBKMajor), "column tails: K-contiguous operands");
     // K tiles of one pass
@@ -828,6 +957,18 @@ struct MfmaDirect4Engine : DirectToLdsEngine<T_, 1> {};
 // of its own: the choice of the last tile's addresses costs the other up to 1.5 %.
 template <typename T_>
 struct ColumnTailEngine : DirectToLdsEngine<T_, 1, true> {};
+// The engine of tiles with at most 32 * kTN rows of B beside E, where it has one (bool) and the
+// LDS a launch takes that may run them all.
+template <class E> constexpr bool kHasNarrowTiles = false;
+template <typename T> constexpr bool kHasNarrowTiles<MfmaDirect4Engine<T>> = true;
+template <typename T, int kTN> using NarrowEngine = DirectToLdsEngine<T, 1, false, kTN>;
+template <class E>
+constexpr int kLaunchSmemBytes =
+    kHasNarrowTiles<E> ? (NarrowEngine<__bf16, 4>::kSmemBytes > E::kSmemBytes
+                              ? NarrowEngine<__bf16, 4>::kSmemBytes
+                              : E::kSmemBytes)
+                       : E::kSmemBytes;
+
 template <class E> constexpr bool kReadsColumnTails = false;
 template <typename T> constexpr bool kReadsColumnTails<ColumnTailEngine<T>> = true;
 // The engine that does so for engine E.

@@ -78,22 +78,10 @@ struct ExpPanelArgs {
 // (a forward value, the unnormalised softmax, not a logit gradient).
 // kRounded: the sums of the entries before and after their rounding go out as well, so that
 // the factor common to a row's rounding errors can be taken out again.
-template <class E, bool kSoftcap, bool kPlain = false, bool kRounded = false>
-__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_panel_kernel(ExpPanelArgs p) {
-  extern __shared__ __align__(16) char smem[];
+// One tile of the panel; a narrow engine's holds fewer tokens.
+template <class E, bool kSoftcap, bool kPlain, bool kRounded>
+__device__ __forceinline__ void exp_logits_tile(ExpPanelArgs p, int tt, int vt, char* smem) {
   using T = typename E::T;
-  static_assert(E::kHasKMajor && sizeof(T) == 2,
-                "written for the four-wave direct-to-LDS engine");
-  if (p.run_flag != nullptr && *p.run_flag == 0) return;
-  if (p.m_dev != nullptr) {
-    p.m = effective_block_rows(p.m, p.m_dev, p.row0);
-    p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
-  }
-  int tt, vt;
-  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_vtiles,
-                (int64_t)E::kTile * p.h * E::kPlanes * sizeof(T), &tt, &vt))
-    return;
-
   E eng;
   typename E::Acc acc;
   const int vbase = vt * E::kTile;
@@ -148,11 +136,11 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
           const int row = eng.row(i + q);
           float z2, dcap = 1.0f;
           if (kSoftcap) {
-            const float t = tanh_of<E::kPrecise>(E::get(acc, j, i + q) * inv_cap);
+            const float t = tanh_of<E::kPrecise>(element_of<E>(acc, j, i + q) * inv_cap);
             z2 = t * to_base2;
             dcap = 1.0f - t * t;
           } else {
-            z2 = E::get(acc, j, i + q) * to_base2;
+            z2 = element_of<E>(acc, j, i + q) * to_base2;
           }
           float e = exp2_of<E::kPrecise>(z2 - ref2[j]);
           if (kEdge) {
@@ -184,6 +172,9 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
             }
           }
         }
+        // summed here: left to the compiler the sums of a column move to where they are used,
+        // and the entries wait for them in scratch memory
+        asm volatile("" : "+v"(s), "+v"(mx));
       }
       col_sum[j] = s;
       col_max[j] = mx;
@@ -191,6 +182,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
         col_entry[j] = kSoftcap ? entry : s;
         col_rounded[j] = rounded;
       }
+      if (E::kReadsWhereUsed) __builtin_amdgcn_sched_barrier(0);
       if (j % E::kStageCols != E::kStageCols - 1) continue;
       __syncthreads();
       if constexpr (E::kPlanes > 1) {
@@ -236,7 +228,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
     sh_max[slot * E::kTile + eng.col(j)] = col_max[j];
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < E::kTile; c += E::kThreads) {
+  for (int c = threadIdx.x; c < E::kTileB; c += E::kThreads) {
     float sum = 0.0f, mx = -INFINITY;
 #pragma unroll
     for (int sl = 0; sl < E::kShare; ++sl) {
@@ -255,7 +247,7 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
       sh_max[slot * E::kTile + eng.col(j)] = col_rounded[j];
     }
     __syncthreads();
-    for (int c = threadIdx.x; c < E::kTile; c += E::kThreads) {
+    for (int c = threadIdx.x; c < E::kTileB; c += E::kThreads) {
       float entry = 0.0f, rounded = 0.0f;
 #pragma unroll
       for (int sl = 0; sl < E::kShare; ++sl) {
@@ -270,9 +262,39 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
 }
 
 template <class E, bool kSoftcap, bool kPlain = false, bool kRounded = false>
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_panel_kernel(ExpPanelArgs p) {
+  extern __shared__ __align__(16) char smem[];
+  using T = typename E::T;
+  static_assert(E::kHasKMajor && sizeof(T) == 2,
+                "written for the four-wave direct-to-LDS engine");
+  if (p.run_flag != nullptr && *p.run_flag == 0) return;
+  if (p.m_dev != nullptr) {
+    p.m = effective_block_rows(p.m, p.m_dev, p.row0);
+    p.n_ttiles = (p.m + E::kTile - 1) / E::kTile;
+  }
+  int tt, vt;
+  if (!xcd_tile(blockIdx.x, p.n_ttiles, p.n_vtiles,
+                (int64_t)E::kTile * p.h * E::kPlanes * sizeof(T), &tt, &vt))
+    return;
+
+  if constexpr (kHasNarrowTiles<E>) {
+    const int tokens = p.m - tt * E::kTile;
+    if (tokens <= 64) {
+      exp_logits_tile<NarrowEngine<T, 2>, kSoftcap, kPlain, kRounded>(p, tt, vt, smem);
+      return;
+    }
+    if (tokens <= 128) {
+      exp_logits_tile<NarrowEngine<T, 4>, kSoftcap, kPlain, kRounded>(p, tt, vt, smem);
+      return;
+    }
+  }
+  exp_logits_tile<E, kSoftcap, kPlain, kRounded>(p, tt, vt, smem);
+}
+
+template <class E, bool kSoftcap, bool kPlain = false, bool kRounded = false>
 int launch_exp_panel_variant(const ExpPanelArgs& a, hipStream_t stream) {
   static LdsOptIn lds;
-  constexpr int kLdsBytes = E::kSmemBytes + E::kTile * (int)sizeof(float);   // stages + stash
+  constexpr int kLdsBytes = kLaunchSmemBytes<E> + E::kTile * (int)sizeof(float);   // stages + stash
   if (int rc = enable_large_lds(lce_exp_logits_panel_kernel<E, kSoftcap, kPlain, kRounded>,
                                 kLdsBytes, lds))
     return rc;

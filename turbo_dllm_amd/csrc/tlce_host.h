@@ -421,7 +421,8 @@ int launch_grad_logits(const GradLogitsArgs& a, hipStream_t stream) {
 template <class E, bool kAKMajor, bool kBKMajor>
 int launch_gemm(GemmArgs a, int ksplit, int cls, hipStream_t stream) {
   static LdsOptIn lds;
-  if (int rc = enable_large_lds(lce_gemm_nt_kernel<E, kAKMajor, kBKMajor>, E::kSmemBytes, lds))
+  constexpr int kLdsBytes = kBKMajor ? E::kSmemBytes : kLaunchSmemBytes<E>;
+  if (int rc = enable_large_lds(lce_gemm_nt_kernel<E, kAKMajor, kBKMajor>, kLdsBytes, lds))
     return rc;
   const int ksteps = (int)ceil_div(a.k, E::kBK);
   a.k_per_split = (int)ceil_div(ksteps, ksplit) * E::kBK;
@@ -429,7 +430,7 @@ int launch_gemm(GemmArgs a, int ksplit, int cls, hipStream_t stream) {
   // kernel may use fewer of them (a.slab_budget then bounds splits x slab)
   dim3 grid(xcd_grid((int64_t)a.ni * a.nj), ksplit, 1);
   ScopedTimer timer(cls, stream);
-  lce_gemm_nt_kernel<E, kAKMajor, kBKMajor><<<grid, E::kThreads, E::kSmemBytes, stream>>>(a);
+  lce_gemm_nt_kernel<E, kAKMajor, kBKMajor><<<grid, E::kThreads, kLdsBytes, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }

@@ -55,6 +55,15 @@ __device__ __forceinline__ void keep_logits(const typename E::Acc& acc, const Ke
   }
 }
 
+// Accumulator element i of owned column j, copied where it is used if the engine asks for it
+// (left to the compiler, the exponentiated-logits panel's epilogue kept up to 70 registers in
+// scratch memory: with top-k 15.39 -> 15.04 ms a step of 8192 rows, H = 4096, V = 151936).
+template <class E>
+__device__ __forceinline__ float element_of(const typename E::Acc& acc, int j, int i) {
+  if constexpr (E::kReadsWhereUsed) return E::read(acc, j, i);
+  else return E::get(acc, j, i);
+}
+
 struct ForwardArgs {
   const void* hidden;   // [m, h]
   const void* weight;   // [v, h], or [h, v] for the kernels instantiated with kWDimFirst
@@ -154,17 +163,13 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_forward_sta
     // online (max, sum-exp) in the base-2 domain: exp(z - m) = exp2(z*log2e - m2), one
     // owned column after the other; `logit` makes a logit of accumulator element i
     auto fold = [&](auto&& logit) {
-      auto element = [&](int j, int i) {
-        if constexpr (E::kReadsWhereUsed) return E::read(acc, j, i);
-        else return E::get(acc, j, i);
-      };
 #pragma unroll
       for (int j = 0; j < E::kCols; ++j) {
         float z[E::kRows];
         float tile_max = -INFINITY;
 #pragma unroll
         for (int i = 0; i < E::kRows; ++i) {
-          z[i] = logit(i, element(j, i));
+          z[i] = logit(i, element_of<E>(acc, j, i));
           tile_max = fmaxf(tile_max, z[i]);
         }
         const float new_max = fmaxf(run_max[j], tile_max * log2e_scaled);
@@ -1536,7 +1541,7 @@ __device__ __forceinline__ void store_tile_f32_by_rows(const E& eng, const typen
     };
     if (kAdd) {
 #pragma unroll
-      for (int b = 0; b < kAhead; ++b) request_old(b);
+      for (int b = 0; b < kAhead && b < kBatches; ++b) request_old(b);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -1546,10 +1551,11 @@ __device__ __forceinline__ void store_tile_f32_by_rows(const E& eng, const typen
 #pragma unroll
       for (int i4 = 0; i4 < E::kRows; i4 += 4) {
         const int chunk = eng.row(i4) >> 2;
-        const f32x4_t quad = {E::get(acc, j, i4), E::get(acc, j, i4 + 1), E::get(acc, j, i4 + 2),
-                              E::get(acc, j, i4 + 3)};
+        const f32x4_t quad = {element_of<E>(acc, j, i4), element_of<E>(acc, j, i4 + 1),
+                              element_of<E>(acc, j, i4 + 2), element_of<E>(acc, j, i4 + 3)};
         *reinterpret_cast<f32x4_t*>(smem + s_row * 1024 + ((chunk ^ (s_row & 63)) * 16)) = quad;
       }
+      if (E::kReadsWhereUsed) __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
 #pragma unroll
@@ -1591,12 +1597,13 @@ __device__ __forceinline__ void store_tile_t_by_rows(const E& eng, const typenam
     for (int i4 = 0; i4 < E::kRows; i4 += 4) {
       const int vq = eng.row(i4) >> 2;
       T* dst = reinterpret_cast<T*>(smem + r * 512 + (((vq >> 1) ^ (r & 31)) * 16) + (vq & 1) * 8);
-      store4<T>(dst, E::get(acc, j, i4), E::get(acc, j, i4 + 1), E::get(acc, j, i4 + 2),
-                E::get(acc, j, i4 + 3));
+      store4<T>(dst, element_of<E>(acc, j, i4), element_of<E>(acc, j, i4 + 1),
+                element_of<E>(acc, j, i4 + 2), element_of<E>(acc, j, i4 + 3));
     }
+    if (E::kReadsWhereUsed) __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
-  constexpr int kMine = (E::kTile * 32) / E::kThreads;   // 16-byte pieces per thread
+  constexpr int kMine = (E::kTileB * 32) / E::kThreads;   // 16-byte pieces per thread
   constexpr int kBatch = 8;
 #pragma unroll
   for (int b0 = 0; b0 < kMine; b0 += kBatch) {
@@ -1620,56 +1627,11 @@ __device__ __forceinline__ void store_tile_t_by_rows(const E& eng, const typenam
   }
 }
 
+// One output tile of a K split, k_begin .. k_end of it.
 template <class E, bool kAKMajor, bool kBKMajor>
-__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_kernel(GemmArgs p) {
-  extern __shared__ __align__(16) char smem[];
+__device__ __forceinline__ void gemm_tile(const GemmArgs& p, int ti, int tj, int k_begin, int k_end,
+                                          char* smem) {
   using T = typename E::T;
-  int n_splits = gridDim.y;
-  if (p.m_dev != nullptr) {
-    if (p.m_role == kRowsFollow) {
-      p.c_rows = effective_block_rows(p.c_rows, p.m_dev, p.m_dev_offset);
-      p.nj = (p.c_rows + E::kTile - 1) / E::kTile;
-      n_splits = dynamic_k_splits(p.nj, p.ni, E::kTile, (int)p.ldc, (int)gridDim.y,
-                                  p.slab_budget, p.k_steps_plan, &p.c_split_stride);
-      p.k_per_split = ((p.k + E::kBK - 1) / E::kBK + n_splits - 1) / n_splits * E::kBK;
-    } else if (p.m_role == kKFollows) {
-      const int rows = effective_block_rows(p.k, p.m_dev, p.m_dev_offset);
-      p.k = (rows + p.m_round - 1) / p.m_round * p.m_round;
-      // nothing to add to an accumulator that already holds earlier blocks of rows
-      if (p.k == 0 && p.mode == kAddF32) return;
-    }
-  }
-  int split, ti, tj;
-  const int tiles = p.ni * p.nj;
-  if (gridDim.y == 1 || tiles >= kSplitMajorBelowTiles) {
-    split = blockIdx.y;
-    if (split >= n_splits) return;
-    if (!xcd_tile(blockIdx.x, p.ni, p.nj,
-                  (int64_t)E::kTile * min(p.k, p.k_per_split) * E::kPlanes * sizeof(T), &ti, &tj))
-      return;
-  } else {
-    // Few output tiles under many K splits (a small head, the last rows of a call
-    // whose row count is on the device): an XCD's share of a split would be 2 or 3 tiles,
-    // and all 8 XCDs would fetch every K range of both operands.  The (split, tile) pairs
-    // in split-major order are dealt to the XCDs in 8 contiguous, equally long runs
-    // instead, so the tiles that stream one K range sit on one XCD (or two) and share
-    // it through that L2.
-    const int total = n_splits * tiles;
-    const int flat = blockIdx.y * gridDim.x + blockIdx.x;   // gridDim.x is a multiple of 8
-    const int xcd = flat % kXcds, slot = flat / kXcds;
-    const int first = (int)((int64_t)xcd * total / kXcds);
-    const int last = (int)((int64_t)(xcd + 1) * total / kXcds);
-    if (slot >= last - first) return;
-    split = (first + slot) / tiles;
-    grouped_tile((first + slot) - split * tiles, p.ni, p.nj, 4, &ti, &tj);
-  }
-  // each K split owns its own output slab: no atomics, reproducible sums; a
-  // split whose K range is empty still writes its (zero) tile
-  const int k_begin = split * p.k_per_split;
-  const int k_end = min(p.k, k_begin + p.k_per_split);
-  p.c = static_cast<char*>(p.c) +
-        (int64_t)split * p.c_split_stride * (p.mode == kStoreT ? sizeof(T) : sizeof(float));
-
   E eng;
   typename E::Acc acc;
   if (k_begin >= k_end) {
@@ -1744,6 +1706,70 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
       }
     }
   }
+}
+
+template <class E, bool kAKMajor, bool kBKMajor>
+__global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_kernel(GemmArgs p) {
+  extern __shared__ __align__(16) char smem[];
+  using T = typename E::T;
+  int n_splits = gridDim.y;
+  if (p.m_dev != nullptr) {
+    if (p.m_role == kRowsFollow) {
+      p.c_rows = effective_block_rows(p.c_rows, p.m_dev, p.m_dev_offset);
+      p.nj = (p.c_rows + E::kTile - 1) / E::kTile;
+      n_splits = dynamic_k_splits(p.nj, p.ni, E::kTile, (int)p.ldc, (int)gridDim.y,
+                                  p.slab_budget, p.k_steps_plan, &p.c_split_stride);
+      p.k_per_split = ((p.k + E::kBK - 1) / E::kBK + n_splits - 1) / n_splits * E::kBK;
+    } else if (p.m_role == kKFollows) {
+      const int rows = effective_block_rows(p.k, p.m_dev, p.m_dev_offset);
+      p.k = (rows + p.m_round - 1) / p.m_round * p.m_round;
+      // nothing to add to an accumulator that already holds earlier blocks of rows
+      if (p.k == 0 && p.mode == kAddF32) return;
+    }
+  }
+  int split, ti, tj;
+  const int tiles = p.ni * p.nj;
+  if (gridDim.y == 1 || tiles >= kSplitMajorBelowTiles) {
+    split = blockIdx.y;
+    if (split >= n_splits) return;
+    if (!xcd_tile(blockIdx.x, p.ni, p.nj,
+                  (int64_t)E::kTile * min(p.k, p.k_per_split) * E::kPlanes * sizeof(T), &ti, &tj))
+      return;
+  } else {
+    // Few output tiles under many K splits (a small head, the last rows of a call
+    // whose row count is on the device): an XCD's share of a split would be 2 or 3 tiles,
+    // and all 8 XCDs would fetch every K range of both operands.  The (split, tile) pairs
+    // in split-major order are dealt to the XCDs in 8 contiguous, equally long runs
+    // instead, so the tiles that stream one K range sit on one XCD (or two) and share
+    // it through that L2.
+    const int total = n_splits * tiles;
+    const int flat = blockIdx.y * gridDim.x + blockIdx.x;   // gridDim.x is a multiple of 8
+    const int xcd = flat % kXcds, slot = flat / kXcds;
+    const int first = (int)((int64_t)xcd * total / kXcds);
+    const int last = (int)((int64_t)(xcd + 1) * total / kXcds);
+    if (slot >= last - first) return;
+    split = (first + slot) / tiles;
+    grouped_tile((first + slot) - split * tiles, p.ni, p.nj, 4, &ti, &tj);
+  }
+  // each K split owns its own output slab: no atomics, reproducible sums; a
+  // split whose K range is empty still writes its (zero) tile
+  const int k_begin = split * p.k_per_split;
+  const int k_end = min(p.k, k_begin + p.k_per_split);
+  p.c = static_cast<char*>(p.c) +
+        (int64_t)split * p.c_split_stride * (p.mode == kStoreT ? sizeof(T) : sizeof(float));
+
+  if constexpr (kHasNarrowTiles<E> && !kBKMajor) {
+    const int rows = p.c_rows - tj * E::kTile;
+    if (rows <= 64) {
+      gemm_tile<NarrowEngine<T, 2>, kAKMajor, kBKMajor>(p, ti, tj, k_begin, k_end, smem);
+      return;
+    }
+    if (rows <= 128) {
+      gemm_tile<NarrowEngine<T, 4>, kAKMajor, kBKMajor>(p, ti, tj, k_begin, k_end, smem);
+      return;
+    }
+  }
+  gemm_tile<E, kAKMajor, kBKMajor>(p, ti, tj, k_begin, k_end, smem);
 }
 
 // out[c][r] = in[r][c] for r < rows, zero for rows <= r < out_cols: the
