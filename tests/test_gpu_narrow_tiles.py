@@ -48,3 +48,20 @@ def test_last_tiles(gpu_device, rows, before, h, v, keywords, dtype):
         hidden[:m], weight, labels[:m], dtype=torch.float32, **keywords)
     assert oracle.relative_max_error(grad_hidden, want_hidden) <= 2e-2
     assert oracle.relative_max_error(grad_weight, want_weight) <= 2e-2
+
+
+@pytest.mark.parametrize("m", [8300, 8448, 8704])
+def test_grad_hidden_in_chunks_of_one_round(gpu_device, m):
+    """15 x 33 and 15 x 34 tiles of grad_hidden, unsplit: two chunks of 17 token tiles, the last
+    one ragged.  Within the operator's 2e-2 relative max-norm of float32."""
+    h, v = 3840, 512
+    gen = torch.Generator(device=gpu_device).manual_seed(m)
+    hidden = torch.randn(m, h, generator=gen, device=gpu_device).bfloat16()
+    weight = (torch.randn(v, h, generator=gen, device=gpu_device) * 0.02).bfloat16()
+    labels = torch.randint(0, v, (m,), generator=gen, device=gpu_device)
+    _, grad_hidden, _ = step(hidden, weight, labels, "sum", True)
+    p = torch.softmax(hidden.float() @ weight.float().t(), 1)
+    p[torch.arange(m, device=gpu_device), labels] -= 1.0
+    want = p @ weight.float()
+    assert oracle.relative_max_error(grad_hidden, want) <= 2e-2
+    assert (grad_hidden.float() - want).norm(dim=1).div(want.norm(dim=1)).max() <= 2e-2

@@ -190,6 +190,12 @@ __device__ __forceinline__ void grouped_tile(int logical, int ni, int nj, int gr
   *tj = within / gsize;
 }
 
+// Whether the eighths of a launch ordered by groups of four tiles begin at the same j (xcd_tile).
+__host__ __device__ static inline bool xcd_aligned(int ni) {
+  const int groups = (ni + 3) / 4;
+  return (ni % 4) == 0 && (groups <= 2 || (groups % 4) == 0);
+}
+
 // Which output tile a workgroup of an ni x nj tile contraction takes (`strip` = bytes of
 // one operand strip of 256 rows over the whole K range); false: none.  The launch has
 // xcd_grid(ni * nj) workgroups.
@@ -228,10 +234,8 @@ __device__ __forceinline__ void grouped_tile(int logical, int ni, int nj, int gr
 __device__ __forceinline__ bool xcd_tile(int bid, int ni, int nj, int64_t strip, int* ti,
                                          int* tj) {
   const int64_t total = (int64_t)ni * nj;
-  const int groups = (ni + 3) / 4;
-  const bool aligned = (ni % 4) == 0 && (groups <= 2 || (groups % 4) == 0);
   const int64_t kib = strip >> 10;
-  if (aligned && (8 * 8 + ni) * kib > 84 * 1024) {
+  if (xcd_aligned(ni) && (8 * 8 + ni) * kib > 84 * 1024) {
     const int logical = xcd_logical_block_of(bid, (int)total);
     if (logical < 0) return false;
     grouped_tile(logical, ni, nj, 4, ti, tj);

@@ -418,17 +418,36 @@ int launch_grad_logits(const GradLogitsArgs& a, hipStream_t stream) {
   return launch_grad_logits_variant<E, false, false>(a, stream);
 }
 
+// Tiles along j of a chunk of an unsplit contraction of ni x nj tiles (GemmArgs::j_chunk), or 0:
+// a chunk is one round of workgroups, so that the second operand's strips are read in one round
+// only and by few XCDs.  In one piece the two rounds of an unaligned launch (xcd_tile) both go
+// over all of j, XCDs drift apart over a long K loop, and what they share is fetched again.  Taken
+// where the chunks need no more rounds than the whole; aligned launches gain nothing (512 tiles of
+// 8192 rows, H = 4096, V = 151936: 7.12 / 7.11 ms).  In one piece / in chunks, grad_hidden, ms:
+//   8704 rows, H = 3840, V = 262144   14.03 / 12.20       9216, H = 3584, V = 65536   3.00 / 2.97
+//   8212 rows, H = 3840, V = 262144   13.15 / 12.68      12288, H = 3840, V = 65536   4.66 / 4.55
+//   8448 rows, H = 3840, V = 151936    6.93 / 6.72       11776, H = 2816, V = 65536   3.00 / 3.00
+inline int round_chunk(int ni, int nj, int tile) {
+  const int resident = resident_workgroups(tile);
+  const int64_t rounds = ceil_div((int64_t)ni * nj, resident);
+  const int width = (int)ceil_div(nj, rounds);
+  return rounds > 1 && !xcd_aligned(ni) && (int64_t)ni * width <= resident ? width : 0;
+}
+
 template <class E, bool kAKMajor, bool kBKMajor>
 int launch_gemm(GemmArgs a, int ksplit, int cls, hipStream_t stream) {
   static LdsOptIn lds;
   constexpr int kLdsBytes = kBKMajor ? E::kSmemBytes : kLaunchSmemBytes<E>;
   if (int rc = enable_large_lds(lce_gemm_nt_kernel<E, kAKMajor, kBKMajor>, kLdsBytes, lds))
     return rc;
+  if (!kBKMajor && ksplit == 1 && a.m_dev == nullptr)
+    a.j_chunk = round_chunk(a.ni, a.nj, E::kTile);
   const int ksteps = (int)ceil_div(a.k, E::kBK);
   a.k_per_split = (int)ceil_div(ksteps, ksplit) * E::kBK;
   // ksplit is the number of splits launched; with a device-side row count the
   // kernel may use fewer of them (a.slab_budget then bounds splits x slab)
-  dim3 grid(xcd_grid((int64_t)a.ni * a.nj), ksplit, 1);
+  dim3 grid(a.j_chunk > 0 ? xcd_grid((int64_t)a.ni * a.j_chunk) * (int)ceil_div(a.nj, a.j_chunk)
+                          : xcd_grid((int64_t)a.ni * a.nj), ksplit, 1);
   ScopedTimer timer(cls, stream);
   lce_gemm_nt_kernel<E, kAKMajor, kBKMajor><<<grid, E::kThreads, kLdsBytes, stream>>>(a);
   TLCE_LAUNCH_CHECK();

@@ -1473,6 +1473,7 @@ struct GemmArgs {
   int a_k_full = 0x7fffffff;
   const void* b_tail = nullptr;
   int b_k_full = 0x7fffffff;
+  int j_chunk = 0;   // unsplit: chunks of this many tiles along j, one after the other; 0: in one piece
 };
 
 // K splits and slab stride the grad_hidden contraction uses for a device-side
@@ -1732,9 +1733,17 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
   if (gridDim.y == 1 || tiles >= kSplitMajorBelowTiles) {
     split = blockIdx.y;
     if (split >= n_splits) return;
-    if (!xcd_tile(blockIdx.x, p.ni, p.nj,
+    int first_j = 0, bid = blockIdx.x, nj = p.nj;
+    if (p.j_chunk > 0) {
+      const int grid = (p.ni * p.j_chunk + kXcds - 1) / kXcds * kXcds;
+      first_j = bid / grid * p.j_chunk;
+      bid %= grid;
+      nj = min(p.j_chunk, p.nj - first_j);
+    }
+    if (!xcd_tile(bid, p.ni, nj,
                   (int64_t)E::kTile * min(p.k, p.k_per_split) * E::kPlanes * sizeof(T), &ti, &tj))
       return;
+    tj += first_j;
   } else {
     // Few output tiles under many K splits (a small head, the last rows of a call
     // whose row count is on the device): an XCD's share of a split would be 2 or 3 tiles,
