@@ -1,0 +1,97 @@
+"""Small calls whose count of rows with a loss stays on the device in the default compaction
+(``native.count_stays_on_device``): no host synchronisation, and the results of a call that
+compacts nothing, for no row with a loss up to all of them, around tiles and 64-row slabs."""
+
+import pytest
+import torch
+
+from turbo_dllm_amd import chunked_linear_ce_native as native, options
+from turbo_dllm_amd.loss import masked_token_loss
+from turbo_dllm_amd.tiled_linear_cross_entropy import tiled_linear_cross_entropy
+
+pytestmark = pytest.mark.gpu
+
+N, H, V = 700, 256, 1088
+
+
+@pytest.fixture(scope="module")
+def operands(gpu_device):
+    gen = torch.Generator(device=gpu_device).manual_seed(2)
+    hidden = torch.randn(N, H, generator=gen, device=gpu_device).bfloat16()
+    weight = (torch.randn(V, H, generator=gen, device=gpu_device) * 0.05).bfloat16()
+    labels = torch.randint(0, V - 1, (N,), generator=gen, device=gpu_device)
+    order = torch.rand(N, generator=gen, device=gpu_device).argsort()
+    up = torch.rand(N, generator=gen, device=gpu_device)
+    return hidden, weight, labels, order, up
+
+
+def without_synchronisation(call):
+    call()          # (allocations and first launches)
+    torch.cuda.synchronize()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        return call()
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+
+
+def close(got, want):
+    for a, b in zip(got, want):
+        assert torch.equal(a.isnan(), b.isnan())
+        a, b = a.nan_to_num().double(), b.nan_to_num().double()
+        # (the same sums in another order, rounded to bf16: half an ulp, 2^-9, on either side)
+        assert (a - b).abs().max() <= 2.0 ** -8 * a.abs().max() + 1e-12
+
+
+@pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
+@pytest.mark.parametrize("trainable", [True, False])
+@pytest.mark.parametrize("kept", [0, 1, 64, 65, 255, 256, 257, 384, 513, N - 1, N])
+def test_cross_entropy(operands, reduction, trainable, kept):
+    hidden, weight, labels, order, up = operands
+    labels = labels.clone()
+    labels[order[kept:]] = -100
+    assert native.count_stays_on_device(N, hidden, weight, None, False)
+
+    def step(compaction):
+        x = hidden.clone().requires_grad_()
+        w = weight.clone().requires_grad_(trainable)
+        loss = tiled_linear_cross_entropy(x, w, labels, reduction=reduction, dtype=x.dtype,
+                                          exclude_index=V - 1, compaction=compaction)
+        (loss * up if reduction == "none" else loss).sum().backward()
+        return [loss.detach(), x.grad] + ([w.grad] if trainable else [])
+
+    got = without_synchronisation(lambda: step("sync"))
+    if kept == 0 and reduction == "mean":
+        assert got[0].isnan()       # the mean over no row, as before
+        return
+    close(got, step("none"))
+
+
+@pytest.mark.parametrize("kept", [0, 1, 257, N])
+def test_masked_token_loss(operands, kept):
+    hidden, weight, labels, order, up = operands
+    labels = labels.clone()
+    labels[order[kept:]] = -100
+    head = torch.nn.Linear(H, V, bias=False, device=hidden.device, dtype=hidden.dtype)
+
+    def step(mode):
+        x = hidden.clone().requires_grad_()
+        head.weight = torch.nn.Parameter(weight.clone())
+        with options.compaction_mode(mode):
+            loss = masked_token_loss(x, labels, up, head, valid_token_count=300.0,
+                                     mask_token_id=V - 1, exclude_mask_token=True,
+                                     output_multiplier=0.5, logit_softcap=20.0)
+            loss.backward()
+        return [loss.detach(), x.grad, head.weight.grad]
+
+    close(without_synchronisation(lambda: step("sync")), step("none"))
+
+
+def test_larger_calls_are_counted(gpu_device):
+    small = torch.empty(4096, 64, dtype=torch.bfloat16, device=gpu_device)
+    for vocab, stays in ((32768, True), (32832, False)):
+        head = torch.empty(vocab, 64, dtype=torch.bfloat16, device=gpu_device)
+        assert native.count_stays_on_device(4096, small, head, None, False) == stays
+    assert not native.count_stays_on_device(256, small[:256], head, None, False)
+    with native.panel_budget(1 << 20):      # several blocks
+        assert not native.count_stays_on_device(4096, small, head[:4096], None, False)

@@ -529,6 +529,24 @@ def _bf16_head(hidden, weight, bias, weight_dim_first) -> bool:
 # count read back, gather: a third of the time of such a step).
 ONE_TILE_ROWS = 256
 
+# Calls whose panel of exponentiated logits is at most this large with every row in it: the row
+# count stays on the device.  Reading it back costs the wait and, after it, 40 to 60 us in which
+# the GPU has nothing to do; launches sized for all rows cost a few us of workgroups that exit.
+# Half of 2048 rows, H = 1024, V = 32000 (125 MiB): 335 -> 280 us a step.  Beyond it a step takes
+# milliseconds, and the panel's memory for rows without a loss is no longer small.
+_UNCOUNTED_PANEL_BYTES = 256 << 20
+
+
+def count_stays_on_device(n: int, hidden: torch.Tensor, weight: torch.Tensor,
+                          bias: torch.Tensor | None, weight_dim_first: bool) -> bool:
+    """Whether the default compaction of ``n`` rows with gradients in the forward leaves the count
+    of those with a loss on the device: bf16 rows in one block, few words and rows."""
+    vocab, h = weight.shape
+    return (n > ONE_TILE_ROWS
+            and (n + 255) // 256 * ((vocab + 255) // 256) << 17 <= _UNCOUNTED_PANEL_BYTES
+            and fused_gradients_supported(hidden, weight, bias, weight_dim_first)
+            and weight_grad_can_wait(n, h, vocab, hidden.dtype))
+
 
 def gradients_in_forward_supported(m: int, hidden: torch.Tensor, weight: torch.Tensor,
                                    bias: torch.Tensor | None, weight_dim_first: bool,

@@ -69,6 +69,9 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
                 and native.fused_gradients_supported(hidden_flat, weight, bias, False)):
             mode = "none"
             rows_copy = torch.empty_like(hidden_flat)
+        elif (mode == "sync" and wants_grad and get_gradient_mode() == "forward"
+              and native.count_stays_on_device(n, hidden_flat, weight, bias, False)):
+            mode = "device"
         rows, targets, token_weights, row_idx, row_count, m = native.compact_loss_rows(
             hidden_flat, labels_flat, weights_flat, -100, mode)
         # gradients while the logits exist (3 contractions instead of 4), where the

@@ -21,7 +21,8 @@ import contextvars
 #   "sync"   (default) compact them away on the device and read the count of
 #            loss-bearing rows back once, so every launch is sized exactly (the
 #            one host synchronisation the reference's call sites incur as well,
-#            nemotron/model.py:4244-4248);
+#            nemotron/model.py:4244-4248); small calls with gradients do without
+#            (native.count_stays_on_device, native.ONE_TILE_ROWS);
 #   "device" compact them away without any host read-back: launches are sized
 #            for all rows and the kernels take the count from device memory, so
 #            the whole loss (forward and backward) can be recorded into a HIP

@@ -281,6 +281,10 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
                                               hidden.dtype)):
             mode = "none"
             rows_copy = torch.empty_like(hidden_flat)
+    elif (mode == "sync" and wants_grad and options.get_gradient_mode() == "forward"
+          and native.count_stays_on_device(n, hidden_flat, weight_vf, bias,
+                                           in_place or weight_dim_first)):
+        mode = "device"
     if in_place and mode == "sync":
         # the entry points that take a device-side row count read a [V, H] head only:
         # compact with the count read back, as the reference's call sites do
