@@ -605,6 +605,10 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     }
   }
 
+  // device-side row count: at least 16 K splits of grad_hidden (or the plan's, if more) are launched
+  // and the kernel picks how many to use for the real count, within the slabs the plan allocated
+  const int dh_launch_ksplit =
+      m_dev == nullptr ? p.dh_ksplit : std::max(p.dh_ksplit, std::min(16, p.dh_max_ksplit));
   for (int panel = 0; panel < p.n_panels; ++panel) {
     const int64_t v0 = (int64_t)panel * p.vc;
     const int64_t width = std::min<int64_t>(p.vc, p.vp - v0);   // multiple of tile
@@ -619,10 +623,6 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     dh.c_split_stride = p.mp * h;
     dh.mode = (panel == 0) ? kStoreF32 : kAddF32;
     dh.m_dev = m_dev; dh.m_role = kRowsFollow;
-    // device-side row count: at least four K splits (or the plan's, if more) are launched
-    // and the kernel picks how many to use for the real count, within the slabs the plan allocated
-    const int dh_launch_ksplit =
-        m_dev == nullptr ? p.dh_ksplit : std::max(p.dh_ksplit, std::min(4, p.dh_max_ksplit));
     dh.slab_budget = (int64_t)p.dh_ksplit * p.mp * h;
     dh.k_steps_plan = (int)(p.vc / p.bk);
     GemmArgs dw;
@@ -707,8 +707,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     ScopedTimer timer(kClassOther, stream);
     lce_finalize_grad_hidden_kernel<T><<<(int)m, 256, 0, stream>>>(
         acc32, p.dh_ksplit, p.mp * h, row_idx, (int)m, (int)h, static_cast<T*>(grad_hidden),
-        m_dev, p.n_htiles, p.tile, std::max(p.dh_ksplit, std::min(4, p.dh_max_ksplit)),
-        (int)(p.vc / p.bk));
+        m_dev, p.n_htiles, p.tile, dh_launch_ksplit, (int)(p.vc / p.bk));
   }
   TLCE_LAUNCH_CHECK();
   return 0;

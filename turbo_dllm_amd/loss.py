@@ -72,6 +72,12 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         elif (mode == "sync" and wants_grad and get_gradient_mode() == "forward"
               and native.count_stays_on_device(n, hidden_flat, weight, bias, False)):
             mode = "device"
+        keeps_uncounted = (
+            mode == "sync" and wants_grad
+            and native.kept_count_stays_on_device(n, hidden_flat, weight, bias,
+                                                  bool(ctx.needs_input_grad[1])))
+        if keeps_uncounted:
+            mode = "device"
         rows, targets, token_weights, row_idx, row_count, m = native.compact_loss_rows(
             hidden_flat, labels_flat, weights_flat, -100, mode)
         # gradients while the logits exist (3 contractions instead of 4), where the
@@ -109,7 +115,7 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             ctx.grad_dtype, ctx.vocab = hidden.dtype, weight.shape[0]
             return loss
         kept = None
-        if mode != "device" and (wants_grad or ctx.needs_input_grad[2]):
+        if (mode != "device" or keeps_uncounted) and (wants_grad or ctx.needs_input_grad[2]):
             kept = native.kept_logits_buffer(m, rows, weight.shape[0], bias)
         _, lse, _, weighted_sum = native.masked_loss_forward(
             rows, weight, bias, targets, token_weights, m=m, row_idx=row_idx,

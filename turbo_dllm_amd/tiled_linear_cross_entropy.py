@@ -285,6 +285,12 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
           and native.count_stays_on_device(n, hidden_flat, weight_vf, bias,
                                            in_place or weight_dim_first)):
         mode = "device"
+    keeps_uncounted = (
+        mode == "sync" and wants_grad and not in_place
+        and native.kept_count_stays_on_device(n, hidden_flat, weight_vf, bias,
+                                              bool(ctx.needs_input_grad[1])))
+    if keeps_uncounted:
+        mode = "device"
     if in_place and mode == "sync":
         # the entry points that take a device-side row count read a [V, H] head only:
         # compact with the count read back, as the reference's call sites do
@@ -348,10 +354,10 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
         ctx.vocab = weight_vf.shape[0]
         return loss.reshape(labels.shape) if reduction == "none" else loss
     # The logits of as many vocabulary tiles as there is room for stay until the backward, which
-    # contracts the others again (not of rows counted on the device: the buffer would be sized
-    # for all of them)
+    # contracts the others again (of rows counted on the device only where a buffer for all of
+    # them is small)
     kept = None
-    if mode != "device" and (wants_grad or ctx.needs_input_grad[2]):
+    if (mode != "device" or keeps_uncounted) and (wants_grad or ctx.needs_input_grad[2]):
         kept = native.kept_logits_buffer(m, rows, weight_vf.shape[1 if in_place else 0], bias)
     if row_count is None and kept is None:
         losses, lse, valid_count = native.forward(
