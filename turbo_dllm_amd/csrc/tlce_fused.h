@@ -1399,7 +1399,8 @@ int kl_forward_with_gradient_impl(const Plan& pd, const Plan& pt, const KlLayout
     ca.label_offset = 0; ca.local_max = nullptr; ca.local_sum = nullptr;
     ca.target_logits = nullptr;
     ScopedTimer timer(kClassCombine, stream);
-    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock), 256, 0, stream>>>(ca);
+    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock),
+                                64 * kCombineRowsPerBlock, 0, stream>>>(ca);
     TLCE_LAUNCH_CHECK();
     return 0;
   };

@@ -18,31 +18,36 @@ namespace tlce {
 // cleared by a launch before, and the losses' sum goes by parts likewise (kLossesPerBlock).  One
 // workgroup for all was most of a step of many rows over few words: 2^20 rows, H = 64, V = 64,
 // frozen, 3.40 ms, now 1.91; 262144 rows, H = 512, V = 256 1.25, now 0.91.
+constexpr int kLabelRows = 16;
+constexpr int kLabelThreads = 64 * kLabelRows;
 constexpr int kClearPerBlock = 4096;
 constexpr int kRowsPerCount = 16384;
 
 template <typename T>
-__global__ __launch_bounds__(256) void lce_label_logit_kernel(LabelLogitArgs p) {
+__global__ __launch_bounds__(kLabelThreads) void lce_label_logit_kernel(LabelLogitArgs p) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const int extra = (int)blockIdx.x - (p.m + 15) / 16;
+  const int extra = (int)blockIdx.x - (p.m + kLabelRows - 1) / kLabelRows;
   p.m = effective_rows(p.m, p.m_dev);
   if (extra >= 0 && extra < p.n_count) {
-    __shared__ int sh_valid[4];
+    __shared__ int sh_valid[kLabelRows];
     if (extra == 0) {
-      for (int i = threadIdx.x; i < p.n_flags; i += 256) p.flags[i] = 0;
+      for (int i = threadIdx.x; i < p.n_flags; i += kLabelThreads) p.flags[i] = 0;
     }
     const int last = (int)min((int64_t)p.m, (int64_t)(extra + 1) * kRowsPerCount);
     int valid = 0;
-#pragma unroll 8
-    for (int r = extra * kRowsPerCount + threadIdx.x; r < last; r += 256)
+#pragma unroll 4
+    for (int r = extra * kRowsPerCount + threadIdx.x; r < last; r += kLabelThreads)
       valid += p.labels[r] != p.ignore ? 1 : 0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) valid += __shfl_xor(valid, o, 64);
     if (lane == 0) sh_valid[wave] = valid;
     __syncthreads();
     if (threadIdx.x == 0) {
-      const float total = (float)(sh_valid[0] + sh_valid[1] + sh_valid[2] + sh_valid[3]);
+      int rows = 0;
+#pragma unroll
+      for (int w = 0; w < kLabelRows; ++w) rows += sh_valid[w];
+      const float total = (float)rows;
       if (p.n_count == 1)
         p.valid_count[0] = total;
       else if (total != 0.0f)
@@ -53,42 +58,40 @@ __global__ __launch_bounds__(256) void lce_label_logit_kernel(LabelLogitArgs p) 
   if (extra >= p.n_count) {
     const int64_t first = (int64_t)(extra - p.n_count) * kClearPerBlock;
     const int64_t last = min(first + kClearPerBlock, p.n_out);
-    for (int64_t i = first + threadIdx.x; i < last; i += 256) {
+    for (int64_t i = first + threadIdx.x; i < last; i += kLabelThreads) {
       if (p.losses != nullptr) p.losses[i] = 0.0f;
       if (p.row_of != nullptr) p.row_of[i] = -1;
     }
     return;
   }
-  for (int i = 0; i < 4; ++i) {
-    const int r = blockIdx.x * 16 + wave * 4 + i;
-    if (r >= p.m) continue;
-    const int64_t label = p.labels[r];
-    const bool valid = label != p.ignore;
-    const bool here = valid && label >= 0 && label < p.v;
-    float z = 0.0f;
-    if (here) {
-      const T* hrow = static_cast<const T*>(p.hidden) + (int64_t)r * p.h;
-      const T* wrow = static_cast<const T*>(p.weight) + label * (int64_t)p.h;
-      z = wave_dot<T>(hrow, wrow, p.h, lane) * p.logit_scale;
-      if (p.softcap > 0.0f) z = p.softcap * tanhf(z / p.softcap);
-    }
-    if (lane == 0) {
-      // a label on the excluded column or outside the vocabulary has no logit in the
-      // loss (ce_forward_kernel, fused_linear_ce_cuda.cu:199-219); as a reference any
-      // real column's logit serves
-      p.target[r] = (here && label != p.exclude) ? z : 0.0f;
-      p.ref[r] = valid ? z : INFINITY;
-      if (p.row_map != nullptr) p.row_map[r] = valid ? r : -1;
-    }
-    if (sizeof(T) == 2 && p.rows_copy != nullptr) {
-      typedef T v8_t __attribute__((ext_vector_type(8)));
-      const v8_t zero = {};
-      const T* from = static_cast<const T*>(p.hidden) + (int64_t)r * p.h;
-      T* to = static_cast<T*>(p.rows_copy) + (int64_t)r * p.h;
-      for (int k = lane * 8; k < p.h; k += 64 * 8)
-        *reinterpret_cast<v8_t*>(to + k) =
-            valid ? *reinterpret_cast<const v8_t*>(from + k) : zero;
-    }
+  const int r = blockIdx.x * kLabelRows + wave;
+  if (r >= p.m) return;
+  const int64_t label = p.labels[r];
+  const bool valid = label != p.ignore;
+  const bool here = valid && label >= 0 && label < p.v;
+  float z = 0.0f;
+  if (here) {
+    const T* hrow = static_cast<const T*>(p.hidden) + (int64_t)r * p.h;
+    const T* wrow = static_cast<const T*>(p.weight) + label * (int64_t)p.h;
+    z = wave_dot<T>(hrow, wrow, p.h, lane) * p.logit_scale;
+    if (p.softcap > 0.0f) z = p.softcap * tanhf(z / p.softcap);
+  }
+  if (lane == 0) {
+    // a label on the excluded column or outside the vocabulary has no logit in the
+    // loss (ce_forward_kernel, fused_linear_ce_cuda.cu:199-219); as a reference any
+    // real column's logit serves
+    p.target[r] = (here && label != p.exclude) ? z : 0.0f;
+    p.ref[r] = valid ? z : INFINITY;
+    if (p.row_map != nullptr) p.row_map[r] = valid ? r : -1;
+  }
+  if (sizeof(T) == 2 && p.rows_copy != nullptr) {
+    typedef T v8_t __attribute__((ext_vector_type(8)));
+    const v8_t zero = {};
+    const T* from = static_cast<const T*>(p.hidden) + (int64_t)r * p.h;
+    T* to = static_cast<T*>(p.rows_copy) + (int64_t)r * p.h;
+    for (int k = lane * 8; k < p.h; k += 64 * 8)
+      *reinterpret_cast<v8_t*>(to + k) =
+          valid ? *reinterpret_cast<const v8_t*>(from + k) : zero;
   }
 }
 

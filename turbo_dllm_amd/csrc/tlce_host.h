@@ -509,7 +509,8 @@ int launch_combine(CombineArgs ca, int n_vtiles, int tile, int64_t m, const Shar
   }
   {
     ScopedTimer timer(kClassCombine, stream);
-    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock), 256, 0, stream>>>(ca);
+    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock),
+                                64 * kCombineRowsPerBlock, 0, stream>>>(ca);
   }
   TLCE_LAUNCH_CHECK();
   if (opt.weighted_sum != nullptr) return launch_sum(ca.weighted, m, opt.weighted_sum, stream);
@@ -917,7 +918,8 @@ int kl_forward_impl(const Plan& pd, const Plan& pt, const KlLayout& l, const voi
   ca.label_offset = 0; ca.local_max = nullptr; ca.local_sum = nullptr; ca.target_logits = nullptr;
   {
     ScopedTimer timer(kClassCombine, stream);
-    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock), 256, 0, stream>>>(ca);
+    lce_combine_loss_kernel<T><<<(int)ceil_div(m, kCombineRowsPerBlock),
+                                64 * kCombineRowsPerBlock, 0, stream>>>(ca);
     TLCE_LAUNCH_CHECK();
     if (int rc = launch_kl_finish(losses, loss_part, tsum_part, pd.n_vtiles, pd.mp, draft_lse, m,
                                   stream))

@@ -308,19 +308,21 @@ struct CombineArgs {
   bool weight_dim_first = false;     // weight is [h, v]: the label's column is read with stride v
 };
 
-// Dot product of two rows of length h by one wave (every lane gets the sum):
-// 16 bytes per lane and load for 2-byte types when the rows allow it.
+// Dot product of two rows of length h by one wave (every lane gets the sum): 16 bytes per lane
+// and load when the rows allow it, several loads in flight.
 template <typename T>
 __device__ __forceinline__ float wave_dot(const T* a_row, const T* b_row, int h, int lane) {
+  constexpr int kVec = 16 / sizeof(T);
   float dot = 0.0f;
-  if (sizeof(T) == 2 && (h % 8) == 0 &&
+  if ((h % kVec) == 0 &&
       ((reinterpret_cast<uintptr_t>(a_row) | reinterpret_cast<uintptr_t>(b_row)) & 15) == 0) {
-    typedef T v8_t __attribute__((ext_vector_type(8)));
-    for (int k = lane * 8; k < h; k += 64 * 8) {
-      const v8_t a = *reinterpret_cast<const v8_t*>(a_row + k);
-      const v8_t b = *reinterpret_cast<const v8_t*>(b_row + k);
+    typedef T vec_t __attribute__((ext_vector_type(kVec)));
+#pragma unroll 4
+    for (int k = lane * kVec; k < h; k += 64 * kVec) {
+      const vec_t a = *reinterpret_cast<const vec_t*>(a_row + k);
+      const vec_t b = *reinterpret_cast<const vec_t*>(b_row + k);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) dot = fmaf(to_float<T>(a[e]), to_float<T>(b[e]), dot);
+      for (int e = 0; e < kVec; ++e) dot = fmaf(to_float<T>(a[e]), to_float<T>(b[e]), dot);
     }
   } else {
     for (int k = lane; k < h; k += 64) dot = fmaf(to_float<T>(a_row[k]), to_float<T>(b_row[k]), dot);
@@ -328,13 +330,77 @@ __device__ __forceinline__ float wave_dot(const T* a_row, const T* b_row, int h,
   return wave_sum(dot);
 }
 
-// Rows per workgroup of lce_combine_loss_kernel: 4 waves x 4 rows, so that the
-// count of valid rows costs one global atomic per 16 rows (one per row
-// serialises 32768 atomics on a single address: two thirds of this kernel).
+// Rows per workgroup of lce_combine_loss_kernel, a wave each: what bounds it is the latency of
+// dependent loads (label, its row of the head), which four rows per wave paid four times: 2741 rows,
+// H = 2048, 23 splits 18 us, now 11.5; 8192 rows with partials of 594 tiles 67 us, now 40.
+// The count of valid rows costs one global atomic per 16 rows (one per row serialises 32768 atomics
+// on a single address: two thirds of this kernel).
 constexpr int kCombineRowsPerBlock = 16;
 
+// One row of it, by one wave; whether the row has a loss.
 template <typename T>
-__global__ __launch_bounds__(256) void lce_combine_loss_kernel(CombineArgs p) {
+__device__ __forceinline__ bool combine_row(const CombineArgs& p, int r, int lane) {
+  float mx = -INFINITY;
+  for (int s = lane; s < p.nsplit; s += 64)
+    mx = fmaxf(mx, p.part_max[(int64_t)s * p.part_ld + r]);
+  mx = wave_max(mx);
+  float sum = 0.0f;
+  for (int s = lane; s < p.nsplit; s += 64) {
+    const float pm = p.part_max[(int64_t)s * p.part_ld + r];
+    if (pm > -INFINITY) sum += p.part_sum[(int64_t)s * p.part_ld + r] * exp2_of<sizeof(T) == 4>(pm - mx);
+  }
+  sum = wave_sum(sum);
+  const float lse = (mx + log2f(sum)) * TLCE_LN2;
+
+  if (p.labels == nullptr) {   // statistics only (soft embedding): no targets, no loss
+    if (lane == 0) p.lse[r] = lse;
+    return false;
+  }
+  const int64_t label = p.labels[r];
+  const bool valid = (label != p.ignore);
+  const int64_t y = label - p.label_offset;   // row of the label in this weight
+  const bool here = valid && y >= 0 && y < p.v;
+  const bool has_target = here && label != p.exclude;
+  float target = 0.0f;
+  if (has_target) {
+    const T* hrow = static_cast<const T*>(p.hidden) + (int64_t)r * p.h;
+    float dot;
+    if (p.weight_dim_first) {
+      const T* wcol = static_cast<const T*>(p.weight) + y;
+      float part = 0.0f;
+      for (int k = lane; k < p.h; k += 64)
+        part = fmaf(to_float<T>(hrow[k]), to_float<T>(wcol[(int64_t)k * p.v]), part);
+      dot = wave_sum(part) * p.logit_scale;
+    } else {
+      const T* wrow = static_cast<const T*>(p.weight) + y * (int64_t)p.h;
+      dot = wave_dot<T>(hrow, wrow, p.h, lane) * p.logit_scale;
+    }
+    if (p.bias != nullptr) dot += p.bias[y];
+    if (p.softcap > 0.0f) dot = p.softcap * tanhf(dot / p.softcap);
+    target = dot;
+  }
+  if (lane == 0) {
+    if (p.local_max != nullptr) {
+      // the partials are in base-2 units: max2 = max * log2(e), sum = sum exp(z - max)
+      p.local_max[r] = mx * TLCE_LN2;
+      p.local_sum[r] = (mx > -INFINITY) ? sum : 0.0f;
+      p.target_logits[r] = (here && label == p.exclude) ? -INFINITY : target;
+    } else {
+      p.lse[r] = lse;
+      const float loss = valid ? (lse - target) : 0.0f;
+      if (p.losses != nullptr) {
+        const int64_t o = (p.row_idx != nullptr) ? p.row_idx[r] : (int64_t)r;
+        p.losses[o] = loss;
+      }
+      if (p.weighted != nullptr)
+        p.weighted[r] = (p.token_weights != nullptr) ? loss * p.token_weights[r] : loss;
+    }
+  }
+  return valid;
+}
+
+template <typename T>
+__global__ __launch_bounds__(64 * kCombineRowsPerBlock) void lce_combine_loss_kernel(CombineArgs p) {
   __shared__ int block_valid;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -346,73 +412,13 @@ __global__ __launch_bounds__(256) void lce_combine_loss_kernel(CombineArgs p) {
     p.nsplit = forward_vocab_splits(n_ttiles, p.n_vtiles, resident_workgroups(p.tile));
     p.part_ld = n_ttiles * p.tile;
   }
-  int wave_valid = 0;
-  for (int i = 0; i < kCombineRowsPerBlock / 4; ++i) {
-    const int r = blockIdx.x * kCombineRowsPerBlock + wave * (kCombineRowsPerBlock / 4) + i;
-    if (r >= p.m) {
-      if (p.weighted != nullptr && r < p.weighted_rows && lane == 0) p.weighted[r] = 0.0f;
-      continue;
-    }
-    float mx = -INFINITY;
-    for (int s = lane; s < p.nsplit; s += 64)
-      mx = fmaxf(mx, p.part_max[(int64_t)s * p.part_ld + r]);
-    mx = wave_max(mx);
-    float sum = 0.0f;
-    for (int s = lane; s < p.nsplit; s += 64) {
-      const float pm = p.part_max[(int64_t)s * p.part_ld + r];
-      if (pm > -INFINITY) sum += p.part_sum[(int64_t)s * p.part_ld + r] * exp2_of<sizeof(T) == 4>(pm - mx);
-    }
-    sum = wave_sum(sum);
-    const float lse = (mx + log2f(sum)) * TLCE_LN2;
-
-    if (p.labels == nullptr) {   // statistics only (soft embedding): no targets, no loss
-      if (lane == 0) p.lse[r] = lse;
-      continue;
-    }
-    const int64_t label = p.labels[r];
-    const bool valid = (label != p.ignore);
-    const int64_t y = label - p.label_offset;   // row of the label in this weight
-    const bool here = valid && y >= 0 && y < p.v;
-    const bool has_target = here && label != p.exclude;
-    float target = 0.0f;
-    if (has_target) {
-      const T* hrow = static_cast<const T*>(p.hidden) + (int64_t)r * p.h;
-      float dot;
-      if (p.weight_dim_first) {
-        const T* wcol = static_cast<const T*>(p.weight) + y;
-        float part = 0.0f;
-        for (int k = lane; k < p.h; k += 64)
-          part = fmaf(to_float<T>(hrow[k]), to_float<T>(wcol[(int64_t)k * p.v]), part);
-        dot = wave_sum(part) * p.logit_scale;
-      } else {
-        const T* wrow = static_cast<const T*>(p.weight) + y * (int64_t)p.h;
-        dot = wave_dot<T>(hrow, wrow, p.h, lane) * p.logit_scale;
-      }
-      if (p.bias != nullptr) dot += p.bias[y];
-      if (p.softcap > 0.0f) dot = p.softcap * tanhf(dot / p.softcap);
-      target = dot;
-    }
-    if (lane == 0) {
-      if (p.local_max != nullptr) {
-        // the partials are in base-2 units: max2 = max * log2(e), sum = sum exp(z - max)
-        p.local_max[r] = mx * TLCE_LN2;
-        p.local_sum[r] = (mx > -INFINITY) ? sum : 0.0f;
-        p.target_logits[r] = (here && label == p.exclude) ? -INFINITY : target;
-      } else {
-        p.lse[r] = lse;
-        const float loss = valid ? (lse - target) : 0.0f;
-        if (p.losses != nullptr) {
-          const int64_t o = (p.row_idx != nullptr) ? p.row_idx[r] : (int64_t)r;
-          p.losses[o] = loss;
-        }
-        if (p.weighted != nullptr)
-          p.weighted[r] = (p.token_weights != nullptr) ? loss * p.token_weights[r] : loss;
-      }
-    }
-    wave_valid += valid ? 1 : 0;
+  const int r = blockIdx.x * kCombineRowsPerBlock + wave;
+  if (r < p.m) {
+    if (combine_row<T>(p, r, lane) && lane == 0) atomicAdd(&block_valid, 1);
+  } else if (p.weighted != nullptr && r < p.weighted_rows && lane == 0) {
+    p.weighted[r] = 0.0f;
   }
   if (p.valid_count == nullptr) return;   // uniform: statistics-only callers
-  if (lane == 0 && wave_valid != 0) atomicAdd(&block_valid, wave_valid);
   __syncthreads();
   if (threadIdx.x == 0 && block_valid != 0) atomicAdd(p.valid_count, (float)block_valid);
 }

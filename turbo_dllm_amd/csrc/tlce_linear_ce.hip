@@ -102,7 +102,8 @@ int launch_label_logit(LabelLogitArgs a, hipStream_t stream) {
   ScopedTimer timer(kClassCombine, stream);
   const int64_t clear =
       a.losses != nullptr || a.row_of != nullptr ? ceil_div(a.n_out, kClearPerBlock) : 0;
-  lce_label_logit_kernel<T><<<(int)(ceil_div(a.m, 16) + a.n_count + clear), 256, 0, stream>>>(a);
+  lce_label_logit_kernel<T><<<(int)(ceil_div(a.m, kLabelRows) + a.n_count + clear),
+                              kLabelThreads, 0, stream>>>(a);
   TLCE_LAUNCH_CHECK();
   return 0;
 }
