@@ -101,17 +101,24 @@ __host__ __device__ static inline int forward_vocab_splits(int n_ttiles, int n_v
 // or 32 wide): the host plan and the kernels that re-plan for a row count known on the
 // device must agree.
 constexpr int kMaxKSplits = 64;
-__host__ __device__ static inline int grad_hidden_k_splits(int64_t tiles, int max_split,
-                                                           int64_t k_steps, int64_t slab_elems,
-                                                           int resident = 256) {
-  const int64_t per_slab = (slab_elems >> 17) > 1 ? (slab_elems >> 17) : 1;
+// The estimate for `ks` splits; per_slab: k_split_slab_cost.
+__host__ __device__ static inline int64_t k_split_cost(int64_t tiles, int ks, int64_t k_steps,
+                                                       int64_t per_slab, int resident) {
   const int shift = 31 - __builtin_clz(resident);
+  const int64_t rounds = (tiles * ks + resident - 1) >> shift;
+  const int64_t steps = ((uint32_t)k_steps + (uint32_t)ks - 1) / (uint32_t)ks;
+  return rounds * 8 * (steps + 8) + ks * per_slab;
+}
+__host__ __device__ static inline int64_t k_split_slab_cost(int64_t slab_elems) {
+  return (slab_elems >> 17) > 1 ? (slab_elems >> 17) : 1;
+}
+static inline int grad_hidden_k_splits(int64_t tiles, int max_split, int64_t k_steps,
+                                       int64_t slab_elems, int resident = 256) {
+  const int64_t per_slab = k_split_slab_cost(slab_elems);
   int pick = 1;
   int64_t best = -1;
   for (int ks = 1; ks <= max_split; ++ks) {
-    const int64_t rounds = (tiles * ks + resident - 1) >> shift;
-    const int64_t steps = ((uint32_t)k_steps + (uint32_t)ks - 1) / (uint32_t)ks;
-    const int64_t cost = rounds * 8 * (steps + 8) + ks * per_slab;
+    const int64_t cost = k_split_cost(tiles, ks, k_steps, per_slab, resident);
     if (best < 0 || cost < best) {
       best = cost;
       pick = ks;

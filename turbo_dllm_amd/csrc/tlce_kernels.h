@@ -1484,16 +1484,30 @@ struct GemmArgs {
 
 // K splits and slab stride the grad_hidden contraction uses for a device-side
 // row count: the host plan's rule applied to the real number of token tiles,
-// limited to the splits launched and to the slab memory the plan allocated.
+// limited to the splits launched (at most kMaxKSplits) and to the slab memory the plan
+// allocated.  A lane per candidate, by all lanes of a wave: one after the other they took 4 us of
+// the slab reduction (16 candidates, 1036 of 2048 rows, H = 1024: 15 -> 12.8 us).
 __device__ __forceinline__ int dynamic_k_splits(int n_ttiles, int n_htiles, int tile, int h,
                                                 int launched, int64_t slab_budget, int k_steps,
                                                 int64_t* stride) {
+  static_assert(kMaxKSplits <= 64, "a lane per candidate");
+  const int lane = threadIdx.x & 63;
   const int64_t slab = (int64_t)n_ttiles * tile * h;
-  int ks = grad_hidden_k_splits((int64_t)n_ttiles * n_htiles, launched, k_steps, slab,
-                                resident_workgroups(tile));
-  while (ks > 1 && ks * slab > slab_budget) --ks;
+  const int64_t cost = lane < launched
+                           ? k_split_cost((int64_t)n_ttiles * n_htiles, lane + 1, k_steps,
+                                          k_split_slab_cost(slab), resident_workgroups(tile))
+                           : INT64_MAX;
+  int64_t best = cost;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const int64_t other = __shfl_xor(best, o, 64);
+    best = other < best ? other : best;
+  }
+  // the first of the cheapest, and no more than the slabs hold
+  const int pick = __builtin_ctzll(__ballot(cost == best)) + 1;
+  const int held = __popcll(__ballot(lane == 0 || (lane + 1) * slab <= slab_budget));
   *stride = slab;
-  return ks;
+  return pick < held ? pick : held;
 }
 enum { kRowsFollow = 1, kKFollows = 2 };
 // Output tiles per K split below which lce_gemm_nt_kernel orders its workgroups
