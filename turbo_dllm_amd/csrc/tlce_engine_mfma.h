@@ -619,6 +619,14 @@ struct DirectToLdsEngine : DirectTileLayout<T_, kTN_> {
     __builtin_amdgcn_sched_barrier(0);
   }
 
+  // Every accumulator as a value of its own, in its register, at this place.
+  static __device__ __forceinline__ void pin(Acc& acc) {
+#pragma unroll
+    for (int q = 0; q < kTM; ++q)
+#pragma unroll
+      for (int t = 0; t < kTN; ++t) asm volatile("" : "+a"(acc.c[q][t]));
+  }
+
   // acc = A-tile * B-tile^T over K in [k_begin, k_end), not empty and a multiple of 64 wide
   // (with column tails, of K-contiguous operands: 65 wide at least and no such multiple, and
   // the rows of B hold zeros up to the next one)
@@ -724,6 +732,9 @@ struct DirectToLdsEngine : DirectTileLayout<T_, kTN_> {
       issue(2);
     }
     Base::zero(acc);
+    // a zero of its own per accumulator: left to the compiler they are copies of one another,
+    // made in front of every loop they enter
+    pin(acc);
     if (nk > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * kTileLoads) : "memory");
     else if (nk == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kTileLoads) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -739,6 +750,12 @@ struct DirectToLdsEngine : DirectTileLayout<T_, kTN_> {
     if (k + 3 == nk) step(k++, Left2{});
     if (k + 2 == nk) step(k++, Left1{});
     step(k, Left0{});
+    // as long as mfma_drain: the builtin's own distance is shorter, and the epilogue's
+    // statements read accumulators without the compiler's knowledge of what wrote them
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 7");
+    pin(acc);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
   }
 
