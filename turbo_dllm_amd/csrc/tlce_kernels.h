@@ -1047,14 +1047,21 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_ke
     const char* tile_in =
         reinterpret_cast<const char*>(panel_in + (int64_t)tt * E::kTile * ld_in + prow);
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
-#pragma unroll 4
-    for (int it = 0; it < (E::kTile * 32) / E::kThreads; ++it) {
-      const int first = (it * E::kThreads + (int)(threadIdx.x & ~63u)) >> 5;   // of two tokens
-      const int tok = first + ((threadIdx.x & 63) >> 5);
-      const int ch = (threadIdx.x & 31) ^ (tok & 31);
-      E::load_to_lds(__builtin_amdgcn_readfirstlane(lds0 + (unsigned)first * 512),
-                     (unsigned)(tok * ld_in * (int)sizeof(T) + ch * 16), tile_in);
+    constexpr int kTokens = E::kThreads / 32;     // of a round of the workgroup
+    constexpr int kRounds = 32 / kTokens;         // until the slots repeat
+    const int first = (int)(threadIdx.x & ~63u) >> 5;   // of two tokens of a wave
+    const unsigned fill = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)first * 512);
+    unsigned off[kRounds];
+#pragma unroll
+    for (int q = 0; q < kRounds; ++q) {
+      const int tok = q * kTokens + first + ((threadIdx.x & 63) >> 5);
+      const int ch = (threadIdx.x & 31) ^ tok;
+      off[q] = (unsigned)(tok * ld_in * (int)sizeof(T) + ch * 16);
     }
+#pragma unroll
+    for (int it = 0; it < E::kTile / kTokens; ++it)
+      E::load_to_lds(fill + (unsigned)(it * kTokens * 512), off[it % kRounds],
+                     tile_in + (int64_t)(it / kRounds) * 32 * ld_in * (int)sizeof(T));
   }
   const float inv_cap = kSoftcap ? 1.0f / p.softcap : 0.0f;
   // Only the last vocabulary tile has rows past v: a workgroup-uniform branch, as the VALU work
