@@ -92,6 +92,7 @@ struct Plan {
   int n_panels;
   int dh_ksplit;
   int dh_max_ksplit;  // upper bound of the rule that chose dh_ksplit
+  int64_t dh_slab_rows;   // rows of all K-split slabs together
 };
 
 inline int engine_class(int64_t h, int dtype) {
@@ -179,6 +180,13 @@ inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_gr
     p.dh_ksplit = grad_hidden_k_splits((int64_t)p.n_ttiles * p.n_htiles, p.dh_max_ksplit,
                                        p.vc / p.bk, p.mp * h, resident_workgroups(p.tile));
   }
+  // A row count on the device may leave fewer tiles, and more splits of them, than m rows have:
+  // slabs for one round of workgroups, so that it gets the splits of a call with that many rows.
+  // 2240 of 3200 rows, H = 2112 (81 of 117 tiles) take three splits and not the plan's two.
+  p.dh_slab_rows =
+      std::max(p.dh_ksplit * p.mp,
+               std::min<int64_t>(ceil_div(resident_workgroups(p.tile), p.n_htiles),
+                                 (int64_t)p.n_ttiles * p.dh_max_ksplit) * p.tile);
   return p;
 }
 
@@ -275,7 +283,7 @@ inline BackwardLayout backward_layout(const Plan& p, int64_t m, int64_t h, int d
   const int64_t es = dtype_bytes(dtype);
   int64_t off = 0;
   l.scale = off; off += align256(p.mp * 4);
-  l.acc32 = off; off += align256(p.mp * h * 4 * p.dh_ksplit);   // one slab per K split
+  l.acc32 = off; off += align256(p.dh_slab_rows * h * 4);   // one slab per K split
   const bool direct = p.engine == 2;
   l.wt = off;    off += direct ? k_tail_bytes(p.v, h) : p.kmajor ? 0 : align256(h * p.vp * es);
   l.ht = off;
@@ -624,7 +632,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     dh.c_split_stride = p.mp * h;
     dh.mode = (panel == 0) ? kStoreF32 : kAddF32;
     dh.m_dev = m_dev; dh.m_role = kRowsFollow;
-    dh.slab_budget = (int64_t)p.dh_ksplit * p.mp * h;
+    dh.slab_budget = p.dh_slab_rows * h;
     dh.k_steps_plan = (int)(p.vc / p.bk);
     GemmArgs dw;
     dw.m_dev = m_dev; dw.m_role = kKFollows; dw.m_round = p.bk;
@@ -707,8 +715,8 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
   {
     ScopedTimer timer(kClassOther, stream);
     lce_finalize_grad_hidden_kernel<T><<<(int)m, 256, 0, stream>>>(
-        acc32, p.dh_ksplit, p.mp * h, row_idx, (int)m, (int)h, static_cast<T*>(grad_hidden),
-        m_dev, p.n_htiles, p.tile, dh_launch_ksplit, (int)(p.vc / p.bk));
+        acc32, p.dh_ksplit, p.mp * h, p.dh_slab_rows * h, row_idx, (int)m, (int)h,
+        static_cast<T*>(grad_hidden), m_dev, p.n_htiles, p.tile, dh_launch_ksplit, (int)(p.vc / p.bk));
   }
   TLCE_LAUNCH_CHECK();
   return 0;

@@ -1874,7 +1874,7 @@ __global__ __launch_bounds__(256) void lce_transpose_pad_kernel(const T* __restr
 // K-split reduction and the un-compaction scatter).
 template <typename T>
 __global__ __launch_bounds__(256) void lce_finalize_grad_hidden_kernel(
-    const float* __restrict__ acc32, int n_splits, int64_t split_stride,
+    const float* __restrict__ acc32, int n_splits, int64_t split_stride, int64_t slab_budget,
     const int64_t* __restrict__ row_idx, int m, int h, T* __restrict__ out,
     const int64_t* __restrict__ m_dev, int n_htiles, int tile, int launched_splits,
     int k_steps_plan) {
@@ -1883,7 +1883,7 @@ __global__ __launch_bounds__(256) void lce_finalize_grad_hidden_kernel(
     // the splits and slab stride the contraction derived from the real row count
     m = effective_rows(m, m_dev);
     n_splits = dynamic_k_splits((m + tile - 1) / tile, n_htiles, tile, h, launched_splits,
-                                (int64_t)n_splits * split_stride, k_steps_plan, &split_stride);
+                                slab_budget, k_steps_plan, &split_stride);
   }
   if (r >= m) return;
   const int64_t o = (row_idx != nullptr) ? row_idx[r] : (int64_t)r;

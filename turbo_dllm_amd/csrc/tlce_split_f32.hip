@@ -177,7 +177,7 @@ int split_backward(const SplitPlan& p, const void* hidden, const void* weight, c
   }
   ScopedTimer timer(kClassOther, stream);
   lce_finalize_grad_hidden_kernel<float><<<(int)m, 256, 0, stream>>>(
-      acc32, p.dh_ksplit, p.mp * h, row_idx, (int)m, (int)h, static_cast<float*>(grad_hidden),
+      acc32, p.dh_ksplit, p.mp * h, 0, row_idx, (int)m, (int)h, static_cast<float*>(grad_hidden),
       nullptr, p.n_htiles, 256, p.dh_ksplit, p.k_steps);
   TLCE_LAUNCH_CHECK();
   return 0;
