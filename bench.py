@@ -581,7 +581,7 @@ def main() -> int:
                     panel_bytes=panel)
             del grad_hidden32, kept
         elif count is not None:
-            keep = (native.kept_logits_buffer(m_rows, rows, v, None)
+            keep = (native.kept_logits_buffer(m_rows, rows, v, None, n)
                     if args.gradients == "forward" and on_device is None else None)
             kw = dict(m=m_rows, row_idx=row_idx, row_count=count, n_out=n, ignore_index=-100,
                       exclude_index=-1, logit_softcap=softcap, kept=keep)

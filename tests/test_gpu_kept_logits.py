@@ -160,3 +160,22 @@ def test_what_keeps_nothing(gpu_device, monkeypatch):
         native.masked_loss_forward(
             hidden.float(), weight.float(), None, labels, None, ignore_index=-100, exclude_index=-1,
             logit_softcap=0.0, kept=torch.empty(1 << 20, dtype=torch.uint8, device=gpu_device))
+
+
+def test_a_backward_without_memory_beside_the_logits(gpu_device, monkeypatch):
+    """It recomputes them in the place they are given back from: the same gradients."""
+    hidden, weight, labels, up = operands(gpu_device, 600, 1024, 3001, ignored=0.4)
+    inner, refused = native.masked_loss_backward, []
+
+    def without_memory(*args, kept=None, **keywords):
+        if kept is not None:
+            refused.append(kept)
+            raise torch.OutOfMemoryError("no room")
+        return inner(*args, kept=kept, **keywords)
+
+    want = step(hidden, weight, labels, up, "none")
+    monkeypatch.setattr(native, "masked_loss_backward", without_memory)
+    got = step(hidden, weight, labels, up, "none")
+    assert len(refused) == 1 and refused[0].untyped_storage().size() == 0
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

@@ -1088,41 +1088,60 @@ def backward_frozen_weight(
 
 
 # ------------------------------------------------- logits kept for the backward --
-# Held between forward and backward without asking how much memory there is: the recomputing
-# backward's own default panel.  Beyond that an eighth of what is free, so that what the backward
-# allocates next finds room, and a twenty-fourth of the device (12 GiB of 288).  Which tiles are
-# kept changes no result, so the answer may differ from call to call.
-_KEEP_UNASKED_BYTES = 1 << 30
+# Which tiles are kept changes no result, so the answer of the two below may differ from call to
+# call.
+def _memory_left(device: torch.device) -> tuple[int, int]:
+    """Bytes that allocations can still get, and those of the device.  Of what torch's allocator
+    holds without using it, whole segments count; pieces of segments in use do not."""
+    free, total = torch.cuda.mem_get_info(device)
+    stats = torch.cuda.memory_stats_as_nested_dict(device)
+    if stats:
+        free += (stats["reserved_bytes"]["all"]["current"]
+                 - stats["active_bytes"]["all"]["current"]
+                 - stats["inactive_split_bytes"]["all"]["current"])
+    return free, total
 
 
-def kept_logits_buffer(m: int, hidden: torch.Tensor, vocab: int,
-                       bias: torch.Tensor | None) -> torch.Tensor | None:
-    """Where the forward of a recomputing cross entropy over ``m`` rows leaves its logits for
-    the backward (``masked_loss_forward(kept=...)``), or None when it is to recompute all of
+def kept_logits_buffer(m: int, hidden: torch.Tensor, vocab: int, bias: torch.Tensor | None,
+                       n_out: int) -> torch.Tensor | None:
+    """Where the forward of a recomputing cross entropy over ``m`` of ``n_out`` rows leaves its
+    logits for the backward (``masked_loss_forward(kept=...)``), or None when it is to recompute all of
     them: operands or sizes that gain nothing, the gradient mode "recompute", a call that is
-    being captured, whose graph would hold the buffer.  A panel budget bounds it as well."""
+    being captured, whose graph would hold the buffer.  A panel budget bounds it as well.
+
+    It takes an eighth of the memory left, so that what is allocated until the backward finds
+    room, a twenty-fourth of the device (12 GiB of 288), and nothing that the backward's own
+    workspace and gradients need beside it.  (Asking takes 10 us.)"""
     if m == 0 or options.get_gradient_mode() != "forward" or hidden.dtype not in _DTYPE_CODES:
         return None
     lib = _lib.library()
     h, code, has_bias = hidden.shape[1], _dtype_code(hidden), int(bias is not None)
-    budget = get_panel_bytes() or (1 << 62)
-    nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, budget)
+    budget = get_panel_bytes()
+    nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, budget or (1 << 62))
     if nbytes <= 0 or torch.cuda.is_current_stream_capturing():
         return None
-    device = hidden.device
-    if nbytes > _KEEP_UNASKED_BYTES:
-        free, total = torch.cuda.mem_get_info(device)
-        stats = torch.cuda.memory_stats_as_nested_dict(device)
-        cached = (stats["reserved_bytes"]["all"]["current"]
-                  - stats["allocated_bytes"]["all"]["current"]) if stats else 0
-        room = max(min((free + cached) // 8, total // 24), _KEEP_UNASKED_BYTES)
-        nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, min(nbytes, room))
-        if nbytes <= 0:
-            return None
+    left, total = _memory_left(hidden.device)
+    backward = (lib.tlce_backward_workspace_bytes(m, h, vocab, code, 1, has_bias, budget)
+                + (n_out + vocab) * h * hidden.element_size())
+    room = min(left // 8, total // 24, left - backward)
+    nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, max(min(nbytes, room), 0))
+    if nbytes <= 0:
+        return None
     try:
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return torch.empty(nbytes, dtype=torch.uint8, device=hidden.device)
     except torch.OutOfMemoryError:
         return None
+
+
+def from_kept_logits(kept: torch.Tensor | None, call):
+    """``call(kept)``; where it finds no memory beside the kept logits, theirs is given back and
+    ``call(None)`` recomputes them."""
+    if kept is not None and kept.untyped_storage().size() > 0:
+        try:
+            return call(kept)
+        except torch.OutOfMemoryError:
+            kept.untyped_storage().resize_(0)   # (a retained graph's next backward finds none)
+    return call(None)
 
 
 # Calls whose logits all fit this with every row in them: the row count stays on the device, as

@@ -116,7 +116,7 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
             return loss
         kept = None
         if (mode != "device" or keeps_uncounted) and (wants_grad or ctx.needs_input_grad[2]):
-            kept = native.kept_logits_buffer(m, rows, weight.shape[0], bias)
+            kept = native.kept_logits_buffer(m, rows, weight.shape[0], bias, n)
         _, lse, _, weighted_sum = native.masked_loss_forward(
             rows, weight, bias, targets, token_weights, m=m, row_idx=row_idx,
             row_count=row_count, n_out=n, ignore_index=-100, exclude_index=exclude_index,
@@ -141,13 +141,14 @@ class _FusedMaskedTokenLoss(torch.autograd.Function):
         rows, weight, bias, targets, token_weights, lse, row_idx, row_count, kept = (
             ctx.saved_tensors)
         with native.panel_budget(ctx.panel_bytes):
-            grad_hidden, grad_weight, grad_bias = native.masked_loss_backward(
-                rows, weight, bias, targets, token_weights, lse, None, grad_output,
-                reduction="sum", m=ctx.m, row_idx=row_idx, row_count=row_count, n_out=ctx.n_rows,
-                ignore_index=-100, exclude_index=ctx.exclude_index,
-                logit_softcap=ctx.logit_softcap, logit_multiplier=ctx.multiplier,
-                compute_weight_grad=ctx.needs_input_grad[1], kept=kept,
-            )
+            grad_hidden, grad_weight, grad_bias = native.from_kept_logits(
+                kept, lambda kept: native.masked_loss_backward(
+                    rows, weight, bias, targets, token_weights, lse, None, grad_output,
+                    reduction="sum", m=ctx.m, row_idx=row_idx, row_count=row_count,
+                    n_out=ctx.n_rows, ignore_index=-100, exclude_index=ctx.exclude_index,
+                    logit_softcap=ctx.logit_softcap, logit_multiplier=ctx.multiplier,
+                    compute_weight_grad=ctx.needs_input_grad[1], kept=kept,
+                ))
         return (
             grad_hidden.reshape(ctx.hidden_shape),
             grad_weight if ctx.needs_input_grad[1] else None,
@@ -225,7 +226,8 @@ class _FusedTokenLosses(torch.autograd.Function):
         weight = weight.contiguous()
         kept = None
         if any(ctx.needs_input_grad[:3]):
-            kept = native.kept_logits_buffer(rows.shape[0], rows, weight.shape[0], bias)
+            kept = native.kept_logits_buffer(rows.shape[0], rows, weight.shape[0], bias,
+                                             rows.shape[0])
         losses, lse, valid_count, _ = native.masked_loss_forward(
             rows, weight, bias, targets, None, ignore_index=-100, exclude_index=-1,
             logit_softcap=logit_softcap, logit_multiplier=multiplier,
@@ -243,12 +245,13 @@ class _FusedTokenLosses(torch.autograd.Function):
 
         rows, weight, bias, targets, lse, valid_count, kept = ctx.saved_tensors
         with native.panel_budget(ctx.panel_bytes):
-            grad_hidden, grad_weight, grad_bias = native.masked_loss_backward(
-                rows, weight, bias, targets, None, lse, valid_count, grad_output,
-                reduction="none", ignore_index=-100, exclude_index=-1,
-                logit_softcap=ctx.logit_softcap, logit_multiplier=ctx.multiplier,
-                compute_weight_grad=ctx.needs_input_grad[1], kept=kept,
-            )
+            grad_hidden, grad_weight, grad_bias = native.from_kept_logits(
+                kept, lambda kept: native.masked_loss_backward(
+                    rows, weight, bias, targets, None, lse, valid_count, grad_output,
+                    reduction="none", ignore_index=-100, exclude_index=-1,
+                    logit_softcap=ctx.logit_softcap, logit_multiplier=ctx.multiplier,
+                    compute_weight_grad=ctx.needs_input_grad[1], kept=kept,
+                ))
         return (
             grad_hidden.reshape(ctx.hidden_shape),
             grad_weight if ctx.needs_input_grad[1] else None,

@@ -358,7 +358,7 @@ def _device_forward(ctx, hidden, weight, bias, labels, reduction, ignore_index, 
     # them is small)
     kept = None
     if (mode != "device" or keeps_uncounted) and (wants_grad or ctx.needs_input_grad[2]):
-        kept = native.kept_logits_buffer(m, rows, weight_vf.shape[1 if in_place else 0], bias)
+        kept = native.kept_logits_buffer(m, rows, weight_vf.shape[1 if in_place else 0], bias, n)
     if row_count is None and kept is None:
         losses, lse, valid_count = native.forward(
             rows, weight_vf, bias, targets,
@@ -413,24 +413,27 @@ def _device_backward(ctx, grad_output, frozen: bool):
         return (grad_hidden.reshape(ctx.hidden_shape), None if frozen else grad_weight,
                 None) + (None,) * 9
     rows, weight_vf, bias, targets, lse, valid_count, row_idx, row_count, kept = ctx.saved_tensors
-    with native.panel_budget(ctx.panel_bytes):
+
+    def gradients(kept):
         if row_count is None and kept is None:
             call = native.backward_frozen_weight if frozen else native.backward
-            grad_hidden, grad_weight, grad_bias = call(
+            return call(
                 rows, weight_vf, bias, targets, lse, valid_count, grad_output,
                 row_block_size=0, reduction=ctx.reduction, ignore_index=ctx.ignore_index,
                 exclude_index=ctx.exclude_index, logit_softcap=ctx.logit_softcap,
                 compute_dtype=ctx.compute_dtype, weight_dim_first=ctx.in_place,
                 row_idx=row_idx, n_out=ctx.n_rows,
             )
-        else:
-            grad_hidden, grad_weight, grad_bias = native.masked_loss_backward(
-                rows, weight_vf, bias, targets, None, lse, valid_count, grad_output,
-                reduction=ctx.reduction, m=ctx.m, row_idx=row_idx, row_count=row_count,
-                n_out=ctx.n_rows, ignore_index=ctx.ignore_index, exclude_index=ctx.exclude_index,
-                logit_softcap=ctx.logit_softcap, compute_weight_grad=not frozen, kept=kept,
-                weight_dim_first=ctx.in_place,
-            )
+        return native.masked_loss_backward(
+            rows, weight_vf, bias, targets, None, lse, valid_count, grad_output,
+            reduction=ctx.reduction, m=ctx.m, row_idx=row_idx, row_count=row_count,
+            n_out=ctx.n_rows, ignore_index=ctx.ignore_index, exclude_index=ctx.exclude_index,
+            logit_softcap=ctx.logit_softcap, compute_weight_grad=not frozen, kept=kept,
+            weight_dim_first=ctx.in_place,
+        )
+
+    with native.panel_budget(ctx.panel_bytes):
+        grad_hidden, grad_weight, grad_bias = native.from_kept_logits(kept, gradients)
     if not frozen and ctx.weight_dim_first and not ctx.in_place:
         grad_weight = grad_weight.t().contiguous()
     return (
