@@ -56,3 +56,18 @@ def test_a_backward_without_memory_gives_the_logits_back():
     assert tried[2:] == [None]
     with pytest.raises(ValueError):                                     # other errors pass
         native.from_kept_logits(torch.empty(8), lambda buffer: (_ for _ in ()).throw(ValueError))
+
+
+def test_memory_left_of_each_allocator(monkeypatch):
+    def stats(device):
+        if backend == "pluggable":
+            raise RuntimeError("CUDAPluggableAllocator does not yet support getDeviceStats.")
+        current = {"reserved_bytes": 100, "active_bytes": 60, "inactive_split_bytes": 30}
+        return {name: {"all": {"current": n}} for name, n in current.items()} if used else {}
+
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (1000, 5000))
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", stats)
+    monkeypatch.setattr(torch.cuda, "get_allocator_backend", lambda: backend)
+    for backend, used, want in (("native", True, 1010), ("native", False, 1000),
+                                ("pluggable", True, 1000)):
+        assert native._memory_left(torch.device("cuda:0")) == (want, 5000)

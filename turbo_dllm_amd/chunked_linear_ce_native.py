@@ -1091,9 +1091,12 @@ def backward_frozen_weight(
 # Which tiles are kept changes no result, so the answer of the two below may differ from call to
 # call.
 def _memory_left(device: torch.device) -> tuple[int, int]:
-    """Bytes that allocations can still get, and those of the device.  Of what torch's allocator
-    holds without using it, whole segments count; pieces of segments in use do not."""
+    """Bytes that allocations can still get, and those of the device.  Of what torch's own
+    allocator holds without using it, whole segments count; pieces of segments in use do not.
+    (Others keep other accounts, and pluggable ones raise when asked for theirs.)"""
     free, total = torch.cuda.mem_get_info(device)
+    if torch.cuda.get_allocator_backend() != "native":
+        return free, total
     stats = torch.cuda.memory_stats_as_nested_dict(device)
     if stats:
         free += (stats["reserved_bytes"]["all"]["current"]
