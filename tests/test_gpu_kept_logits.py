@@ -6,6 +6,7 @@ a panel of the backward."""
 
 import pytest
 import torch
+import torch.utils.checkpoint
 
 from turbo_dllm_amd import _lib, options
 from turbo_dllm_amd import chunked_linear_ce_native as native
@@ -177,5 +178,39 @@ def test_a_backward_without_memory_beside_the_logits(gpu_device, monkeypatch):
     monkeypatch.setattr(native, "masked_loss_backward", without_memory)
     got = step(hidden, weight, labels, up, "none")
     assert len(refused) == 1 and refused[0].untyped_storage().size() == 0
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("loss", ["ce", "tokens", "masked"])
+def test_checkpointing_while_free_memory_changes(gpu_device, monkeypatch, loss):
+    """Non-reentrant checkpointing compares what the forward and its repetition save: logits for
+    which there is room in one of them only must not be among it."""
+    hidden, weight, labels, up = operands(gpu_device, 600, 1024, 3001)
+    head = torch.nn.Linear(1024, 3001, bias=False, device="meta")
+    left = [1 << 40]
+    monkeypatch.setattr(native, "_memory_left", lambda device: (left[0], 1 << 40))
+
+    def gradients(wrap):
+        x = hidden.clone().requires_grad_()
+        head.weight = w = torch.nn.Parameter(weight.clone())
+
+        def forward(x):
+            if loss == "ce":
+                return (tiled_linear_cross_entropy(x, w, labels, reduction="none",
+                                                   dtype=x.dtype) * up).sum()
+            if loss == "tokens":
+                return (native_token_cross_entropy(x, labels, head) * up).sum()
+            return masked_token_loss(x, labels, up, head, valid_token_count=600.0)
+
+        left[0] = 1 << 40
+        result = wrap(forward, x)
+        left[0] = 0
+        result.backward()
+        return [result.detach(), x.grad, w.grad]
+
+    want = gradients(lambda forward, x: forward(x))
+    got = gradients(lambda forward, x: torch.utils.checkpoint.checkpoint(
+        forward, x, use_reentrant=False))
     for a, b in zip(got, want):
         assert torch.equal(a, b)

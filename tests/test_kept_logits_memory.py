@@ -4,6 +4,7 @@ queries run on the host; what the allocator would answer is given."""
 
 import pytest
 import torch
+import torch.utils.checkpoint
 
 from turbo_dllm_amd import _lib
 from turbo_dllm_amd import chunked_linear_ce_native as native
@@ -71,3 +72,20 @@ def test_memory_left_of_each_allocator(monkeypatch):
     for backend, used, want in (("native", True, 1010), ("native", False, 1000),
                                 ("pluggable", True, 1000)):
         assert native._memory_left(torch.device("cuda:0")) == (want, 5000)
+
+
+def test_nothing_is_kept_where_saved_tensors_are_packed(monkeypatch):
+    assert buffer(monkeypatch, 8 * GIB) > 0
+    with torch.autograd.graph.save_on_cpu():
+        assert buffer(monkeypatch, 8 * GIB) == 0
+    seen = []
+
+    def layer(x):
+        seen.append(buffer(monkeypatch, 8 * GIB))
+        return x.sin()
+
+    x = torch.ones(3, requires_grad=True)
+    torch.utils.checkpoint.checkpoint(layer, x, use_reentrant=False).sum().backward()
+    assert seen == [0, 0] and buffer(monkeypatch, 8 * GIB) > 0
+    monkeypatch.delattr(torch._C._autograd, "_top_saved_tensors_default_hooks")
+    assert buffer(monkeypatch, 8 * GIB) == 0

@@ -1088,8 +1088,17 @@ def backward_frozen_weight(
 
 
 # ------------------------------------------------- logits kept for the backward --
-# Which tiles are kept changes no result, so the answer of the two below may differ from call to
-# call.
+# Which tiles are kept changes no result, so the answer of kept_logits_buffer may differ from call
+# to call.  Saved tensors may not where a hook packs them: activation checkpointing compares their
+# number and shapes between a forward and its repetition.
+def _saved_tensors_are_packed() -> bool:
+    """Whether ``torch.autograd.graph.saved_tensors_hooks`` are in force here, as they are under
+    ``torch.utils.checkpoint`` and ``save_on_cpu``.  (torch offers no public question; where it
+    has lost this one, the answer is yes.)"""
+    top = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
+    return top is None or top(True) is not None
+
+
 def _memory_left(device: torch.device) -> tuple[int, int]:
     """Bytes that allocations can still get, and those of the device.  Of what torch's own
     allocator holds without using it, whole segments count; pieces of segments in use do not.
@@ -1110,7 +1119,8 @@ def kept_logits_buffer(m: int, hidden: torch.Tensor, vocab: int, bias: torch.Ten
     """Where the forward of a recomputing cross entropy over ``m`` of ``n_out`` rows leaves its
     logits for the backward (``masked_loss_forward(kept=...)``), or None when it is to recompute all of
     them: operands or sizes that gain nothing, the gradient mode "recompute", a call that is
-    being captured, whose graph would hold the buffer.  A panel budget bounds it as well.
+    being captured, whose graph would hold the buffer, a caller that checkpoints or moves away
+    what is saved for the backward.  A panel budget bounds it as well.
 
     It takes an eighth of the memory left, so that what is allocated until the backward finds
     room, a twenty-fourth of the device (12 GiB of 288), and nothing that the backward's own
@@ -1121,7 +1131,8 @@ def kept_logits_buffer(m: int, hidden: torch.Tensor, vocab: int, bias: torch.Ten
     h, code, has_bias = hidden.shape[1], _dtype_code(hidden), int(bias is not None)
     budget = get_panel_bytes()
     nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, budget or (1 << 62))
-    if nbytes <= 0 or torch.cuda.is_current_stream_capturing():
+    if (nbytes <= 0 or torch.cuda.is_current_stream_capturing()
+            or _saved_tensors_are_packed()):
         return None
     left, total = _memory_left(hidden.device)
     backward = (lib.tlce_backward_workspace_bytes(m, h, vocab, code, 1, has_bias, budget)
