@@ -5,9 +5,10 @@ import pytest
 import torch
 
 from turbo_dllm_amd import _lib
+from turbo_dllm_amd import chunked_linear_ce_native as native
 from turbo_dllm_amd.dflash_kl import frozen_linear_kl
 from turbo_dllm_amd.dflash_linear_topk import frozen_linear_ce_topk
-from turbo_dllm_amd.loss import dflash_token_loss, masked_token_loss
+from turbo_dllm_amd.loss import dflash_token_loss, masked_token_loss, native_token_cross_entropy
 from turbo_dllm_amd.tiled_linear_cross_entropy import tiled_linear_cross_entropy
 
 pytestmark = pytest.mark.gpu
@@ -37,6 +38,12 @@ def drafter(x, w, y, up):
                              loss_kind="paper_ce", normalization_count=counts)
 
 
+def tokens(x, w, y, up):
+    head = torch.nn.Linear(w.shape[1], w.shape[0], bias=False, device="meta")
+    head.weight = w
+    return native_token_cross_entropy(x, y, head, output_multiplier=0.5)
+
+
 def top_k(x, w, y, up):
     return torch.cat([t.flatten().double() for t in
                       frozen_linear_ce_topk(x, w.detach(), y.clamp(min=0), top_k=4)])
@@ -48,7 +55,7 @@ def kl(x, w, y, up):
 
 CALLS = {"none": cross_entropy("none"), "mean": cross_entropy("mean"),
          "dim_first": cross_entropy("sum", dim_first=True), "masked": masked, "drafter": drafter,
-         "top_k": top_k, "kl": kl}
+         "tokens": tokens, "top_k": top_k, "kl": kl}
 SIZES = [
     (200, 192, 1600, torch.bfloat16),       # rows of one tile
     (700, 256, 3008, torch.bfloat16),
@@ -62,7 +69,7 @@ SIZES = [
     (*size, kind) for size in SIZES for kind in CALLS
     if size[3] != torch.float32 or kind != "top_k"])    # (which is plain torch there)
 @pytest.mark.parametrize("inference", [False, True])
-def test_no_gradients_are_formed(gpu_device, m, h, v, dtype, kind, inference):
+def test_no_gradients_are_formed(gpu_device, monkeypatch, m, h, v, dtype, kind, inference):
     print("[case]", m, h, v, dtype, kind, inference, flush=True)
     gen = torch.Generator().manual_seed(m)
     x = torch.randn(m, h, generator=gen).to(dtype).to(gpu_device)
@@ -72,6 +79,11 @@ def test_no_gradients_are_formed(gpu_device, m, h, v, dtype, kind, inference):
     y = y.to(gpu_device)
     up = (torch.rand(m, generator=gen) + 0.5).to(gpu_device)
     call = CALLS[kind]
+
+    def keep(*args):
+        raise AssertionError("logits kept for no backward")
+
+    monkeypatch.setattr(native, "kept_logits_buffer", keep)
     with torch.no_grad():
         want = call(x, torch.nn.Parameter(w, requires_grad=False), y, up)
     x = x.requires_grad_()

@@ -364,7 +364,7 @@ def native_token_cross_entropy(
     if isinstance(weight, torch.Tensor) and weight.dim() == 2 and _fused_path_applies(
             hidden_states, weight, bias, labels, multiplier) and labels.numel() > 0:
         return _FusedTokenLosses.apply(
-            hidden_states, weight, bias, labels, multiplier,
+            *grad_mode_operands(hidden_states, weight, bias), labels, multiplier,
             0.0 if logit_softcap is None else float(logit_softcap),
         )
     if output_multiplier is not None:
