@@ -96,6 +96,32 @@ def test_masked_token_loss(operands, kept):
     close(without_synchronisation(lambda: step("sync")), step("none"))
 
 
+@pytest.mark.parametrize("h,v,trainable", [(256, 16384, True), (320, 9024, True),   # fused
+                                            (1024, 9001, True), (1032, 20001, False)])   # kept
+@pytest.mark.parametrize("kept", [1, 64, 65, 256, 300, 513, N - 1])
+def test_the_bits_of_a_counted_call(gpu_device, monkeypatch, h, v, trainable, kept):
+    """Few tiles over many words: as many K splits, and so the same sums, as with a known count."""
+    print("[case]", h, v, trainable, kept, flush=True)
+    gen = torch.Generator(device=gpu_device).manual_seed(h + kept)
+    hidden = torch.randn(N, h, generator=gen, device=gpu_device).bfloat16()
+    weight = (torch.randn(v, h, generator=gen, device=gpu_device) * 0.05).bfloat16()
+    labels = torch.randint(0, v, (N,), generator=gen, device=gpu_device)
+    labels[torch.rand(N, generator=gen, device=gpu_device).argsort()[kept:]] = -100
+
+    def step():
+        x = hidden.clone().requires_grad_()
+        w = weight.clone().requires_grad_(trainable)
+        loss = tiled_linear_cross_entropy(x, w, labels, dtype=x.dtype)
+        loss.backward()
+        return [loss.detach(), x.grad] + ([w.grad] if trainable else [])
+
+    got = without_synchronisation(step)
+    for rule in ("count_stays_on_device", "kept_count_stays_on_device"):
+        monkeypatch.setattr(native, rule, lambda *args: False)
+    for a, b in zip(got, step()):
+        assert torch.equal(a, b)
+
+
 def test_larger_calls_are_counted(gpu_device):
     for n, h, stays in ((4096, 1024, True), (4097, 1024, False), (4096, 960, False)):
         rows = torch.empty(n, h, dtype=torch.float16, device=gpu_device)

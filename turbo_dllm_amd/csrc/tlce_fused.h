@@ -411,7 +411,7 @@ struct ReduceSlabsArgs {
   int64_t row0 = 0;                 // first row among the counted rows
   // with a device row count the contraction derives its K splits and slab stride from
   // the real rows of the block (dynamic_k_splits); the same inputs reproduce them here
-  int n_htiles = 0, tile = 0, launched_splits = 0, k_steps = 0;
+  int n_htiles = 0, tile = 0, max_splits = 1, k_steps = 0;
   int64_t slab_budget = 0;
   // non-null: row r also gets sum_j fix_value[r, j] * weight[fix_id[r, j], :] (j < kTopkFix),
   // before the row factor
@@ -516,6 +516,7 @@ struct FusedPlan {
   int64_t block_rows;   // rows per block, a multiple of the tile
   int n_blocks;
   int dh_ksplit;        // K splits of the grad_hidden contraction of a full block
+  int dh_max_ksplit;    // upper bound of the rule that chose them
   int64_t k_steps;      // of its K loop, unsplit
 };
 
@@ -580,8 +581,8 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
   p.n_blocks = (int)ceil_div(total, per);
   // (in planes, six steps of the K loop per 64 vocabulary rows)
   p.k_steps = p.vp / 64 * (dtype == TLCE_DTYPE_F32 ? SplitF32Engine::kPasses : 1);
-  const int max_split = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxKSplits, p.k_steps / 8));
-  p.dh_ksplit = grad_hidden_k_splits((p.block_rows / tile) * p.n_htiles, max_split, p.k_steps,
+  p.dh_max_ksplit = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxKSplits, p.k_steps / 8));
+  p.dh_ksplit = grad_hidden_k_splits((p.block_rows / tile) * p.n_htiles, p.dh_max_ksplit, p.k_steps,
                                      std::min(p.block_rows, std::max<int64_t>(m, 1)) * h);
   return p;
 }
@@ -824,14 +825,13 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
                                                      p.k_steps, rows * h));
     ReduceSlabsArgs rs;
     if (m_dev != nullptr) {
-      // The block may hold far fewer rows than it was sized for (down to none): at least
-      // 16 splits (or the plan's, if more) are launched and the kernel takes as many as the
-      // real rows call for, within the slab memory the plan allocated; the others exit at once.
+      // The block may hold far fewer rows than it was sized for (down to none): the kernel
+      // takes as many splits as the real rows call for, within the slabs the plan allocated.
       dh.m_dev = m_dev; dh.m_role = kRowsFollow; dh.m_dev_offset = r0;
       dh.slab_budget = (int64_t)p.dh_ksplit * p.block_rows * h;
       dh.k_steps_plan = (int)p.k_steps;
-      ksplit = (int)std::max<int64_t>(p.dh_ksplit, std::min<int64_t>(16, p.vp / 64 / 8));
-      rs.n_htiles = p.n_htiles; rs.tile = E::kTile; rs.launched_splits = ksplit;
+      dh.max_splits = p.dh_max_ksplit;
+      rs.n_htiles = p.n_htiles; rs.tile = E::kTile; rs.max_splits = dh.max_splits;
       rs.k_steps = dh.k_steps_plan; rs.slab_budget = dh.slab_budget;
     }
     if (int rc = launch_gemm<E, true, false>(dh, ksplit, kClassGradHidden, stream)) return rc;

@@ -442,6 +442,26 @@ inline int round_chunk(int ni, int nj, int tile) {
   return rounds > 1 && !xcd_aligned(ni) && (int64_t)ni * width <= resident ? width : 0;
 }
 
+// Workgroups of a contraction whose row count, up to nj tiles of them, is on the device: those of
+// the count that needs the most, for the splits it gets.  The most splits of the most tiles are
+// mostly workgroups that exit, and a bound on the splits leaves few tiles without theirs.  16
+// splits launched at most / this, grad_hidden and the step:
+//    256 of 1024 rows, H = 2048, V = 131072   222 / 142 us   706 / 633 us  (32 splits of 8 tiles)
+//    102 of 2048, H = 1024, V = 32000          34 /  22
+//   1036 of 2048, H = 4096, V = 32000         454 / 232     1056 / 833
+//   8212 recomputed, H = 3840, V = 262144                   51.6 / 51.2 ms
+inline int counted_rows_grid(const GemmArgs& a, int tile) {
+  int64_t grid = kXcds;
+  for (int64_t j = 1; j <= a.nj; ++j) {
+    const int64_t slab = j * tile * a.ldc;
+    const int ks = grad_hidden_k_splits(j * a.ni, a.max_splits, a.k_steps_plan, slab,
+                                        resident_workgroups(tile));
+    const int64_t held = std::max<int64_t>(1, a.slab_budget / slab);
+    grid = std::max(grid, std::min<int64_t>(ks, held) * xcd_grid(j * a.ni));
+  }
+  return (int)grid;
+}
+
 template <class E, bool kAKMajor, bool kBKMajor>
 int launch_gemm(GemmArgs a, int ksplit, int cls, hipStream_t stream) {
   static LdsOptIn lds;
@@ -452,10 +472,11 @@ int launch_gemm(GemmArgs a, int ksplit, int cls, hipStream_t stream) {
     a.j_chunk = round_chunk(a.ni, a.nj, E::kTile);
   const int ksteps = (int)ceil_div(a.k, E::kBK);
   a.k_per_split = (int)ceil_div(ksteps, ksplit) * E::kBK;
-  // ksplit is the number of splits launched; with a device-side row count the
-  // kernel may use fewer of them (a.slab_budget then bounds splits x slab)
-  dim3 grid(a.j_chunk > 0 ? xcd_grid((int64_t)a.ni * a.j_chunk) * (int)ceil_div(a.nj, a.j_chunk)
-                          : xcd_grid((int64_t)a.ni * a.nj), ksplit, 1);
+  // (with a device-side row count the kernel finds its number of splits itself)
+  const bool counted = a.m_dev != nullptr && a.m_role == kRowsFollow;
+  dim3 grid(counted ? counted_rows_grid(a, E::kTile)
+            : a.j_chunk > 0 ? xcd_grid((int64_t)a.ni * a.j_chunk) * (int)ceil_div(a.nj, a.j_chunk)
+                            : xcd_grid((int64_t)a.ni * a.nj), counted ? 1 : ksplit, 1);
   ScopedTimer timer(cls, stream);
   lce_gemm_nt_kernel<E, kAKMajor, kBKMajor><<<grid, E::kThreads, kLdsBytes, stream>>>(a);
   TLCE_LAUNCH_CHECK();
@@ -614,10 +635,6 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     }
   }
 
-  // device-side row count: at least 16 K splits of grad_hidden (or the plan's, if more) are launched
-  // and the kernel picks how many to use for the real count, within the slabs the plan allocated
-  const int dh_launch_ksplit =
-      m_dev == nullptr ? p.dh_ksplit : std::max(p.dh_ksplit, std::min(16, p.dh_max_ksplit));
   for (int panel = 0; panel < p.n_panels; ++panel) {
     const int64_t v0 = (int64_t)panel * p.vc;
     const int64_t width = std::min<int64_t>(p.vc, p.vp - v0);   // multiple of tile
@@ -633,6 +650,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     dh.mode = (panel == 0) ? kStoreF32 : kAddF32;
     dh.m_dev = m_dev; dh.m_role = kRowsFollow;
     dh.slab_budget = p.dh_slab_rows * h;
+    dh.max_splits = p.dh_max_ksplit;
     dh.k_steps_plan = (int)(p.vc / p.bk);
     GemmArgs dw;
     dw.m_dev = m_dev; dw.m_role = kKFollows; dw.m_round = p.bk;
@@ -649,7 +667,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
           // are K-contiguous rows of the stored matrix; B = G.
           dh.a = weight_t + v0; dh.lda = v; dh.a_rows = (int)h;
           dh.k = (int)round_up(rows_valid, kSlab);
-          if (int rc = launch_gemm<E, false, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
+          if (int rc = launch_gemm<E, false, false>(dh, p.dh_ksplit, kClassGradHidden, stream))
             return rc;
           if (weight_grad) {
             // grad_weight [h, v]: the roles of the operands swap so that the hidden axis
@@ -678,7 +696,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
           dh.a_tail = wt;
           dh.a_k_full = dh.k - kSlab;
         }
-        if (int rc = launch_gemm<E, true, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
+        if (int rc = launch_gemm<E, true, false>(dh, p.dh_ksplit, kClassGradHidden, stream))
           return rc;
         if (weight_grad) {
           // grad_weight: A = hidden as stored, B = G as stored, both K-major (K = token)
@@ -696,7 +714,7 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     }
     dh.a = wt + v0; dh.lda = p.vp; dh.a_rows = (int)h;
     dh.k = (int)width;
-    if (int rc = launch_gemm<E, false, false>(dh, dh_launch_ksplit, kClassGradHidden, stream))
+    if (int rc = launch_gemm<E, false, false>(dh, p.dh_ksplit, kClassGradHidden, stream))
       return rc;
     if (weight_grad) {
       dw.a = ht; dw.lda = p.mp; dw.a_rows = (int)h;
@@ -716,7 +734,8 @@ int panel_contractions(const Plan& p, const BackwardLayout& l, const void* hidde
     ScopedTimer timer(kClassOther, stream);
     lce_finalize_grad_hidden_kernel<T><<<(int)m, 256, 0, stream>>>(
         acc32, p.dh_ksplit, p.mp * h, p.dh_slab_rows * h, row_idx, (int)m, (int)h,
-        static_cast<T*>(grad_hidden), m_dev, p.n_htiles, p.tile, dh_launch_ksplit, (int)(p.vc / p.bk));
+        static_cast<T*>(grad_hidden), m_dev, p.n_htiles, p.tile, p.dh_max_ksplit,
+        (int)(p.vc / p.bk));
   }
   TLCE_LAUNCH_CHECK();
   return 0;

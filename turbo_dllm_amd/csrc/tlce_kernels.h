@@ -1509,6 +1509,7 @@ struct GemmArgs {
   int m_role = 0, m_round = 1;
   int64_t m_dev_offset = 0;  // the operand's first token row is row m_dev_offset of the counted rows
   int64_t slab_budget = 0;   // kRowsFollow: float32 elements all K-split slabs may take
+  int max_splits = 1;        // kRowsFollow: the split rule's own bound
   int k_steps_plan = 0;      // kRowsFollow: K steps of a full panel, what the split rule plans on
   // K-major operands whose K rows end inside a 64-row slab (Operand::tail)
   const void* a_tail = nullptr;
@@ -1520,16 +1521,15 @@ struct GemmArgs {
 
 // K splits and slab stride the grad_hidden contraction uses for a device-side
 // row count: the host plan's rule applied to the real number of token tiles,
-// limited to the splits launched (at most kMaxKSplits) and to the slab memory the plan
-// allocated.  A lane per candidate, by all lanes of a wave: one after the other they took 4 us of
+// limited to the slab memory the plan allocated.  A lane per candidate, by all lanes of a wave: one after the other they took 4 us of
 // the slab reduction (16 candidates, 1036 of 2048 rows, H = 1024: 15 -> 12.8 us).
 __device__ __forceinline__ int dynamic_k_splits(int n_ttiles, int n_htiles, int tile, int h,
-                                                int launched, int64_t slab_budget, int k_steps,
-                                                int64_t* stride) {
+                                                int max_splits, int64_t slab_budget,
+                                                int k_steps, int64_t* stride) {
   static_assert(kMaxKSplits <= 64, "a lane per candidate");
   const int lane = threadIdx.x & 63;
   const int64_t slab = (int64_t)n_ttiles * tile * h;
-  const int64_t cost = lane < launched
+  const int64_t cost = lane < max_splits
                            ? k_split_cost((int64_t)n_ttiles * n_htiles, lane + 1, k_steps,
                                           k_split_slab_cost(slab), resident_workgroups(tile))
                            : INT64_MAX;
@@ -1770,12 +1770,15 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
   extern __shared__ __align__(16) char smem[];
   using T = typename E::T;
   int n_splits = gridDim.y;
+  bool counted_here = false;   // the splits are: workgroups in one row (counted_rows_grid)
   if (p.m_dev != nullptr) {
     if (p.m_role == kRowsFollow) {
       p.c_rows = effective_block_rows(p.c_rows, p.m_dev, p.m_dev_offset);
       p.nj = (p.c_rows + E::kTile - 1) / E::kTile;
-      n_splits = dynamic_k_splits(p.nj, p.ni, E::kTile, (int)p.ldc, (int)gridDim.y,
-                                  p.slab_budget, p.k_steps_plan, &p.c_split_stride);
+      if (p.nj == 0) return;
+      counted_here = true;
+      n_splits = dynamic_k_splits(p.nj, p.ni, E::kTile, (int)p.ldc, p.max_splits, p.slab_budget,
+                                  p.k_steps_plan, &p.c_split_stride);
       p.k_per_split = ((p.k + E::kBK - 1) / E::kBK + n_splits - 1) / n_splits * E::kBK;
     } else if (p.m_role == kKFollows) {
       const int rows = effective_block_rows(p.k, p.m_dev, p.m_dev_offset);
@@ -1786,10 +1789,15 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
   }
   int split, ti, tj;
   const int tiles = p.ni * p.nj;
-  if (gridDim.y == 1 || tiles >= kSplitMajorBelowTiles) {
+  if (n_splits == 1 || tiles >= kSplitMajorBelowTiles) {
     split = blockIdx.y;
-    if (split >= n_splits) return;
     int first_j = 0, bid = blockIdx.x, nj = p.nj;
+    if (counted_here) {
+      const int grid = (tiles + kXcds - 1) / kXcds * kXcds;
+      split = bid / grid;
+      bid -= split * grid;
+    }
+    if (split >= n_splits) return;
     if (p.j_chunk > 0) {
       const int grid = (p.ni * p.j_chunk + kXcds - 1) / kXcds * kXcds;
       first_j = bid / grid * p.j_chunk;
@@ -1876,14 +1884,14 @@ template <typename T>
 __global__ __launch_bounds__(256) void lce_finalize_grad_hidden_kernel(
     const float* __restrict__ acc32, int n_splits, int64_t split_stride, int64_t slab_budget,
     const int64_t* __restrict__ row_idx, int m, int h, T* __restrict__ out,
-    const int64_t* __restrict__ m_dev, int n_htiles, int tile, int launched_splits,
+    const int64_t* __restrict__ m_dev, int n_htiles, int tile, int max_splits,
     int k_steps_plan) {
   const int r = blockIdx.x;
   if (m_dev != nullptr) {
     // the splits and slab stride the contraction derived from the real row count
     m = effective_rows(m, m_dev);
-    n_splits = dynamic_k_splits((m + tile - 1) / tile, n_htiles, tile, h, launched_splits,
-                                slab_budget, k_steps_plan, &split_stride);
+    n_splits = dynamic_k_splits((m + tile - 1) / tile, n_htiles, tile, h, max_splits, slab_budget,
+                                k_steps_plan, &split_stride);
   }
   if (r >= m) return;
   const int64_t o = (row_idx != nullptr) ? row_idx[r] : (int64_t)r;
