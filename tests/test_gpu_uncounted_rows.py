@@ -96,8 +96,10 @@ def test_masked_token_loss(operands, kept):
     close(without_synchronisation(lambda: step("sync")), step("none"))
 
 
-@pytest.mark.parametrize("h,v,trainable", [(256, 16384, True), (320, 9024, True),   # fused
-                                            (1024, 9001, True), (1032, 20001, False)])   # kept
+@pytest.mark.parametrize("h,v,trainable", [
+    (256, 16384, True), (320, 9024, True),       # gradients in the forward,
+    (3840, 16384, True),                         # 8 splits of 2 tiles, 5 of 3,
+    (1024, 9001, True), (1032, 20001, False)])   # kept logits
 @pytest.mark.parametrize("kept", [1, 64, 65, 256, 300, 513, N - 1])
 def test_the_bits_of_a_counted_call(gpu_device, monkeypatch, h, v, trainable, kept):
     """Few tiles over many words: as many K splits, and so the same sums, as with a known count."""

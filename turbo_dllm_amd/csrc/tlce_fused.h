@@ -517,6 +517,7 @@ struct FusedPlan {
   int n_blocks;
   int dh_ksplit;        // K splits of the grad_hidden contraction of a full block
   int dh_max_ksplit;    // upper bound of the rule that chose them
+  int64_t dh_slab_rows; // k_split_slab_rows of a full block
   int64_t k_steps;      // of its K loop, unsplit
 };
 
@@ -584,6 +585,8 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
   p.dh_max_ksplit = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxKSplits, p.k_steps / 8));
   p.dh_ksplit = grad_hidden_k_splits((p.block_rows / tile) * p.n_htiles, p.dh_max_ksplit, p.k_steps,
                                      std::min(p.block_rows, std::max<int64_t>(m, 1)) * h);
+  p.dh_slab_rows = k_split_slab_rows(p.dh_ksplit, p.dh_max_ksplit, (int)(p.block_rows / tile),
+                                     p.n_htiles, (int)tile);
   return p;
 }
 
@@ -626,7 +629,7 @@ inline FusedLayout fused_layout(const FusedPlan& p, int64_t m, int64_t h, int dt
   l.row_scale = off;  off += align256(p.block_rows * 4);
   l.scaled_hidden = off;
   if (weight_grad) off += align256(p.block_rows * hp * es);
-  l.slabs = off;      off += align256((int64_t)p.dh_ksplit * p.block_rows * h * 4);
+  l.slabs = off;      off += align256(p.dh_slab_rows * h * 4);
   l.redo = off;       off += align256((int64_t)p.n_blocks * 4);
   l.hidden_planes = off;
   if (planes) off += align256(p.block_rows * hp * es);
@@ -828,7 +831,7 @@ int fused_gradients_impl(const FusedPlan& p, const void* hidden, const void* wei
       // The block may hold far fewer rows than it was sized for (down to none): the kernel
       // takes as many splits as the real rows call for, within the slabs the plan allocated.
       dh.m_dev = m_dev; dh.m_role = kRowsFollow; dh.m_dev_offset = r0;
-      dh.slab_budget = (int64_t)p.dh_ksplit * p.block_rows * h;
+      dh.slab_budget = p.dh_slab_rows * h; dh.split_by_rows = true;
       dh.k_steps_plan = (int)p.k_steps;
       dh.max_splits = p.dh_max_ksplit;
       rs.n_htiles = p.n_htiles; rs.tile = E::kTile; rs.max_splits = dh.max_splits;

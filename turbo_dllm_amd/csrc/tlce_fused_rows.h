@@ -397,8 +397,8 @@ __global__ __launch_bounds__(256) void lce_reduce_scaled_slabs_kernel(ReduceSlab
   if (p.m_dev != nullptr) {
     const int rows = effective_block_rows(p.m, p.m_dev, p.row0);
     if (r >= rows) return;
-    p.n_splits = dynamic_k_splits((rows + p.tile - 1) / p.tile, p.n_htiles, p.tile, p.h,
-                                  p.max_splits, p.slab_budget, p.k_steps, &p.split_stride);
+    p.n_splits = dynamic_k_splits(rows, true, p.n_htiles, p.tile, p.h, p.max_splits, p.slab_budget,
+                                  p.k_steps, &p.split_stride);
   }
   const float s = p.row_scale[r];
   const float* src = p.slabs + (int64_t)r * p.h;

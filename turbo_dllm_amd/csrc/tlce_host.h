@@ -101,6 +101,16 @@ inline int engine_class(int64_t h, int dtype) {
   return (h % 64) == 0 ? 2 : 1;
 }
 
+// Rows of all K-split slabs of a grad_hidden contraction together.  A row count on the device may
+// leave fewer tiles, and more splits of them, than n_ttiles have: slabs for one round of workgroups
+// (64 MiB at most), so that it gets the splits of a call with that many rows where they make one.
+// 2240 of 3200 rows, H = 2112 (81 of 117 tiles) take three splits and not the plan's two.
+inline int64_t k_split_slab_rows(int ksplit, int max_split, int n_ttiles, int n_htiles, int tile) {
+  const int64_t round = std::min<int64_t>(ceil_div(resident_workgroups(tile), n_htiles),
+                                          (int64_t)n_ttiles * max_split);
+  return std::max((int64_t)ksplit * n_ttiles, round) * tile;
+}
+
 // Whether the caller has scratch for copies of operands (column tails), and what for.
 enum ColumnTails { kNoColumnTails, kForwardTails, kBackwardTails };
 
@@ -180,13 +190,7 @@ inline Plan make_plan(int64_t m, int64_t h, int64_t v, int dtype, bool weight_gr
     p.dh_ksplit = grad_hidden_k_splits((int64_t)p.n_ttiles * p.n_htiles, p.dh_max_ksplit,
                                        p.vc / p.bk, p.mp * h, resident_workgroups(p.tile));
   }
-  // A row count on the device may leave fewer tiles, and more splits of them, than m rows have:
-  // slabs for one round of workgroups, so that it gets the splits of a call with that many rows.
-  // 2240 of 3200 rows, H = 2112 (81 of 117 tiles) take three splits and not the plan's two.
-  p.dh_slab_rows =
-      std::max(p.dh_ksplit * p.mp,
-               std::min<int64_t>(ceil_div(resident_workgroups(p.tile), p.n_htiles),
-                                 (int64_t)p.n_ttiles * p.dh_max_ksplit) * p.tile);
+  p.dh_slab_rows = k_split_slab_rows(p.dh_ksplit, p.dh_max_ksplit, p.n_ttiles, p.n_htiles, p.tile);
   return p;
 }
 
@@ -454,7 +458,9 @@ inline int counted_rows_grid(const GemmArgs& a, int tile) {
   int64_t grid = kXcds;
   for (int64_t j = 1; j <= a.nj; ++j) {
     const int64_t slab = j * tile * a.ldc;
-    const int ks = grad_hidden_k_splits(j * a.ni, a.max_splits, a.k_steps_plan, slab,
+    // (no count of j tiles takes more splits than the smallest)
+    const int64_t rows = a.split_by_rows ? (j - 1) * tile + 1 : j * tile;
+    const int ks = grad_hidden_k_splits(j * a.ni, a.max_splits, a.k_steps_plan, rows * a.ldc,
                                         resident_workgroups(tile));
     const int64_t held = std::max<int64_t>(1, a.slab_budget / slab);
     grid = std::max(grid, std::min<int64_t>(ks, held) * xcd_grid(j * a.ni));

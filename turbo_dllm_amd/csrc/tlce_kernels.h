@@ -1510,6 +1510,7 @@ struct GemmArgs {
   int64_t m_dev_offset = 0;  // the operand's first token row is row m_dev_offset of the counted rows
   int64_t slab_budget = 0;   // kRowsFollow: float32 elements all K-split slabs may take
   int max_splits = 1;        // kRowsFollow: the split rule's own bound
+  bool split_by_rows = false;   // kRowsFollow: it prices slabs by their rows, not whole tiles
   int k_steps_plan = 0;      // kRowsFollow: K steps of a full panel, what the split rule plans on
   // K-major operands whose K rows end inside a 64-row slab (Operand::tail)
   const void* a_tail = nullptr;
@@ -1523,15 +1524,18 @@ struct GemmArgs {
 // row count: the host plan's rule applied to the real number of token tiles,
 // limited to the slab memory the plan allocated.  A lane per candidate, by all lanes of a wave: one after the other they took 4 us of
 // the slab reduction (16 candidates, 1036 of 2048 rows, H = 1024: 15 -> 12.8 us).
-__device__ __forceinline__ int dynamic_k_splits(int n_ttiles, int n_htiles, int tile, int h,
-                                                int max_splits, int64_t slab_budget,
-                                                int k_steps, int64_t* stride) {
+__device__ __forceinline__ int dynamic_k_splits(int rows, bool split_by_rows, int n_htiles,
+                                                int tile, int h, int max_splits,
+                                                int64_t slab_budget, int k_steps,
+                                                int64_t* stride) {
   static_assert(kMaxKSplits <= 64, "a lane per candidate");
   const int lane = threadIdx.x & 63;
+  const int n_ttiles = (rows + tile - 1) / tile;
   const int64_t slab = (int64_t)n_ttiles * tile * h;
+  const int64_t priced = split_by_rows ? (int64_t)rows * h : slab;
   const int64_t cost = lane < max_splits
                            ? k_split_cost((int64_t)n_ttiles * n_htiles, lane + 1, k_steps,
-                                          k_split_slab_cost(slab), resident_workgroups(tile))
+                                          k_split_slab_cost(priced), resident_workgroups(tile))
                            : INT64_MAX;
   int64_t best = cost;
 #pragma unroll
@@ -1777,8 +1781,8 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_gemm_nt_ker
       p.nj = (p.c_rows + E::kTile - 1) / E::kTile;
       if (p.nj == 0) return;
       counted_here = true;
-      n_splits = dynamic_k_splits(p.nj, p.ni, E::kTile, (int)p.ldc, p.max_splits, p.slab_budget,
-                                  p.k_steps_plan, &p.c_split_stride);
+      n_splits = dynamic_k_splits(p.c_rows, p.split_by_rows, p.ni, E::kTile, (int)p.ldc,
+                                  p.max_splits, p.slab_budget, p.k_steps_plan, &p.c_split_stride);
       p.k_per_split = ((p.k + E::kBK - 1) / E::kBK + n_splits - 1) / n_splits * E::kBK;
     } else if (p.m_role == kKFollows) {
       const int rows = effective_block_rows(p.k, p.m_dev, p.m_dev_offset);
@@ -1890,7 +1894,7 @@ __global__ __launch_bounds__(256) void lce_finalize_grad_hidden_kernel(
   if (m_dev != nullptr) {
     // the splits and slab stride the contraction derived from the real row count
     m = effective_rows(m, m_dev);
-    n_splits = dynamic_k_splits((m + tile - 1) / tile, n_htiles, tile, h, max_splits, slab_budget,
+    n_splits = dynamic_k_splits(m, false, n_htiles, tile, h, max_splits, slab_budget,
                                 k_steps_plan, &split_stride);
   }
   if (r >= m) return;
