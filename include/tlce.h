@@ -619,8 +619,9 @@ int tlce_query_fused_plan(int64_t m, int64_t h, int64_t v, int dtype,
 
 /* The panel_bytes with which a call with a trainable head and a loss reduced to one number runs
  * best: 0 (the default), or the size of a panel of all its rows where that is more than the
- * default but the step's peak stays that of several blocks (a default panel and a float32
- * [v, h] sum).  The same value goes to the workspace query, the forward and the backward. */
+ * default but, with the 16-bit gradient, no more than several blocks may take (a default panel
+ * and a float32 [v, h] sum; the block's row buffers, 6 h + v / 32 bytes a row, come on top).  The
+ * same value goes to the workspace query, the forward and the backward. */
 int64_t tlce_reduced_loss_panel_bytes(int64_t m, int64_t h, int64_t v, int dtype);
 
 int64_t tlce_forward_with_gradients_workspace_bytes(int64_t m, int64_t h, int64_t v,

@@ -532,8 +532,14 @@ ONE_TILE_ROWS = 256
 # Calls whose panel of exponentiated logits is at most this large with every row in it: the row
 # count stays on the device.  Reading it back costs the wait and, after it, 40 to 60 us in which
 # the GPU has nothing to do; launches sized for all rows cost a few us of workgroups that exit.
-# Half of 2048 rows, H = 1024, V = 32000 (125 MiB): 335 -> 280 us a step.  Beyond it a step takes
-# milliseconds, and the panel's memory for rows without a loss is no longer small.
+# A step in us, count read back -> left, of 1 or 2 / 5 / 50 / 97 % of the rows with a loss:
+#   2048 rows, H = 1024, V = 32000 (125 MiB)   ...        258 -> 240  314 -> 265  449 -> 396
+#   1024 rows, H = 1024, V = 131072 (256 MiB)  315 -> 262  318 -> 264  531 -> 481  844 -> 788
+#   8192 rows, H = 1024, V = 16384 (256 MiB)   260 -> 250  261 -> 250  467 -> 421  783 -> 738
+#   2048 rows, H = 1024, V = 131072 (512 MiB)  316 -> 265  339 -> 290  844 -> 801 1454 -> 1420
+#   32768 rows, H = 512, V = 8192 (512 MiB)    249 -> 245  254 -> 249  730 -> 707 1296 -> 1272
+# Time would allow twice as much (at 1 GiB over V = 131072 few rows lose: 396 -> 466 at 5 %); the
+# line is for the memory that rows without a loss take until the backward.
 _UNCOUNTED_PANEL_BYTES = 256 << 20
 
 
@@ -809,8 +815,8 @@ def forward_with_gradients(
 
 def reduced_loss_panel_bytes(m: int, h: int, v: int, dtype: torch.dtype) -> int:
     """The panel budget for ``m`` rows, whose count the host knows, of a trainable head under a
-    loss reduced to one number: the one in force, or, where none is and it costs no memory at
-    the step's peak, one that takes them as one block."""
+    loss reduced to one number: the one in force, or, where none is and the step's peak stays
+    about what several blocks may take, one that takes them as one block."""
     panel = get_panel_bytes()
     if panel or dtype != torch.bfloat16:
         return panel
@@ -1161,7 +1167,12 @@ def from_kept_logits(kept: torch.Tensor | None, call):
 # Calls whose logits all fit this with every row in them: the row count stays on the device, as
 # where the gradients leave the forward (count_stays_on_device).  2741 of 4096 rows, H = 2048,
 # V = 32003 (504 MiB): 1.17 -> 1.12 ms a step; 1036 of 2048, H = 1024 390 -> 350 us; 600 of 1024
-# float16 rows, H = 2048, V = 32000 415 -> 387.
+# float16 rows, H = 2048, V = 32000 415 -> 387.  At 1 or 2 / 5 / 50 / 97 % of H = 1024 rows:
+#   1024 rows, V = 130817 (512 MiB)   415 -> 333  410 -> 335   652 -> 579  1030 -> 958
+#   8192 rows, V = 16129 (512 MiB)    342 -> 331  344 -> 335   579 -> 493   956 -> 872
+#   2048 rows, V = 131073 (1026 MiB)  455 -> 363  479 -> 389  1095 -> 1014 1912 -> 1825
+#   16384 rows, V = 16385 (1040 MiB)  324 -> 312  345 -> 317  1155 -> 1078 2094 -> 2013
+# Twice as much would still gain; the line is for the memory of the rows without a loss.
 _UNCOUNTED_KEPT_BYTES = 512 << 20
 
 

@@ -305,13 +305,22 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_exp_logits_
 }
 
 // Heads up to this size are well within the last-level cache when the narrow tiles of the last
-// tokens come to read them a second time; there they come last and end the launch evenly (1036
-// rows, H = 1024, V = 32000: 89 -> 81 us, the step 274 -> 261).  Larger heads are read once, by
-// neighbouring wide and narrow tiles: narrow ones alone wait for memory, 1.5 us a K step instead of
-// 0.6.  With the head's bytes, a step in us, neighbours / last:
-//   62 MiB   8250 rows, H = 1024  1521 / 1519     128 MiB   600 rows, H = 1024        329 / 321
-//  117 MiB   1610, H = 1024        473 / 484      128 MiB   600, H = 1024, top-8      361 / 374
-//  125 MiB   2100, H = 2048        762 / 749      125 MiB  1400, H = 2048             525 / 531
+// tokens come to read them a second time; there they come last and fill the wide tiles' last
+// round.  Larger heads are read once, by neighbouring wide and narrow tiles: narrow ones alone wait
+// for memory, 1.5 us a K step instead of 0.6.  Exponentiated logits in us, neighbours / last, of
+// 612, 1036, 2081 and 8212 rows:
+//   16 MiB  H =  256, V = 32000   36 /  33    48 /  43    73 /  69   226 / 228
+//   31 MiB  H =  512, V = 32000   45 /  42    64 /  56   103 /  99   312 / 317
+//   32 MiB  H = 1024, V = 16384   37 /  37    63 /  52    95 /  85   279 / 267
+//   62 MiB  H = 1024, V = 32000   65 /  59    94 /  86   150 / 146   497 / 494
+//   64 MiB  H = 2048, V = 16384   58 /  58   101 /  82   154 / 135   460 / 448
+// Above the line it goes either way, by how the wide tiles fill whole rounds and by the cache:
+//   74 MiB  H =  768, V = 50304   78 /  75   113 / 117   186 / 190   625 / 633
+//   98 MiB  H = 1024, V = 50048   92 /  85   135 / 138   217 / 229   761 / 758
+//  125 MiB  H = 2048, V = 32000  102 /  96   152 / 137   247 / 236
+//  125 MiB  H = 1024, V = 64000   98 / 101   156 / 156   268 / 270
+//  256 MiB  H = 1024, V = 131072 199 / 195   322 / 311   543 / 549   (269 rows 131 / 154)
+// The line gives up gains beyond it; below, what loses loses 2 % of the kernel at most.
 constexpr int64_t kTailLastWeightBytes = 64ll << 20;
 
 template <class E, bool kSoftcap, bool kPlain = false, bool kRounded = false>
@@ -593,9 +602,11 @@ inline FusedPlan make_fused_plan(int64_t m, int64_t h, int64_t v, int dtype, int
 // Panel budget (0: the default) of a call with a trainable head whose loss is reduced to one
 // number.  In one block the panel waits for the backward, in several the float32 [v, h] sum does,
 // which every block but the first reads and writes and a last pass rounds.  One block is taken
-// beyond the default as well where the step's peak stays what it is: the panel and the 16-bit
-// gradient in the backward against a default panel and the float32 sum in the forward, i.e. up to
-// the default and one 16-bit gradient.  Several blocks / one, ms a step and GB at its peak:
+// beyond the default as well where the panel and the 16-bit gradient in the backward take no more
+// than a default panel and the float32 sum in the forward, i.e. up to the default and one 16-bit
+// gradient.  The step's peak then grows by no more than several blocks stay under a default panel
+// (half of it at most) and by the larger block's row buffers, 6 h + v / 32 bytes for each row
+// more (0.13 GB in the first line).  Several blocks / one, ms a step and GB at its peak:
 //   8212 rows, H = 3840, V = 262144, cap 30   39.7 / 38.8   6.5 / 6.6
 //   6000 rows, H = 4096, V = 262144           33.8 / 28.2   6.5 / 5.5    (16 and 8 token tiles)
 //  10000 rows, H = 4096, V = 151936           29.8 / 27.4   5.2 / 4.7    (32 and 8)
