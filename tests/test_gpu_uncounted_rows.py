@@ -1,6 +1,7 @@
 """Small calls whose count of rows with a loss stays on the device in the default compaction
 (``native.count_stays_on_device``): no host synchronisation, and the results of a call that
-compacts nothing, for no row with a loss up to all of them, around tiles and 64-row slabs."""
+compacts nothing, for no row with a loss up to all of them, around tiles and 64-row slabs.  The
+same with the count read back, as larger calls have it."""
 
 import pytest
 import torch
@@ -30,6 +31,11 @@ def operands(gpu_device, request):
     return hidden, weight, labels, order, up
 
 
+def read_back(monkeypatch):
+    for rule in ("count_stays_on_device", "kept_count_stays_on_device"):
+        monkeypatch.setattr(native, rule, lambda *args: False)
+
+
 def without_synchronisation(call):
     call()          # (allocations and first launches)
     torch.cuda.synchronize()
@@ -52,7 +58,8 @@ def close(got, want):
 @pytest.mark.parametrize("reduction", ["mean", "sum", "none"])
 @pytest.mark.parametrize("trainable", [True, False])
 @pytest.mark.parametrize("kept", [0, 1, 64, 65, 255, 256, 257, 384, 513, N - 1, N])
-def test_cross_entropy(operands, reduction, trainable, kept):
+@pytest.mark.parametrize("counted", [False, True])
+def test_cross_entropy(operands, monkeypatch, reduction, trainable, kept, counted):
     hidden, weight, labels, order, up = operands
     labels = labels.clone()
     labels[order[kept:]] = -100
@@ -68,7 +75,11 @@ def test_cross_entropy(operands, reduction, trainable, kept):
         (loss * up if reduction == "none" else loss).sum().backward()
         return [loss.detach(), x.grad] + ([w.grad] if trainable else [])
 
-    got = without_synchronisation(lambda: step("sync"))
+    if counted:
+        read_back(monkeypatch)
+        got = step("sync")
+    else:
+        got = without_synchronisation(lambda: step("sync"))
     if kept == 0 and reduction == "mean":
         assert got[0].isnan()       # the mean over no row, as before
         return
@@ -76,7 +87,8 @@ def test_cross_entropy(operands, reduction, trainable, kept):
 
 
 @pytest.mark.parametrize("kept", [0, 1, 257, N])
-def test_masked_token_loss(operands, kept):
+@pytest.mark.parametrize("counted", [False, True])
+def test_masked_token_loss(operands, monkeypatch, kept, counted):
     hidden, weight, labels, order, up = operands
     labels = labels.clone()
     labels[order[kept:]] = -100
@@ -93,7 +105,12 @@ def test_masked_token_loss(operands, kept):
             loss.backward()
         return [loss.detach(), x.grad, head.weight.grad]
 
-    close(without_synchronisation(lambda: step("sync")), step("none"))
+    want = step("none")
+    if counted:
+        read_back(monkeypatch)
+        close(step("sync"), want)
+    else:
+        close(without_synchronisation(lambda: step("sync")), want)
 
 
 @pytest.mark.parametrize("h,v,trainable", [
@@ -118,8 +135,7 @@ def test_the_bits_of_a_counted_call(gpu_device, monkeypatch, h, v, trainable, ke
         return [loss.detach(), x.grad] + ([w.grad] if trainable else [])
 
     got = without_synchronisation(step)
-    for rule in ("count_stays_on_device", "kept_count_stays_on_device"):
-        monkeypatch.setattr(native, rule, lambda *args: False)
+    read_back(monkeypatch)
     for a, b in zip(got, step()):
         assert torch.equal(a, b)
 
