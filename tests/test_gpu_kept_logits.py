@@ -189,7 +189,9 @@ def test_checkpointing_while_free_memory_changes(gpu_device, monkeypatch, loss):
     hidden, weight, labels, up = operands(gpu_device, 600, 1024, 3001)
     head = torch.nn.Linear(1024, 3001, bias=False, device="meta")
     left = [1 << 40]
-    monkeypatch.setattr(native, "_memory_left", lambda device: (left[0], 1 << 40))
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (left[0], 1 << 40))
+    monkeypatch.setattr(native, "_memory_cached", lambda device: 0)
+    monkeypatch.setattr(native, "_KEEP_UNASKED_BYTES", 0)
 
     def gradients(wrap):
         x = hidden.clone().requires_grad_()

@@ -19,9 +19,11 @@ def backward_needs(n_out):
             + (n_out + V) * H * 2)
 
 
-def buffer(monkeypatch, left, total=288 * GIB, n_out=M):
+def buffer(monkeypatch, left, total=288 * GIB, n_out=M, cached=0, unasked=0):
+    monkeypatch.setattr(native, "_KEEP_UNASKED_BYTES", unasked)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
-    monkeypatch.setattr(native, "_memory_left", lambda device: (left, total))
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (left - cached, total))
+    monkeypatch.setattr(native, "_memory_cached", lambda device: cached)
     rows = torch.empty(M, H, dtype=torch.bfloat16)
     kept = native.kept_logits_buffer(M, rows, V, None, n_out)
     return 0 if kept is None else kept.numel()
@@ -34,9 +36,12 @@ def test_what_is_taken_of_the_memory_left(monkeypatch):
     for left in (need + 3 * COLUMN, 8 * 11 * COLUMN, 8 * 19 * COLUMN + 5):
         want = min(left // 8, left - need, 20 * COLUMN) // COLUMN * COLUMN
         assert buffer(monkeypatch, left) == max(want, 0)
+        assert buffer(monkeypatch, left, cached=left - MIB) == max(want, 0)
     assert buffer(monkeypatch, 8 * GIB, total=24 * 5 * COLUMN) == 5 * COLUMN
     for left in (0, MIB, need, need + COLUMN - 1):                      # the backward alone
         assert buffer(monkeypatch, left) == 0
+    assert buffer(monkeypatch, 0, unasked=20 * COLUMN) == 20 * COLUMN   # small: not asked
+    assert buffer(monkeypatch, 0, unasked=20 * COLUMN - 1) == 0
     # un-compacted gradients count as they are: 100 000 rows, 205 MB
     assert buffer(monkeypatch, backward_needs(100_000), n_out=100_000) == 0
 
@@ -59,19 +64,17 @@ def test_a_backward_without_memory_gives_the_logits_back():
         native.from_kept_logits(torch.empty(8), lambda buffer: (_ for _ in ()).throw(ValueError))
 
 
-def test_memory_left_of_each_allocator(monkeypatch):
+def test_what_each_allocator_holds(monkeypatch):
     def stats(device):
         if backend == "pluggable":
             raise RuntimeError("CUDAPluggableAllocator does not yet support getDeviceStats.")
         current = {"reserved_bytes": 100, "active_bytes": 60, "inactive_split_bytes": 30}
         return {name: {"all": {"current": n}} for name, n in current.items()} if used else {}
 
-    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (1000, 5000))
     monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", stats)
     monkeypatch.setattr(torch.cuda, "get_allocator_backend", lambda: backend)
-    for backend, used, want in (("native", True, 1010), ("native", False, 1000),
-                                ("pluggable", True, 1000)):
-        assert native._memory_left(torch.device("cuda:0")) == (want, 5000)
+    for backend, used, want in (("native", True, 10), ("native", False, 0), ("pluggable", True, 0)):
+        assert native._memory_cached(torch.device("cuda:0")) == want
 
 
 def test_nothing_is_kept_where_saved_tensors_are_packed(monkeypatch):

@@ -1094,6 +1094,12 @@ def backward_frozen_weight(
 
 
 # ------------------------------------------------- logits kept for the backward --
+# Buffers up to this size are taken without asking how much memory is left: 18 us in a running step,
+# of 260 that 300 rows over H = 1024, V = 16001 take.  A backward that finds none beside them gives
+# them back.
+_KEEP_UNASKED_BYTES = 128 << 20
+
+
 # Which tiles are kept changes no result, so the answer of kept_logits_buffer may differ from call
 # to call.  Saved tensors may not where a hook packs them: activation checkpointing compares their
 # number and shapes between a forward and its repetition.
@@ -1105,32 +1111,30 @@ def _saved_tensors_are_packed() -> bool:
     return top is None or top(True) is not None
 
 
-def _memory_left(device: torch.device) -> tuple[int, int]:
-    """Bytes that allocations can still get, and those of the device.  Of what torch's own
-    allocator holds without using it, whole segments count; pieces of segments in use do not.
-    (Others keep other accounts, and pluggable ones raise when asked for theirs.)"""
-    free, total = torch.cuda.mem_get_info(device)
+def _memory_cached(device: torch.device) -> int:
+    """Bytes that torch's own allocator holds without using them: whole segments count, pieces of
+    segments in use do not.  (Others keep other accounts, and pluggable ones raise when asked for
+    theirs.)"""
     if torch.cuda.get_allocator_backend() != "native":
-        return free, total
+        return 0
     stats = torch.cuda.memory_stats_as_nested_dict(device)
-    if stats:
-        free += (stats["reserved_bytes"]["all"]["current"]
-                 - stats["active_bytes"]["all"]["current"]
-                 - stats["inactive_split_bytes"]["all"]["current"])
-    return free, total
+    if not stats:
+        return 0
+    return (stats["reserved_bytes"]["all"]["current"] - stats["active_bytes"]["all"]["current"]
+            - stats["inactive_split_bytes"]["all"]["current"])
 
 
 def kept_logits_buffer(m: int, hidden: torch.Tensor, vocab: int, bias: torch.Tensor | None,
                        n_out: int) -> torch.Tensor | None:
     """Where the forward of a recomputing cross entropy over ``m`` of ``n_out`` rows leaves its
-    logits for the backward (``masked_loss_forward(kept=...)``), or None when it is to recompute all of
-    them: operands or sizes that gain nothing, the gradient mode "recompute", a call that is
+    logits for the backward (``masked_loss_forward(kept=...)``), or None when it is to recompute
+    all of them: operands and sizes that gain nothing, the gradient mode "recompute", a call that is
     being captured, whose graph would hold the buffer, a caller that checkpoints or moves away
     what is saved for the backward.  A panel budget bounds it as well.
 
-    It takes an eighth of the memory left, so that what is allocated until the backward finds
-    room, a twenty-fourth of the device (12 GiB of 288), and nothing that the backward's own
-    workspace and gradients need beside it.  (Asking takes 10 us.)"""
+    A large one takes an eighth of the memory left, so that what is allocated until the backward
+    finds room, a twenty-fourth of the device (12 GiB of 288), and nothing that the backward's
+    own workspace and gradients need beside it."""
     if m == 0 or options.get_gradient_mode() != "forward" or hidden.dtype not in _DTYPE_CODES:
         return None
     lib = _lib.library()
@@ -1140,13 +1144,17 @@ def kept_logits_buffer(m: int, hidden: torch.Tensor, vocab: int, bias: torch.Ten
     if (nbytes <= 0 or torch.cuda.is_current_stream_capturing()
             or _saved_tensors_are_packed()):
         return None
-    left, total = _memory_left(hidden.device)
-    backward = (lib.tlce_backward_workspace_bytes(m, h, vocab, code, 1, has_bias, budget)
-                + (n_out + vocab) * h * hidden.element_size())
-    room = min(left // 8, total // 24, left - backward)
-    nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, max(min(nbytes, room), 0))
-    if nbytes <= 0:
-        return None
+    if nbytes > _KEEP_UNASKED_BYTES:
+        backward = (lib.tlce_backward_workspace_bytes(m, h, vocab, code, 1, has_bias, budget)
+                    + (n_out + vocab) * h * hidden.element_size())
+        left, total = torch.cuda.mem_get_info(hidden.device)
+        if min(left // 8, left - backward) < nbytes:
+            left += _memory_cached(hidden.device)
+        room = min(left // 8, total // 24, left - backward)
+        if room < nbytes:
+            nbytes = lib.tlce_kept_logits_bytes(m, h, vocab, code, has_bias, max(room, 0))
+            if nbytes <= 0:
+                return None
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=hidden.device)
     except torch.OutOfMemoryError:
@@ -1178,8 +1186,8 @@ _UNCOUNTED_KEPT_BYTES = 512 << 20
 
 def kept_count_stays_on_device(n: int, hidden: torch.Tensor, weight: torch.Tensor,
                                bias: torch.Tensor | None, trainable: bool) -> bool:
-    """``count_stays_on_device`` for the calls that keep their logits: all of them in a small
-    buffer (no panel budget), and gradients that no count moves into the forward."""
+    """``count_stays_on_device`` for the calls that keep their logits or recompute them: a small
+    buffer for all (no panel budget), and gradients that no count moves into the forward."""
     vocab, h = weight.shape
     tiles = (n + 255) // 256 * ((vocab + 255) // 256)
     if (n <= ONE_TILE_ROWS or tiles << 18 > _UNCOUNTED_KEPT_BYTES or bias is not None
