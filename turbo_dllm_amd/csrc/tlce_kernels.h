@@ -854,11 +854,11 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_grad_logits
 // The panel of logit gradients from kept products instead of a contraction: the same entries,
 // bit for bit.  One workgroup per quarter of a tile (64 tokens, all of its 256 words): 64 KiB in,
 // a transposition through 32 KiB of LDS, 64 rows of 512 bytes out; a CU holds several, so that
-// one's loads pass under another's stores.  Bound by memory: 6 bytes a logit.  In the place of
-// the recomputing panels, a step of 16384 per-token losses of a trainable head, H = 4096,
-// V = 151936, takes 47.0 ms instead of 58.9, of 2741 rows, H = 2048, V = 32003 1.160 instead
-// of 1.339; the statistics' contraction, which writes the products, 15.2 instead of 14.5 and
-// 0.33 instead of 0.31.
+// one's loads pass under another's stores.  Bound by memory: 6 bytes a logit.  Traced, in the
+// place of the recomputing panels: 16384 per-token losses of a trainable head, H = 4096,
+// V = 151936 2.5 ms instead of 14.9 (the step 46.7 instead of 58.5), 2741 rows, H = 2048,
+// V = 32003 94 us instead of 350; the statistics' contraction, which writes the products, 15.2
+// instead of 14.4 ms and 336 instead of 301 us.
 template <typename T, bool kSoftcap>
 __global__ __launch_bounds__(256) void lce_grad_from_kept_kernel(GradLogitsArgs p, KeptLogits kept) {
   using E = DirectTileLayout<T>;
@@ -1066,8 +1066,8 @@ __global__ __launch_bounds__(E::kThreads, E::kWavesPerSimd) void lce_kl_panel_ke
   const float inv_cap = kSoftcap ? 1.0f / p.softcap : 0.0f;
   // Only the last vocabulary tile has rows past v: a workgroup-uniform branch, as the VALU work
   // below is a tenth of the draft pass.  With the accumulators read where they are used and the
-  // sums kept in place, 8192 rows, H = 4096, V = 151936: draft pass 8.10 -> 7.83 ms, teacher's
-  // 7.29 -> 7.16.
+  // sums kept in place, and the teacher's tile requested without a loop, 8192 rows, H = 4096,
+  // V = 151936, traced: draft pass 8.47 -> 8.23 ms, teacher's 7.81 -> 7.69.
   // Capped logits replace their accumulators; those are left to the compiler.
   constexpr bool kReads = E::kReadsWhereUsed && (kGrad || !kSoftcap);
   auto epilogue = [&](auto edge_tag) {
