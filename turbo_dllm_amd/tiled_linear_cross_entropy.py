@@ -507,6 +507,12 @@ def tiled_linear_cross_entropy(
 ) -> torch.Tensor:
     """Linear projection plus cross entropy without materializing [N, V] logits.
 
+    Calls whose gradients are not formed in the forward (16-bit, no bias, a hidden size of 1024 or
+    more; float16, odd vocabularies, per-token losses of a trainable head) do hold float32 logits of
+    as many vocabulary tiles as there is room for until the backward: an eighth of the memory left,
+    12 GiB at most.  ``options.gradient_mode("recompute")`` holds none, ``options.panel_budget``
+    bounds them.
+
     Args:
       hidden: token representations, [B, S, D] or [N, D].
       lm_head: output projection, [V, D] ("vocab_first") or [D, V] ("dim_first");
