@@ -113,6 +113,36 @@ def test_masked_token_loss(operands, monkeypatch, kept, counted):
         close(without_synchronisation(lambda: step("sync")), want)
 
 
+def test_captured_with_any_count(operands):
+    """No synchronisation, so such a call can be captured in the default compaction: replayed with
+    other counts and eager steps in between, the bits of the eager step (which keeps logits where
+    the captured one recomputes them)."""
+    hidden, weight, labels, order, _ = operands
+    x = hidden.clone().requires_grad_()
+    w = weight.clone().requires_grad_()
+    y = labels.clone()
+
+    def step():
+        loss = tiled_linear_cross_entropy(x, w, y, reduction="sum", dtype=x.dtype)
+        return [loss.detach(), *torch.autograd.grad(loss, (x, w))]
+
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outputs = step()
+    for kept in (N, 3, 257, 0, 600):
+        y.copy_(labels)
+        y[order[kept:]] = -100
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in outputs]
+        for a, b in zip(got, step()):
+            assert torch.equal(a, b), kept
+
+
 @pytest.mark.parametrize("h,v,trainable", [
     (256, 16384, True), (320, 9024, True),       # gradients in the forward,
     (3840, 16384, True),                         # 8 splits of 2 tiles, 5 of 3,
